@@ -20,10 +20,12 @@
 //   4. pixel-sequential phase: each lane owns one pixel and applies the
 //      order-dependent recurrence of its pairs in depth order (compositing in
 //      the forward; transmittance undo and the d(log T) chain in the adjoint);
-//   5. adjoint only, pair-parallel again: gradient terms per pair, a segmented
-//      wave64 scan keyed by tet sums each tet's terms, segment tails add them
-//      into an LDS accumulator, and the batch is flushed with one hardware
-//      float atomic per term per (tile, tet) — the reference's atomic count.
+//   5. adjoint only, pair-parallel again, each pair on the lane that evaluated
+//      it in step 3 (its slab and exponential stay in registers): gradient
+//      terms per pair, a segmented scan keyed by tet inside each 16-lane row,
+//      each row's sum of a tet stored to a slot of its own, and the batch is
+//      flushed with one hardware float atomic per term per (tile, tet) — the
+//      reference's atomic count.
 // Per-pixel state lives in VGPRs; ray directions and d(image) live in LDS.
 //
 // Per-pixel semantics (coverage rules, skip thresholds, clamps, undo order)
@@ -52,12 +54,9 @@ __device__ __forceinline__ TileCtx tile_ctx(const ViewParams& vw, uint32_t gtile
     return c;
 }
 
-// Row span packing: tiles up to 16 pixels wide keep a span in a byte
-// (xl | xr << 4), wider tiles (32) in 16 bits (xl | xr << 8); the empty span
-// has xl = all ones > xr = 0.
+// Row spans, xl | xr << SH; the empty span has xl = all ones > xr = 0.
 template <int TS>
 struct SpanFmt {
-    using T = typename std::conditional<(TS <= 16), uint8_t, uint16_t>::type;
     static constexpr uint32_t SH = TS <= 16 ? 4u : 8u;
     static constexpr uint32_t MASK = (1u << SH) - 1u;
     static constexpr uint32_t EMPTY = MASK;
@@ -166,12 +165,10 @@ struct BatchLDS {
     static constexpr int TR = 7;
     float4 tr[B * TR];
     float pxy[8][B];        // tile-local projected vertices (x0..x3, y0..y3)
-    uint32_t behind[B];
     uint32_t rows[B];       // tile rows the tet's projected y-range touches: r0 | r1 << 8 (r0 > r1: none)
-    typename SpanFmt<TS>::T span[B * SP];  // [tet][row] span (SpanFmt)
     uint16_t rpref[B * SP];  // [tet][row] record base of the row - its first column (mod 2^16)
     uint32_t wsum[(TS * TS + 63) / 64];  // layout scan carry per wave (one wave per 64 pixels of the tile)
-    uint32_t nbp;           // chunk count << 8 | tets processed this batch (capacity cut)
+    uint32_t nbp;           // record count << 8 | tets processed this batch (capacity cut)
     // adjoint only: per face (grad lambda_a, lambda_a(v0), grad lambda_b,
     // lambda_b(v0)) in face order, then per face the sign s of the stored
     // inward normal n = s * raw normal; 36 floats per tet so that lanes reading
@@ -179,6 +176,7 @@ struct BatchLDS {
     static constexpr int FS = 4 * 8 + 4;
     alignas(16) float face[BWD ? B * FS : 1];
     uint32_t tid[BWD ? B : 1];
+    uint32_t recs[B];  // record range of the tet: first | end << 16
 };
 
 // Global loads of one tet (issued one batch ahead, consumed by store_tet).
@@ -268,7 +266,6 @@ __device__ __forceinline__ void store_rest(BatchLDS<TS, B, BWD>& L, int k, const
 #pragma unroll
     for (int i = 0; i < 4; ++i) mul_vp(vw.vp, v[i], clip[i]);
     bool behind = (clip[0][3] <= 0.0f) || (clip[1][3] <= 0.0f) || (clip[2][3] <= 0.0f) || (clip[3][3] <= 0.0f);
-    L.behind[k] = behind ? 1u : 0u;
     uint32_t rr = 0xFFu;
     if (!behind) {
         float py_[4];
@@ -373,7 +370,6 @@ __device__ __forceinline__ void store_quad(BatchLDS<TS, B, BWD>& L, const QuadFe
         const V3 g = mk3(g1, g2, g3);
         const float bo = dot3(g, sub3(cam, v0));
         L.tr[k * L.TR + 4] = make_float4(f.col.x + bo, f.col.y + bo, f.col.z + bo, f.r.w);
-        L.behind[k] = behind ? 1u : 0u;
         uint32_t rr = 0xFFu;
         if (!behind) {
             // rows whose pixel band [row, row + 1] meets [ymin, ymax] (as store_rest)
@@ -452,42 +448,31 @@ __device__ __forceinline__ uint32_t group_last(uint32_t v) {
     else return v;
 }
 
-// Chunk table entry: up to R consecutive covered pixels of one tet (in row,
-// col order), packed as
-//   tet k (6 bits) | row (5) | first column (5) | first record slot (11) | count (5).
-// With R = 1 the table holds one 16-bit entry (tet, row, first column) per
-// row segment, at the segment's first record slot, and a bit mask marks those
-// slots: record j belongs to the segment starting at the last marked slot <= j.
-constexpr int chunk_capacity(int CAP, int R, int B) { return CAP / R + B; }
-template <int R>
-using chunk_t = typename std::conditional<R == 1, uint16_t, uint32_t>::type;
-template <int R>
-__device__ __forceinline__ chunk_t<R> chunk_entry(uint32_t k, uint32_t row, uint32_t col, uint32_t slot0,
-                                                  uint32_t cnt) {
-    const uint32_t lo = k | (row << 6) | (col << 11);
-    if constexpr (R == 1) return (uint16_t)lo;
-    else return lo | (slot0 << 16) | (cnt << 27);
+// Segment table: one 16-bit entry (tet k in 6 bits, row in 5, first column in
+// 5) per row segment, at the segment's first record slot, and a bit mask marks
+// those slots: record j belongs to the segment starting at the last marked
+// slot <= j.
+__device__ __forceinline__ uint16_t segment_entry(uint32_t k, uint32_t row, uint32_t col) {
+    return (uint16_t)(k | (row << 6) | (col << 11));
 }
 
-// Layout of a batch in one pass: spans, record slots, chunk table and the
+// Layout of a batch in one pass: spans, record slots, segment table and the
 // capacity cut (records <= CAP).  LPT lanes per tet, each over a contiguous
 // block of the rows of the tet's projected y-range (rows outside it are empty
-// and never read).  One wave scan of the lanes' pixel counts, packed with the
-// per-tet chunk counts in the high half-word and carried across waves through
-// L.wsum, gives every lane its record base and its tet's chunk base.  Leaves
-//   span[tet][row], rpref[tet][row] = record base of the row - its first column,
-//   tab[] = chunk table, nbp = chunk count << 8 | tets kept,
+// and never read).  One wave scan of the lanes' pixel counts, carried across
+// waves through L.wsum, gives every lane its record base.  Leaves
+//   rpref[tet][row] = record base of the row - its first column,
+//   seg[], starts[] = segment table, nbp = record count << 8 | tets kept,
 // published by the caller's barrier.  Contains one barrier; every thread of
 // the block calls it.
-template <int TS, int B, bool BWD, bool FORWARD_RULE, int CAP, int R, int NT>
-__device__ __forceinline__ void batch_layout(BatchLDS<TS, B, BWD>& L, int nb, chunk_t<R>* __restrict__ tab,
+template <int TS, int B, bool BWD, bool FORWARD_RULE, int CAP, int NT>
+__device__ __forceinline__ void batch_layout(BatchLDS<TS, B, BWD>& L, int nb, uint16_t* __restrict__ seg,
                                              uint32_t* __restrict__ starts) {
     constexpr int SP = TS + 1;
     constexpr int LPT = NT >= 8 * B ? 8 : NT >= 4 * B ? 4 : NT >= 2 * B ? 2 : 1;
     constexpr int QMAX = (TS + LPT - 1) / LPT;
     static_assert(LPT * B <= NT && B <= 64, "one pass over the batch");
     static_assert(NT / 64 <= (int)(sizeof(L.wsum) / sizeof(L.wsum[0])), "a scan carry per wave");
-    static_assert(B * TS * TS < 65536, "packed scan fields");
     const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
     const int k = t / LPT, j = t % LPT;
     const bool valid = k < nb;
@@ -510,7 +495,6 @@ __device__ __forceinline__ void batch_layout(BatchLDS<TS, B, BWD>& L, int nb, ch
             for (int i = 0; i < QMAX; ++i) {
                 if (i < nr) {
                     sp[i] = tr.span<FORWARD_RULE, TS>((uint32_t)(ra + i));
-                    L.span[k * SP + ra + i] = (typename SpanFmt<TS>::T)sp[i];
                     s += (uint32_t)max(span_xr<TS>(sp[i]) - span_xl<TS>(sp[i]) + 1, 0);
                 }
             }
@@ -533,44 +517,32 @@ __device__ __forceinline__ void batch_layout(BatchLDS<TS, B, BWD>& L, int nb, ch
     }
     const uint32_t tot = group_last<LPT>(g);
     const uint32_t pl = g - s;
-    const uint32_t cc = (tot + R - 1) / R;
-    const bool last = j == LPT - 1;
-    uint32_t inc = wave_scan_dpp(s | (valid && last ? cc << 16 : 0u));
+    uint32_t inc = wave_scan_dpp(s);
     if (lane == 63) L.wsum[wid] = inc;
     __syncthreads();
     for (int w = 0; w < wid; ++w) inc += L.wsum[w];
-    const uint32_t texc = (inc & 0xFFFFu) - s - pl;               // records of the tets before k
-    const uint32_t cexc = (inc >> 16) - (valid && last ? cc : 0u);  // chunks of the tets before k
+    const uint32_t texc = inc - s - pl;  // records of the tets before k
     const bool kept = valid && texc + tot <= (uint32_t)CAP;
     if (kept) {
-        uint32_t base = pl;  // tet-local record index of the row's first pixel
+        uint32_t b = texc + pl;  // the row segment's first record slot
 #pragma unroll
         for (int i = 0; i < QMAX; ++i) {
             if (i < nr) {
                 const uint32_t row = (uint32_t)(ra + i);
                 const int xl = span_xl<TS>(sp[i]), w = span_xr<TS>(sp[i]) - xl + 1;
                 if (w > 0) {
-                    if constexpr (R == 1) {
-                        const uint32_t b = texc + base;  // the row segment's first record slot
-                        tab[b] = chunk_entry<1>((uint32_t)k, row, (uint32_t)xl, 0u, 0u);
-                        atomicOr(&starts[b >> 5], 1u << (b & 31u));
-                    } else {
-                        const uint32_t c0 = (base + R - 1) / R, c1 = (base + (uint32_t)w - 1) / R;
-                        for (uint32_t c = c0; c <= c1; ++c) {
-                            const uint32_t l = c * R;
-                            tab[cexc + c] = chunk_entry<R>((uint32_t)k, row, (uint32_t)(xl + (int)(l - base)),
-                                                           texc + l, min((uint32_t)R, tot - l));
-                        }
-                    }
-                    L.rpref[k * SP + row] = (uint16_t)(texc + base - (uint32_t)xl);
-                    base += (uint32_t)w;
+                    seg[b] = segment_entry((uint32_t)k, row, (uint32_t)xl);
+                    atomicOr(&starts[b >> 5], 1u << (b & 31u));
+                    L.rpref[k * SP + row] = (uint16_t)(b - (uint32_t)xl);
+                    b += (uint32_t)w;
                 }
             }
         }
     }
+    if (kept && j == LPT - 1) L.recs[k] = texc | ((texc + tot) << 16);
     // kept tets are a prefix of the batch: the highest one carries the totals
-    const uint64_t m = __ballot(kept && last);
-    if (m && lane == 63 - __clzll((long long)m)) atomicMax(&L.nbp, ((cexc + cc) << 8) | (uint32_t)(k + 1));
+    const uint64_t m = __ballot(kept && j == LPT - 1);
+    if (m && lane == 63 - __clzll((long long)m)) atomicMax(&L.nbp, ((texc + tot) << 8) | (uint32_t)(k + 1));
 }
 
 // Tets to stage for the next batch.  Tets staged past the capacity cut are
@@ -585,57 +557,33 @@ __device__ __forceinline__ int next_batch(uint32_t nbp, int nb, uint32_t left) {
     return (int)min(want, left);
 }
 
-struct ChunkRef {
+struct RecordRef {
     int k, row, col;
-    uint32_t slot0, cnt;
 };
-// R = 1: record slot j.  A row segment spans at most 16 slots, so its start
-// lies in j's mask word or the one before.
-__device__ __forceinline__ ChunkRef record_at(const uint16_t* seg, const uint32_t* starts, uint32_t j) {
-    const uint32_t wd = j >> 5;
-    const uint32_t m = starts[wd] & ((2u << (j & 31u)) - 1u);
-    const uint32_t s0 = m ? (wd << 5) + 31u - (uint32_t)__clz((int)m)
-                          : ((wd - 1u) << 5) + 31u - (uint32_t)__clz((int)starts[wd - 1u]);
+// Record slot j.  A row segment spans at most 32 slots, so its start
+// lies in j's mask word or the one before; both are read (starts[-1] is a
+// word of padding, never the one used: slot 0 starts a segment) so that the
+// lanes of a wave do not split.
+__device__ __forceinline__ RecordRef record_at(const uint16_t* seg, const uint32_t* starts, uint32_t j) {
+    const int wd = (int)(j >> 5);
+    const uint32_t lo = starts[wd - 1], hi = starts[wd] & ((2u << (j & 31u)) - 1u);
+    const uint32_t m = hi ? hi : lo;
+    const uint32_t s0 = (j & ~31u) + (hi ? 31u : ~0u) - (uint32_t)__builtin_clz(m | 1u);
     const uint32_t e = seg[s0];
-    return ChunkRef{(int)(e & 63u), (int)((e >> 6) & 31u), (int)((e >> 11) & 31u) + (int)(j - s0), j, 1u};
+    return RecordRef{(int)(e & 63u), (int)((e >> 6) & 31u), (int)(e >> 11) + (int)(j - s0)};
 }
-template <int R>
-__device__ __forceinline__ ChunkRef chunk_at(const chunk_t<R>* tab, uint32_t j) {
-    const uint32_t e = tab[j];
-    if constexpr (R == 1) return ChunkRef{(int)(e & 63u), (int)((e >> 6) & 31u), (int)((e >> 11) & 31u), j, 1u};
-    return ChunkRef{(int)(e & 63u), (int)((e >> 6) & 31u), (int)((e >> 11) & 31u), (e >> 16) & 2047u, e >> 27};
-}
-
-// Walks the covered pixels of one tet in (row, col) order starting at local index l.
-template <int TS>
-struct PixWalk {
-    int row, col, xr, r1;
-    template <int B, bool BWD>
-    __device__ __forceinline__ void init(const BatchLDS<TS, B, BWD>& L, const ChunkRef& c) {
-        row = c.row;
-        col = c.col;
-        xr = span_xr<TS>(L.span[c.k * (TS + 1) + c.row]);
-        r1 = (int)(L.rows[c.k] >> 8);
-    }
-    template <int B, bool BWD>
-    __device__ __forceinline__ void next(const BatchLDS<TS, B, BWD>& L, int k) {
-        constexpr int SP = TS + 1;
-        if (++col > xr) {
-            for (int r = row + 1; r <= r1; ++r) {
-                uint32_t sp = L.span[k * SP + r];
-                if (span_xr<TS>(sp) >= span_xl<TS>(sp)) {
-                    row = r;
-                    col = span_xl<TS>(sp);
-                    xr = span_xr<TS>(sp);
-                    return;
-                }
-            }
-            row = TS;
-        }
-    }
+// LDS of a batch's segment table: CAP entries and the slot mask behind one
+// word of padding (record_at).
+template <int CAP>
+struct SegTab {
+    static_assert(CAP % 32 == 0 && CAP <= 2048, "segment start mask");
+    static constexpr int WORDS = CAP / 32;
+    uint32_t start_[WORDS + 1];
+    uint16_t seg[CAP];
+    __device__ __forceinline__ uint32_t* starts() { return start_ + 1; }
 };
 
-// Per-tet data held in registers while a lane walks its chunk.
+// Per-tet data in registers.
 struct TetRegs {
     V3 n[4];
     float num[4];
@@ -665,50 +613,70 @@ __device__ __forceinline__ void tet_regs(const BatchLDS<TS, B, BWD>& L, int k, T
 // vertex gradients magnify a one-ulp change of t through grazing faces).
 __device__ __forceinline__ float fdot3(V3 a, V3 b) { return fmaf(a.x, b.x, fmaf(a.y, b.y, a.z * b.z)); }
 
-// Ray–tet slab intersection against inward planes (rasterize_compute.wgsl:354-390).
-__device__ __forceinline__ bool intersect(const TetRegs& T, V3 rd, float min_t, float& t_min, float& t_max, int& fmin,
-                                          int& fmax) {
+// Ray–tet slab intersection against inward planes (rasterize_compute.wgsl:354-390),
+// without branches: the four faces' quotients are independent, so their
+// reciprocals overlap, and a wave never splits over the faces.  The reference
+// skips a face whose |n . d| is below 1e-20 and calls the tet missed if its
+// plane faces the ray (num > 0).  Sorting the faces by the sign bit of n . d
+// gives the same without the test: an (almost) parallel face divides to
+// +-inf, entry +inf or exit -inf where num > 0 (no slab left), a value that
+// max / min ignore otherwise (0 * inf = NaN for num = 0 included).
+// min_face / max_face: the first face in table order that attains the bound
+// (0 where no face does, as the reference's adjoint assumes).
+// Written with per-face branches, a face cost 14 scalar and branch
+// instructions and a serial reciprocal latency.
+constexpr float kNoEntry = -3.402823e38f;
+__device__ __forceinline__ bool intersect(const TetRegs& T, V3 rd, float min_t, float& t_min, float& t_max,
+                                          int& min_face, int& max_face) {
 #pragma clang fp contract(fast)
-    t_min = -3.402823e38f;
-    t_max = 3.402823e38f;
-    fmin = 4;
-    fmax = 0;
-    bool valid = true;
+    float ta[4], tb[4];
 #pragma unroll
     for (int fi = 0; fi < 4; ++fi) {
-        float den = dot3(T.n[fi], rd);
+        const float den = dot3(T.n[fi], rd);
         float num = T.num[fi];
         if (min_t != 0.0f) num = num - min_t * den;
-        if (fabsf(den) < 1e-20f) {
-            if (num > 0.0f) valid = false;
-            continue;
-        }
-        float t = fast_div(num, den);
-        if (den > 0.0f) {
-            if (t > t_min) {
-                t_min = t;
-                fmin = fi;
-            }
-        } else if (t < t_max) {
-            t_max = t;
-            fmax = fi;
-        }
+        const float t = fast_div(num, den);
+        const bool entry = __float_as_int(den) >= 0;
+        ta[fi] = entry ? t : kNoEntry;
+        tb[fi] = entry ? -kNoEntry : t;
     }
-    return valid && t_min < t_max;
+    t_min = fmaxf(fmaxf(fmaxf(fmaxf(ta[0], ta[1]), ta[2]), ta[3]), kNoEntry);
+    t_max = fminf(fminf(fminf(fminf(tb[0], tb[1]), tb[2]), tb[3]), -kNoEntry);
+    min_face = ta[0] == t_min ? 0 : (ta[1] == t_min ? 1 : (ta[2] == t_min ? 2 : (ta[3] == t_min ? 3 : 0)));
+    max_face = tb[0] == t_max ? 0 : (tb[1] == t_max ? 1 : (tb[2] == t_max ? 2 : (tb[3] == t_max ? 3 : 0)));
+    return t_min < t_max;
+}
+
+// phi(x) = (1 - e^-x) / x and its derivative (e^-x - phi) / x for an optical
+// depth x in [1e-8, 88] (the clamp on x makes the reference's guards of the
+// division and the exponential no-ops), both sides of the series' switch
+// computed: a select, no divergent branch.  The derivative's form loses no
+// digits in e^-x (x + 1) - 1 (of the order x^2).
+__device__ __forceinline__ float od_phi(float x, float ex) {
+#pragma clang fp contract(fast)
+    const float ser = 1.0f + x * (-0.5f + x * ((float)(1.0 / 6.0) + x * ((float)(-1.0 / 24.0))));
+    const float q = fast_div(1.0f - ex, x);
+    return x < 0.02f ? ser : q;
+}
+__device__ __forceinline__ float od_dphi(float x, float ex, float ph) {
+#pragma clang fp contract(fast)
+    const float ser = -0.5f + x * ((float)(1.0 / 3.0) + x * ((float)(-1.0 / 8.0) + x * ((float)(1.0 / 30.0))));
+    const float q = fast_div(ex - ph, x);
+    return x < 0.02f ? ser : q;
 }
 
 // Volume integral of the linear colour field over [t_min, t_max]
 // (rasterize_compute.wgsl:394-410): optical depth, premultiplied colour.
 struct Integral {
-    float od, alpha_t, w0, w1;
+    float od, alpha_t, ph, w0, w1;
     float cs[3], ce[3], csr[3], cer[3];
     float cp[3];
 };
-// EXTRA = false: bo_extra is 0 and not added (x + 0 only differs from x in
-// the sign of a zero, which no use of b sees).
-template <bool EXTRA = true>
-__device__ __forceinline__ void integral(const TetRegs& T, V3 rd, float t_min, float t_max, float bo_extra, float clip_lo,
-                                         Integral& I) {
+// The colours at the slab's ends (EXTRA = false: bo_extra is 0 and not added;
+// x + 0 only differs from x in the sign of a zero, which no use of b sees).
+template <bool EXTRA>
+__device__ __forceinline__ void slab_colors(const TetRegs& T, V3 rd, float t_min, float t_max, float bo_extra,
+                                            Integral& I) {
 #pragma clang fp contract(fast)
     float dc_dt = dot3(T.g, rd);
     float a0 = dc_dt * t_min, a1 = dc_dt * t_max;
@@ -720,12 +688,18 @@ __device__ __forceinline__ void integral(const TetRegs& T, V3 rd, float t_min, f
         I.cs[c] = relu(I.csr[c]);
         I.ce[c] = relu(I.cer[c]);
     }
+}
+template <bool EXTRA = true>
+__device__ __forceinline__ void integral(const TetRegs& T, V3 rd, float t_min, float t_max, float bo_extra, float clip_lo,
+                                         Integral& I) {
+#pragma clang fp contract(fast)
+    slab_colors<EXTRA>(T, rd, t_min, t_max, bo_extra, I);
     float dist = t_max - t_min;
     I.od = med_clip(T.dens * dist, 1e-8f, 88.0f);
-    I.alpha_t = fast_safe_exp(-I.od);
-    float ph = fast_phi(I.od, I.alpha_t);
-    I.w0 = ph - I.alpha_t;
-    I.w1 = 1.0f - ph;
+    I.alpha_t = fast_exp(-I.od);
+    I.ph = od_phi(I.od, I.alpha_t);
+    I.w0 = I.ph - I.alpha_t;
+    I.w1 = 1.0f - I.ph;
 #pragma unroll
     for (int c = 0; c < 3; ++c) I.cp[c] = med_clip(I.ce[c] * I.w0 + I.cs[c] * I.w1, clip_lo, kMaxVal);
 }
@@ -734,17 +708,16 @@ __device__ __forceinline__ void integral(const TetRegs& T, V3 rd, float t_min, f
 // Forward
 // ---------------------------------------------------------------------------
 // Batch geometry of the forward: B tets per LDS batch (<= 64, one mask bit
-// each), CAP (pixel, tet) records per batch, R pixels per lane in the pair
-// phase, PF = fetch the next batch's records while this batch runs.
+// each), CAP (pixel, tet) records per batch, PF = fetch the next batch's
+// records while this batch runs.
 // WPE_: minimum waves per SIMD the register allocation must allow (0: the
 // compiler's choice); a cap on VGPRs that trades recomputation for occupancy.
-template <int TS_, int B_, int CAP_, int R_, int PF_, int WPE_ = 0>
+template <int TS_, int B_, int CAP_, int PF_, int WPE_ = 0>
 struct FwdCfg {
     static constexpr int TS = TS_;
     static constexpr int NT = (TS * TS + 63) / 64 * 64;
     static constexpr int B = B_;
     static constexpr int CAP = CAP_;
-    static constexpr int R = R_;
     // next batch's records: 0 at batch start, 1 in registers, 2 LDS DMA, 3 in
     // registers by quads (4 lanes per tet: falls back to 1 where 4 B > NT)
     static constexpr int PF = (PF_ == 3 && 4 * B_ > NT) ? 1 : PF_;
@@ -762,7 +735,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     const uint32_t* __restrict__ sorted_vals, const uint32_t* __restrict__ ranges, const ViewParams* __restrict__ views,
     const uint32_t* __restrict__ tile_view, const uint32_t* __restrict__ tile_order, float* __restrict__ rgba,
     float* __restrict__ aux, float* __restrict__ ck, float2* __restrict__ fin) {
-    constexpr int TS = C::TS, NT = C::NT, B = C::B, CAP = C::CAP, R = C::R, SP = TS + 1;
+    constexpr int TS = C::TS, NT = C::NT, B = C::B, CAP = C::CAP, SP = TS + 1;
     constexpr int NA = AUX ? CAP : 1;
     static_assert(B <= 64, "pixel masks hold 64 tets; the layout scan is one wave");
     static_assert(CAP >= TS * TS, "one tet's pixels of a tile must fit a batch");
@@ -774,10 +747,8 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     __shared__ float s_ray[3][TS * TS];
     __shared__ uint32_t s_live[TS * TS];  // pixel inside the image and not yet saturated (log T >= -13.8)
     __shared__ unsigned long long s_mask[TS * TS];  // covered tets of the batch per pixel
-    __shared__ chunk_t<R> s_chunk[chunk_capacity(CAP, R, B)];
-    __shared__ uint32_t s_start[R == 1 ? CAP / 32 : 1];  // R = 1: record slots that start a row segment
-    static_assert(CAP <= 2048 && TS <= 32 && R <= 31, "chunk table packing");
-    static_assert(R != 1 || (CAP % 32 == 0 && CAP / 32 <= NT), "segment start mask");
+    __shared__ SegTab<CAP> G;
+    static_assert(CAP / 32 <= NT && TS <= 32, "segment table");
 
     const uint32_t gtile = tile_order ? tile_order[blockIdx.x] : blockIdx.x;
     const uint32_t view = tile_view[gtile];
@@ -831,7 +802,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         if constexpr (C::PF == 3) store_quad<TS, B, false>(L, qf, tid >> 2, tid & 3, tid < 4 * nbs, vw, tc);
         else if (tid < nbs) store_tet<TS, B, false>(L, tid, f, vw, tc);
         if (tid < TS * TS) s_mask[tid] = 0ull;
-        if (R == 1 && tid < CAP / 32) s_start[tid] = 0u;
+        if (tid < CAP / 32) G.starts()[tid] = 0u;
     };
     if constexpr (MERGE) {
         if (count) stage(nb, 0u);
@@ -851,16 +822,16 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             if constexpr (C::PF == 2) {
                 store_batch_staged<TS, B, false, NT>(L, S, nb, vw, tc);
                 if (tid < TS * TS) s_mask[tid] = 0ull;
-                if (R == 1 && tid < CAP / 32) s_start[tid] = 0u;
+                if (tid < CAP / 32) G.starts()[tid] = 0u;
             } else {
                 stage(nb, done);
             }
             __syncthreads();
         }
-        batch_layout<TS, B, false, true, CAP, R, NT>(L, nb, s_chunk, s_start);
+        batch_layout<TS, B, false, true, CAP, NT>(L, nb, G.seg, G.starts());
         __syncthreads();
         const uint32_t nbp = L.nbp & 0xFFu;
-        const uint32_t nchunks = L.nbp >> 8;
+        const uint32_t nrec = L.nbp >> 8;
         // prefetch the next batch's tet records while this one is processed
         const uint32_t next = done + nbp;
         const int nb_next = next_batch<B>(nbp, nb, count - next);
@@ -872,45 +843,31 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             stage_async<false>(S, tn, lane < nb_next, rec, nullptr, col_v);
         }
         // record-parallel: intersection + volume integral of one (pixel, tet)
-        // record per lane (R = 1), or of a chunk of R pixels of one tet
-        for (uint32_t j = tid; j < nchunks; j += NT) {
-            ChunkRef c;
-            if constexpr (R == 1) c = record_at(s_chunk, s_start, j);
-            else c = chunk_at<R>(s_chunk, j);
-            const int k = c.k;
-            TetRegs T;
-            tet_regs(L, k, T);
-            auto one = [&](uint32_t slot, int p) {
-                // saturated pixels skip the rest of the tile's tets (their compositing loop would)
-                if (s_live[p]) {
-                    V3 rd = mk3(s_ray[0][p], s_ray[1][p], s_ray[2][p]);
-                    float t_min, t_max;
-                    int fmin, fmax;
-                    if (intersect(T, rd, min_t, t_min, t_max, fmin, fmax)) {
-                        Integral I;
-                        integral(T, rd, t_min, t_max, min_t != 0.0f ? min_t * dot3(T.g, rd) : 0.0f, 0.0f, I);
-                        s_od[slot] = I.od;
-                        s_cp[0][slot] = I.cp[0];
-                        s_cp[1][slot] = I.cp[1];
-                        s_cp[2][slot] = I.cp[2];
-                        if (AUX) {
-                            s_aux[0][slot] = t_min;
-                            s_aux[1][slot] = t_max;
-                            s_aux[2][slot] = I.w0;
-                            s_ent[slot] = (uint32_t)fmin;
-                        }
-                        atomicOr(&s_mask[p], 1ull << k);
+        // record per lane
+        for (uint32_t j = tid; j < nrec; j += NT) {
+            const RecordRef c = record_at(G.seg, G.starts(), j);
+            const int p = c.row * TS + c.col;
+            // saturated pixels skip the rest of the tile's tets (their compositing loop would)
+            if (s_live[p]) {
+                TetRegs T;
+                tet_regs(L, c.k, T);
+                const V3 rd = mk3(s_ray[0][p], s_ray[1][p], s_ray[2][p]);
+                float t_min, t_max;
+                int fmin, fmax;
+                if (intersect(T, rd, min_t, t_min, t_max, fmin, fmax)) {
+                    Integral I;
+                    integral(T, rd, t_min, t_max, min_t != 0.0f ? min_t * dot3(T.g, rd) : 0.0f, 0.0f, I);
+                    s_od[j] = I.od;
+                    s_cp[0][j] = I.cp[0];
+                    s_cp[1][j] = I.cp[1];
+                    s_cp[2][j] = I.cp[2];
+                    if (AUX) {
+                        s_aux[0][j] = t_min;
+                        s_aux[1][j] = t_max;
+                        s_aux[2][j] = I.w0;
+                        s_ent[j] = t_min == kNoEntry ? 4u : (uint32_t)fmin;
                     }
-                }
-            };
-            if constexpr (R == 1) {
-                one(j, c.row * TS + c.col);
-            } else {
-                PixWalk<TS> w;
-                w.init(L, c);
-                for (uint32_t q = 0; q < c.cnt; ++q) {
-                    one(c.slot0 + q, w.row * TS + w.col);
-                    w.next(L, k);
+                    atomicOr(&s_mask[p], 1ull << c.k);
                 }
             }
         }
@@ -929,40 +886,40 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                 }
                 const uint32_t slot = (L.rpref[k * SP + row] + (uint32_t)colp) & 0xFFFFu;
                 const float od = s_od[slot];
-                const float Tj = fast_safe_exp(log_t);
-                if (Tj >= 1e-6f) {
-                    cr = cr + s_cp[0][slot] * Tj;
-                    cg = cg + s_cp[1][slot] * Tj;
-                    cb = cb + s_cp[2][slot] * Tj;
-                    log_t = log_t - od;
-                    if constexpr (CK) stop = done + k + 1u;
-                    if (AUX) {
-                        // rasterize_compute.wgsl:434-456
-                        float alpha_t = fast_safe_exp(-od);
-                        float alpha = 1.0f - alpha_t;
-                        float w0 = s_aux[2][slot];
-                        float w1 = 1.0f - (w0 + alpha_t);
-                        float t_min = s_aux[0][slot], t_max = s_aux[1][slot];
-                        int entry = (int)s_ent[slot];
-                        V3 en = mk3(0.f, 0.f, 0.f);
-                        if (entry < 4) {
-                            const float4 q = L.tr[k * L.TR + entry];
-                            en = normalize3(neg3(mk3(q.x, q.y, q.z)));
-                        }
-                        float depth_premul = w0 * t_max + w1 * t_min;
-                        float ta = Tj * alpha;
-                        nx = nx + ta * en.x;
-                        ny = ny + ta * en.y;
-                        nz = nz + ta * en.z;
-                        dep = dep + Tj * depth_premul;
-                        float wt = alpha * Tj;
-                        float c_mid = (t_min + t_max) * 0.5f;
-                        float wc = wt * c_mid;
-                        e0 = e0 + wt;
-                        e1 = e1 + (wt > 1e-20f ? wt * logf(wt) : 0.0f);
-                        e2 = e2 + wt * c_mid;
-                        e3 = e3 + (wc > 1e-20f ? wc * logf(wc) : 0.0f);
+                // log_t is in [-13.8, 0] here: the reference's clamp of the
+                // exponent and its test T >= 1e-6 (exp(-13.8) = 1.01e-6) hold
+                const float Tj = fast_exp(log_t);
+                cr = cr + s_cp[0][slot] * Tj;
+                cg = cg + s_cp[1][slot] * Tj;
+                cb = cb + s_cp[2][slot] * Tj;
+                log_t = log_t - od;
+                if constexpr (CK) stop = done + k + 1u;
+                if (AUX) {
+                    // rasterize_compute.wgsl:434-456
+                    float alpha_t = fast_safe_exp(-od);
+                    float alpha = 1.0f - alpha_t;
+                    float w0 = s_aux[2][slot];
+                    float w1 = 1.0f - (w0 + alpha_t);
+                    float t_min = s_aux[0][slot], t_max = s_aux[1][slot];
+                    int entry = (int)s_ent[slot];
+                    V3 en = mk3(0.f, 0.f, 0.f);
+                    if (entry < 4) {
+                        const float4 q = L.tr[k * L.TR + entry];
+                        en = normalize3(neg3(mk3(q.x, q.y, q.z)));
                     }
+                    float depth_premul = w0 * t_max + w1 * t_min;
+                    float ta = Tj * alpha;
+                    nx = nx + ta * en.x;
+                    ny = ny + ta * en.y;
+                    nz = nz + ta * en.z;
+                    dep = dep + Tj * depth_premul;
+                    float wt = alpha * Tj;
+                    float c_mid = (t_min + t_max) * 0.5f;
+                    float wc = wt * c_mid;
+                    e0 = e0 + wt;
+                    e1 = e1 + (wt > 1e-20f ? wt * logf(wt) : 0.0f);
+                    e2 = e2 + wt * c_mid;
+                    e3 = e3 + (wc > 1e-20f ? wc * logf(wc) : 0.0f);
                 }
             }
             if (log_t < -13.8f) s_live[tid] = 0u;
@@ -993,53 +950,27 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
 // ---------------------------------------------------------------------------
 constexpr int kTerms = 19;  // d_density, d_v[4][3], d_grad[3], d_colour[3]
 
-// Batch geometry of the adjoint (B <= 32, one mask bit each); SCAN = how a
-// wave sums each tet's terms before the LDS adds: 2 segmented scan on DPP,
-// 1 segmented scan on ds_bpermute, 0 none (every lane adds its own terms).
-template <int TS_, int B_, int CAP_, int R_, int PF_, int SCAN_, int WPE_ = 0>
+// Batch geometry of the adjoint: B tets (<= 64, one mask bit each), CAP records
+// per batch, PF and WPE as FwdCfg.
+template <int TS_, int B_, int CAP_, int PF_, int WPE_ = 0>
 struct BwdCfg {
     static constexpr int TS = TS_;
     static constexpr int NT = (TS * TS + 63) / 64 * 64;
     static constexpr int B = B_;
     static constexpr int CAP = CAP_;
-    static constexpr int R = R_;
     static constexpr int PF = (PF_ == 3 && 4 * B_ > NT) ? 1 : PF_;  // as FwdCfg::PF
-    static constexpr int SCAN = SCAN_;
     static constexpr int WPE = WPE_ > 0 ? WPE_ : 1;
     static constexpr int PF_ARG = PF_;
     static constexpr int WPE_ARG = WPE_;
+    static constexpr int NREC = (CAP + NT - 1) / NT;  // records per lane
 };
 
-// Segmented inclusive sum across the wave; lanes with equal `key` form
-// contiguous segments (keys non-decreasing with the lane index).
-struct SegMasks {
-    bool m[6];
-};
-__device__ __forceinline__ SegMasks seg_masks(int key) {
-    SegMasks s;
-    const int lane = (int)__lane_id();
-#pragma unroll
-    for (int j = 0; j < 6; ++j) {
-        const int o = 1 << j;
-        int up = __shfl_up(key, o, 64);
-        s.m[j] = lane >= o && up == key;
-    }
-    return s;
-}
-__device__ __forceinline__ float seg_scan(float v, const SegMasks& s) {
-#pragma unroll
-    for (int j = 0; j < 6; ++j) {
-        float up = __shfl_up(v, 1 << j, 64);
-        if (s.m[j]) v += up;
-    }
-    return v;
-}
-
-// The same segmented inclusive sum on DPP: four row_shr steps inside each
-// 16-lane row, then row_bcast:15 (rows 1, 3) and row_bcast:31 (rows 2, 3)
-// carry the previous rows' partial sums.  Lanes whose DPP source lies outside
-// the row or the row mask read 0.  Masks are 0/1 floats (the summands are
-// finite: every gradient term is clamped to +-1e20 before it is summed).
+// Segmented inclusive sum on DPP; lanes with equal `key` form contiguous
+// segments (keys non-decreasing with the lane index).  Four row_shr steps sum
+// inside each 16-lane row, then row_bcast:15 (rows 1, 3) and row_bcast:31 (rows
+// 2, 3) carry the previous rows' partial sums.  Lanes whose DPP source lies
+// outside the row or the row mask read 0.  Masks are 0/1 floats (the summands
+// are finite: every gradient term is clamped to +-1e20 before it is summed).
 template <int CTRL, int ROWS>
 __device__ __forceinline__ int dpp_i(int v, int old) {
     return __builtin_amdgcn_update_dpp(old, v, CTRL, ROWS, 0xF, false);
@@ -1079,11 +1010,14 @@ __device__ __forceinline__ void seg_scan_dpp(float* v, const SegMasksDpp& s) {
     for (int q = 0; q < N; ++q) v[q] = fmaf(dpp_f<0x143, 0xC>(v[q]), s.m[5], v[q]);
 }
 
-// The same scan of 19 sums with the shift folded into the accumulate: one
-// v_fmac_f32_dpp (v += dpp(v) * m) per sum and level.  Each level is one asm
-// block opened by s_nop 1, the two wait states a DPP read needs after a VALU
-// write of its source; inside a level every register is written once, and
-// its next DPP read is 18 instructions later.
+// The adjoint's scan of its 19 sums stays inside the 16-lane rows: four levels
+// instead of six.  A row's last lane ends its segment, so a tet leaves
+// one sum per row, and the flush adds the rows.  (The sums used to be added into
+// one LDS accumulator per tet with ds_add_f32: about 20 LDS cycles an
+// instruction, a third of the kernel's time.)  Each level is one asm block of v_fmac_f32_dpp (v += dpp(v) * m,
+// the shift folded into the accumulate) opened by s_nop 1, the two wait states
+// a DPP read needs after a VALU write of its source; inside a level every
+// register is written once, and its next DPP read is 18 instructions later.
 #define RMESH_FMAC_DPP(i, CTRL) "v_fmac_f32_dpp %" #i ", %" #i ", %19 " CTRL "\n"
 #define RMESH_SCAN_LEVEL(M, CTRL)                                                                              \
     asm volatile("s_nop 1\n" RMESH_FMAC_DPP(0, CTRL) RMESH_FMAC_DPP(1, CTRL) RMESH_FMAC_DPP(2, CTRL)            \
@@ -1096,13 +1030,22 @@ __device__ __forceinline__ void seg_scan_dpp(float* v, const SegMasksDpp& s) {
                    "+v"(v[8]), "+v"(v[9]), "+v"(v[10]), "+v"(v[11]), "+v"(v[12]), "+v"(v[13]), "+v"(v[14]),         \
                    "+v"(v[15]), "+v"(v[16]), "+v"(v[17]), "+v"(v[18])                                             \
                  : "v"(M))
-__device__ __forceinline__ void seg_scan_dpp19(float* v, const SegMasksDpp& s) {
+struct RowMasks {
+    float m[4];
+};
+__device__ __forceinline__ RowMasks row_masks(int key) {
+    RowMasks s;
+    s.m[0] = dpp_i<0x111, 0xF>(key, -1) == key ? 1.0f : 0.0f;  // row_shr:1
+    s.m[1] = dpp_i<0x112, 0xF>(key, -1) == key ? 1.0f : 0.0f;  // row_shr:2
+    s.m[2] = dpp_i<0x114, 0xF>(key, -1) == key ? 1.0f : 0.0f;  // row_shr:4
+    s.m[3] = dpp_i<0x118, 0xF>(key, -1) == key ? 1.0f : 0.0f;  // row_shr:8
+    return s;
+}
+__device__ __forceinline__ void row_scan19(float* v, const RowMasks& s) {
     RMESH_SCAN_LEVEL(s.m[0], "row_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1");
     RMESH_SCAN_LEVEL(s.m[1], "row_shr:2 row_mask:0xf bank_mask:0xf bound_ctrl:1");
     RMESH_SCAN_LEVEL(s.m[2], "row_shr:4 row_mask:0xf bank_mask:0xf bound_ctrl:1");
     RMESH_SCAN_LEVEL(s.m[3], "row_shr:8 row_mask:0xf bank_mask:0xf bound_ctrl:1");
-    RMESH_SCAN_LEVEL(s.m[4], "row_bcast:15 row_mask:0xa bank_mask:0xf");
-    RMESH_SCAN_LEVEL(s.m[5], "row_bcast:31 row_mask:0xc bank_mask:0xf");
 }
 #undef RMESH_SCAN_LEVEL
 #undef RMESH_FMAC_DPP
@@ -1121,7 +1064,7 @@ __device__ __forceinline__ void face_slot_weights(int fi, float la, float lb, fl
     w[3] = f0 ? 0.0f : (f1 ? lc : (f2 ? lb : la));
 }
 
-// Gradient terms of one covered (pixel, tet) pair, accumulated into acc
+// Gradient terms of one covered (pixel, tet) pair, assigned to acc
 // (backward_tiled_compute.wgsl:446-543, per-pixel clipping as there).  The
 // intersection derivatives use dt/dva = ((vc - hit) x (vb - hit)) / den (and
 // cyclic), algebraically identical to the reference's
@@ -1138,23 +1081,35 @@ __device__ __forceinline__ void face_slot_weights(int fi, float la, float lb, fl
 // |g| |dbo|; |cam - v0| |dbo| + |rd| |d_dcdt| for dg) cannot reach a clip,
 // so it accumulates n (k w) with fused multiply-adds and no clips; any other
 // pair (and NaN) takes the clipped path, term by term as the reference.
-// FIRST: acc holds nothing yet (one pair per lane): terms are assigned, not
-// added to zeros.
-template <int TS, int B, bool FIRST>
-__device__ __forceinline__ void pair_grad(const BatchLDS<TS, B, true>& L, int k, const TetRegs& T, V3 v0, V3 cam,
-                                          V3 rd, float dc0, float dc1, float dc2, float t_prev, float d_log_t_b,
-                                          float t_min, float t_max, int min_face, int max_face, float* acc) {
+// The slab and the integral's exponential and phi come from the lane's phase-A
+// evaluation of the same pair.
+template <int TS, int B>
+__device__ __forceinline__ void pair_grad(const BatchLDS<TS, B, true>& L, int k, V3 cam, V3 rd, float dc0, float dc1,
+                                          float dc2, float t_prev, float d_log_t_b, float t_min, float t_max,
+                                          float alpha_t, float ph, int min_face, int max_face, float* acc) {
 #pragma clang fp contract(fast)
+    TetRegs T;
+    const float4 cq = L.tr[k * L.TR + 4], gq = L.tr[k * L.TR + 5], v0q = L.tr[k * L.TR + 6];
+    T.bc[0] = cq.x;
+    T.bc[1] = cq.y;
+    T.bc[2] = cq.z;
+    T.dens = cq.w;
+    T.g = mk3(gq.x, gq.y, gq.z);
+    const V3 v0 = mk3(v0q.x, v0q.y, v0q.z);
     Integral I;
-    integral<false>(T, rd, t_min, t_max, 0.0f, kMinVal, I);
+    slab_colors<false>(T, rd, t_min, t_max, 0.0f, I);
     const float dist = t_max - t_min;
     const float dens = T.dens;
+    I.od = med_clip(dens * dist, 1e-8f, 88.0f);
+    I.alpha_t = alpha_t;
+    I.w0 = ph - alpha_t;
+    I.w1 = 1.0f - ph;
     const float dc_dt = fdot3(T.g, rd);
     float dcp0 = med_clip(dc0 * t_prev, kMinVal, kMaxVal);
     float dcp1 = med_clip(dc1 * t_prev, kMinVal, kMaxVal);
     float dcp2 = med_clip(dc2 * t_prev, kMinVal, kMaxVal);
     float d_od_state = -d_log_t_b;
-    float dphi = fast_dphi(I.od, I.alpha_t);
+    float dphi = od_dphi(I.od, I.alpha_t, ph);
     float dw0 = dphi + I.alpha_t, dw1 = -dphi;
     float d_od_int = fmaf(dcp0, fmaf(I.ce[0], dw0, I.cs[0] * dw1),
                           fmaf(dcp1, fmaf(I.ce[1], dw0, I.cs[1] * dw1), dcp2 * fmaf(I.ce[2], dw0, I.cs[2] * dw1)));
@@ -1207,12 +1162,9 @@ __device__ __forceinline__ void pair_grad(const BatchLDS<TS, B, true>& L, int k,
     const float rmax = fmaxf(fmaxf(fabsf(rd.x), fabsf(rd.y)), fabsf(rd.z));
     bound = fmaf(gmax, fabsf(dbo), bound);
     const float bound_g = fmaf(cmax, fabsf(dbo), rmax * fabsf(d_dcdt));
-    auto put = [&](int q, float x) { acc[q] = FIRST ? x : acc[q] + x; };
-    // x1 k1 + x0 k0 (+ acc)
-    auto put2 = [&](int q, float x0, float k0, float x1, float k1) {
-        acc[q] = FIRST ? fmaf(x1, k1, x0 * k0) : fmaf(x1, k1, fmaf(x0, k0, acc[q]));
-    };
-    put(0, med_clip(d_dens_l, kMinVal, kMaxVal));
+    auto put = [&](int q, float x) { acc[q] = x; };
+    auto put2 = [&](int q, float x0, float k0, float x1, float k1) { acc[q] = fmaf(x1, k1, x0 * k0); };
+    put(0, d_dens_l);
     if (bound <= 1e19f && bound_g <= 1e19f) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
@@ -1262,26 +1214,30 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     const float* __restrict__ rgba, const float* __restrict__ dl_img, const float* __restrict__ gt, uint32_t loss_type,
     float* __restrict__ loss_partial, float* __restrict__ tet_g, float* __restrict__ d_colors,
     const float* __restrict__ ck, const float2* __restrict__ fin, uint64_t* __restrict__ scene_done) {
-    constexpr int TS = C::TS, NT = C::NT, B = C::B, CAP = C::CAP, R = C::R, SP = TS + 1, NW = NT / 64;
+    constexpr int TS = C::TS, NT = C::NT, B = C::B, CAP = C::CAP, SP = TS + 1, NW = NT / 64, NREC = C::NREC;
     __shared__ BatchLDS<TS, B, true> L;
-    // per-pair record: od -> t_prev, dc . cp -> d_log_t before, t_min, t_max
-    // (dc . cp, the pixel's image gradient dotted with the pair's premultiplied
-    // colour, is all the d(log T) chain needs of the colour)
-    __shared__ float s_r[4][CAP];
-    __shared__ uint8_t s_meta[CAP];    // fmin | fmax << 2 | valid << 4 | did << 5
+    // per-pair record: od -> -t_prev (the sign marks a pair that takes part),
+    // dc . cp -> d_log_t before (dc . cp, the pixel's image gradient dotted with
+    // the pair's premultiplied colour, is all the d(log T) chain needs of the
+    // colour).  What else phase C needs of a pair stays in registers of the
+    // lane that evaluated it in phase A: the same lane takes it in phase C.
+    __shared__ float s_od[CAP], s_dl[CAP];
     __shared__ float s_ray[3][TS * TS];
     __shared__ float s_dc[3][TS * TS];
-    __shared__ float s_acc[B][kTerms];
-    __shared__ uint32_t s_ftid[B];  // tet ids of the batch whose terms s_acc holds
+    // Row sums of phase C: the sum over the records of tet k in the 16-record
+    // row r (records 16 r .. 16 r + 15) at slot k + r.  Along the batch's records
+    // k and r never decrease and one of them steps from each such run to the
+    // next, so the slots are distinct, and the writes are plain stores.
+    constexpr int NPART = B + CAP / 16, PS = (kTerms + 3) / 4;
+    __shared__ float4 s_part[NPART][PS];
+    __shared__ uint32_t s_ftid[B];  // tet ids of the batch whose sums s_part holds
     // covered tets of the batch per pixel, one bit per tet
     using MaskT = typename std::conditional<(B > 32), unsigned long long, unsigned int>::type;
     __shared__ MaskT s_mask[TS * TS];
-    __shared__ chunk_t<R> s_chunk[chunk_capacity(CAP, R, B)];
-    static_assert(CAP <= 2048 && TS <= 32 && R <= 31, "chunk table packing");
+    __shared__ SegTab<CAP> G;
     __shared__ float s_loss[NW];
     static_assert(B <= 64, "pixel masks hold 64 tets");
-    __shared__ uint32_t s_start[R == 1 ? CAP / 32 : 1];  // R = 1: record slots that start a row segment
-    static_assert(R != 1 || (CAP % 32 == 0 && CAP / 32 <= NT), "segment start mask");
+    static_assert(CAP / 32 <= NT && TS <= 32, "segment table");
     static_assert(CAP >= TS * TS, "one tet's pixels of a tile must fit a batch");
 
     const uint32_t gtile = tile_order ? tile_order[blockIdx.x] : blockIdx.x;
@@ -1385,13 +1341,18 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         // tet), the colour terms into the view's colour gradients
         for (int it = tid; it < (int)flush_n * kTerms; it += NT) {
             const int k = it / kTerms, q = it % kTerms;
-            const float s = s_acc[k][q];
+            const uint32_t rr = L.recs[k], lo = rr & 0xFFFFu, hi = rr >> 16;
+            if (lo == hi) continue;  // no records
+            float s = 0.0f;
+            for (uint32_t r = lo >> 4; r << 4 < hi; ++r) s += reinterpret_cast<const float*>(s_part[k + r])[q];
             if (s == 0.0f) continue;
             const uint32_t t = s_ftid[k];
             float* dst = q < 16 ? tet_g + 16ull * t + q : dcol_v + 3ull * t + (q - 16);
             unsafeAtomicAdd(dst, s);
         }
     };
+    // tile columns and rows inside the image
+    const int in_w = (int)min<uint32_t>(TS, vw.width - tc.tile_x * TS), in_h = (int)min<uint32_t>(TS, vw.height - tc.tile_y * TS);
     while (done < count) {
         if (C::PF == 2) __builtin_amdgcn_s_waitcnt(0);  // staged records of this batch have landed
         __syncthreads();
@@ -1406,12 +1367,12 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         else if constexpr (C::PF == 3) store_quad<TS, B, true>(L, qf, tid >> 2, tid & 3, tid < 4 * nb, vw, tc);
         else if (tid < nb) store_tet<TS, B, true>(L, tid, f, vw, tc);
         if (tid < TS * TS) s_mask[tid] = 0u;
-        if (R == 1 && tid < CAP / 32) s_start[tid] = 0u;
+        if (tid < CAP / 32) G.starts()[tid] = 0u;
         __syncthreads();
-        batch_layout<TS, B, true, false, CAP, R, NT>(L, nb, s_chunk, s_start);
+        batch_layout<TS, B, true, false, CAP, NT>(L, nb, G.seg, G.starts());
         __syncthreads();
         const uint32_t nbp = L.nbp & 0xFFu;
-        const uint32_t nchunks = L.nbp >> 8;
+        const uint32_t nrec = L.nbp >> 8;
         const uint32_t next = done + nbp;
         const int nb_next = next_batch<B>(nbp, nb, count - next);
         // CK: log T at the end of the (at most two) groups this batch spans,
@@ -1431,48 +1392,36 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             const uint32_t tn = window_id<B>(win, win1, (int)nbp + lane);
             stage_async<true>(S, tn, lane < nb_next, rec, idx, col_v);
         }
-        // the flush above has read s_acc and s_ftid (two barriers ago)
-        for (int i = tid; i < B * kTerms; i += NT) (&s_acc[0][0])[i] = 0.0f;
+        // the flush above has read s_ftid (two barriers ago)
         if (tid < (int)nbp) s_ftid[tid] = L.tid[tid];
-        // phase A (record- or chunk-parallel): intersection + integral
-        for (uint32_t j = tid; j < nchunks; j += NT) {
-            ChunkRef c;
-            if constexpr (R == 1) c = record_at(s_chunk, s_start, j);
-            else c = chunk_at<R>(s_chunk, j);
-            const int k = c.k;
-            TetRegs T;
-            tet_regs(L, k, T);
-            auto one = [&](uint32_t slot, int prow, int pcol) {
-                const uint32_t gx = tc.tile_x * TS + pcol, gy = tc.tile_y * TS + prow;
-                uint32_t meta = 0;
-                if (gx < vw.width && gy < vw.height) {
-                    const int p = prow * TS + pcol;
-                    V3 rd = mk3(s_ray[0][p], s_ray[1][p], s_ray[2][p]);
-                    float t_min, t_max;
-                    int fmin, fmax;
-                    if (intersect(T, rd, 0.0f, t_min, t_max, fmin, fmax)) {
-                        // the reference's adjoint defaults both faces to 0 (backward_tiled_compute.wgsl:365-366)
-                        if (fmin == 4) fmin = 0;
-                        Integral I;
-                        integral<false>(T, rd, t_min, t_max, 0.0f, kMinVal, I);
-                        s_r[0][slot] = I.od;
-                        s_r[1][slot] = (s_dc[0][p] * I.cp[0] + s_dc[1][p] * I.cp[1]) + s_dc[2][p] * I.cp[2];
-                        s_r[2][slot] = t_min;
-                        s_r[3][slot] = t_max;
-                        meta = (uint32_t)fmin | ((uint32_t)fmax << 2) | (1u << 4);
-                        atomicOr(&s_mask[p], (MaskT)1 << k);
-                    }
-                }
-                s_meta[slot] = (uint8_t)meta;
-            };
-            if constexpr (R == 1) {
-                one(j, c.row, c.col);
-            } else {
-                PixWalk<TS> w;
-                w.init(L, c);
-                for (uint32_t q = 0; q < c.cnt; ++q) {
-                    one(c.slot0 + q, w.row, w.col);
-                    w.next(L, k);
+        // phase A (record-parallel): intersection + integral; lane tid takes
+        // records tid, tid + NT, ... here and in phase C
+        float r_t0[NREC], r_t1[NREC], r_at[NREC], r_ph[NREC];
+        uint32_t r_m[NREC];  // tet | pixel << 6 | entry face << 16 | exit face << 18 | hit << 20
+#pragma unroll
+        for (int n = 0; n < NREC; ++n) {
+            const uint32_t j = (uint32_t)(n * NT + tid);
+            r_m[n] = 0u;
+            if (j < nrec) {
+                const RecordRef c = record_at(G.seg, G.starts(), j);
+                const int p = c.row * TS + c.col;
+                TetRegs T;
+                tet_regs(L, c.k, T);
+                const V3 rd = mk3(s_ray[0][p], s_ray[1][p], s_ray[2][p]);
+                float t_min, t_max;
+                int fmin, fmax;
+                r_m[n] = (uint32_t)c.k;
+                if (intersect(T, rd, 0.0f, t_min, t_max, fmin, fmax) && c.row < in_h && c.col < in_w) {
+                    Integral I;
+                    integral<false>(T, rd, t_min, t_max, 0.0f, kMinVal, I);
+                    s_od[j] = I.od;
+                    s_dl[j] = (s_dc[0][p] * I.cp[0] + s_dc[1][p] * I.cp[1]) + s_dc[2][p] * I.cp[2];
+                    r_t0[n] = t_min;
+                    r_t1[n] = t_max;
+                    r_at[n] = I.alpha_t;
+                    r_ph[n] = I.ph;
+                    r_m[n] |= ((uint32_t)p << 6) | ((uint32_t)fmin << 16) | ((uint32_t)fmax << 18) | (1u << 20);
+                    atomicOr(&s_mask[p], (MaskT)1 << c.k);
                 }
             }
         }
@@ -1494,98 +1443,53 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                     }
                 }
                 const uint32_t slot = (L.rpref[k * SP + row] + (uint32_t)colp) & 0xFFFFu;
-                const float od = s_r[0][slot];
+                const float od = s_od[slot];
                 const float prev_log_t = fminf(log_t + od, 0.0f);
-                const float t_prev = fast_safe_exp(prev_log_t);
+                // (no clamp of the exponent: below -88 the value is under 1e-6 all the same)
+                const float t_prev = fast_exp(prev_log_t);
                 log_t = prev_log_t;
                 if (t_prev < 1e-6f) continue;
-                const float dcp = s_r[1][slot];
-                s_r[0][slot] = t_prev;
-                s_r[1][slot] = d_log_t;
-                s_meta[slot] = (uint8_t)(s_meta[slot] | 32u);
+                const float dcp = s_dl[slot];
+                s_od[slot] = -t_prev;
+                s_dl[slot] = d_log_t;
                 d_log_t = safe_clip(d_log_t + dcp * t_prev, kMinVal, kMaxVal);
             }
         }
         __syncthreads();
-        // phase C (chunk-parallel): gradient terms of R pixels of one tet per
-        // lane, then a segmented wave sum keyed by tet
-        for (uint32_t base = (uint32_t)wid * 64; base < nchunks; base += NT) {
-            const uint32_t j = base + lane;
+        // phase C (record-parallel): gradient terms of one pair per lane, then a
+        // segmented sum keyed by tet inside each 16-lane row
+#pragma unroll
+        for (int n = 0; n < NREC; ++n) {
+            const uint32_t j = (uint32_t)(n * NT + tid);
+            if ((uint32_t)(n * NT + wid * 64) >= nrec) break;  // per wave
             float acc[kTerms];
-            if constexpr (R != 1) {
+            bool have = false;  // acc assigned by the lane's pair
+            const int key = j < nrec ? (int)(r_m[n] & 63u) : -2;  // a tet's records are contiguous, hit or not
+            if (r_m[n] >> 20) {
+                const float tp = s_od[j];
+                if (tp < 0.0f) {
+                    const int p = (int)((r_m[n] >> 6) & 1023u);
+                    const V3 rd = mk3(s_ray[0][p], s_ray[1][p], s_ray[2][p]);
+                    pair_grad<TS, B>(L, key, cam, rd, s_dc[0][p], s_dc[1][p], s_dc[2][p], -tp, s_dl[j], r_t0[n],
+                                     r_t1[n], r_at[n], r_ph[n], (int)((r_m[n] >> 16) & 3u), (int)((r_m[n] >> 18) & 3u),
+                                     acc);
+                    have = true;
+                }
+            }
+            if (!have) {
 #pragma unroll
                 for (int q = 0; q < kTerms; ++q) acc[q] = 0.0f;
             }
-            bool have = false;  // R = 1: acc assigned by the lane's one pair
-            int key = 0x7fffffff;
-            if (j < nchunks) {
-                ChunkRef c;
-                if constexpr (R == 1) c = record_at(s_chunk, s_start, j);
-                else c = chunk_at<R>(s_chunk, j);
-                const int k = c.k;
-                key = k;
-                TetRegs T;
-                tet_regs(L, k, T);
-                const float4 v0q = L.tr[k * L.TR + 6];
-                const V3 v0 = mk3(v0q.x, v0q.y, v0q.z);
-                auto one = [&](uint32_t slot, int p) {
-                    const uint32_t meta = s_meta[slot];
-                    if (meta & 32u) {
-                        const V3 rd = mk3(s_ray[0][p], s_ray[1][p], s_ray[2][p]);
-                        pair_grad<TS, B, R == 1>(L, k, T, v0, cam, rd, s_dc[0][p], s_dc[1][p], s_dc[2][p],
-                                                 s_r[0][slot], s_r[1][slot], s_r[2][slot], s_r[3][slot],
-                                                 (int)(meta & 3u), (int)((meta >> 2) & 3u), acc);
-                        have = true;
-                    }
-                };
-                if constexpr (R == 1) {
-                    one(j, c.row * TS + c.col);
-                } else {
-                    PixWalk<TS> w;
-                    w.init(L, c);
-                    for (uint32_t q = 0; q < c.cnt; ++q) {
-                        one(c.slot0 + q, w.row * TS + w.col);
-                        w.next(L, k);
-                    }
-                }
-            }
-            if constexpr (R == 1) {
-                if (!have) {
+            const RowMasks sm = row_masks(key);
+            const int next_key = dpp_i<0x101, 0xF>(key, -1);  // row_shl:1 (a row's last lane reads -1)
+            const bool tail = key >= 0 && next_key != key;
+            static_assert(kTerms == 19, "the asm scan holds 19 sums");
+            row_scan19(acc, sm);
+            if (tail) {
+                float4* o = s_part[key + (int)(j >> 4)];
 #pragma unroll
-                    for (int q = 0; q < kTerms; ++q) acc[q] = 0.0f;
-                }
-            }
-            if (C::SCAN >= 2) {
-                // lanes of one tet are contiguous: a segmented wave scan leaves
-                // each tet's sum in its last lane, which adds it to LDS
-                const SegMasksDpp sm = seg_masks_dpp(key);
-                const int next_key = dpp_i<0x130, 0xF>(key, -1);  // wave_shl:1 (lane 63 reads -1)
-                const bool tail = key != 0x7fffffff && next_key != key;
-                if constexpr (C::SCAN == 3) {
-                    static_assert(kTerms == 19, "the asm scan holds 19 sums");
-                    seg_scan_dpp19(acc, sm);
-                } else {
-                    seg_scan_dpp<kTerms>(acc, sm);
-                }
-                // no zero test per term: a tail's adds are one LDS atomic per
-                // term for the few tail lanes, cheaper than 19 compares and branches
-                if (tail) {
-#pragma unroll
-                    for (int q = 0; q < kTerms; ++q) atomicAdd(&s_acc[key][q], acc[q]);
-                }
-            } else if (C::SCAN == 1) {
-                const SegMasks sm = seg_masks(key);
-                const int next_key = __shfl_down(key, 1, 64);
-                const bool tail = key != 0x7fffffff && (lane == 63 || next_key != key);
-#pragma unroll
-                for (int q = 0; q < kTerms; ++q) {
-                    float s = seg_scan(acc[q], sm);
-                    if (tail && s != 0.0f) atomicAdd(&s_acc[key][q], s);
-                }
-            } else if (key != 0x7fffffff) {
-#pragma unroll
-                for (int q = 0; q < kTerms; ++q)
-                    if (acc[q] != 0.0f) atomicAdd(&s_acc[key][q], acc[q]);
+                for (int q = 0; q < PS; ++q)
+                    o[q] = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], 4 * q + 3 < kTerms ? acc[4 * q + 3] : 0.0f);
             }
         }
         flush_n = nbp;
@@ -1622,14 +1526,14 @@ static void fwd_launch(const FwdArgs& a, hipStream_t s) {
 template <int TS>
 static bool fwd_variant(const FwdArgs& a, int v, hipStream_t s) {
     switch (v) {
-        case 0: fwd_launch<FwdCfg<TS, 48, 768, 1, 3>>(a, s); return true;
-        case 1: fwd_launch<FwdCfg<TS, 48, 704, 1, 3, 5>>(a, s); return true;
-        case 2: fwd_launch<FwdCfg<TS, 32, 704, 1, 3, 5>>(a, s); return true;
-        case 3: fwd_launch<FwdCfg<TS, 64, 1024, 1, 3>>(a, s); return true;
-        case 4: fwd_launch<FwdCfg<TS, 64, 768, 1, 3, 5>>(a, s); return true;
-        case 5: fwd_launch<FwdCfg<TS, 56, 896, 1, 3>>(a, s); return true;
-        case 6: fwd_launch<FwdCfg<TS, 56, 768, 1, 3, 5>>(a, s); return true;
-        case 7: fwd_launch<FwdCfg<TS, 64, 896, 1, 3>>(a, s); return true;
+        case 0: fwd_launch<FwdCfg<TS, 48, 768, 3>>(a, s); return true;
+        case 1: fwd_launch<FwdCfg<TS, 48, 704, 3, 5>>(a, s); return true;
+        case 2: fwd_launch<FwdCfg<TS, 32, 704, 3, 5>>(a, s); return true;
+        case 3: fwd_launch<FwdCfg<TS, 64, 1024, 3>>(a, s); return true;
+        case 4: fwd_launch<FwdCfg<TS, 64, 768, 3, 5>>(a, s); return true;
+        case 5: fwd_launch<FwdCfg<TS, 56, 896, 3>>(a, s); return true;
+        case 6: fwd_launch<FwdCfg<TS, 56, 768, 3, 5>>(a, s); return true;
+        case 7: fwd_launch<FwdCfg<TS, 64, 896, 3>>(a, s); return true;
         default: return false;
     }
 }
@@ -1638,8 +1542,8 @@ static bool fwd_variant(const FwdArgs& a, int v, hipStream_t s) {
 // (CAP >= TS^2), so two geometries only.
 static bool fwd_variant32(const FwdArgs& a, int v, hipStream_t s) {
     switch (v) {
-        case 0: fwd_launch<FwdCfg<32, 32, 1024, 1, 3>>(a, s); return true;
-        case 1: fwd_launch<FwdCfg<32, 48, 1536, 1, 3>>(a, s); return true;
+        case 0: fwd_launch<FwdCfg<32, 32, 1024, 3>>(a, s); return true;
+        case 1: fwd_launch<FwdCfg<32, 48, 1536, 3>>(a, s); return true;
         default: return false;
     }
 }
@@ -1659,7 +1563,7 @@ static void bwd_launch(const BwdArgs& a, hipStream_t s) {
     if (a.ck) {
         if constexpr (C::B > 32) {
             // the checkpointed adjoint's batches span at most two checkpoint groups (B <= 32)
-            bwd_launch<BwdCfg<C::TS, 32, C::CAP, C::R, C::PF_ARG, C::SCAN, C::WPE_ARG>>(a, s);
+            bwd_launch<BwdCfg<C::TS, 32, C::CAP, C::PF_ARG, C::WPE_ARG>>(a, s);
         } else {
             hipLaunchKernelGGL((k_backward<C, true>), dim3(a.num_gtiles), dim3(C::NT), 0, s, a.rec, a.idx, a.colors,
                                a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order,
@@ -1673,30 +1577,36 @@ static void bwd_launch(const BwdArgs& a, hipStream_t s) {
                            nullptr, a.scene_done);
 }
 
+// Adjoint geometries, by tets B and records per lane N (CAP = N NT) of a batch at
+// 4 waves per SIMD (128 VGPRs): with a pair's state kept in registers from
+// phase A to phase C the record capacity costs 8 bytes of LDS a record, and
+// three records a lane measured best at tiles 12 and 16 (config C, tile 16, B
+// 48: N 2 13.25 ms, N 3 12.31 ms; B 64 leaves 3 workgroups per CU: 13.9 ms).
+// One-wave workgroups (tile 8) take half the tets and one record a lane more.
+template <int TS, int B, int N, int PF>
+using BwdGeo = BwdCfg<TS, (TS == 8 ? B / 2 : B), (TS == 8 ? N + 1 : N) * ((TS * TS + 63) / 64 * 64), PF, 4>;
 template <int TS>
 static bool bwd_variant(const BwdArgs& a, int v, hipStream_t s) {
     switch (v) {
-        case 0: bwd_launch<BwdCfg<TS, 32, 480, 1, 3, 3, 5>>(a, s); return true;
-        case 1: bwd_launch<BwdCfg<TS, 32, 512, 1, 3, 3, 4>>(a, s); return true;
-        case 2: bwd_launch<BwdCfg<TS, 32, 512, 1, 2, 3, 4>>(a, s); return true;
-        case 3: bwd_launch<BwdCfg<TS, 32, 576, 1, 3, 3, 4>>(a, s); return true;
-        case 4: bwd_launch<BwdCfg<TS, 32, 640, 1, 2, 3, 4>>(a, s); return true;
-        case 5: bwd_launch<BwdCfg<TS, 32, 640, 1, 3, 3, 4>>(a, s); return true;
-        // 31.5 KB of LDS and 96 VGPRs at tile 16: 5 workgroups (20 waves) per CU
-        case 6: bwd_launch<BwdCfg<TS, 32, 544, 1, 3, 3, 5>>(a, s); return true;
-        // more tets per batch where they are small (the checkpointed mode runs these with B 32)
-        case 7: bwd_launch<BwdCfg<TS, 48, 576, 1, 3, 3, 4>>(a, s); return true;
-        case 8: bwd_launch<BwdCfg<TS, 64, 512, 1, 3, 3, 4>>(a, s); return true;
-        case 9: bwd_launch<BwdCfg<TS, 40, 576, 1, 3, 3, 4>>(a, s); return true;
-        case 10: bwd_launch<BwdCfg<TS, 48, 512, 1, 3, 3, 4>>(a, s); return true;
+        case 0:
+        case 10: bwd_launch<BwdGeo<TS, 48, 3, 3>>(a, s); return true;
+        case 1: bwd_launch<BwdGeo<TS, 32, 3, 3>>(a, s); return true;
+        case 2: bwd_launch<BwdGeo<TS, 32, 2, 2>>(a, s); return true;
+        case 3: bwd_launch<BwdGeo<TS, 48, 2, 3>>(a, s); return true;
+        case 4: bwd_launch<BwdGeo<TS, 32, 3, 2>>(a, s); return true;
+        case 5: bwd_launch<BwdGeo<TS, 64, 3, 3>>(a, s); return true;
+        case 6: bwd_launch<BwdGeo<TS, 40, 3, 3>>(a, s); return true;
+        case 7: bwd_launch<BwdGeo<TS, 56, 3, 3>>(a, s); return true;
+        case 8: bwd_launch<BwdGeo<TS, 64, 2, 3>>(a, s); return true;
+        case 9: bwd_launch<BwdGeo<TS, 40, 2, 3>>(a, s); return true;
         default: return false;
     }
 }
 
 static bool bwd_variant32(const BwdArgs& a, int v, hipStream_t s) {
     switch (v) {
-        case 0: bwd_launch<BwdCfg<32, 32, 1024, 1, 3, 3, 4>>(a, s); return true;
-        case 1: bwd_launch<BwdCfg<32, 16, 1024, 1, 3, 3, 4>>(a, s); return true;
+        case 0: bwd_launch<BwdCfg<32, 32, 1024, 3, 4>>(a, s); return true;
+        case 1: bwd_launch<BwdCfg<32, 16, 1024, 3, 4>>(a, s); return true;
         default: return false;
     }
 }
@@ -1735,15 +1645,14 @@ __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec,
                                                  const float* __restrict__ ssim_err, float* __restrict__ tet_err,
                                                  int32_t* __restrict__ tet_count) {
     constexpr int TS = C::TS, NT = C::NT, B = C::B, CAP = C::CAP, SP = TS + 1;
-    static_assert(C::R == 1 && B <= 64 && CAP % 32 == 0 && CAP / 32 <= NT && CAP >= TS * TS, "error pass geometry");
+    static_assert(B <= 64 && CAP % 32 == 0 && CAP / 32 <= NT && CAP >= TS * TS, "error pass geometry");
     __shared__ BatchLDS<TS, B, false> L;
     __shared__ float s_r[3][CAP];  // t_min, t_max, optical depth -> weight (0: none)
     __shared__ float s_ray[3][TS * TS];
     __shared__ float s_pe[TS * TS], s_se[TS * TS];
     __shared__ uint32_t s_live[TS * TS];            // inside the image, log T >= -5.5
     __shared__ unsigned long long s_mask[TS * TS];  // covered tets of the batch per pixel
-    __shared__ chunk_t<1> s_chunk[chunk_capacity(CAP, 1, B)];
-    __shared__ uint32_t s_start[CAP / 32];
+    __shared__ SegTab<CAP> G;
     __shared__ float4 s_cen[B];
     __shared__ uint32_t s_tid[B];  // tet ids of the batch (the forward's LDS image has none)
     __shared__ float s_acc[B][kErrStats];
@@ -1804,11 +1713,11 @@ __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec,
             s_tid[tid] = f.t;
         }
         if (tid < TS * TS) s_mask[tid] = 0ull;
-        if (tid < CAP / 32) s_start[tid] = 0u;
+        if (tid < CAP / 32) G.starts()[tid] = 0u;
         for (int i = tid; i < B * kErrStats; i += NT) (&s_acc[0][0])[i] = 0.0f;
         if (tid < B) s_max[tid] = 0;
         __syncthreads();
-        batch_layout<TS, B, false, true, CAP, 1, NT>(L, nb, s_chunk, s_start);
+        batch_layout<TS, B, false, true, CAP, NT>(L, nb, G.seg, G.starts());
         __syncthreads();
         const uint32_t nbp = L.nbp & 0xFFu;
         const uint32_t nrec = L.nbp >> 8;
@@ -1819,7 +1728,7 @@ __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec,
             fetch_quad<false>(qf, sorted_vals[re - 1 - next - (tid >> 2)], tid & 3, rec, nullptr, rec);
         // phase A: slab and optical depth of every covered pair
         for (uint32_t j = tid; j < nrec; j += NT) {
-            const ChunkRef c = record_at(s_chunk, s_start, j);
+            const RecordRef c = record_at(G.seg, G.starts(), j);
             const int p = c.row * TS + c.col;
             if (s_live[p]) {
                 TetRegs T;
@@ -1865,7 +1774,7 @@ __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec,
             for (int q = 0; q < kErrStats; ++q) acc[q] = 0.0f;
             int key = 0x7fffffff;
             if (j < nrec) {
-                const ChunkRef c = record_at(s_chunk, s_start, j);
+                const RecordRef c = record_at(G.seg, G.starts(), j);
                 key = c.k;
                 const int p = c.row * TS + c.col;
                 const float tv = (s_mask[p] >> c.k) & 1ull ? s_r[2][j] : 0.0f;
@@ -1923,7 +1832,7 @@ __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec,
 
 template <int TS>
 static void err_launch(const ErrArgs& a, hipStream_t s) {
-    using C = FwdCfg<TS, 32, (TS * TS > 512 ? TS * TS : 512), 1, 3>;
+    using C = FwdCfg<TS, 32, (TS * TS > 512 ? TS * TS : 512), 3>;
     hipLaunchKernelGGL((k_error<C>), dim3(a.num_tiles), dim3(C::NT), 0, s, a.rec, a.sorted_vals, a.ranges, a.views,
                        a.pixel_err, a.ssim_err, a.tet_err, a.tet_count);
 }
@@ -2174,8 +2083,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     __shared__ float s_rsc[TS * TS];
     __shared__ uint32_t s_live[TS * TS];
     __shared__ unsigned long long s_mask[TS * TS];
-    __shared__ uint16_t s_chunk[chunk_capacity(CAP, 1, B)];
-    __shared__ uint32_t s_start[CAP / 32];
+    __shared__ SegTab<CAP> G;
 
     const uint32_t gtile = tile_order ? tile_order[blockIdx.x] : blockIdx.x;
     const ViewParams& vw = views[0];
@@ -2236,9 +2144,9 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             L.rows[k] = rr;
         }
         if (tid < TS * TS) s_mask[tid] = 0ull;
-        if (tid < CAP / 32) s_start[tid] = 0u;
+        if (tid < CAP / 32) G.starts()[tid] = 0u;
         __syncthreads();
-        batch_layout<TS, B, false, true, CAP, 1, NT>(L, nb, s_chunk, s_start);
+        batch_layout<TS, B, false, true, CAP, NT>(L, nb, G.seg, G.starts());
         __syncthreads();
         const uint32_t nbp = L.nbp & 0xFFu;
         const uint32_t nrec = L.nbp >> 8;
@@ -2248,7 +2156,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         // record-parallel: fan triangle, interpolation and the per-pair terms
         // (interval_tiled_rasterize.wgsl:248-400)
         for (uint32_t j = tid; j < nrec; j += NT) {
-            const ChunkRef c = record_at(s_chunk, s_start, j);
+            const RecordRef c = record_at(G.seg, G.starts(), j);
             const int p = c.row * TS + c.col;
             if (!s_live[p]) continue;
             const float4* T = &L.tr[c.k * kIvlRec];
@@ -2442,8 +2350,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     __shared__ float s_dl[7][TS * TS];  // d colour rgb, d xyzd
     __shared__ uint32_t s_live[TS * TS];
     __shared__ unsigned long long s_mask[TS * TS];
-    __shared__ uint16_t s_chunk[chunk_capacity(CAP, 1, B)];
-    __shared__ uint32_t s_start[CAP / 32];
+    __shared__ SegTab<CAP> G;
     __shared__ float s_acc[B][KT];
     __shared__ uint32_t s_tid[B];
 
@@ -2536,10 +2443,10 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             L.rows[k] = rr;
         }
         if (tid < TS * TS) s_mask[tid] = 0ull;
-        if (tid < CAP / 32) s_start[tid] = 0u;
+        if (tid < CAP / 32) G.starts()[tid] = 0u;
         for (int i = tid; i < B * KT; i += NT) (&s_acc[0][0])[i] = 0.0f;
         __syncthreads();
-        batch_layout<TS, B, false, true, CAP, 1, NT>(L, nb, s_chunk, s_start);
+        batch_layout<TS, B, false, true, CAP, NT>(L, nb, G.seg, G.starts());
         __syncthreads();
         const uint32_t nbp = L.nbp & 0xFFu;
         const uint32_t nrec = L.nbp >> 8;
@@ -2548,7 +2455,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         if (tid < nb_next) fetch(sorted_vals[rs_ + next + tid]);
         // phase A: the pair's colour, optical depth and distortion factors
         for (uint32_t j = tid; j < nrec; j += NT) {
-            const ChunkRef c = record_at(s_chunk, s_start, j);
+            const RecordRef c = record_at(G.seg, G.starts(), j);
             const int p = c.row * TS + c.col;
             if (!s_live[p]) continue;
             const float4* T = &L.tr[c.k * kIvlRec];
@@ -2611,7 +2518,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             for (int i = 0; i < kIvlNormalTerms; ++i) accn[i] = 0.0f;
             int key = 0x7fffffff;
             if (j < nrec) {
-                const ChunkRef c = record_at(s_chunk, s_start, j);
+                const RecordRef c = record_at(G.seg, G.starts(), j);
                 key = c.k;
                 const int p = c.row * TS + c.col;
                 const float tp = (s_mask[p] >> c.k) & 1ull ? s_r[0][j] : 0.0f;
@@ -2954,7 +2861,7 @@ __global__ __launch_bounds__(256) void k_vertex_gather(const uint32_t* __restric
 
 template <int TS>
 static void ivl_bwd_launch(const IvlBwdArgs& a, hipStream_t s) {
-    using C = FwdCfg<TS, (TS > 16 ? 16 : 32), (TS * TS > 512 ? TS * TS : 512), 1, 1>;
+    using C = FwdCfg<TS, (TS > 16 ? 16 : 32), (TS * TS > 512 ? TS * TS : 512), 1>;
     hipLaunchKernelGGL((k_interval_backward<C>), dim3(a.num_tiles), dim3(C::NT), 0, s, a.ivr, a.sorted_vals, a.ranges,
                        a.views, a.tile_order, a.rgba, a.dist, a.dl_img, a.dl_xyzd, a.dl_dist, a.d_ivr);
 }
@@ -2978,7 +2885,7 @@ bool launch_interval_backward(const IvlBwdArgs& a, uint32_t tile_size, hipStream
 
 template <int TS>
 static void ivl_launch(const IvlArgs& a, hipStream_t s) {
-    using C = FwdCfg<TS, (TS > 16 ? 16 : 32), (TS * TS > 512 ? TS * TS : 512), 1, 1>;
+    using C = FwdCfg<TS, (TS > 16 ? 16 : 32), (TS * TS > 512 ? TS * TS : 512), 1>;
     hipLaunchKernelGGL((k_interval_forward<C>), dim3(a.num_tiles), dim3(C::NT), 0, s, a.ivr, a.sorted_vals, a.ranges,
                        a.views, a.tile_order, a.rgba, a.xyzd, a.dist);
 }
