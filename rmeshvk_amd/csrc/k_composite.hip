@@ -39,6 +39,13 @@
 
 namespace rmesh {
 
+// x, recomputed where it is used: what depends on it is not hoisted out of the
+// batch loop, where it would hold registers through every phase.
+__device__ __forceinline__ int opaque(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
 struct TileCtx {
     uint32_t tile, tile_x, tile_y;
     float tile_ox, tile_oy;
@@ -156,7 +163,10 @@ struct TetRows {
 // LDS image of one batch of tets.  Row arrays use an odd stride (TS + 1) so
 // the pixel-sequential phase (fixed tet, lanes on different rows) is free of
 // bank conflicts.
-template <int TS, int B, bool BWD>
+// U: two floats per record for U records (the adjoint's per-pair values), in the
+// place of the projected vertices: those are read last by the layout, the
+// records are written after it and read last before the next batch is stored.
+template <int TS, int B, bool BWD, int U = 0>
 struct BatchLDS {
     static constexpr int SP = TS + 1;
     // per tet, 7 float4 (112 B: lanes reading different tets spread over the
@@ -164,7 +174,10 @@ struct BatchLDS {
     // density), (g, 0), (v0, 0)
     static constexpr int TR = 7;
     float4 tr[B * TR];
-    float pxy[8][B];        // tile-local projected vertices (x0..x3, y0..y3)
+    union {
+        float pxy[8][B];    // tile-local projected vertices (x0..x3, y0..y3)
+        float2 pair[U > 0 ? U : 1];
+    };
     uint32_t rows[B];       // tile rows the tet's projected y-range touches: r0 | r1 << 8 (r0 > r1: none)
     uint16_t rpref[B * SP];  // [tet][row] record base of the row - its first column (mod 2^16)
     uint32_t wsum[(TS * TS + 63) / 64];  // layout scan carry per wave (one wave per 64 pixels of the tile)
@@ -175,7 +188,6 @@ struct BatchLDS {
     // different tets start on different banks; tet id
     static constexpr int FS = 4 * 8 + 4;
     alignas(16) float face[BWD ? B * FS : 1];
-    uint32_t tid[BWD ? B : 1];
     uint32_t recs[B];  // record range of the tet: first | end << 16
 };
 
@@ -183,53 +195,18 @@ struct BatchLDS {
 struct TetFetch {
     float4 r[4];
     float4 col;
-    uint32_t t;
 };
 
-template <bool BWD>
 __device__ __forceinline__ void fetch_tet(TetFetch& f, uint32_t t, const float4* __restrict__ rec,
-                                          const uint32_t* __restrict__ idx, const float4* __restrict__ colors) {
-    f.t = t;
+                                          const float4* __restrict__ colors) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) f.r[i] = rec[4ull * t + i];
     f.col = colors[t];
 }
 
-// LDS staging of a batch's tet data, filled by direct global -> LDS loads
-// (global_load_lds_dwordx4: lane l's 16 bytes land at base + 16 l), so the
-// next batch's gather is in flight during this batch without holding VGPRs.
-template <int B>
-struct Staging {
-    float4 rec[4][B];
-    float4 col[B];
-    uint32_t t[B];
-};
-
-// Wave 0 only (lane == tet slot): start loading tet t for the lanes with `on`.
-template <bool BWD, int B>
-__device__ __forceinline__ void stage_async(Staging<B>& S, uint32_t t, bool on, const float4* __restrict__ rec,
-                                            const uint32_t* __restrict__ idx, const float4* __restrict__ colors) {
-    typedef __attribute__((address_space(3))) void* lds_ptr;
-    if (on) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            __builtin_amdgcn_global_load_lds((const void*)(rec + 4ull * t + i), (lds_ptr)&S.rec[i][0], 16, 0, 0);
-        __builtin_amdgcn_global_load_lds((const void*)(colors + t), (lds_ptr)&S.col[0], 16, 0, 0);
-        S.t[__lane_id()] = t;
-    }
-}
-
-template <bool BWD, int B>
-__device__ __forceinline__ void staged_tet(const Staging<B>& S, int k, TetFetch& f) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) f.r[i] = S.rec[i][k];
-    f.col = S.col[k];
-    f.t = S.t[k];
-}
-
 // Face fi of tet k: inward plane (and, for the adjoint, the face table entry).
-template <int TS, int B, bool BWD>
-__device__ __forceinline__ void store_face(BatchLDS<TS, B, BWD>& L, int k, int fi, V3 va, V3 vb, V3 vc, V3 vo, V3 v0,
+template <int TS, int B, bool BWD, int U>
+__device__ __forceinline__ void store_face(BatchLDS<TS, B, BWD, U>& L, int k, int fi, V3 va, V3 vb, V3 vc, V3 vo, V3 v0,
                                            V3 cam) {
     V3 raw = cross3(sub3(vc, va), sub3(vb, va));
     V3 nn = raw;
@@ -253,8 +230,8 @@ __device__ __forceinline__ void store_face(BatchLDS<TS, B, BWD>& L, int k, int f
 
 // Per-tet data of tet k: base colour at the camera, density, g, v0, the
 // tile-local projected vertices, vertex ids and tet id.
-template <int TS, int B, bool BWD>
-__device__ __forceinline__ void store_rest(BatchLDS<TS, B, BWD>& L, int k, const TetFetch& f, const V3* v,
+template <int TS, int B, bool BWD, int U>
+__device__ __forceinline__ void store_rest(BatchLDS<TS, B, BWD, U>& L, int k, const TetFetch& f, const V3* v,
                                            const ViewParams& vw, const TileCtx& tc) {
     const V3 g = mk3(f.r[1].w, f.r[2].w, f.r[3].w);
     const V3 cam = mk3(vw.cam[0], vw.cam[1], vw.cam[2]);
@@ -284,14 +261,11 @@ __device__ __forceinline__ void store_rest(BatchLDS<TS, B, BWD>& L, int k, const
         if (r0 <= r1) rr = (uint32_t)r0 | ((uint32_t)r1 << 8);
     }
     L.rows[k] = rr;
-    if (BWD) {
-        L.tid[k] = f.t;
-    }
 }
 
 // One lane stages a whole tet (records in registers).
-template <int TS, int B, bool BWD>
-__device__ __forceinline__ void store_tet(BatchLDS<TS, B, BWD>& L, int k, const TetFetch& f, const ViewParams& vw,
+template <int TS, int B, bool BWD, int U>
+__device__ __forceinline__ void store_tet(BatchLDS<TS, B, BWD, U>& L, int k, const TetFetch& f, const ViewParams& vw,
                                           const TileCtx& tc) {
     V3 v[4] = {mk3(f.r[0].x, f.r[0].y, f.r[0].z), mk3(f.r[1].x, f.r[1].y, f.r[1].z), mk3(f.r[2].x, f.r[2].y, f.r[2].z),
                mk3(f.r[3].x, f.r[3].y, f.r[3].z)};
@@ -307,17 +281,14 @@ __device__ __forceinline__ void store_tet(BatchLDS<TS, B, BWD>& L, int k, const 
 
 // Quad prefetch: lane j of the four lanes 4k..4k+3 of tet slot k holds the
 // tet's vertex record j (vertex j; w = density for j = 0, else g component
-// j - 1), its colour and the tet id.
+// j - 1) and its colour.
 struct QuadFetch {
     float4 r;
     float4 col;
-    uint32_t t;
 };
 
-template <bool BWD>
 __device__ __forceinline__ void fetch_quad(QuadFetch& f, uint32_t t, int j, const float4* __restrict__ rec,
-                                           const uint32_t* __restrict__ idx, const float4* __restrict__ colors) {
-    f.t = t;
+                                           const float4* __restrict__ colors) {
     f.r = rec[4ull * t + j];
     f.col = colors[t];
 }
@@ -337,8 +308,8 @@ __device__ __forceinline__ V3 qperm3(float4 v) {
 // each: FACES = {0,2,1,3}, {1,2,3,0}, {0,3,2,1}, {3,0,1,2}) and projects
 // vertex j; lanes 0-2 write the per-tet rows.  Every lane of the block calls
 // it (DPP reads the whole quad); `on` marks the lanes of the batch's tets.
-template <int TS, int B, bool BWD>
-__device__ __forceinline__ void store_quad(BatchLDS<TS, B, BWD>& L, const QuadFetch& f, int k, int j, bool on,
+template <int TS, int B, bool BWD, int U>
+__device__ __forceinline__ void store_quad(BatchLDS<TS, B, BWD, U>& L, const QuadFetch& f, int k, int j, bool on,
                                            const ViewParams& vw, const TileCtx& tc) {
     const V3 va = qperm3<0xC4>(f.r);  // [0,1,0,3]
     const V3 vb = qperm3<0x3A>(f.r);  // [2,2,3,0]
@@ -378,48 +349,11 @@ __device__ __forceinline__ void store_quad(BatchLDS<TS, B, BWD>& L, const QuadFe
             if (r0 <= r1) rr = (uint32_t)r0 | ((uint32_t)r1 << 8);
         }
         L.rows[k] = rr;
-        if (BWD) L.tid[k] = f.t;
     } else if (j == 1) {
         L.tr[k * L.TR + 5] = make_float4(g1, g2, g3, 0.0f);
     } else if (j == 2) {
         L.tr[k * L.TR + 6] = make_float4(v0.x, v0.y, v0.z, 0.0f);
     }
-}
-
-// Five lanes per tet stage the batch from the LDS staging area: lanes 0-3 a
-// face each, lane 4 the per-tet data.
-template <int TS, int B, bool BWD, int NT>
-__device__ __forceinline__ void store_batch_staged(BatchLDS<TS, B, BWD>& L, const Staging<B>& S, int nb,
-                                                   const ViewParams& vw, const TileCtx& tc) {
-    const V3 cam = mk3(vw.cam[0], vw.cam[1], vw.cam[2]);
-    for (int it = threadIdx.x; it < 5 * nb; it += NT) {
-        const int k = it / 5, part = it % 5;
-        auto vtx = [&](int i) {
-            const float4 r = S.rec[i][k];
-            return mk3(r.x, r.y, r.z);
-        };
-        if (part < 4) {
-            int a, b, c, o;
-            face_idx(part, a, b, c, o);
-            store_face(L, k, part, vtx(a), vtx(b), vtx(c), vtx(o), vtx(0), cam);
-        } else {
-            TetFetch f;
-            staged_tet<BWD>(S, k, f);
-            const V3 v[4] = {vtx(0), vtx(1), vtx(2), vtx(3)};
-            store_rest(L, k, f, v, vw, tc);
-        }
-    }
-}
-
-// Entry i < 128 of a wave's two-register id window (entries 0-63 in w0, 64-127 in w1).
-template <int B>
-__device__ __forceinline__ uint32_t window_id(uint32_t w0, uint32_t w1, int i) {
-    const uint32_t a = (uint32_t)__shfl((int)w0, i & 63, 64);
-    if constexpr (B > 32) {
-        const uint32_t b = (uint32_t)__shfl((int)w1, i & 63, 64);
-        return i < 64 ? a : b;
-    }
-    return a;
 }
 
 template <int CTRL, int ROWS>
@@ -465,8 +399,8 @@ __device__ __forceinline__ uint16_t segment_entry(uint32_t k, uint32_t row, uint
 //   seg[], starts[] = segment table, nbp = record count << 8 | tets kept,
 // published by the caller's barrier.  Contains one barrier; every thread of
 // the block calls it.
-template <int TS, int B, bool BWD, bool FORWARD_RULE, int CAP, int NT>
-__device__ __forceinline__ void batch_layout(BatchLDS<TS, B, BWD>& L, int nb, uint16_t* __restrict__ seg,
+template <int TS, int B, bool BWD, bool FORWARD_RULE, int CAP, int NT, int U>
+__device__ __forceinline__ void batch_layout(BatchLDS<TS, B, BWD, U>& L, int nb, uint16_t* __restrict__ seg,
                                              uint32_t* __restrict__ starts) {
     constexpr int SP = TS + 1;
     constexpr int LPT = NT >= 8 * B ? 8 : NT >= 4 * B ? 4 : NT >= 2 * B ? 2 : 1;
@@ -592,8 +526,8 @@ struct TetRegs {
     float dens;
 };
 
-template <int TS, int B, bool BWD>
-__device__ __forceinline__ void tet_regs(const BatchLDS<TS, B, BWD>& L, int k, TetRegs& T) {
+template <int TS, int B, bool BWD, int U>
+__device__ __forceinline__ void tet_regs(const BatchLDS<TS, B, BWD, U>& L, int k, TetRegs& T) {
 #pragma unroll
     for (int fi = 0; fi < 4; ++fi) {
         const float4 q = L.tr[k * L.TR + fi];
@@ -708,8 +642,8 @@ __device__ __forceinline__ void integral(const TetRegs& T, V3 rd, float t_min, f
 // Forward
 // ---------------------------------------------------------------------------
 // Batch geometry of the forward: B tets per LDS batch (<= 64, one mask bit
-// each), CAP (pixel, tet) records per batch, PF = fetch the next batch's
-// records while this batch runs.
+// each), CAP (pixel, tet) records per batch, PF how the next batch's records are
+// fetched while this batch runs.
 // WPE_: minimum waves per SIMD the register allocation must allow (0: the
 // compiler's choice); a cap on VGPRs that trades recomputation for occupancy.
 template <int TS_, int B_, int CAP_, int PF_, int WPE_ = 0>
@@ -718,9 +652,10 @@ struct FwdCfg {
     static constexpr int NT = (TS * TS + 63) / 64 * 64;
     static constexpr int B = B_;
     static constexpr int CAP = CAP_;
-    // next batch's records: 0 at batch start, 1 in registers, 2 LDS DMA, 3 in
-    // registers by quads (4 lanes per tet: falls back to 1 where 4 B > NT)
+    // next batch's records in registers: 1 one lane per tet, 3 quads (4 lanes
+    // per tet: falls back to 1 where 4 B > NT)
     static constexpr int PF = (PF_ == 3 && 4 * B_ > NT) ? 1 : PF_;
+    static_assert(PF == 1 || PF == 3, "prefetch mode");
     static constexpr int WPE = WPE_ > 0 ? WPE_ : 1;
 };
 
@@ -740,14 +675,17 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     static_assert(B <= 64, "pixel masks hold 64 tets; the layout scan is one wave");
     static_assert(CAP >= TS * TS, "one tet's pixels of a tile must fit a batch");
     __shared__ BatchLDS<TS, B, false> L;
-    __shared__ float s_od[CAP];
-    __shared__ float s_cp[3][CAP];
+    __shared__ float4 s_pr[CAP];       // per pair: premultiplied colour, optical depth
     __shared__ float s_aux[3][NA];     // t_min, t_max, w0
     __shared__ uint32_t s_ent[NA];
-    __shared__ float s_ray[3][TS * TS];
-    __shared__ uint32_t s_live[TS * TS];  // pixel inside the image and not yet saturated (log T >= -13.8)
+    // ray direction; w: 1 while the pixel is inside the image and not yet saturated (log T >= -13.8)
+    __shared__ float4 s_ray[TS * TS];
     __shared__ unsigned long long s_mask[TS * TS];  // covered tets of the batch per pixel
     __shared__ SegTab<CAP> G;
+    // tet ids at list positions done .. done + 2 B - 1, so the next batch's record
+    // loads (which start where this batch is cut) wait for no id
+    constexpr int IDW = (2 * B + NT - 1) / NT;
+    __shared__ uint32_t s_ids[2 * B];
     static_assert(CAP / 32 <= NT && TS <= 32, "segment table");
 
     const uint32_t gtile = tile_order ? tile_order[blockIdx.x] : blockIdx.x;
@@ -764,10 +702,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     if (tid < TS * TS) {
         V3 rd = mk3(0.f, 0.f, 1.f);
         if (active) rd = pixel_ray(vw, px, py);
-        s_ray[0][tid] = rd.x;
-        s_ray[1][tid] = rd.y;
-        s_ray[2][tid] = rd.z;
-        s_live[tid] = active ? 1u : 0u;
+        s_ray[tid] = make_float4(rd.x, rd.y, rd.z, active ? 1.0f : 0.0f);
     }
     float cr = 0.f, cg = 0.f, cb = 0.f, log_t = 0.f;
     float nx = 0.f, ny = 0.f, nz = 0.f, dep = 0.f, e0 = 0.f, e1 = 0.f, e2 = 0.f, e3 = 0.f;
@@ -779,88 +714,68 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     // checkpoints: next position to store, stop position, slot base
     uint32_t next_ck = kCkGroup, stop = 0u;
     const uint64_t ck_base = ((uint64_t)(rs >> 5) + gtile - 1u) * (uint64_t)(TS * TS) + (uint64_t)tid;
-    TetFetch f;
-    static_assert(C::PF != 2 || B <= 64, "LDS-DMA staging: one wave, next batch inside a 128-entry id window");
-    __shared__ Staging<C::PF == 2 ? B : 1> S;
-    const int wid = tid / 64, lane = (int)__lane_id();
-    QuadFetch qf{};
-    if (C::PF == 1 && tid < nb) fetch_tet<false>(f, sorted_vals[re - 1 - tid], rec, nullptr, col_v);
-    if (C::PF == 3 && tid < 4 * nb) fetch_quad<false>(qf, sorted_vals[re - 1 - (tid >> 2)], tid & 3, rec, nullptr, col_v);
-    if (C::PF == 2 && wid == 0) {
-        const uint32_t t = lane < nb ? sorted_vals[re - 1 - lane] : 0u;
-        stage_async<false>(S, t, lane < nb, rec, nullptr, col_v);
-    }
-    // MERGE: a batch's LDS image is built right after the previous batch's
-    // pixel-sequential phase, without a barrier between them (that phase
-    // reads only the row bases and the pair records, which the image does not
-    // touch; each lane clears its own pixel's mask after reading it), so one
-    // barrier phase per batch goes.  Not with the aux outputs (their phase
-    // reads the face planes) or LDS-DMA staging (its loads need a barrier).
-    constexpr bool MERGE = !AUX && C::PF != 2;
-    auto stage = [&](int nbs, uint32_t d) {
-        if (C::PF == 0 && tid < nbs) fetch_tet<false>(f, sorted_vals[re - 1 - d - tid], rec, nullptr, col_v);
-        if constexpr (C::PF == 3) store_quad<TS, B, false>(L, qf, tid >> 2, tid & 3, tid < 4 * nbs, vw, tc);
-        else if (tid < nbs) store_tet<TS, B, false>(L, tid, f, vw, tc);
+    auto fetch = [&](TetFetch& f, QuadFetch& qf, const uint32_t* ids, int dir, int n) {  // the tets ids[0], ids[dir], ...
+        if constexpr (C::PF == 3) fetch_quad(qf, ids[dir * min(tid >> 2, n - 1)], tid & 3, rec, col_v);
+        else fetch_tet(f, ids[dir * min(tid, n - 1)], rec, col_v);
+    };
+    auto load_ids = [&](uint32_t* idw, uint32_t d) {  // list positions d .. d + 2 B - 1 (past the end: the last)
+#pragma unroll
+        for (int u = 0; u < IDW; ++u)
+            idw[u] = sorted_vals[re - 1 - min(d + (uint32_t)(u * NT + tid), count - 1u)];
+    };
+    auto stage = [&](const TetFetch& f, const QuadFetch& qf, const uint32_t* idw, int n) {
+        if constexpr (C::PF == 3) store_quad<TS, B, false>(L, qf, tid >> 2, tid & 3, tid < 4 * n, vw, tc);
+        else if (tid < n) store_tet<TS, B, false>(L, tid, f, vw, tc);
         if (tid < TS * TS) s_mask[tid] = 0ull;
         if (tid < CAP / 32) G.starts()[tid] = 0u;
+#pragma unroll
+        for (int u = 0; u < IDW; ++u)
+            if (u * NT + tid < 2 * B) s_ids[u * NT + tid] = idw[u];
     };
-    if constexpr (MERGE) {
-        if (count) stage(nb, 0u);
+    if (count) {
+        TetFetch f;
+        QuadFetch qf;
+        uint32_t idw[IDW];
+        fetch(f, qf, sorted_vals + (re - 1), -1, nb);
+        load_ids(idw, 0u);
+        stage(f, qf, idw, nb);
     }
     while (done < count) {
-        // staged records of this batch have landed (and none is in flight at an early exit)
-        if (C::PF == 2) __builtin_amdgcn_s_waitcnt(0);
         if (__syncthreads_and(!active || log_t < -13.8f)) break;
-        // wave 0: tet ids of this and the next batch (back to front of the
-        // sorted list), 64 per register
-        uint32_t win = 0, win1 = 0;
-        if (C::PF == 2 && wid == 0) {
-            win = done + lane < count ? sorted_vals[re - 1 - done - lane] : 0u;
-            if constexpr (B > 32) win1 = done + 64 + lane < count ? sorted_vals[re - 1 - done - 64 - lane] : 0u;
-        }
-        if constexpr (!MERGE) {
-            if constexpr (C::PF == 2) {
-                store_batch_staged<TS, B, false, NT>(L, S, nb, vw, tc);
-                if (tid < TS * TS) s_mask[tid] = 0ull;
-                if (tid < CAP / 32) G.starts()[tid] = 0u;
-            } else {
-                stage(nb, done);
-            }
-            __syncthreads();
-        }
         batch_layout<TS, B, false, true, CAP, NT>(L, nb, G.seg, G.starts());
         __syncthreads();
         const uint32_t nbp = L.nbp & 0xFFu;
         const uint32_t nrec = L.nbp >> 8;
-        // prefetch the next batch's tet records while this one is processed
+        // The next batch's tet records and the ids of the one after it are
+        // loaded while this batch is processed, by every lane (a lane without a
+        // tet takes the last one) into registers declared here and consumed in
+        // this iteration: joined with an older value, by a branch or around
+        // the loop, they were copied right behind the loads, and every batch
+        // waited for the whole latency.
         const uint32_t next = done + nbp;
         const int nb_next = next_batch<B>(nbp, nb, count - next);
-        if (C::PF == 1 && tid < nb_next) fetch_tet<false>(f, sorted_vals[re - 1 - next - tid], rec, nullptr, col_v);
-        if (C::PF == 3 && tid < 4 * nb_next)
-            fetch_quad<false>(qf, sorted_vals[re - 1 - next - (tid >> 2)], tid & 3, rec, nullptr, col_v);
-        if (C::PF == 2 && wid == 0) {
-            const uint32_t tn = window_id<B>(win, win1, (int)nbp + lane);
-            stage_async<false>(S, tn, lane < nb_next, rec, nullptr, col_v);
-        }
+        TetFetch f;
+        QuadFetch qf;
+        uint32_t idw[IDW];
+        fetch(f, qf, s_ids + nbp, 1, B);
+        load_ids(idw, next);
         // record-parallel: intersection + volume integral of one (pixel, tet)
         // record per lane
         for (uint32_t j = tid; j < nrec; j += NT) {
             const RecordRef c = record_at(G.seg, G.starts(), j);
             const int p = c.row * TS + c.col;
+            const float4 rq = s_ray[p];
             // saturated pixels skip the rest of the tile's tets (their compositing loop would)
-            if (s_live[p]) {
+            if (rq.w != 0.0f) {
                 TetRegs T;
                 tet_regs(L, c.k, T);
-                const V3 rd = mk3(s_ray[0][p], s_ray[1][p], s_ray[2][p]);
+                const V3 rd = mk3(rq.x, rq.y, rq.z);
                 float t_min, t_max;
                 int fmin, fmax;
                 if (intersect(T, rd, min_t, t_min, t_max, fmin, fmax)) {
                     Integral I;
                     integral(T, rd, t_min, t_max, min_t != 0.0f ? min_t * dot3(T.g, rd) : 0.0f, 0.0f, I);
-                    s_od[j] = I.od;
-                    s_cp[0][j] = I.cp[0];
-                    s_cp[1][j] = I.cp[1];
-                    s_cp[2][j] = I.cp[2];
+                    s_pr[j] = make_float4(I.cp[0], I.cp[1], I.cp[2], I.od);
                     if (AUX) {
                         s_aux[0][j] = t_min;
                         s_aux[1][j] = t_max;
@@ -873,67 +788,81 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         }
         __syncthreads();
         // pixel-sequential compositing in depth order over this pixel's covered
-        // tets (rasterize_compute.wgsl:336-463)
+        // tets (rasterize_compute.wgsl:336-463), two tets per round: both
+        // records' LDS reads (row base, then record) are in flight together,
+        // and only the arithmetic on log T stays sequential
         if (active) {
             unsigned long long m = s_mask[tid];
-            while (m) {
-                const uint32_t k = (uint32_t)__ffsll((long long)m) - 1u;
+            while (m != 0ull && !(log_t < -13.8f)) {
+                const uint32_t k0 = (uint32_t)__ffsll((long long)m) - 1u;
                 m &= m - 1ull;
-                if (log_t < -13.8f) break;
-                if constexpr (CK) {
-                    const uint32_t q = done + k;
-                    for (; next_ck <= q; next_ck += kCkGroup) ck[ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)] = log_t;
-                }
-                const uint32_t slot = (L.rpref[k * SP + row] + (uint32_t)colp) & 0xFFFFu;
-                const float od = s_od[slot];
-                // log_t is in [-13.8, 0] here: the reference's clamp of the
-                // exponent and its test T >= 1e-6 (exp(-13.8) = 1.01e-6) hold
-                const float Tj = fast_exp(log_t);
-                cr = cr + s_cp[0][slot] * Tj;
-                cg = cg + s_cp[1][slot] * Tj;
-                cb = cb + s_cp[2][slot] * Tj;
-                log_t = log_t - od;
-                if constexpr (CK) stop = done + k + 1u;
-                if (AUX) {
-                    // rasterize_compute.wgsl:434-456
-                    float alpha_t = fast_safe_exp(-od);
-                    float alpha = 1.0f - alpha_t;
-                    float w0 = s_aux[2][slot];
-                    float w1 = 1.0f - (w0 + alpha_t);
-                    float t_min = s_aux[0][slot], t_max = s_aux[1][slot];
-                    int entry = (int)s_ent[slot];
-                    V3 en = mk3(0.f, 0.f, 0.f);
-                    if (entry < 4) {
-                        const float4 q = L.tr[k * L.TR + entry];
-                        en = normalize3(neg3(mk3(q.x, q.y, q.z)));
+                const bool two = m != 0ull;
+                const uint32_t k1 = two ? (uint32_t)__ffsll((long long)m) - 1u : k0;
+                m &= m - 1ull;
+                const uint32_t slot0 = (L.rpref[k0 * SP + row] + (uint32_t)colp) & 0xFFFFu;
+                const uint32_t slot1 = (L.rpref[k1 * SP + row] + (uint32_t)colp) & 0xFFFFu;
+                const float4 q0 = s_pr[slot0], q1 = s_pr[slot1];
+                auto step = [&](uint32_t k, uint32_t slot, float4 q) {
+                    if constexpr (CK) {
+                        const uint32_t pos = done + k;
+                        for (; next_ck <= pos; next_ck += kCkGroup)
+                            ck[ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)] = log_t;
+                        stop = pos + 1u;
                     }
-                    float depth_premul = w0 * t_max + w1 * t_min;
-                    float ta = Tj * alpha;
-                    nx = nx + ta * en.x;
-                    ny = ny + ta * en.y;
-                    nz = nz + ta * en.z;
-                    dep = dep + Tj * depth_premul;
-                    float wt = alpha * Tj;
-                    float c_mid = (t_min + t_max) * 0.5f;
-                    float wc = wt * c_mid;
-                    e0 = e0 + wt;
-                    e1 = e1 + (wt > 1e-20f ? wt * logf(wt) : 0.0f);
-                    e2 = e2 + wt * c_mid;
-                    e3 = e3 + (wc > 1e-20f ? wc * logf(wc) : 0.0f);
-                }
+                    // log_t is in [-13.8, 0] here: the reference's clamp of the
+                    // exponent and its test T >= 1e-6 (exp(-13.8) = 1.01e-6) hold
+                    const float Tj = fast_exp(log_t);
+                    const float od = q.w;
+                    cr = cr + q.x * Tj;
+                    cg = cg + q.y * Tj;
+                    cb = cb + q.z * Tj;
+                    log_t = log_t - od;
+                    if (AUX) {
+                        // rasterize_compute.wgsl:434-456
+                        float alpha_t = fast_safe_exp(-od);
+                        float alpha = 1.0f - alpha_t;
+                        float w0 = s_aux[2][slot];
+                        float w1 = 1.0f - (w0 + alpha_t);
+                        float t_min = s_aux[0][slot], t_max = s_aux[1][slot];
+                        int entry = (int)s_ent[slot];
+                        V3 en = mk3(0.f, 0.f, 0.f);
+                        if (entry < 4) {
+                            const float4 q = L.tr[k * L.TR + entry];
+                            en = normalize3(neg3(mk3(q.x, q.y, q.z)));
+                        }
+                        float depth_premul = w0 * t_max + w1 * t_min;
+                        float ta = Tj * alpha;
+                        nx = nx + ta * en.x;
+                        ny = ny + ta * en.y;
+                        nz = nz + ta * en.z;
+                        dep = dep + Tj * depth_premul;
+                        float wt = alpha * Tj;
+                        float c_mid = (t_min + t_max) * 0.5f;
+                        float wc = wt * c_mid;
+                        e0 = e0 + wt;
+                        e1 = e1 + (wt > 1e-20f ? wt * logf(wt) : 0.0f);
+                        e2 = e2 + wt * c_mid;
+                        e3 = e3 + (wc > 1e-20f ? wc * logf(wc) : 0.0f);
+                    }
+                };
+                step(k0, slot0, q0);
+                if (two && !(log_t < -13.8f)) step(k1, slot1, q1);
             }
-            if (log_t < -13.8f) s_live[tid] = 0u;
+            if (log_t < -13.8f) s_ray[tid].w = 0.0f;
             else if constexpr (CK)  // positions up to the batch's end that this pixel passed uncovered
                 for (; next_ck <= next && next_ck < count; next_ck += kCkGroup)
                     ck[ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)] = log_t;
         }
-        if constexpr (MERGE) {
-            if (nb_next > 0) stage(nb_next, next);
-        }
+        // The next batch's LDS image follows the pixel phase without a barrier
+        // between them (that phase reads only the row bases and the pair
+        // records, which the image does not touch; each lane clears its own
+        // pixel's mask after reading it).  The aux outputs' phase reads the
+        // face planes too.
+        if (AUX) __syncthreads();
+        if (nb_next > 0) stage(f, qf, idw, nb_next);
         done = next;
         nb = nb_next;
     }
-    if (C::PF == 2) __builtin_amdgcn_s_waitcnt(0);  // no LDS DMA outlives the workgroup
     if (active) {
         const uint64_t pix = vw.pix_base + (uint64_t)py * vw.width + px;
         if constexpr (CK) fin[pix] = make_float2(log_t, __uint_as_float(stop));
@@ -1083,8 +1012,8 @@ __device__ __forceinline__ void face_slot_weights(int fi, float la, float lb, fl
 // pair (and NaN) takes the clipped path, term by term as the reference.
 // The slab and the integral's exponential and phi come from the lane's phase-A
 // evaluation of the same pair.
-template <int TS, int B>
-__device__ __forceinline__ void pair_grad(const BatchLDS<TS, B, true>& L, int k, V3 cam, V3 rd, float dc0, float dc1,
+template <int TS, int B, int U>
+__device__ __forceinline__ void pair_grad(const BatchLDS<TS, B, true, U>& L, int k, V3 cam, V3 rd, float dc0, float dc1,
                                           float dc2, float t_prev, float d_log_t_b, float t_min, float t_max,
                                           float alpha_t, float ph, int min_face, int max_face, float* acc) {
 #pragma clang fp contract(fast)
@@ -1208,22 +1137,22 @@ __device__ __forceinline__ void pair_grad(const BatchLDS<TS, B, true>& L, int k,
 // forward.  Without CK: the reference's undo from log(1 - alpha).
 template <class C, bool CK>
 __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE))) void k_backward(
-    const float4* __restrict__ rec, const uint32_t* __restrict__ idx, const float4* __restrict__ colors,
+    const float4* __restrict__ rec, const float4* __restrict__ colors,
     const uint32_t* __restrict__ sorted_vals, const uint32_t* __restrict__ ranges,
     const ViewParams* __restrict__ views, const uint32_t* __restrict__ tile_view, const uint32_t* __restrict__ tile_order,
     const float* __restrict__ rgba, const float* __restrict__ dl_img, const float* __restrict__ gt, uint32_t loss_type,
     float* __restrict__ loss_partial, float* __restrict__ tet_g, float* __restrict__ d_colors,
     const float* __restrict__ ck, const float2* __restrict__ fin, uint64_t* __restrict__ scene_done) {
     constexpr int TS = C::TS, NT = C::NT, B = C::B, CAP = C::CAP, SP = TS + 1, NW = NT / 64, NREC = C::NREC;
-    __shared__ BatchLDS<TS, B, true> L;
+    __shared__ BatchLDS<TS, B, true, CAP> L;
     // per-pair record: od -> -t_prev (the sign marks a pair that takes part),
     // dc . cp -> d_log_t before (dc . cp, the pixel's image gradient dotted with
     // the pair's premultiplied colour, is all the d(log T) chain needs of the
     // colour).  What else phase C needs of a pair stays in registers of the
     // lane that evaluated it in phase A: the same lane takes it in phase C.
-    __shared__ float s_od[CAP], s_dl[CAP];
-    __shared__ float s_ray[3][TS * TS];
-    __shared__ float s_dc[3][TS * TS];
+    float2* const s_pr = L.pair;
+    __shared__ float4 s_ray[TS * TS];  // ray direction, image gradient r
+    __shared__ float2 s_dc[TS * TS];   // image gradient g, b
     // Row sums of phase C: the sum over the records of tet k in the 16-record
     // row r (records 16 r .. 16 r + 15) at slot k + r.  Along the batch's records
     // k and r never decrease and one of them steps from each such run to the
@@ -1235,6 +1164,10 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     using MaskT = typename std::conditional<(B > 32), unsigned long long, unsigned int>::type;
     __shared__ MaskT s_mask[TS * TS];
     __shared__ SegTab<CAP> G;
+    // tet ids at list positions done .. done + 2 B - 1, so the next batch's
+    // record loads (which start where this batch is cut) wait for no id
+    constexpr int IDW = (2 * B + NT - 1) / NT;
+    __shared__ uint32_t s_ids[2 * B];
     __shared__ float s_loss[NW];
     static_assert(B <= 64, "pixel masks hold 64 tets");
     static_assert(CAP / 32 <= NT && TS <= 32, "segment table");
@@ -1295,12 +1228,8 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                 d_log_t = -d.w * (CK ? safe_exp(fin_lt) : 1.0f - im.w);
             }
         }
-        s_ray[0][tid] = rd.x;
-        s_ray[1][tid] = rd.y;
-        s_ray[2][tid] = rd.z;
-        s_dc[0][tid] = dcv[0];
-        s_dc[1][tid] = dcv[1];
-        s_dc[2][tid] = dcv[2];
+        s_ray[tid] = make_float4(rd.x, rd.y, rd.z, dcv[0]);
+        s_dc[tid] = make_float2(dcv[1], dcv[2]);
     }
     if (gt && loss_partial) {
         float ws = wave_sum(lsum);
@@ -1320,54 +1249,72 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     // CK: slot of checkpoint j + 1 (the end of group j) is ck_base + j
     const uint64_t ck_base = ((uint64_t)(rs >> 5) + gtile) * (uint64_t)(TS * TS) + (uint64_t)tid;
     int32_t cur = -1;  // CK: group the pixel's undo is in
-    TetFetch f;
-    static_assert(C::PF != 2 || B <= 64, "LDS-DMA staging: one wave, next batch inside a 128-entry id window");
     static_assert(!CK || B <= (int)kCkGroup, "a batch spans at most two checkpoint groups");
-    __shared__ Staging<C::PF == 2 ? B : 1> S;
-    QuadFetch qf{};
-    if (C::PF == 1 && tid < nb) fetch_tet<true>(f, sorted_vals[rs + tid], rec, idx, col_v);
-    if (C::PF == 3 && tid < 4 * nb) fetch_quad<true>(qf, sorted_vals[rs + (tid >> 2)], tid & 3, rec, idx, col_v);
-    if (C::PF == 2 && wid == 0) {
-        const uint32_t t = lane < nb ? sorted_vals[rs + lane] : 0u;
-        stage_async<true>(S, t, lane < nb, rec, idx, col_v);
-    }
-    // The flush of a batch's terms runs at the top of the next iteration, in
-    // the same phase as the next batch's LDS image (they touch disjoint LDS):
-    // one barrier phase fewer per batch, and the atomics overlap the staging.
-    uint32_t flush_n = 0;  // tets of the previous batch to flush
-    auto flush = [&]() {
+    auto fetch = [&](TetFetch& f, QuadFetch& qf, const uint32_t* ids, int n) {
+        if constexpr (C::PF == 3) fetch_quad(qf, ids[min(tid >> 2, n - 1)], tid & 3, rec, col_v);
+        else fetch_tet(f, ids[min(tid, n - 1)], rec, col_v);
+    };
+    auto load_ids = [&](uint32_t* idw, uint32_t d) {  // list positions d .. d + 2 B - 1 (past the end: the last)
+#pragma unroll
+        for (int u = 0; u < IDW; ++u)
+            idw[u] = sorted_vals[rs + min(d + (uint32_t)(u * NT + opaque(threadIdx.x)), count - 1u)];
+    };
+    auto stage = [&](const TetFetch& f, const QuadFetch& qf, const uint32_t* idw, int n) {
+        if constexpr (C::PF == 3) store_quad<TS, B, true>(L, qf, tid >> 2, tid & 3, tid < 4 * n, vw, tc);
+        else if (tid < n) store_tet<TS, B, true>(L, tid, f, vw, tc);
+        if (tid < TS * TS) s_mask[tid] = 0u;
+        if (tid < CAP / 32) G.starts()[tid] = 0u;
+#pragma unroll
+        for (int u = 0; u < IDW; ++u)
+            if (u * NT + opaque(threadIdx.x) < 2 * B) s_ids[u * NT + opaque(threadIdx.x)] = idw[u];
+    };
+    auto flush = [&](int flush_n) {
         // one atomic per non-zero term per (tile, tet), the first 16 into the
         // tet's 64-byte staging record (one L2 request for the lanes of a
-        // tet), the colour terms into the view's colour gradients
-        for (int it = tid; it < (int)flush_n * kTerms; it += NT) {
-            const int k = it / kTerms, q = it % kTerms;
-            const uint32_t rr = L.recs[k], lo = rr & 0xFFFFu, hi = rr >> 16;
-            if (lo == hi) continue;  // no records
-            float s = 0.0f;
-            for (uint32_t r = lo >> 4; r << 4 < hi; ++r) s += reinterpret_cast<const float*>(s_part[k + r])[q];
-            if (s == 0.0f) continue;
-            const uint32_t t = s_ftid[k];
-            float* dst = q < 16 ? tet_g + 16ull * t + q : dcol_v + 3ull * t + (q - 16);
-            unsafeAtomicAdd(dst, s);
+        // tet), the colour terms into the view's colour gradients.  All of a
+        // lane's LDS reads are issued before the first atomic; a tet has
+        // seldom more than two rows.
+        constexpr int IT = (B * kTerms + NT - 1) / NT;
+        float sum[IT];
+        uint32_t id[IT];
+        const int tid = opaque(threadIdx.x);
+#pragma unroll
+        for (int u = 0; u < IT; ++u) {
+            const int it = u * NT + tid;
+            sum[u] = 0.0f;
+            if (it < flush_n * kTerms) {
+                const int k = it / kTerms, q = it % kTerms;
+                const uint32_t rr = L.recs[k], lo = rr & 0xFFFFu, hi = rr >> 16;
+                const uint32_t r0 = lo >> 4, r1 = (hi + 15u) >> 4;  // rows [r0, r1)
+                id[u] = s_ftid[k];
+                const float x0 = reinterpret_cast<const float*>(s_part[k + r0])[q];
+                const float x1 = reinterpret_cast<const float*>(s_part[min((int)(k + r0) + 1, NPART - 1)])[q];
+                float x = lo < hi ? x0 : 0.0f;
+                if (lo < hi && r0 + 1u < r1) x += x1;
+                for (uint32_t r = r0 + 2u; r < r1; ++r) x += reinterpret_cast<const float*>(s_part[k + r])[q];
+                sum[u] = x;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < IT; ++u) {
+            if (sum[u] == 0.0f) continue;
+            const int q = (u * NT + tid) % kTerms;
+            float* dst = q < 16 ? tet_g + 16ull * id[u] + q : dcol_v + 3ull * id[u] + (q - 16);
+            unsafeAtomicAdd(dst, sum[u]);
         }
     };
     // tile columns and rows inside the image
     const int in_w = (int)min<uint32_t>(TS, vw.width - tc.tile_x * TS), in_h = (int)min<uint32_t>(TS, vw.height - tc.tile_y * TS);
+    if (count) {
+        TetFetch f;
+        QuadFetch qf;
+        uint32_t idw[IDW];
+        fetch(f, qf, sorted_vals + rs, nb);
+        load_ids(idw, 0u);
+        stage(f, qf, idw, nb);
+    }
     while (done < count) {
-        if (C::PF == 2) __builtin_amdgcn_s_waitcnt(0);  // staged records of this batch have landed
-        __syncthreads();
-        flush();
-        uint32_t win = 0, win1 = 0;  // wave 0: tet ids of this and the next batch, 64 per register
-        if (C::PF == 2 && wid == 0) {
-            win = done + lane < count ? sorted_vals[rs + done + lane] : 0u;
-            if constexpr (B > 32) win1 = done + 64 + lane < count ? sorted_vals[rs + done + 64 + lane] : 0u;
-        }
-        if (C::PF == 0 && tid < nb) fetch_tet<true>(f, sorted_vals[rs + done + tid], rec, idx, col_v);
-        if constexpr (C::PF == 2) store_batch_staged<TS, B, true, NT>(L, S, nb, vw, tc);
-        else if constexpr (C::PF == 3) store_quad<TS, B, true>(L, qf, tid >> 2, tid & 3, tid < 4 * nb, vw, tc);
-        else if (tid < nb) store_tet<TS, B, true>(L, tid, f, vw, tc);
-        if (tid < TS * TS) s_mask[tid] = 0u;
-        if (tid < CAP / 32) G.starts()[tid] = 0u;
+        const int tid = opaque(threadIdx.x);
         __syncthreads();
         batch_layout<TS, B, true, false, CAP, NT>(L, nb, G.seg, G.starts());
         __syncthreads();
@@ -1385,15 +1332,13 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             ck_hi = (uint32_t)(j_hi + 1) * kCkGroup < stop ? ck[ck_base + (uint64_t)j_hi * (TS * TS)] : fin_lt;
             ck_lo = (uint32_t)(j_lo + 1) * kCkGroup < stop ? ck[ck_base + (uint64_t)j_lo * (TS * TS)] : fin_lt;
         }
-        if (C::PF == 1 && tid < nb_next) fetch_tet<true>(f, sorted_vals[rs + next + tid], rec, idx, col_v);
-        if (C::PF == 3 && tid < 4 * nb_next)
-            fetch_quad<true>(qf, sorted_vals[rs + next + (tid >> 2)], tid & 3, rec, idx, col_v);
-        if (C::PF == 2 && wid == 0) {
-            const uint32_t tn = window_id<B>(win, win1, (int)nbp + lane);
-            stage_async<true>(S, tn, lane < nb_next, rec, idx, col_v);
-        }
-        // the flush above has read s_ftid (two barriers ago)
-        if (tid < (int)nbp) s_ftid[tid] = L.tid[tid];
+        // loaded for the end of this iteration (as in the forward)
+        TetFetch f;
+        QuadFetch qf;
+        uint32_t idw[IDW];
+        fetch(f, qf, s_ids + nbp, B);
+        load_ids(idw, next);
+        if (tid < (int)nbp) s_ftid[tid] = s_ids[tid];
         // phase A (record-parallel): intersection + integral; lane tid takes
         // records tid, tid + NT, ... here and in phase C
         float r_t0[NREC], r_t1[NREC], r_at[NREC], r_ph[NREC];
@@ -1407,15 +1352,16 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                 const int p = c.row * TS + c.col;
                 TetRegs T;
                 tet_regs(L, c.k, T);
-                const V3 rd = mk3(s_ray[0][p], s_ray[1][p], s_ray[2][p]);
+                const float4 rq = s_ray[p];
+                const float2 dq = s_dc[p];
+                const V3 rd = mk3(rq.x, rq.y, rq.z);
                 float t_min, t_max;
                 int fmin, fmax;
                 r_m[n] = (uint32_t)c.k;
                 if (intersect(T, rd, 0.0f, t_min, t_max, fmin, fmax) && c.row < in_h && c.col < in_w) {
                     Integral I;
                     integral<false>(T, rd, t_min, t_max, 0.0f, kMinVal, I);
-                    s_od[j] = I.od;
-                    s_dl[j] = (s_dc[0][p] * I.cp[0] + s_dc[1][p] * I.cp[1]) + s_dc[2][p] * I.cp[2];
+                    s_pr[j] = make_float2(I.od, (rq.w * I.cp[0] + dq.x * I.cp[1]) + dq.y * I.cp[2]);
                     r_t0[n] = t_min;
                     r_t1[n] = t_max;
                     r_at[n] = I.alpha_t;
@@ -1427,32 +1373,41 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         }
         __syncthreads();
         // phase B (pixel-sequential, back to front over this pixel's covered
-        // tets): undo and the d(log T) chain (backward_tiled_compute.wgsl:419-451)
+        // tets): undo and the d(log T) chain (backward_tiled_compute.wgsl:419-451),
+        // two tets per round as in the forward
         if (active) {
             MaskT m = s_mask[tid];
+            auto first = [](MaskT x) {
+                return B > 32 ? (uint32_t)__ffsll((long long)x) - 1u : (uint32_t)__ffs((int)x) - 1u;
+            };
             while (m) {
-                const uint32_t k = B > 32 ? (uint32_t)__ffsll((long long)m) - 1u : (uint32_t)__ffs((int)m) - 1u;
+                const uint32_t k0 = first(m);
                 m &= m - (MaskT)1;
-                if constexpr (CK) {
-                    const uint32_t q = count - 1u - done - k;  // position in compositing order
-                    if (q >= stop) continue;
-                    const int32_t j = (int32_t)(q / kCkGroup);
-                    if (j != cur) {
-                        log_t = j == j_hi ? ck_hi : ck_lo;
-                        cur = j;
+                const bool two = m != 0;
+                const uint32_t k1 = two ? first(m) : k0;
+                m &= m - (MaskT)1;
+                const uint32_t slot0 = (L.rpref[k0 * SP + row] + (uint32_t)colp) & 0xFFFFu;
+                const uint32_t slot1 = (L.rpref[k1 * SP + row] + (uint32_t)colp) & 0xFFFFu;
+                const float2 q0 = s_pr[slot0], q1 = s_pr[slot1];
+                auto step = [&](uint32_t k, uint32_t slot, float2 q) {
+                    if constexpr (CK) {
+                        const uint32_t pos = count - 1u - done - k;  // position in compositing order
+                        if (pos >= stop) return;
+                        const int32_t j = (int32_t)(pos / kCkGroup);
+                        if (j != cur) {
+                            log_t = j == j_hi ? ck_hi : ck_lo;
+                            cur = j;
+                        }
                     }
-                }
-                const uint32_t slot = (L.rpref[k * SP + row] + (uint32_t)colp) & 0xFFFFu;
-                const float od = s_od[slot];
-                const float prev_log_t = fminf(log_t + od, 0.0f);
-                // (no clamp of the exponent: below -88 the value is under 1e-6 all the same)
-                const float t_prev = fast_exp(prev_log_t);
-                log_t = prev_log_t;
-                if (t_prev < 1e-6f) continue;
-                const float dcp = s_dl[slot];
-                s_od[slot] = -t_prev;
-                s_dl[slot] = d_log_t;
-                d_log_t = safe_clip(d_log_t + dcp * t_prev, kMinVal, kMaxVal);
+                    log_t = fminf(log_t + q.x, 0.0f);
+                    // (no clamp of the exponent: below -88 the value is under 1e-6 all the same)
+                    const float t_prev = fast_exp(log_t);
+                    if (t_prev < 1e-6f) return;
+                    s_pr[slot] = make_float2(-t_prev, d_log_t);
+                    d_log_t = safe_clip(d_log_t + q.y * t_prev, kMinVal, kMaxVal);
+                };
+                step(k0, slot0, q0);
+                if (two) step(k1, slot1, q1);
             }
         }
         __syncthreads();
@@ -1466,12 +1421,12 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             bool have = false;  // acc assigned by the lane's pair
             const int key = j < nrec ? (int)(r_m[n] & 63u) : -2;  // a tet's records are contiguous, hit or not
             if (r_m[n] >> 20) {
-                const float tp = s_od[j];
-                if (tp < 0.0f) {
+                const float2 q = s_pr[j];
+                if (q.x < 0.0f) {
                     const int p = (int)((r_m[n] >> 6) & 1023u);
-                    const V3 rd = mk3(s_ray[0][p], s_ray[1][p], s_ray[2][p]);
-                    pair_grad<TS, B>(L, key, cam, rd, s_dc[0][p], s_dc[1][p], s_dc[2][p], -tp, s_dl[j], r_t0[n],
-                                     r_t1[n], r_at[n], r_ph[n], (int)((r_m[n] >> 16) & 3u), (int)((r_m[n] >> 18) & 3u),
+                    const float4 rq = s_ray[p];
+                    const float2 dq = s_dc[p];
+                    pair_grad<TS, B>(L, key, cam, mk3(rq.x, rq.y, rq.z), rq.w, dq.x, dq.y, -q.x, q.y, r_t0[n], r_t1[n], r_at[n], r_ph[n], (int)((r_m[n] >> 16) & 3u), (int)((r_m[n] >> 18) & 3u),
                                      acc);
                     have = true;
                 }
@@ -1492,13 +1447,16 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                     o[q] = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], 4 * q + 3 < kTerms ? acc[4 * q + 3] : 0.0f);
             }
         }
-        flush_n = nbp;
+        __syncthreads();
+        // The next batch's LDS image and this batch's flush share a phase (they
+        // touch disjoint LDS).  The atomics come last: loads and atomics
+        // complete in order, so a wait for a load would also wait for the
+        // atomics issued before it.
+        if (nb_next > 0) stage(f, qf, idw, nb_next);
+        flush((int)nbp);
         done = next;
         nb = nb_next;
     }
-    __syncthreads();
-    flush();
-    if (C::PF == 2) __builtin_amdgcn_s_waitcnt(0);  // no LDS DMA outlives the workgroup
     if (scene_done && tid == 0) atomicMax(reinterpret_cast<unsigned long long*>(scene_done) + vw.scene,
                                           (unsigned long long)wall_clock64());
 }
@@ -1565,13 +1523,13 @@ static void bwd_launch(const BwdArgs& a, hipStream_t s) {
             // the checkpointed adjoint's batches span at most two checkpoint groups (B <= 32)
             bwd_launch<BwdCfg<C::TS, 32, C::CAP, C::PF_ARG, C::WPE_ARG>>(a, s);
         } else {
-            hipLaunchKernelGGL((k_backward<C, true>), dim3(a.num_gtiles), dim3(C::NT), 0, s, a.rec, a.idx, a.colors,
+            hipLaunchKernelGGL((k_backward<C, true>), dim3(a.num_gtiles), dim3(C::NT), 0, s, a.rec, a.colors,
                                a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order,
                                a.rgba, a.dl_img, a.gt, a.loss_type, a.loss_partial, a.tet_g, a.d_colors, a.ck, a.fin,
                                a.scene_done);
         }
     } else
-        hipLaunchKernelGGL((k_backward<C, false>), dim3(a.num_gtiles), dim3(C::NT), 0, s, a.rec, a.idx, a.colors,
+        hipLaunchKernelGGL((k_backward<C, false>), dim3(a.num_gtiles), dim3(C::NT), 0, s, a.rec, a.colors,
                            a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order,
                            a.rgba, a.dl_img, a.gt, a.loss_type, a.loss_partial, a.tet_g, a.d_colors, nullptr,
                            nullptr, a.scene_done);
@@ -1583,22 +1541,22 @@ static void bwd_launch(const BwdArgs& a, hipStream_t s) {
 // three records a lane measured best at tiles 12 and 16 (config C, tile 16, B
 // 48: N 2 13.25 ms, N 3 12.31 ms; B 64 leaves 3 workgroups per CU: 13.9 ms).
 // One-wave workgroups (tile 8) take half the tets and one record a lane more.
-template <int TS, int B, int N, int PF>
-using BwdGeo = BwdCfg<TS, (TS == 8 ? B / 2 : B), (TS == 8 ? N + 1 : N) * ((TS * TS + 63) / 64 * 64), PF, 4>;
+template <int TS, int B, int N>
+using BwdGeo = BwdCfg<TS, (TS == 8 ? B / 2 : B), (TS == 8 ? N + 1 : N) * ((TS * TS + 63) / 64 * 64), 3, 4>;
 template <int TS>
 static bool bwd_variant(const BwdArgs& a, int v, hipStream_t s) {
     switch (v) {
         case 0:
-        case 10: bwd_launch<BwdGeo<TS, 48, 3, 3>>(a, s); return true;
-        case 1: bwd_launch<BwdGeo<TS, 32, 3, 3>>(a, s); return true;
-        case 2: bwd_launch<BwdGeo<TS, 32, 2, 2>>(a, s); return true;
-        case 3: bwd_launch<BwdGeo<TS, 48, 2, 3>>(a, s); return true;
-        case 4: bwd_launch<BwdGeo<TS, 32, 3, 2>>(a, s); return true;
-        case 5: bwd_launch<BwdGeo<TS, 64, 3, 3>>(a, s); return true;
-        case 6: bwd_launch<BwdGeo<TS, 40, 3, 3>>(a, s); return true;
-        case 7: bwd_launch<BwdGeo<TS, 56, 3, 3>>(a, s); return true;
-        case 8: bwd_launch<BwdGeo<TS, 64, 2, 3>>(a, s); return true;
-        case 9: bwd_launch<BwdGeo<TS, 40, 2, 3>>(a, s); return true;
+        case 10: bwd_launch<BwdGeo<TS, 48, 3>>(a, s); return true;
+        case 1: bwd_launch<BwdGeo<TS, 32, 3>>(a, s); return true;
+        case 2: bwd_launch<BwdGeo<TS, 32, 2>>(a, s); return true;
+        case 3: bwd_launch<BwdGeo<TS, 48, 2>>(a, s); return true;
+        case 4: bwd_launch<BwdGeo<TS, 24, 3>>(a, s); return true;
+        case 5: bwd_launch<BwdGeo<TS, 64, 3>>(a, s); return true;
+        case 6: bwd_launch<BwdGeo<TS, 40, 3>>(a, s); return true;
+        case 7: bwd_launch<BwdGeo<TS, 56, 3>>(a, s); return true;
+        case 8: bwd_launch<BwdGeo<TS, 64, 2>>(a, s); return true;
+        case 9: bwd_launch<BwdGeo<TS, 40, 2>>(a, s); return true;
         default: return false;
     }
 }
@@ -1692,8 +1650,9 @@ __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec,
     int nb = (int)min<uint32_t>(B, count);
     TetFetch f;
     QuadFetch qf{};
-    if (C::PF == 1 && tid < nb) fetch_tet<false>(f, sorted_vals[re - 1 - tid], rec, nullptr, rec);
-    if (C::PF == 3 && tid < 4 * nb) fetch_quad<false>(qf, sorted_vals[re - 1 - (tid >> 2)], tid & 3, rec, nullptr, rec);
+    uint32_t ft = 0;
+    if (C::PF == 1 && tid < nb) fetch_tet(f, ft = sorted_vals[re - 1 - tid], rec, rec);
+    if (C::PF == 3 && tid < 4 * nb) fetch_quad(qf, ft = sorted_vals[re - 1 - (tid >> 2)], tid & 3, rec, rec);
     while (done < count) {
         if (__syncthreads_and(!active || log_t < -5.5f)) break;
         if constexpr (C::PF == 3) {
@@ -1702,7 +1661,7 @@ __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec,
             const V3 cen = scl3(add3(add3(add3(a, b), c), d), 0.25f);
             if (tid < 4 * nb && (tid & 3) == 0) {
                 s_cen[tid >> 2] = make_float4(cen.x, cen.y, cen.z, 0.0f);
-                s_tid[tid >> 2] = qf.t;
+                s_tid[tid >> 2] = ft;
             }
         } else if (tid < nb) {
             store_tet<TS, B, false>(L, tid, f, vw, tc);
@@ -1710,7 +1669,7 @@ __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec,
                      c = mk3(f.r[2].x, f.r[2].y, f.r[2].z), d = mk3(f.r[3].x, f.r[3].y, f.r[3].z);
             const V3 cen = scl3(add3(add3(add3(a, b), c), d), 0.25f);
             s_cen[tid] = make_float4(cen.x, cen.y, cen.z, 0.0f);
-            s_tid[tid] = f.t;
+            s_tid[tid] = ft;
         }
         if (tid < TS * TS) s_mask[tid] = 0ull;
         if (tid < CAP / 32) G.starts()[tid] = 0u;
@@ -1723,9 +1682,8 @@ __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec,
         const uint32_t nrec = L.nbp >> 8;
         const uint32_t next = done + nbp;
         const int nb_next = (int)min<uint32_t>(B, count - next);
-        if (C::PF == 1 && tid < nb_next) fetch_tet<false>(f, sorted_vals[re - 1 - next - tid], rec, nullptr, rec);
-        if (C::PF == 3 && tid < 4 * nb_next)
-            fetch_quad<false>(qf, sorted_vals[re - 1 - next - (tid >> 2)], tid & 3, rec, nullptr, rec);
+        if (C::PF == 1 && tid < nb_next) fetch_tet(f, ft = sorted_vals[re - 1 - next - tid], rec, rec);
+        if (C::PF == 3 && tid < 4 * nb_next) fetch_quad(qf, ft = sorted_vals[re - 1 - next - (tid >> 2)], tid & 3, rec, rec);
         // phase A: slab and optical depth of every covered pair
         for (uint32_t j = tid; j < nrec; j += NT) {
             const RecordRef c = record_at(G.seg, G.starts(), j);
