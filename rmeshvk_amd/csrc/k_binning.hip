@@ -764,66 +764,113 @@ void launch_pairs_depth_ordered(const float4* rec, const SceneRange* scenes, uin
         hipLaunchKernelGGL(k_pairs_sorted<false>, gr, bl, 0, s, rec, scenes, n_scenes, sval, n_items, views, counts,
                            block_sums, keys, vals, cap, overflow);
 }
-// Tiles heaviest first: the compositing grids take their tiles in this order,
-// so the few very dense tiles (tens of times the median pair count) start
-// early instead of running alone at the end of the grid (longest-processing-
-// time-first).  A bucket sort by the pair count's bit length and its next two
-// bits (four buckets per octave), descending; the order inside a bucket is
-// whatever the LDS atomics give (every tile's result is independent of when
-// it runs).
-constexpr int kOrderBuckets = 33 * 4;
-__device__ __forceinline__ uint32_t tile_bucket(const uint32_t* __restrict__ ranges, uint32_t t) {
+// Work items of the compositing grids, heaviest first: the few very dense tiles
+// (tens of times the median pair count) start early instead of running alone at
+// the end of the grid (longest-processing-time-first).  With a SplitPlan a tile
+// whose list is longer than a segment gives one item per segment, and gets its
+// segment slots.  A bucket sort by the item's pair count, its bit length and the
+// next two bits (four buckets per octave), descending; among segments of a bucket
+// those nearer the camera first (a segment behind others that already block the
+// tile's light need not run).  The order inside a bucket and the slot bases are
+// whatever the LDS atomics give (no result depends on either).
+constexpr int kPairBuckets = 33 * 4;
+constexpr int kSegBuckets = 16;   // per pair bucket that segments fall into: segments 0 .. 14, 15 and later
+constexpr int kOrderBuckets = kPairBuckets + 5 * kSegBuckets;  // (unit / 2 .. unit pairs: at most five)
+__device__ __forceinline__ uint32_t tile_pairs(const uint32_t* __restrict__ ranges, uint32_t t) {
     const uint32_t rs = ranges[2ull * t], re = ranges[2ull * t + 1];
-    const uint32_t c = re > rs ? re - rs : 0u;
+    return re > rs ? re - rs : 0u;
+}
+__device__ __forceinline__ uint32_t pair_bucket(uint32_t c) {
     if (c < 4u) return c;
     const uint32_t len = 32u - (uint32_t)__clz((int)c);  // >= 3
     return len * 4u + ((c >> (len - 3u)) & 3u);           // 3 leading bits: 1xx
 }
-
+// Bucket of segment seg of a tile whose segments hold c pairs, or (seg -1) of a
+// whole tile of c pairs.  Whole tiles come first in their pair bucket.
+__device__ __forceinline__ uint32_t item_bucket(uint32_t c, int seg, const SplitPlan& sp) {
+    const uint32_t b = pair_bucket(c);
+    if (!sp.seg) return b;
+    const uint32_t lo = pair_bucket(sp.unit / 2u), hi = pair_bucket(sp.unit);
+    if (b < lo) return b;
+    const uint32_t in = seg < 0 ? (uint32_t)kSegBuckets : (uint32_t)kSegBuckets - 1u - min((uint32_t)seg, (uint32_t)kSegBuckets - 1u);
+    return lo + (min(b, hi) - lo) * (uint32_t)(kSegBuckets + 1) + in;
+}
+// cnt: the tile's bucket counters (its scene's).
+__device__ __forceinline__ void count_items(uint32_t* cnt, uint32_t pairs, const SplitPlan& sp) {
+    const uint32_t n = sp.seg ? split_segments(pairs, sp.unit) : 1u;
+    if (n == 1u) atomicAdd(&cnt[item_bucket(pairs, -1, sp)], 1u);
+    else
+        for (uint32_t g = 0; g < n; ++g) atomicAdd(&cnt[item_bucket(split_length(pairs, sp.unit), (int)g, sp)], 1u);
+}
+// off: the buckets' running item offsets; n_slots: the running slot count.
+__device__ __forceinline__ void place_items(uint32_t* off, uint32_t* n_slots, uint32_t t, uint32_t pairs,
+                                            uint32_t* __restrict__ order, const SplitPlan& sp) {
+    const uint32_t n = sp.seg ? split_segments(pairs, sp.unit) : 1u;
+    if (n == 1u) {
+        const uint32_t i = atomicAdd(&off[item_bucket(pairs, -1, sp)], 1u);
+        order[i] = t;
+        if (sp.seg) sp.seg[i] = 0u;
+        return;
+    }
+    const uint32_t slot = atomicAdd(n_slots, n);
+    sp.slot[t] = slot;
+    sp.arrived[t] = 0u;
+    sp.serial[t] = 0u;
+    for (uint32_t g = 0; g < n; ++g) {
+        const uint32_t i = atomicAdd(&off[item_bucket(split_length(pairs, sp.unit), (int)g, sp)], 1u);
+        order[i] = t;
+        sp.seg[i] = g;
+        sp.dark[slot + g] = 0.0f;
+    }
+}
 
 __global__ __launch_bounds__(1024) void k_tile_order(const uint32_t* __restrict__ ranges, uint32_t n,
-                                                      uint32_t* __restrict__ order) {
+                                                      uint32_t* __restrict__ order, SplitPlan sp) {
     __shared__ uint32_t cnt[kOrderBuckets];
-    __shared__ uint32_t off[kOrderBuckets];
+    __shared__ uint32_t n_slots;
     const uint32_t tid = threadIdx.x;
     if (tid < kOrderBuckets) cnt[tid] = 0u;
+    if (tid == 0) n_slots = 0u;
     __syncthreads();
-    for (uint32_t t = tid; t < n; t += blockDim.x) atomicAdd(&cnt[tile_bucket(ranges, t)], 1u);
+    for (uint32_t t = tid; t < n; t += blockDim.x) count_items(cnt, tile_pairs(ranges, t), sp);
     __syncthreads();
     if (tid == 0) {
         uint32_t run = 0;
         for (int b = kOrderBuckets - 1; b >= 0; --b) {
-            off[b] = run;
-            run += cnt[b];
+            const uint32_t k = cnt[b];
+            cnt[b] = run;
+            run += k;
         }
+        if (sp.seg) *sp.n_items = run;
     }
     __syncthreads();
-    for (uint32_t t = tid; t < n; t += blockDim.x) order[atomicAdd(&off[tile_bucket(ranges, t)], 1u)] = t;
+    for (uint32_t t = tid; t < n; t += blockDim.x) place_items(cnt, &n_slots, t, tile_pairs(ranges, t), order, sp);
 }
 
 // Scene-major order for batches of several scenes: the scenes one after
 // another, the one with the fewest pairs first (ties: the caller's order), and
-// the tiles of each scene heaviest first as above.  A scene's tiles then finish
+// the items of each scene in the order above.  A scene's tiles then finish
 // together early in the step instead of all scenes finishing at its end; the
-// tile grid is the same, so the total work is too.  Counts per (scene, bucket)
+// items are the same, so the total work is too.  Counts per (scene, bucket)
 // in LDS, then offsets by one thread.
 constexpr uint32_t kOrderMaxScenes = 64;
 __global__ __launch_bounds__(1024) void k_tile_order_scenes(const uint32_t* __restrict__ ranges, uint32_t n,
                                                             const uint32_t* __restrict__ tile_view,
                                                             const ViewParams* __restrict__ views, uint32_t n_scenes,
-                                                            uint32_t* __restrict__ order) {
+                                                            uint32_t* __restrict__ order, SplitPlan sp) {
     __shared__ uint32_t cnt[kOrderMaxScenes * kOrderBuckets];  // counts, then running offsets
     __shared__ unsigned long long s_pairs[kOrderMaxScenes];
     __shared__ uint32_t s_by_rank[kOrderMaxScenes];
+    __shared__ uint32_t n_slots;
     const uint32_t tid = threadIdx.x;
     for (uint32_t i = tid; i < n_scenes * kOrderBuckets; i += blockDim.x) cnt[i] = 0u;
     if (tid < n_scenes) s_pairs[tid] = 0ull;
+    if (tid == 0) n_slots = 0u;
     __syncthreads();
     for (uint32_t t = tid; t < n; t += blockDim.x) {
-        const uint32_t sc = views[tile_view[t]].scene;
-        atomicAdd(&cnt[sc * kOrderBuckets + tile_bucket(ranges, t)], 1u);
-        const uint32_t rs = ranges[2ull * t], re = ranges[2ull * t + 1];
-        atomicAdd(&s_pairs[sc], (unsigned long long)(re > rs ? re - rs : 0u));
+        const uint32_t sc = views[tile_view[t]].scene, c = tile_pairs(ranges, t);
+        count_items(cnt + sc * kOrderBuckets, c, sp);
+        atomicAdd(&s_pairs[sc], (unsigned long long)c);
     }
     __syncthreads();
     if (tid < n_scenes) {
@@ -842,11 +889,12 @@ __global__ __launch_bounds__(1024) void k_tile_order_scenes(const uint32_t* __re
                 run += k;
             }
         }
+        if (sp.seg) *sp.n_items = run;
     }
     __syncthreads();
     for (uint32_t t = tid; t < n; t += blockDim.x) {
         const uint32_t sc = views[tile_view[t]].scene;
-        order[atomicAdd(&cnt[sc * kOrderBuckets + tile_bucket(ranges, t)], 1u)] = t;
+        place_items(cnt + sc * kOrderBuckets, &n_slots, t, tile_pairs(ranges, t), order, sp);
     }
 }
 
@@ -858,16 +906,17 @@ void launch_stamp_start(uint64_t* p, uint32_t n, hipStream_t s) {
     hipLaunchKernelGGL(k_stamp_start, dim3(1), dim3(64), 0, s, p, n);
 }
 
-void launch_tile_order(const uint32_t* ranges, uint32_t n_tiles, uint32_t* order, hipStream_t s) {
-    if (n_tiles) hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, s, ranges, n_tiles, order);
+void launch_tile_order(const uint32_t* ranges, uint32_t n_tiles, uint32_t* order, const SplitPlan& sp, hipStream_t s) {
+    if (n_tiles) hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, s, ranges, n_tiles, order, sp);
 }
 
 bool launch_tile_order_scenes(const uint32_t* ranges, uint32_t n_tiles, const uint32_t* tile_view,
-                              const ViewParams* views, uint32_t n_scenes, uint32_t* order, hipStream_t s) {
+                              const ViewParams* views, uint32_t n_scenes, uint32_t* order, const SplitPlan& sp,
+                              hipStream_t s) {
     if (n_scenes == 0 || n_scenes > kOrderMaxScenes) return false;
     if (n_tiles)
         hipLaunchKernelGGL(k_tile_order_scenes, dim3(1), dim3(1024), 0, s, ranges, n_tiles, tile_view, views, n_scenes,
-                           order);
+                           order, sp);
     return true;
 }
 

@@ -659,6 +659,40 @@ struct FwdCfg {
     static constexpr int WPE = WPE_ > 0 ? WPE_ : 1;
 };
 
+// Values that workgroups of one grid pass to each other: stored through to the
+// level all XCDs share and loaded from there.  A fence at device scope instead
+// writes back and invalidates the XCD's whole L2, and with one or two per segment
+// the segmented forward of config C took twice as long (10.4 ms for 5.2).
+template <class T>
+__device__ __forceinline__ void store_shared(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ T load_shared(const T* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_shared(float4* p, float4 v) {
+    float* f = reinterpret_cast<float*>(p);
+    store_shared(f, v.x);
+    store_shared(f + 1, v.y);
+    store_shared(f + 2, v.z);
+    store_shared(f + 3, v.w);
+}
+__device__ __forceinline__ float4 load_shared(const float4* p) {
+    const float* f = reinterpret_cast<const float*>(p);
+    return make_float4(load_shared(f), load_shared(f + 1), load_shared(f + 2), load_shared(f + 3));
+}
+// Every store of this wave is done.
+__device__ __forceinline__ void drain_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// A workgroup composites a tile's list, or one segment of a long one (SplitPlan)
+// as if it were the first.  The tile's last workgroup to finish joins the
+// segments, T and colour being a product and a sum along the list.  Where that
+// shows a pixel saturating (log T < -13.8, from where the serial pass composites
+// nothing), it runs the list again from the segment in which the first such
+// pixel does, for those pixels alone, and marks the tile for a serial adjoint
+// (the undo from the image alpha passes over the pairs behind the stop too).
+//
 // CK: also store the transmittance checkpoints of the checkpointed adjoint:
 // a pixel still compositing writes its log T before every tile-list position
 // 32 j it reaches (coalesced: the tile's pixels write one 4 TS^2-byte slot),
@@ -668,8 +702,8 @@ template <class C, bool AUX, bool CK>
 __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE))) void k_forward(
     const float4* __restrict__ rec, const float4* __restrict__ colors,
     const uint32_t* __restrict__ sorted_vals, const uint32_t* __restrict__ ranges, const ViewParams* __restrict__ views,
-    const uint32_t* __restrict__ tile_view, const uint32_t* __restrict__ tile_order, float* __restrict__ rgba,
-    float* __restrict__ aux, float* __restrict__ ck, float2* __restrict__ fin) {
+    const uint32_t* __restrict__ tile_view, const uint32_t* __restrict__ tile_order, const SplitPlan split,
+    float* __restrict__ rgba, float* __restrict__ aux, float* __restrict__ ck, float2* __restrict__ fin) {
     constexpr int TS = C::TS, NT = C::NT, B = C::B, CAP = C::CAP, SP = TS + 1;
     constexpr int NA = AUX ? CAP : 1;
     static_assert(B <= 64, "pixel masks hold 64 tets; the layout scan is one wave");
@@ -686,8 +720,12 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     // loads (which start where this batch is cut) wait for no id
     constexpr int IDW = (2 * B + NT - 1) / NT;
     __shared__ uint32_t s_ids[2 * B];
+    __shared__ float s_red[NT / 64];
+    __shared__ int s_arrived, s_first;
+    __shared__ uint32_t s_plan[4];  // segment, segments, their length, the tile's first slot
     static_assert(CAP / 32 <= NT && TS <= 32, "segment table");
 
+    if (split.seg && blockIdx.x >= *split.n_items) return;
     const uint32_t gtile = tile_order ? tile_order[blockIdx.x] : blockIdx.x;
     const uint32_t view = tile_view[gtile];
     const ViewParams& vw = views[view];
@@ -709,10 +747,37 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
 
     const uint32_t rs = ranges[2ull * gtile], re = ranges[2ull * gtile + 1];
     const uint32_t count = re > rs ? re - rs : 0u;
-    uint32_t done = 0;
-    int nb = (int)min<uint32_t>(B, count);
+    // list positions [done, end) of this workgroup
+    uint32_t done = 0, end = count;
+    bool whole = AUX || !split.seg || split_segments(count, split.unit) == 1u;  // one workgroup, one list
+    if (!whole) {
+        const uint32_t seg = split.seg[blockIdx.x], seg_len = split_length(count, split.unit);
+        const uint32_t slot = split.slot[gtile];
+        done = seg * seg_len;
+        end = min(done + seg_len, count);
+        if (tid == 0) {  // (kept out of the registers until behind the loop)
+            s_plan[0] = seg;
+            s_plan[1] = split_segments(count, split.unit);
+            s_plan[2] = seg_len;
+            s_plan[3] = slot;
+        }
+        // nothing to do once the segments in front are known to saturate every
+        // pixel (with a margin for the rounding of the sum): their last pixel
+        // records show that, and this segment's is not read
+        float d = 0.0f;
+        for (uint32_t g = tid; g < seg; g += NT)
+            d += load_shared(split.dark + slot + g);
+        d = wave_sum(d);
+        if ((tid & 63) == 0) s_red[tid >> 6] = d;
+        __syncthreads();
+        d = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NT / 64; ++w) d += s_red[w];
+        if (d < -13.9f) done = end;
+    }
     // checkpoints: next position to store, stop position, slot base
-    uint32_t next_ck = kCkGroup, stop = 0u;
+    uint32_t next_ck = done + kCkGroup, stop = 0u;
+    bool run = active;  // the pixel composites in the loop below
     const uint64_t ck_base = ((uint64_t)(rs >> 5) + gtile - 1u) * (uint64_t)(TS * TS) + (uint64_t)tid;
     auto fetch = [&](TetFetch& f, QuadFetch& qf, const uint32_t* ids, int dir, int n) {  // the tets ids[0], ids[dir], ...
         if constexpr (C::PF == 3) fetch_quad(qf, ids[dir * min(tid >> 2, n - 1)], tid & 3, rec, col_v);
@@ -721,7 +786,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     auto load_ids = [&](uint32_t* idw, uint32_t d) {  // list positions d .. d + 2 B - 1 (past the end: the last)
 #pragma unroll
         for (int u = 0; u < IDW; ++u)
-            idw[u] = sorted_vals[re - 1 - min(d + (uint32_t)(u * NT + tid), count - 1u)];
+            idw[u] = sorted_vals[re - 1 - min(d + (uint32_t)(u * NT + tid), end - 1u)];
     };
     auto stage = [&](const TetFetch& f, const QuadFetch& qf, const uint32_t* idw, int n) {
         if constexpr (C::PF == 3) store_quad<TS, B, false>(L, qf, tid >> 2, tid & 3, tid < 4 * n, vw, tc);
@@ -732,16 +797,18 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         for (int u = 0; u < IDW; ++u)
             if (u * NT + tid < 2 * B) s_ids[u * NT + tid] = idw[u];
     };
-    if (count) {
+    for (;;) {
+    int nb = (int)min<uint32_t>(B, end - done);
+    if (nb > 0) {
         TetFetch f;
         QuadFetch qf;
         uint32_t idw[IDW];
-        fetch(f, qf, sorted_vals + (re - 1), -1, nb);
-        load_ids(idw, 0u);
+        fetch(f, qf, sorted_vals + (re - 1 - done), -1, nb);
+        load_ids(idw, done);
         stage(f, qf, idw, nb);
     }
-    while (done < count) {
-        if (__syncthreads_and(!active || log_t < -13.8f)) break;
+    while (done < end) {
+        if (__syncthreads_and(!run || log_t < -13.8f)) break;
         batch_layout<TS, B, false, true, CAP, NT>(L, nb, G.seg, G.starts());
         __syncthreads();
         const uint32_t nbp = L.nbp & 0xFFu;
@@ -753,7 +820,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         // the loop, they were copied right behind the loads, and every batch
         // waited for the whole latency.
         const uint32_t next = done + nbp;
-        const int nb_next = next_batch<B>(nbp, nb, count - next);
+        const int nb_next = next_batch<B>(nbp, nb, end - next);
         TetFetch f;
         QuadFetch qf;
         uint32_t idw[IDW];
@@ -791,7 +858,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         // tets (rasterize_compute.wgsl:336-463), two tets per round: both
         // records' LDS reads (row base, then record) are in flight together,
         // and only the arithmetic on log T stays sequential
-        if (active) {
+        if (run) {
             unsigned long long m = s_mask[tid];
             while (m != 0ull && !(log_t < -13.8f)) {
                 const uint32_t k0 = (uint32_t)__ffsll((long long)m) - 1u;
@@ -806,7 +873,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                     if constexpr (CK) {
                         const uint32_t pos = done + k;
                         for (; next_ck <= pos; next_ck += kCkGroup)
-                            ck[ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)] = log_t;
+                            store_shared(ck + (ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)), log_t);
                         stop = pos + 1u;
                     }
                     // log_t is in [-13.8, 0] here: the reference's clamp of the
@@ -851,7 +918,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             if (log_t < -13.8f) s_ray[tid].w = 0.0f;
             else if constexpr (CK)  // positions up to the batch's end that this pixel passed uncovered
                 for (; next_ck <= next && next_ck < count; next_ck += kCkGroup)
-                    ck[ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)] = log_t;
+                    store_shared(ck + (ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)), log_t);
         }
         // The next batch's LDS image follows the pixel phase without a barrier
         // between them (that phase reads only the row bases and the pair
@@ -862,6 +929,127 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         if (nb_next > 0) stage(f, qf, idw, nb_next);
         done = next;
         nb = nb_next;
+    }
+    if (whole) break;
+    const uint32_t seg = s_plan[0], n_seg = s_plan[1], seg_len = s_plan[2], slot = s_plan[3];
+    // One segment of several: its pixel states go to its slot, and the tile's
+    // last workgroup to get here joins them.
+    const uint64_t px0 = (uint64_t)slot * (TS * TS) + (uint64_t)tid;
+    if (tid < TS * TS) {
+        store_shared(split.px + (px0 + (uint64_t)seg * (TS * TS)), make_float4(cr, cg, cb, log_t));
+        if constexpr (CK) store_shared(split.stop + (px0 + (uint64_t)seg * (TS * TS)), stop);
+    }
+    {
+        float d = active ? log_t : -3.0e38f;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) d = fmaxf(d, __shfl_xor(d, o, 64));
+        __syncthreads();  // s_red's readers at the start are done
+        if ((tid & 63) == 0) s_red[tid >> 6] = d;
+        drain_stores();  // this wave's states and checkpoints
+        __syncthreads();
+        if (tid == 0) {
+            for (int w = 1; w < NT / 64; ++w) d = fmaxf(d, s_red[w]);
+            store_shared(split.dark + slot + seg, d);
+            drain_stores();
+            s_arrived = (int)atomicAdd(split.arrived + gtile, 1u);
+            s_first = (int)n_seg;
+        }
+        __syncthreads();
+        if (s_arrived != (int)n_seg - 1) return;
+    }
+    // Front to back: each segment as seen from the camera.  sat: the segment in
+    // which the pixel saturates.
+    float lt = 0.0f;
+    int sat = (int)n_seg;
+    cr = cg = cb = 0.0f;
+    stop = 0u;
+    if (active) {
+        constexpr int U = 4;
+        for (uint32_t g0 = 0; g0 < n_seg; g0 += U) {
+            float4 q[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) q[u] = load_shared(split.px + (px0 + (uint64_t)min(g0 + u, n_seg - 1u) * (TS * TS)));
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint32_t g = g0 + u;
+                if (g >= n_seg || (int)g > sat) continue;
+                const float w = expf(lt);
+                lt += q[u].w;
+                q[u] = make_float4(q[u].x * w, q[u].y * w, q[u].z * w, lt);
+                cr += q[u].x;
+                cg += q[u].y;
+                cb += q[u].z;
+                if constexpr (CK) stop = max(stop, load_shared(split.stop + (px0 + (uint64_t)g * (TS * TS))));
+                split.px[px0 + (uint64_t)g * (TS * TS)] = q[u];
+                if (lt < -13.8f) sat = (int)g;
+            }
+        }
+    }
+    log_t = lt;
+    // the plan's counters are zero between forwards
+    for (uint32_t g = tid; g < n_seg; g += NT) split.dark[slot + g] = 0.0f;
+    if (tid == 0) split.arrived[gtile] = 0u;
+    const bool any = __syncthreads_or(active && sat < (int)n_seg);
+    if (tid == 0) split.serial[gtile] = any ? 1u : 0u;
+    if (!any) {
+        // Back to front: what lies behind each segment, for the adjoint.
+        if (active) {
+            constexpr int U = 4;
+            float br = 0.f, bg = 0.f, bb = 0.f;
+            for (int g0 = (int)n_seg - 1; g0 >= 0; g0 -= U) {
+                float4 q[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) q[u] = split.px[px0 + (uint64_t)max(g0 - u, 0) * (TS * TS)];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (g0 - u < 0) continue;
+                    split.px[px0 + (uint64_t)(g0 - u) * (TS * TS)] = make_float4(br, bg, bb, q[u].w);
+                    br += q[u].x;
+                    bg += q[u].y;
+                    bb += q[u].z;
+                }
+            }
+        }
+        break;
+    }
+    // Some pixel saturates.  A pixel that does so in the first segment is done; the
+    // others that do are composited again from the first segment with such a pixel
+    // on, so that each stops behind the pair that saturates it; the rest are done.
+    // The adjoint takes this tile's list as one.
+    if constexpr (CK) {  // checkpoints as seen from the camera
+        if (active) {
+            uint32_t g = 0;
+            float base = 0.0f;
+            for (uint32_t c = kCkGroup; c < count; c += kCkGroup) {
+                while (c > (g + 1u) * seg_len) base = split.px[px0 + (uint64_t)g++ * (TS * TS)].w;
+                if ((int)g > sat) break;
+                float* const p = ck + (ck_base + (uint64_t)(c / kCkGroup) * (TS * TS));
+                if (g > 0u) store_shared(p, load_shared(p) + base);
+            }
+        }
+    }
+    run = active && sat > 0 && sat < (int)n_seg;
+    if (run) atomicMin(&s_first, sat);
+    __syncthreads();
+    const int first = s_first;
+    if (first == (int)n_seg) break;  // all of them in the first segment
+    if (run) {
+        cr = cg = cb = 0.0f;
+        stop = 0u;
+        for (int g = 0; g < first; ++g) {
+            const float4 q = split.px[px0 + (uint64_t)g * (TS * TS)];
+            cr += q.x;
+            cg += q.y;
+            cb += q.z;
+            log_t = q.w;
+            if constexpr (CK) stop = max(stop, load_shared(split.stop + (px0 + (uint64_t)g * (TS * TS))));
+        }
+    }
+    if (tid < TS * TS) s_ray[tid].w = run ? 1.0f : 0.0f;
+    done = (uint32_t)first * seg_len;
+    next_ck = done + kCkGroup;
+    end = ranges[2ull * gtile + 1] - ranges[2ull * gtile];
+    whole = true;
     }
     if (active) {
         const uint64_t pix = vw.pix_base + (uint64_t)py * vw.width + px;
@@ -1140,7 +1328,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     const float4* __restrict__ rec, const float4* __restrict__ colors,
     const uint32_t* __restrict__ sorted_vals, const uint32_t* __restrict__ ranges,
     const ViewParams* __restrict__ views, const uint32_t* __restrict__ tile_view, const uint32_t* __restrict__ tile_order,
-    const float* __restrict__ rgba, const float* __restrict__ dl_img, const float* __restrict__ gt, uint32_t loss_type,
+    const SplitPlan split, const float* __restrict__ rgba, const float* __restrict__ dl_img, const float* __restrict__ gt, uint32_t loss_type,
     float* __restrict__ loss_partial, float* __restrict__ tet_g, float* __restrict__ d_colors,
     const float* __restrict__ ck, const float2* __restrict__ fin, uint64_t* __restrict__ scene_done) {
     constexpr int TS = C::TS, NT = C::NT, B = C::B, CAP = C::CAP, SP = TS + 1, NW = NT / 64, NREC = C::NREC;
@@ -1169,11 +1357,21 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     constexpr int IDW = (2 * B + NT - 1) / NT;
     __shared__ uint32_t s_ids[2 * B];
     __shared__ float s_loss[NW];
+    __shared__ float s_front[CK ? TS * TS : 1];  // CK: log T in front of the segment, which its checkpoints start from
     static_assert(B <= 64, "pixel masks hold 64 tets");
     static_assert(CAP / 32 <= NT && TS <= 32, "segment table");
     static_assert(CAP >= TS * TS, "one tet's pixels of a tile must fit a batch");
 
+    if (split.seg && blockIdx.x >= *split.n_items) return;
     const uint32_t gtile = tile_order ? tile_order[blockIdx.x] : blockIdx.x;
+    const uint32_t seg = split.seg ? split.seg[blockIdx.x] : 0u;
+    const uint32_t rs = ranges[2ull * gtile], re = ranges[2ull * gtile + 1];
+    const uint32_t count = re > rs ? re - rs : 0u;
+    // a list whose segment states the forward left is taken by segments too
+    const bool by_seg = split.px && split_segments(count, split.unit) > 1u && split.serial[gtile] == 0u;
+    if (!by_seg && seg > 0u) return;
+    const uint32_t seg_len = by_seg ? split_length(count, split.unit) : count;
+    const uint32_t slot = by_seg ? split.slot[gtile] + seg : 0u;
     const uint32_t view = tile_view[gtile];
     const ViewParams& vw = views[view];
     const TileCtx tc = tile_ctx(vw, gtile);
@@ -1227,6 +1425,12 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                 dcv[2] = d.z;
                 d_log_t = -d.w * (CK ? safe_exp(fin_lt) : 1.0f - im.w);
             }
+            if (CK) s_front[tid] = by_seg && seg > 0u ? split.px[(uint64_t)(slot - 1u) * (TS * TS) + (uint64_t)tid].w : 0.0f;
+            if (by_seg) {  // what lies behind the segment
+                const float4 q = split.px[(uint64_t)slot * (TS * TS) + (uint64_t)tid];
+                log_t = q.w;
+                d_log_t = safe_clip(d_log_t + (dcv[0] * q.x + dcv[1] * q.y + dcv[2] * q.z), kMinVal, kMaxVal);
+            }
         }
         s_ray[tid] = make_float4(rd.x, rd.y, rd.z, dcv[0]);
         s_dc[tid] = make_float2(dcv[1], dcv[2]);
@@ -1235,17 +1439,17 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         float ws = wave_sum(lsum);
         if (lane == 0) s_loss[wid] = ws;
         __syncthreads();
-        if (tid == 0) {
+        if (tid == 0 && seg == 0u) {
             float s = 0.f;
             for (int w = 0; w < NW; ++w) s += s_loss[w];
             loss_partial[gtile] = s;
         }
     }
 
-    const uint32_t rs = ranges[2ull * gtile], re = ranges[2ull * gtile + 1];
-    const uint32_t count = re > rs ? re - rs : 0u;
-    uint32_t done = 0;
-    int nb = (int)min<uint32_t>(B, count);
+    // list positions from the back, [done, end) here
+    const uint32_t end = count - seg * seg_len;
+    uint32_t done = by_seg ? count - min(seg * seg_len + seg_len, count) : 0u;
+    int nb = (int)min<uint32_t>(B, end - done);
     // CK: slot of checkpoint j + 1 (the end of group j) is ck_base + j
     const uint64_t ck_base = ((uint64_t)(rs >> 5) + gtile) * (uint64_t)(TS * TS) + (uint64_t)tid;
     int32_t cur = -1;  // CK: group the pixel's undo is in
@@ -1257,7 +1461,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     auto load_ids = [&](uint32_t* idw, uint32_t d) {  // list positions d .. d + 2 B - 1 (past the end: the last)
 #pragma unroll
         for (int u = 0; u < IDW; ++u)
-            idw[u] = sorted_vals[rs + min(d + (uint32_t)(u * NT + opaque(threadIdx.x)), count - 1u)];
+            idw[u] = sorted_vals[rs + min(d + (uint32_t)(u * NT + opaque(threadIdx.x)), end - 1u)];
     };
     auto stage = [&](const TetFetch& f, const QuadFetch& qf, const uint32_t* idw, int n) {
         if constexpr (C::PF == 3) store_quad<TS, B, true>(L, qf, tid >> 2, tid & 3, tid < 4 * n, vw, tc);
@@ -1309,11 +1513,11 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         TetFetch f;
         QuadFetch qf;
         uint32_t idw[IDW];
-        fetch(f, qf, sorted_vals + rs, nb);
-        load_ids(idw, 0u);
+        fetch(f, qf, sorted_vals + rs + done, nb);
+        load_ids(idw, done);
         stage(f, qf, idw, nb);
     }
-    while (done < count) {
+    while (done < end) {
         const int tid = opaque(threadIdx.x);
         __syncthreads();
         batch_layout<TS, B, true, false, CAP, NT>(L, nb, G.seg, G.starts());
@@ -1321,7 +1525,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         const uint32_t nbp = L.nbp & 0xFFu;
         const uint32_t nrec = L.nbp >> 8;
         const uint32_t next = done + nbp;
-        const int nb_next = next_batch<B>(nbp, nb, count - next);
+        const int nb_next = next_batch<B>(nbp, nb, end - next);
         // CK: log T at the end of the (at most two) groups this batch spans,
         // positions [count - next, count - 1 - done] in compositing order
         float ck_hi = 0.f, ck_lo = 0.f;
@@ -1329,8 +1533,8 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         if (CK && active) {
             j_hi = (int32_t)((count - 1u - done) / kCkGroup);
             const int32_t j_lo = (int32_t)((count - next) / kCkGroup);
-            ck_hi = (uint32_t)(j_hi + 1) * kCkGroup < stop ? ck[ck_base + (uint64_t)j_hi * (TS * TS)] : fin_lt;
-            ck_lo = (uint32_t)(j_lo + 1) * kCkGroup < stop ? ck[ck_base + (uint64_t)j_lo * (TS * TS)] : fin_lt;
+            ck_hi = (uint32_t)(j_hi + 1) * kCkGroup < stop ? ck[ck_base + (uint64_t)j_hi * (TS * TS)] + s_front[tid] : fin_lt;
+            ck_lo = (uint32_t)(j_lo + 1) * kCkGroup < stop ? ck[ck_base + (uint64_t)j_lo * (TS * TS)] + s_front[tid] : fin_lt;
         }
         // loaded for the end of this iteration (as in the forward)
         TetFetch f;
@@ -1467,30 +1671,47 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
 // ---------------------------------------------------------------------------
 template <class C>
 static void fwd_launch(const FwdArgs& a, hipStream_t s) {
+    const dim3 grid(a.split.seg ? a.split.grid : a.num_gtiles);
     if (a.aux)  // the aux outputs serve the forward-only API: no checkpoints with them
-        hipLaunchKernelGGL((k_forward<C, true, false>), dim3(a.num_gtiles), dim3(C::NT), 0, s, a.rec, a.colors,
-                           a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order,
+        hipLaunchKernelGGL((k_forward<C, true, false>), grid, dim3(C::NT), 0, s, a.rec, a.colors,
+                           a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order, a.split,
                            a.rgba, a.aux, nullptr, nullptr);
     else if (a.ck)
-        hipLaunchKernelGGL((k_forward<C, false, true>), dim3(a.num_gtiles), dim3(C::NT), 0, s, a.rec, a.colors,
-                           a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order,
+        hipLaunchKernelGGL((k_forward<C, false, true>), grid, dim3(C::NT), 0, s, a.rec, a.colors,
+                           a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order, a.split,
                            a.rgba, nullptr, a.ck, a.fin);
     else
-        hipLaunchKernelGGL((k_forward<C, false, false>), dim3(a.num_gtiles), dim3(C::NT), 0, s, a.rec, a.colors,
-                           a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order,
+        hipLaunchKernelGGL((k_forward<C, false, false>), grid, dim3(C::NT), 0, s, a.rec, a.colors,
+                           a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order, a.split,
                            a.rgba, nullptr, nullptr, nullptr);
 }
 
+// Forward geometries.  The defaults measured best over a batch of small views,
+// a full-HD scene and config C: tile 12 B 32, CAP 1152 (six records a lane; 8
+// views of a 10,000-point scene 0.89 ms, B 48 with CAP 768 1.03, CAP 1344 0.98),
+// tile 16 B 64, CAP 1024 at four waves per SIMD (config C 5.30 ms, B 56 with CAP
+// 768 at five 5.42, B 48 with CAP 1024 5.74; two full-HD views 1.38 ms in all
+// for 1.50 with B 48, CAP 768).
 template <int TS>
 static bool fwd_variant(const FwdArgs& a, int v, hipStream_t s) {
     switch (v) {
-        case 0: fwd_launch<FwdCfg<TS, 48, 768, 3>>(a, s); return true;
+        case 0:
+            if constexpr (TS == 12) fwd_launch<FwdCfg<TS, 32, 1152, 3>>(a, s);
+            else if constexpr (TS == 16) fwd_launch<FwdCfg<TS, 64, 1024, 3, 4>>(a, s);
+            else fwd_launch<FwdCfg<TS, 48, 768, 3>>(a, s);
+            return true;
         case 1: fwd_launch<FwdCfg<TS, 48, 704, 3, 5>>(a, s); return true;
         case 2: fwd_launch<FwdCfg<TS, 32, 704, 3, 5>>(a, s); return true;
-        case 3: fwd_launch<FwdCfg<TS, 64, 1024, 3>>(a, s); return true;
+        case 3:
+            if constexpr (TS == 8) fwd_launch<FwdCfg<TS, 64, 1024, 3>>(a, s);
+            else fwd_launch<FwdCfg<TS, 48, 768, 3>>(a, s);
+            return true;
         case 4: fwd_launch<FwdCfg<TS, 64, 768, 3, 5>>(a, s); return true;
         case 5: fwd_launch<FwdCfg<TS, 56, 896, 3>>(a, s); return true;
-        case 6: fwd_launch<FwdCfg<TS, 56, 768, 3, 5>>(a, s); return true;
+        case 6:
+            if constexpr (TS == 16) fwd_launch<FwdCfg<TS, 64, 1024, 3, 4>>(a, s);
+            else fwd_launch<FwdCfg<TS, 56, 768, 3, 5>>(a, s);
+            return true;
         case 7: fwd_launch<FwdCfg<TS, 64, 896, 3>>(a, s); return true;
         default: return false;
     }
@@ -1518,28 +1739,30 @@ bool launch_forward(const FwdArgs& a, uint32_t tile_size, int variant, hipStream
 
 template <class C>
 static void bwd_launch(const BwdArgs& a, hipStream_t s) {
+    const dim3 grid(a.split.seg ? a.split.grid : a.num_gtiles);
     if (a.ck) {
         if constexpr (C::B > 32) {
             // the checkpointed adjoint's batches span at most two checkpoint groups (B <= 32)
             bwd_launch<BwdCfg<C::TS, 32, C::CAP, C::PF_ARG, C::WPE_ARG>>(a, s);
         } else {
-            hipLaunchKernelGGL((k_backward<C, true>), dim3(a.num_gtiles), dim3(C::NT), 0, s, a.rec, a.colors,
-                               a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order,
+            hipLaunchKernelGGL((k_backward<C, true>), grid, dim3(C::NT), 0, s, a.rec, a.colors,
+                               a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order, a.split,
                                a.rgba, a.dl_img, a.gt, a.loss_type, a.loss_partial, a.tet_g, a.d_colors, a.ck, a.fin,
                                a.scene_done);
         }
     } else
-        hipLaunchKernelGGL((k_backward<C, false>), dim3(a.num_gtiles), dim3(C::NT), 0, s, a.rec, a.colors,
-                           a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order,
+        hipLaunchKernelGGL((k_backward<C, false>), grid, dim3(C::NT), 0, s, a.rec, a.colors,
+                           a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order, a.split,
                            a.rgba, a.dl_img, a.gt, a.loss_type, a.loss_partial, a.tet_g, a.d_colors, nullptr,
                            nullptr, a.scene_done);
 }
 
 // Adjoint geometries, by tets B and records per lane N (CAP = N NT) of a batch at
 // 4 waves per SIMD (128 VGPRs): with a pair's state kept in registers from
-// phase A to phase C the record capacity costs 8 bytes of LDS a record, and
-// three records a lane measured best at tiles 12 and 16 (config C, tile 16, B
-// 48: N 2 13.25 ms, N 3 12.31 ms; B 64 leaves 3 workgroups per CU: 13.9 ms).
+// phase A to phase C the record capacity costs 8 bytes of LDS a record.  Measured
+// best: tile 16 B 48, N 3 (config C 11.9 ms; B 32 12.6, B 32 with N 4 12.6, B 44
+// 12.2; B 64 leaves 3 workgroups per CU: 13.9), tile 12 B 32, N 5 (8 views of a
+// 10,000-point scene 2.23 ms; N 3 2.43, N 4 2.30, N 6 2.36, B 48 with N 3 2.49).
 // One-wave workgroups (tile 8) take half the tets and one record a lane more.
 template <int TS, int B, int N>
 using BwdGeo = BwdCfg<TS, (TS == 8 ? B / 2 : B), (TS == 8 ? N + 1 : N) * ((TS * TS + 63) / 64 * 64), 3, 4>;
@@ -1547,12 +1770,18 @@ template <int TS>
 static bool bwd_variant(const BwdArgs& a, int v, hipStream_t s) {
     switch (v) {
         case 0:
-        case 10: bwd_launch<BwdGeo<TS, 48, 3>>(a, s); return true;
+        case 10:
+            if constexpr (TS == 12) bwd_launch<BwdGeo<TS, 32, 5>>(a, s);
+            else bwd_launch<BwdGeo<TS, 48, 3>>(a, s);
+            return true;
         case 1: bwd_launch<BwdGeo<TS, 32, 3>>(a, s); return true;
         case 2: bwd_launch<BwdGeo<TS, 32, 2>>(a, s); return true;
         case 3: bwd_launch<BwdGeo<TS, 48, 2>>(a, s); return true;
         case 4: bwd_launch<BwdGeo<TS, 24, 3>>(a, s); return true;
-        case 5: bwd_launch<BwdGeo<TS, 64, 3>>(a, s); return true;
+        case 5:
+            if constexpr (TS == 12) bwd_launch<BwdGeo<TS, 48, 3>>(a, s);
+            else bwd_launch<BwdGeo<TS, 64, 3>>(a, s);
+            return true;
         case 6: bwd_launch<BwdGeo<TS, 40, 3>>(a, s); return true;
         case 7: bwd_launch<BwdGeo<TS, 56, 3>>(a, s); return true;
         case 8: bwd_launch<BwdGeo<TS, 64, 2>>(a, s); return true;

@@ -138,7 +138,14 @@ struct rmesh_renderer {
     uint32_t *ihist = nullptr, *d_nitems = nullptr, *block_sums2 = nullptr;
     bool pairs_depth_ordered = false;  // the last pair generation emitted items in depth order
     uint32_t* ranges = nullptr;
-    uint32_t* tile_order = nullptr;  // compositing workgroup -> global tile, heaviest first
+    uint32_t* tile_order = nullptr;  // compositing work item -> global tile, heaviest first
+    // segments of long tile lists (SplitPlan); px also per tet-sorted pair capacity
+    uint32_t *seg = nullptr, *n_seg_items = nullptr, *seg_slot = nullptr, *seg_arrived = nullptr, *seg_serial = nullptr;
+    float* seg_dark = nullptr;
+    float4* seg_px = nullptr;
+    uint32_t* seg_stop = nullptr;
+    bool order_split = false;        // tile_order holds (tile, segment) items
+    bool have_segs = false;          // the last forward left segment states for these tile lists
     bool sorted_in_b = false;
     // adjoint mode: false = the reference's undo from the image alpha, true =
     // the checkpointed adjoint (transmittance checkpoints stored by the forward)
@@ -345,8 +352,15 @@ void set_tiles(rmesh_renderer* h, uint32_t ts) {
     drop_graph(h);
 }
 
+// Pixel records of the segment slots for P pairs, at the tile size that needs most.
+uint64_t segment_pixels(uint64_t P) {
+    uint64_t n = 0;
+    for (uint32_t ts : {8u, 12u, 16u, 32u}) n = std::max<uint64_t>(n, split_slots(P, split_unit(ts)) * ts * ts);
+    return n;
+}
+
 rmesh_status ensure_capacity(rmesh_renderer* h, uint64_t need) {
-    if (need <= h->cap && h->keys_a && h->hist) return RMESH_OK;
+    if (need <= h->cap && h->keys_a && h->hist && h->seg_px) return RMESH_OK;
     if (need > 0xFFFFFFF0ull) return fail(RMESH_ERR_CAPACITY, "tile-tet pair count exceeds 2^32");
     uint64_t c = std::max<uint64_t>(need + need / 4 + (1u << 16), 1u << 20);
     if (c > 0xFFFFFFF0ull) c = 0xFFFFFFF0ull;
@@ -356,15 +370,28 @@ rmesh_status ensure_capacity(rmesh_renderer* h, uint64_t need) {
     (void)hipFree(h->vals_a);
     (void)hipFree(h->vals_b);
     (void)hipFree(h->hist);
+    (void)hipFree(h->tile_order);
+    (void)hipFree(h->seg);
+    (void)hipFree(h->seg_dark);
+    (void)hipFree(h->seg_px);
+    (void)hipFree(h->seg_stop);
     h->keys_a = h->keys_b = nullptr;
     h->vals_a = h->vals_b = nullptr;
     h->hist = nullptr;
+    h->tile_order = h->seg = h->seg_stop = nullptr;
+    h->seg_dark = nullptr;
+    h->seg_px = nullptr;
     h->cap = 0;
     HIP_TRY(dalloc(&h->keys_a, c));
     HIP_TRY(dalloc(&h->keys_b, c));
     HIP_TRY(dalloc(&h->vals_a, c));
     HIP_TRY(dalloc(&h->vals_b, c));
     HIP_TRY(dalloc(&h->hist, std::max(radix_hist_words((uint32_t)c), radix_hist_words32((uint32_t)c))));
+    // work items and segment slots of any tile size (most at the smallest)
+    HIP_TRY(dalloc(&h->tile_order, h->tile_cap + split_extra_items(c, split_unit(8))));
+    HIP_TRY(dalloc(&h->seg, h->tile_cap + split_extra_items(c, split_unit(8))));
+    HIP_TRY(dalloc(&h->seg_dark, split_slots(c, split_unit(8))));
+    HIP_TRY(dalloc(&h->seg_px, segment_pixels(c)));
     h->cap = (uint32_t)c;
     drop_graph(h);
     return RMESH_OK;
@@ -383,6 +410,10 @@ rmesh_status ensure_checkpoints(rmesh_renderer* h, uint32_t V) {
         const uint64_t c = need + need / 8;
         HIP_TRY(dalloc(&h->ck, c));
         h->ck_floats = c;
+        drop_graph(h);
+    }
+    if (!h->seg_stop) {
+        HIP_TRY(dalloc(&h->seg_stop, segment_pixels(h->cap)));
         drop_graph(h);
     }
     if (!h->fin) HIP_TRY(dalloc(&h->fin, (size_t)h->pix_cap));
@@ -459,22 +490,42 @@ void launch_sort_stage(rmesh_renderer* h, hipStream_t s) {
         h->sorted_in_b = launch_radix_sort(h->keys_a, h->vals_a, h->keys_b, h->vals_b, h->n_pairs, h->cap,
                                            h->sorting_bits(0), h->hist, s, h->sort_db);
 }
-void launch_ranges_stage(rmesh_renderer* h, hipStream_t s) {
+// The segment plan of the current tile size, for the order kernel and the forward.
+SplitPlan split_plan(const rmesh_renderer* h) {
+    SplitPlan p;
+    p.unit = split_unit(h->TS);
+    p.seg = h->seg;
+    p.n_items = h->n_seg_items;
+    p.slot = h->seg_slot;
+    p.arrived = h->seg_arrived;
+    p.serial = h->seg_serial;
+    p.dark = h->seg_dark;
+    p.px = h->seg_px;
+    p.stop = h->seg_stop;
+    p.grid = h->n_gt + (uint32_t)split_extra_items(h->cap, p.unit);
+    return p;
+}
+// split: long lists as several work items (the plain forward and the adjoint);
+// the aux, error and interval kernels take whole tiles.
+void launch_ranges_stage(rmesh_renderer* h, bool split, hipStream_t s) {
+    const SplitPlan sp = split ? split_plan(h) : SplitPlan();
+    h->order_split = split;
+    h->have_segs = false;
     launch_fill_u32(h->ranges, 0u, 2ull * h->n_gt, s);
     uint64_t* sk = h->sorted_in_b ? h->keys_b : h->keys_a;
     if (h->pairs_depth_ordered) launch_ranges32(keys32(sk), h->n_pairs, h->cap, h->ranges, h->d_ktile, h->n_kt, s);
     else launch_ranges(sk, h->n_pairs, h->cap, h->ranges, h->d_ktile, h->n_kt, s);
     if (h->scene_order != RMESH_SCENE_ORDER_BY_SCENE ||
         !launch_tile_order_scenes(h->ranges, h->n_gt, h->d_tile_view, h->d_views, (uint32_t)h->sc.size(),
-                                  h->tile_order, s))
-        launch_tile_order(h->ranges, h->n_gt, h->tile_order, s);
+                                  h->tile_order, sp, s))
+        launch_tile_order(h->ranges, h->n_gt, h->tile_order, sp, s);
 }
 
-rmesh_status stage_binning_back(rmesh_renderer* h, uint32_t V) {
+rmesh_status stage_binning_back(rmesh_renderer* h, uint32_t V, bool split) {
     hipStream_t s = h->stream;
     launch_pair_gen(h, s);
     launch_sort_stage(h, s);
-    launch_ranges_stage(h, s);
+    launch_ranges_stage(h, split, s);
     return RMESH_OK;
 }
 
@@ -491,6 +542,7 @@ rmesh_status stage_forward(rmesh_renderer* h, uint32_t V, bool want_aux) {
     a.tile_view = h->d_tile_view;
     a.num_gtiles = h->n_gt;
     a.tile_order = h->tile_order;
+    if (h->order_split) a.split = split_plan(h);
     a.rgba = h->rgba;
     a.aux = want_aux ? h->aux : nullptr;
     const bool ck = h->adj_ck && !want_aux;  // the aux forward keeps no checkpoints
@@ -498,6 +550,9 @@ rmesh_status stage_forward(rmesh_renderer* h, uint32_t V, bool want_aux) {
     a.fin = ck ? h->fin : nullptr;
     if (!launch_forward(a, h->TS, h->fwd_var, h->stream)) return fail(RMESH_ERR_INVALID, "unsupported tile size");
     h->have_ck = ck;
+    // A near limit cuts the forward's slabs and not the adjoint's, whose undo runs
+    // from the image alpha alone: its list stays one chain then.
+    h->have_segs = h->order_split && (h->min_t == 0.0f || ck);
     return RMESH_OK;
 }
 
@@ -513,7 +568,6 @@ void zero_grads(rmesh_renderer* h, uint32_t V) {
 rmesh_status stage_backward(rmesh_renderer* h, uint32_t V, const float* dl, const float* gt, uint32_t loss_type) {
     BwdArgs a;
     a.rec = h->rec;
-    a.idx = h->idx;
     a.colors = h->colors;
     a.sorted_vals = sorted_vals(h);
     a.ranges = h->ranges;
@@ -521,6 +575,10 @@ rmesh_status stage_backward(rmesh_renderer* h, uint32_t V, const float* dl, cons
     a.tile_view = h->d_tile_view;
     a.num_gtiles = h->n_gt;
     a.tile_order = h->tile_order;
+    if (h->order_split) {
+        a.split = split_plan(h);
+        if (!h->have_segs) a.split.px = nullptr;
+    }
     a.rgba = h->rgba;
     a.dl_img = dl;
     a.gt = gt;
@@ -650,7 +708,7 @@ rmesh_status record_stage(rmesh_renderer* h, int stage, uint32_t V, const float*
             launch_sort_stage(h, s);
             return RMESH_OK;
         case 3:
-            launch_ranges_stage(h, s);
+            launch_ranges_stage(h, true, s);
             return RMESH_OK;
         case 4: return stage_forward(h, V, false);
         case 5: return stage_backward(h, V, nullptr, gt, loss_type);
@@ -681,7 +739,8 @@ void free_all(rmesh_renderer* h) {
                     h->ivl_ddist, h->ivl_dgrad, h->ivl_dvn, h->ivl_tv, h->v2t_off, h->v2t, h->ck, h->fin,
                     h->d_scenes, h->d_tile_view, h->d_ktile, h->scene_clock, h->tet_g, h->dkey_a, h->dkey_b,
                     h->ditem_a, h->ditem_b, h->ihist, h->d_nitems, h->block_sums2, h->block_vis, h->spine_part,
-                    h->spine_aux};
+                    h->spine_aux, h->seg, h->n_seg_items, h->seg_slot, h->seg_arrived, h->seg_serial, h->seg_dark,
+                    h->seg_px, h->seg_stop};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (hipEvent_t e : h->ev)
@@ -876,7 +935,10 @@ static rmesh_status create_impl(const rmesh_scene_desc* descs, uint32_t n_scenes
     CREATE_TRY(dalloc(&h->d_step, 1));
     CREATE_TRY(hipMemset(h->d_step, 0, 4));
     CREATE_TRY(dalloc(&h->ranges, 2ull * h->tile_cap));
-    CREATE_TRY(dalloc(&h->tile_order, (size_t)h->tile_cap));
+    CREATE_TRY(dalloc(&h->n_seg_items, 1));
+    CREATE_TRY(dalloc(&h->seg_slot, (size_t)h->tile_cap));
+    CREATE_TRY(dalloc(&h->seg_arrived, (size_t)h->tile_cap));
+    CREATE_TRY(dalloc(&h->seg_serial, (size_t)h->tile_cap));
     CREATE_TRY(dalloc(&h->rgba, 4 * h->pix_cap));
     CREATE_TRY(dalloc(&h->dl, 4ull * h->W * h->H));
     CREATE_TRY(dalloc(&h->gt, 3 * h->pix_cap));
@@ -905,6 +967,7 @@ extern "C" void rmesh_destroy(rmesh_renderer* h) {
 
 extern "C" rmesh_status rmesh_set_min_t(rmesh_renderer* h, float min_t) {
     if (!h) return fail(RMESH_ERR_INVALID, "null handle");
+    if ((min_t != 0.0f) != (h->min_t != 0.0f)) drop_graph(h);  // the captured adjoint depends on it
     h->min_t = min_t;
     return RMESH_OK;
 }
@@ -926,7 +989,7 @@ static rmesh_status forward_views(rmesh_renderer* h, uint32_t V, const float* ca
     if (st != RMESH_OK) return st;
     st = stage_binning_front(h, V, false);
     if (st != RMESH_OK) return st;
-    st = stage_binning_back(h, V);
+    st = stage_binning_back(h, V, !want_aux);
     if (st != RMESH_OK) return st;
     if (want_aux && !h->aux_alloc) {
         HIP_TRY(dalloc(&h->aux, 8ull * h->W * h->H * h->max_views));
@@ -1012,7 +1075,7 @@ extern "C" rmesh_status rmesh_forward_interval_tiled(rmesh_renderer* h, const fl
     if (st != RMESH_OK) return st;
     st = stage_binning_front(h, 1, false);
     if (st != RMESH_OK) return st;
-    st = stage_binning_back(h, 1);
+    st = stage_binning_back(h, 1, false);
     if (st != RMESH_OK) return st;
     IvlArgs a;
     a.rec = h->rec;
@@ -1255,8 +1318,10 @@ extern "C" rmesh_status rmesh_set_adjoint_mode(rmesh_renderer* h, int32_t mode) 
             HIP_TRY(hipStreamSynchronize(h->stream));
             (void)hipFree(h->ck);
             (void)hipFree(h->fin);
+            (void)hipFree(h->seg_stop);
             h->ck = nullptr;
             h->fin = nullptr;
+            h->seg_stop = nullptr;
             h->ck_floats = 0;
         }
     }
@@ -1280,7 +1345,8 @@ extern "C" rmesh_status rmesh_device_bytes(rmesh_renderer* h, uint64_t* out) {
                           h->ivl_xyzd, h->ivl_dist, h->ivl_dxyzd, h->ivl_ddist, h->ivl_dgrad, h->ivl_dvn,
                           h->ivl_tv, h->v2t_off, h->v2t, h->ck, h->fin, h->d_scenes, h->d_tile_view, h->d_ktile,
                           h->tet_g, h->dkey_a, h->dkey_b, h->ditem_a, h->ditem_b, h->ihist, h->d_nitems,
-                          h->block_sums2, h->block_vis, h->spine_part, h->spine_aux};
+                          h->block_sums2, h->block_vis, h->spine_part, h->spine_aux, h->seg, h->n_seg_items,
+                          h->seg_slot, h->seg_arrived, h->seg_serial, h->seg_dark, h->seg_px, h->seg_stop};
     uint64_t total = 0;
     for (const void* p : ptrs) {
         if (!p) continue;
@@ -1443,7 +1509,7 @@ static rmesh_status autotune_layout(rmesh_renderer* h, const uint32_t* per_user,
             result = timed([&]() {
                 rmesh_status s2 = stage_binning_front(h, V, true);
                 if (s2 != RMESH_OK) return s2;
-                return stage_binning_back(h, V);
+                return stage_binning_back(h, V, true);
             }, t);
             if (result != RMESH_OK) break;
             if (t < t_bin) {
@@ -1453,7 +1519,7 @@ static rmesh_status autotune_layout(rmesh_renderer* h, const uint32_t* per_user,
         }
         if (result != RMESH_OK) break;
         h->sort_db = bdb;
-        if ((result = stage_binning_back(h, V)) != RMESH_OK) break;  // lists of the chosen width
+        if ((result = stage_binning_back(h, V, true)) != RMESH_OK) break;  // lists of the chosen width
         for (int f = 0; f < fwd_variants(ts) && result == RMESH_OK; ++f) {
             h->fwd_var = f;
             float t = 0.0f;
@@ -1631,7 +1697,7 @@ extern "C" rmesh_status rmesh_forward_multi(rmesh_renderer* h, const uint32_t* v
     if (st != RMESH_OK) return st;
     const uint32_t V = h->n_views;
     if ((st = stage_binning_front(h, V, false)) != RMESH_OK) return st;
-    if ((st = stage_binning_back(h, V)) != RMESH_OK) return st;
+    if ((st = stage_binning_back(h, V, true)) != RMESH_OK) return st;
     if ((st = stage_forward(h, V, false)) != RMESH_OK) return st;
     h->last_views = V;
     h->have_forward = !h->multi();

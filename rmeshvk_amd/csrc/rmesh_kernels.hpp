@@ -9,6 +9,49 @@ namespace rmesh {
 
 struct ViewParams;
 
+// Tile lists longer than a unit are composited by several workgroups, a segment
+// of at most `unit` pairs each (a rule of the list's own length, so a view's
+// image does not depend on what it is batched with).  Segments start at
+// multiples of 32 positions, as the transmittance checkpoints do.
+// The unit, 6 pairs per pixel: a tile's workgroup is a serial chain over its
+// list, and the chip holds some 1300 of them, so a list far above (all pairs) /
+// 1300 runs on after the rest of the grid is done (12 scenes, longest list 33,800
+// pairs at tile 16: forward 2.1 ms, adjoint 3.6 unsplit, 0.37 and 0.84 split; 4
+// clustered views, longest 16,300: 1.5 and 2.9, 0.34 and 0.79).  A segment costs a
+// pixel record (16 bytes a pixel written, read by the tile's last workgroup and
+// by the adjoint) and the start of a workgroup: where no list is long for the
+// grid (config C) 2 % at 6, 4 % at 4 and 1 % at 8 pairs a pixel, while 8 leaves
+// the clustered views 7 % slower than 6.
+constexpr uint32_t split_unit(uint32_t tile_size) { return 6u * tile_size * tile_size; }
+__host__ __device__ inline uint32_t split_length(uint32_t pairs, uint32_t unit) {
+    if (pairs <= unit) return pairs;
+    const uint32_t n = (pairs - 1u) / unit + 1u;
+    return ((pairs - 1u) / n + 1u + 31u) & ~31u;  // <= unit, a multiple of 32
+}
+__host__ __device__ inline uint32_t split_segments(uint32_t pairs, uint32_t unit) {
+    return pairs <= unit ? 1u : (pairs - 1u) / split_length(pairs, unit) + 1u;
+}
+// Bounds for P pairs: items beyond one per tile, and segment slots.  A tile of c >
+// unit pairs has at most (c - 1) / unit + 1 < 2 c / unit segments.
+inline uint64_t split_extra_items(uint64_t P, uint32_t unit) { return P / unit; }
+inline uint64_t split_slots(uint64_t P, uint32_t unit) { return 2u * (P / unit) + 2u; }
+
+struct SplitPlan {
+    uint32_t unit = 0;
+    uint32_t* seg = nullptr;      // [item] segment of the item's tile; null: one item per tile, no segments
+    uint32_t* n_items = nullptr;
+    uint32_t* slot = nullptr;     // [tile] first segment slot (tiles with more than one segment)
+    uint32_t* arrived = nullptr;  // [tile] segments composited
+    uint32_t* serial = nullptr;   // [tile] 1: a pixel saturated, the adjoint takes the list as one
+    float* dark = nullptr;        // [slot] the segment's largest log transmittance over the tile's pixels (0: not known)
+    // [slot][TS TS] the segment alone: premultiplied colour, log T; once the tile
+    // is complete: colour behind the segment, log T at its end, both seen from
+    // the camera.  Null in the adjoint: every list as one.
+    float4* px = nullptr;
+    uint32_t* stop = nullptr;     // [slot][TS TS] with checkpoints: stop position in the segment
+    uint32_t grid = 0;            // workgroups to launch: at least *n_items
+};
+
 // binning (k_binning.hip)
 void launch_prep_records(const float* verts, const uint32_t* idx, const float* dens, const float* grads, uint32_t M,
                          float4* rec, hipStream_t s);
@@ -51,12 +94,15 @@ void launch_ranges(const uint64_t* keys, const uint32_t* n_ptr, uint32_t cap, ui
                    const uint32_t* ktile_gtile, uint32_t n_ktiles, hipStream_t s);
 void launch_ranges32(const uint32_t* keys, const uint32_t* n_ptr, uint32_t cap, uint32_t* ranges,
                      const uint32_t* ktile_gtile, uint32_t n_ktiles, hipStream_t s);
-// Permutation of the global tiles, heaviest (most pairs) first.
-void launch_tile_order(const uint32_t* ranges, uint32_t n_tiles, uint32_t* order, hipStream_t s);
+// Work items (tile, segment) in launch order, heaviest first: order[item] the
+// global tile, sp.seg[item] its segment; without a plan (sp.seg null) a
+// permutation of the tiles.
+void launch_tile_order(const uint32_t* ranges, uint32_t n_tiles, uint32_t* order, const SplitPlan& sp, hipStream_t s);
 // Scene-major heaviest-first order (scenes by ascending pair count); false
 // (nothing launched) above 64 scenes.
 bool launch_tile_order_scenes(const uint32_t* ranges, uint32_t n_tiles, const uint32_t* tile_view,
-                              const ViewParams* views, uint32_t n_scenes, uint32_t* order, hipStream_t s);
+                              const ViewParams* views, uint32_t n_scenes, uint32_t* order, const SplitPlan& sp,
+                              hipStream_t s);
 // p[0..n) = 0, p[n] = the wall clock now (start of a step's per-scene timing)
 void launch_stamp_start(uint64_t* p, uint32_t n, hipStream_t s);
 
@@ -82,7 +128,8 @@ struct FwdArgs {
     const ViewParams* views;
     const uint32_t* tile_view;   // global tile -> view
     uint32_t num_gtiles;
-    const uint32_t* tile_order;  // nullable: workgroup -> global tile (identity when null)
+    const uint32_t* tile_order;  // nullable: work item -> global tile (identity when null)
+    SplitPlan split;             // the plan tile_order was made with
     float* rgba;
     float* aux;  // nullable: [V][H][W][8]
     // nullable: transmittance checkpoints for the checkpointed adjoint.
@@ -164,7 +211,6 @@ bool launch_interval_backward(const IvlBwdArgs& a, uint32_t tile_size, hipStream
 
 struct BwdArgs {
     const float4* rec;
-    const uint32_t* idx;
     const float4* colors;
     const uint32_t* sorted_vals;
     const uint32_t* ranges;
@@ -172,6 +218,7 @@ struct BwdArgs {
     const uint32_t* tile_view;
     uint32_t num_gtiles;
     const uint32_t* tile_order;  // nullable, as FwdArgs::tile_order
+    SplitPlan split;             // as FwdArgs::split, px null where the forward left no segment states
     const float* rgba;
     const float* dl_img;      // used when gt == nullptr
     const float* gt;          // [V][H][W][3] or nullptr
