@@ -815,7 +815,7 @@ __device__ __forceinline__ void place_items(uint32_t* off, uint32_t* n_slots, ui
     const uint32_t slot = atomicAdd(n_slots, n);
     sp.slot[t] = slot;
     sp.arrived[t] = 0u;
-    sp.serial[t] = 0u;
+    sp.merged[t] = 0u;
     for (uint32_t g = 0; g < n; ++g) {
         const uint32_t i = atomicAdd(&off[item_bucket(split_length(pairs, sp.unit), (int)g, sp)], 1u);
         order[i] = t;

@@ -687,11 +687,10 @@ __device__ __forceinline__ void drain_stores() { asm volatile("s_waitcnt vmcnt(0
 
 // A workgroup composites a tile's list, or one segment of a long one (SplitPlan)
 // as if it were the first.  The tile's last workgroup to finish joins the
-// segments, T and colour being a product and a sum along the list.  Where that
-// shows a pixel saturating (log T < -13.8, from where the serial pass composites
-// nothing), it runs the list again from the segment in which the first such
-// pixel does, for those pixels alone, and marks the tile for a serial adjoint
-// (the undo from the image alpha passes over the pairs behind the stop too).
+// segments, T and colour being a product and a sum along the list.  A pixel that
+// this shows to saturate (log T < -13.8, from where the serial pass composites
+// nothing) in a later segment than the first is composited again from that
+// segment's start, so that it stops behind the same pair as in a serial pass.
 //
 // CK: also store the transmittance checkpoints of the checkpointed adjoint:
 // a pixel still compositing writes its log T before every tile-list position
@@ -721,7 +720,8 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     constexpr int IDW = (2 * B + NT - 1) / NT;
     __shared__ uint32_t s_ids[2 * B];
     __shared__ float s_red[NT / 64];
-    __shared__ int s_arrived, s_first;
+    __shared__ int s_arrived, s_first, s_merge;
+    __shared__ uint32_t s_sat[AUX ? 1 : TS * TS];  // segment in which the pixel saturates
     __shared__ uint32_t s_plan[4];  // segment, segments, their length, the tile's first slot
     static_assert(CAP / 32 <= NT && TS <= 32, "segment table");
 
@@ -749,6 +749,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     const uint32_t count = re > rs ? re - rs : 0u;
     // list positions [done, end) of this workgroup
     uint32_t done = 0, end = count;
+    bool skipped = false;
     bool whole = AUX || !split.seg || split_segments(count, split.unit) == 1u;  // one workgroup, one list
     if (!whole) {
         const uint32_t seg = split.seg[blockIdx.x], seg_len = split_length(count, split.unit);
@@ -773,11 +774,14 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         d = 0.0f;
 #pragma unroll
         for (int w = 0; w < NT / 64; ++w) d += s_red[w];
-        if (d < -13.9f) done = end;
+        skipped = d < -13.9f;
+        if (skipped) done = end;
     }
     // checkpoints: next position to store, stop position, slot base
     uint32_t next_ck = done + kCkGroup, stop = 0u;
-    bool run = active;  // the pixel composites in the loop below
+    bool run = active;     // the pixel composites in the loop below
+    bool joined = false;   // the pixel states are the tile's, in front of segment `again` for pixels still to run
+    uint32_t again = 0u;
     const uint64_t ck_base = ((uint64_t)(rs >> 5) + gtile - 1u) * (uint64_t)(TS * TS) + (uint64_t)tid;
     auto fetch = [&](TetFetch& f, QuadFetch& qf, const uint32_t* ids, int dir, int n) {  // the tets ids[0], ids[dir], ...
         if constexpr (C::PF == 3) fetch_quad(qf, ids[dir * min(tid >> 2, n - 1)], tid & 3, rec, col_v);
@@ -931,16 +935,18 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         nb = nb_next;
     }
     if (whole) break;
-    const uint32_t seg = s_plan[0], n_seg = s_plan[1], seg_len = s_plan[2], slot = s_plan[3];
-    // One segment of several: its pixel states go to its slot, and the tile's
-    // last workgroup to get here joins them.
-    const uint64_t px0 = (uint64_t)slot * (TS * TS) + (uint64_t)tid;
-    if (tid < TS * TS) {
-        store_shared(split.px + (px0 + (uint64_t)seg * (TS * TS)), make_float4(cr, cg, cb, log_t));
-        if constexpr (CK) store_shared(split.stop + (px0 + (uint64_t)seg * (TS * TS)), stop);
-    }
-    {
-        float d = active ? log_t : -3.0e38f;
+    const uint32_t seg = s_plan[0], n_seg = s_plan[1], seg_len = s_plan[2];
+    float4* const px = split.px + ((uint64_t)s_plan[3] * (TS * TS) + (uint64_t)tid);
+    if (!joined) {
+        // One segment: its pixel states go to its slot, and all but the tile's
+        // last workgroup to get here are done.  (log T of a segment that was
+        // skipped, or in which the pixel saturated by itself, is short of its
+        // pairs: below -13.8.)
+        if (tid < TS * TS) {
+            store_shared(px + (uint64_t)seg * (TS * TS), make_float4(cr, cg, cb, skipped ? -1e30f : log_t));
+            if constexpr (CK) store_shared(split.stop + (px - split.px) + (uint64_t)seg * (TS * TS), stop);
+        }
+        float d = active ? (skipped ? 0.0f : log_t) : -3.0e38f;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) d = fmaxf(d, __shfl_xor(d, o, 64));
         __syncthreads();  // s_red's readers at the start are done
@@ -949,107 +955,137 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         __syncthreads();
         if (tid == 0) {
             for (int w = 1; w < NT / 64; ++w) d = fmaxf(d, s_red[w]);
-            store_shared(split.dark + slot + seg, d);
+            store_shared(split.dark + s_plan[3] + seg, d);
             drain_stores();
             s_arrived = (int)atomicAdd(split.arrived + gtile, 1u);
-            s_first = (int)n_seg;
         }
         __syncthreads();
         if (s_arrived != (int)n_seg - 1) return;
-    }
-    // Front to back: each segment as seen from the camera.  sat: the segment in
-    // which the pixel saturates.
-    float lt = 0.0f;
-    int sat = (int)n_seg;
-    cr = cg = cb = 0.0f;
-    stop = 0u;
-    if (active) {
-        constexpr int U = 4;
-        for (uint32_t g0 = 0; g0 < n_seg; g0 += U) {
-            float4 q[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) q[u] = load_shared(split.px + (px0 + (uint64_t)min(g0 + u, n_seg - 1u) * (TS * TS)));
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const uint32_t g = g0 + u;
-                if (g >= n_seg || (int)g > sat) continue;
-                const float w = expf(lt);
-                lt += q[u].w;
-                q[u] = make_float4(q[u].x * w, q[u].y * w, q[u].z * w, lt);
-                cr += q[u].x;
-                cg += q[u].y;
-                cb += q[u].z;
-                if constexpr (CK) stop = max(stop, load_shared(split.stop + (px0 + (uint64_t)g * (TS * TS))));
-                split.px[px0 + (uint64_t)g * (TS * TS)] = q[u];
-                if (lt < -13.8f) sat = (int)g;
-            }
-        }
-    }
-    log_t = lt;
-    // the plan's counters are zero between forwards
-    for (uint32_t g = tid; g < n_seg; g += NT) split.dark[slot + g] = 0.0f;
-    if (tid == 0) split.arrived[gtile] = 0u;
-    const bool any = __syncthreads_or(active && sat < (int)n_seg);
-    if (tid == 0) split.serial[gtile] = any ? 1u : 0u;
-    if (!any) {
-        // Back to front: what lies behind each segment, for the adjoint.
+        joined = true;
+        // Front to back: log T at each segment's end, colour and log T of the
+        // pixel, up to the segment in which it saturates (s_sat).
+        uint32_t sat = n_seg;
+        cr = cg = cb = log_t = 0.0f;
+        stop = 0u;
         if (active) {
             constexpr int U = 4;
-            float br = 0.f, bg = 0.f, bb = 0.f;
-            for (int g0 = (int)n_seg - 1; g0 >= 0; g0 -= U) {
+            for (uint32_t g0 = 0; g0 < n_seg && sat == n_seg; g0 += U) {
                 float4 q[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) q[u] = split.px[px0 + (uint64_t)max(g0 - u, 0) * (TS * TS)];
+                for (int u = 0; u < U; ++u) q[u] = load_shared(px + (uint64_t)min(g0 + u, n_seg - 1u) * (TS * TS));
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    if (g0 - u < 0) continue;
-                    split.px[px0 + (uint64_t)(g0 - u) * (TS * TS)] = make_float4(br, bg, bb, q[u].w);
-                    br += q[u].x;
-                    bg += q[u].y;
-                    bb += q[u].z;
+                    const uint32_t g = g0 + u;
+                    if (g >= n_seg || sat < n_seg) continue;
+                    const float lt = log_t + q[u].w;
+                    store_shared(&px[(uint64_t)g * (TS * TS)].w, lt);
+                    if (lt < -13.8f) sat = g;
+                    if (sat == n_seg || g == 0u) {  // (in the first segment the pixel stopped where it has to)
+                        const float w = expf(log_t);
+                        cr += q[u].x * w;
+                        cg += q[u].y * w;
+                        cb += q[u].z * w;
+                        log_t = lt;
+                        if constexpr (CK)
+                            stop = max(stop, load_shared(split.stop + (px - split.px) + (uint64_t)g * (TS * TS)));
+                    }
                 }
             }
         }
-        break;
+        if (tid < TS * TS) s_sat[tid] = sat;
+        // the plan's counters are zero between forwards
+        for (uint32_t g = tid; g < n_seg; g += NT) split.dark[s_plan[3] + g] = 0.0f;
+        if (tid == 0) {
+            split.arrived[gtile] = 0u;
+            s_merge = 0;
+        }
     }
-    // Some pixel saturates.  A pixel that does so in the first segment is done; the
-    // others that do are composited again from the first segment with such a pixel
-    // on, so that each stops behind the pair that saturates it; the rest are done.
-    // The adjoint takes this tile's list as one.
-    if constexpr (CK) {  // checkpoints as seen from the camera
+    // Pixels that saturate in a later segment run in it once more, segment by
+    // segment, from the pixel state in front of it; their colour starts from 0.
+    if (tid == 0) s_first = (int)n_seg;
+    __syncthreads();
+    const uint32_t sat = tid < TS * TS ? s_sat[tid] : 0u;
+    if (active && sat > again && sat < n_seg) atomicMin(&s_first, (int)sat);
+    __syncthreads();
+    again = (uint32_t)s_first;
+    if (again == n_seg) break;
+    run = active && sat == again;
+    if (run) cr = cg = cb = 0.0f;
+    if (tid < TS * TS) s_ray[tid].w = run ? 1.0f : 0.0f;
+    done = again * seg_len;
+    end = min(done + seg_len, ranges[2ull * gtile + 1] - ranges[2ull * gtile]);
+    next_ck = 0xFFFFFFFFu;  // the segment's checkpoints stand
+    }
+    if (!whole) {
+        // Back to front: every segment's slot gets what lies behind the segment, the
+        // adjoint's start: colour and log T.  The undo of a saturated pixel begins
+        // at its alpha and passes over the pairs behind its stop too, so that it
+        // reaches log T = 0, and stays there, before the front: from a segment in
+        // which it does (or whose sum is short) on, the adjoint takes the rest of
+        // the list in one.
+        const uint32_t n_seg = s_plan[1];
+        float4* const px = split.px + ((uint64_t)s_plan[3] * (TS * TS) + (uint64_t)tid);
+        const uint32_t sat = tid < TS * TS ? s_sat[tid] : 0u;
+        uint32_t merge = 0u;
         if (active) {
-            uint32_t g = 0;
-            float base = 0.0f;
-            for (uint32_t c = kCkGroup; c < count; c += kCkGroup) {
-                while (c > (g + 1u) * seg_len) base = split.px[px0 + (uint64_t)g++ * (TS * TS)].w;
-                if ((int)g > sat) break;
-                float* const p = ck + (ck_base + (uint64_t)(c / kCkGroup) * (TS * TS));
-                if (g > 0u) store_shared(p, load_shared(p) + base);
+            const bool undo = !CK && sat < n_seg;
+            const float end_r = cr, end_g = cg, end_b = cb;  // of the saturating segment
+            float br = 0.f, bg = 0.f, bb = 0.f;              // behind the segment
+            float tr = 0.f, tg = 0.f, tb = 0.f;              // the pixel's, if it ran again
+            float x = undo ? logf(fmaxf(1.0f - (1.0f - safe_exp(log_t)), 1e-20f)) : 0.0f;
+            bool lost = false;
+            constexpr int U = 4;
+            for (int g0 = (int)n_seg - 1; g0 >= 0; g0 -= U) {
+                float4 q[U + 1];
+#pragma unroll
+                for (int u = 0; u <= U; ++u) q[u] = load_shared(px + (uint64_t)max(g0 - u, 0) * (TS * TS));
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int g = g0 - u;
+                    if (g < 0) continue;
+                    const float front = g > 0 ? q[u + 1].w : 0.0f;  // log T in front (up to the saturating segment)
+                    const bool seen = (uint32_t)g < sat;
+                    px[(uint64_t)g * (TS * TS)] = make_float4(br, bg, bb, undo ? x : q[u].w);
+                    const float w = expf(front);
+                    if (seen) {
+                        tr += q[u].x * w;
+                        tg += q[u].y * w;
+                        tb += q[u].z * w;
+                    }
+                    if (undo) {
+                        const float sum = (uint32_t)g <= sat ? q[u].w - front : q[u].w;
+                        const float xf = x - sum;
+                        if (!lost && (sum < -13.79f || xf > 0.0f)) {
+                            lost = true;
+                            merge = (uint32_t)g;
+                        }
+                        if (!lost) {
+                            const float wx = expf(xf);
+                            br += q[u].x * wx;
+                            bg += q[u].y * wx;
+                            bb += q[u].z * wx;
+                            x = xf;
+                        }
+                    } else if (seen) {
+                        br += q[u].x * w;
+                        bg += q[u].y * w;
+                        bb += q[u].z * w;
+                    } else if ((uint32_t)g == sat) {
+                        br = end_r;
+                        bg = end_g;
+                        bb = end_b;
+                    }
+                }
+            }
+            if (sat > 0u && sat < n_seg) {
+                cr = tr + end_r;
+                cg = tg + end_g;
+                cb = tb + end_b;
             }
         }
-    }
-    run = active && sat > 0 && sat < (int)n_seg;
-    if (run) atomicMin(&s_first, sat);
-    __syncthreads();
-    const int first = s_first;
-    if (first == (int)n_seg) break;  // all of them in the first segment
-    if (run) {
-        cr = cg = cb = 0.0f;
-        stop = 0u;
-        for (int g = 0; g < first; ++g) {
-            const float4 q = split.px[px0 + (uint64_t)g * (TS * TS)];
-            cr += q.x;
-            cg += q.y;
-            cb += q.z;
-            log_t = q.w;
-            if constexpr (CK) stop = max(stop, load_shared(split.stop + (px0 + (uint64_t)g * (TS * TS))));
-        }
-    }
-    if (tid < TS * TS) s_ray[tid].w = run ? 1.0f : 0.0f;
-    done = (uint32_t)first * seg_len;
-    next_ck = done + kCkGroup;
-    end = ranges[2ull * gtile + 1] - ranges[2ull * gtile];
-    whole = true;
+        if (merge) atomicMax(&s_merge, (int)merge);
+        __syncthreads();
+        if (tid == 0) split.merged[gtile] = (uint32_t)s_merge;
     }
     if (active) {
         const uint64_t pix = vw.pix_base + (uint64_t)py * vw.width + px;
@@ -1367,9 +1403,11 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     const uint32_t seg = split.seg ? split.seg[blockIdx.x] : 0u;
     const uint32_t rs = ranges[2ull * gtile], re = ranges[2ull * gtile + 1];
     const uint32_t count = re > rs ? re - rs : 0u;
-    // a list whose segment states the forward left is taken by segments too
-    const bool by_seg = split.px && split_segments(count, split.unit) > 1u && split.serial[gtile] == 0u;
-    if (!by_seg && seg > 0u) return;
+    // a list whose segment states the forward left is taken by segments too, the
+    // first `merged` of them with the one behind
+    const bool by_seg = split.px && split_segments(count, split.unit) > 1u;
+    const uint32_t merged = by_seg ? split.merged[gtile] : 0u;
+    if (by_seg ? seg < merged : seg > 0u) return;
     const uint32_t seg_len = by_seg ? split_length(count, split.unit) : count;
     const uint32_t slot = by_seg ? split.slot[gtile] + seg : 0u;
     const uint32_t view = tile_view[gtile];
@@ -1439,7 +1477,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         float ws = wave_sum(lsum);
         if (lane == 0) s_loss[wid] = ws;
         __syncthreads();
-        if (tid == 0 && seg == 0u) {
+        if (tid == 0 && seg == merged) {
             float s = 0.f;
             for (int w = 0; w < NW; ++w) s += s_loss[w];
             loss_partial[gtile] = s;
@@ -1447,7 +1485,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     }
 
     // list positions from the back, [done, end) here
-    const uint32_t end = count - seg * seg_len;
+    const uint32_t end = count - (seg == merged ? 0u : seg * seg_len);
     uint32_t done = by_seg ? count - min(seg * seg_len + seg_len, count) : 0u;
     int nb = (int)min<uint32_t>(B, end - done);
     // CK: slot of checkpoint j + 1 (the end of group j) is ck_base + j

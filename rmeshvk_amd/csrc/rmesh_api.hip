@@ -140,7 +140,7 @@ struct rmesh_renderer {
     uint32_t* ranges = nullptr;
     uint32_t* tile_order = nullptr;  // compositing work item -> global tile, heaviest first
     // segments of long tile lists (SplitPlan); px also per tet-sorted pair capacity
-    uint32_t *seg = nullptr, *n_seg_items = nullptr, *seg_slot = nullptr, *seg_arrived = nullptr, *seg_serial = nullptr;
+    uint32_t *seg = nullptr, *n_seg_items = nullptr, *seg_slot = nullptr, *seg_arrived = nullptr, *seg_merged = nullptr;
     float* seg_dark = nullptr;
     float4* seg_px = nullptr;
     uint32_t* seg_stop = nullptr;
@@ -498,7 +498,7 @@ SplitPlan split_plan(const rmesh_renderer* h) {
     p.n_items = h->n_seg_items;
     p.slot = h->seg_slot;
     p.arrived = h->seg_arrived;
-    p.serial = h->seg_serial;
+    p.merged = h->seg_merged;
     p.dark = h->seg_dark;
     p.px = h->seg_px;
     p.stop = h->seg_stop;
@@ -739,7 +739,7 @@ void free_all(rmesh_renderer* h) {
                     h->ivl_ddist, h->ivl_dgrad, h->ivl_dvn, h->ivl_tv, h->v2t_off, h->v2t, h->ck, h->fin,
                     h->d_scenes, h->d_tile_view, h->d_ktile, h->scene_clock, h->tet_g, h->dkey_a, h->dkey_b,
                     h->ditem_a, h->ditem_b, h->ihist, h->d_nitems, h->block_sums2, h->block_vis, h->spine_part,
-                    h->spine_aux, h->seg, h->n_seg_items, h->seg_slot, h->seg_arrived, h->seg_serial, h->seg_dark,
+                    h->spine_aux, h->seg, h->n_seg_items, h->seg_slot, h->seg_arrived, h->seg_merged, h->seg_dark,
                     h->seg_px, h->seg_stop};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -938,7 +938,7 @@ static rmesh_status create_impl(const rmesh_scene_desc* descs, uint32_t n_scenes
     CREATE_TRY(dalloc(&h->n_seg_items, 1));
     CREATE_TRY(dalloc(&h->seg_slot, (size_t)h->tile_cap));
     CREATE_TRY(dalloc(&h->seg_arrived, (size_t)h->tile_cap));
-    CREATE_TRY(dalloc(&h->seg_serial, (size_t)h->tile_cap));
+    CREATE_TRY(dalloc(&h->seg_merged, (size_t)h->tile_cap));
     CREATE_TRY(dalloc(&h->rgba, 4 * h->pix_cap));
     CREATE_TRY(dalloc(&h->dl, 4ull * h->W * h->H));
     CREATE_TRY(dalloc(&h->gt, 3 * h->pix_cap));
@@ -1346,7 +1346,7 @@ extern "C" rmesh_status rmesh_device_bytes(rmesh_renderer* h, uint64_t* out) {
                           h->ivl_tv, h->v2t_off, h->v2t, h->ck, h->fin, h->d_scenes, h->d_tile_view, h->d_ktile,
                           h->tet_g, h->dkey_a, h->dkey_b, h->ditem_a, h->ditem_b, h->ihist, h->d_nitems,
                           h->block_sums2, h->block_vis, h->spine_part, h->spine_aux, h->seg, h->n_seg_items,
-                          h->seg_slot, h->seg_arrived, h->seg_serial, h->seg_dark, h->seg_px, h->seg_stop};
+                          h->seg_slot, h->seg_arrived, h->seg_merged, h->seg_dark, h->seg_px, h->seg_stop};
     uint64_t total = 0;
     for (const void* p : ptrs) {
         if (!p) continue;

@@ -42,7 +42,7 @@ struct SplitPlan {
     uint32_t* n_items = nullptr;
     uint32_t* slot = nullptr;     // [tile] first segment slot (tiles with more than one segment)
     uint32_t* arrived = nullptr;  // [tile] segments composited
-    uint32_t* serial = nullptr;   // [tile] 1: a pixel saturated, the adjoint takes the list as one
+    uint32_t* merged = nullptr;   // [tile] the adjoint takes segments 0 .. merged in one
     float* dark = nullptr;        // [slot] the segment's largest log transmittance over the tile's pixels (0: not known)
     // [slot][TS TS] the segment alone: premultiplied colour, log T; once the tile
     // is complete: colour behind the segment, log T at its end, both seen from

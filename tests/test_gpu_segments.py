@@ -7,8 +7,7 @@ several workgroups composite, against the oracle's single pass over each list.
   pixel saturates but some come close, and in one where pixels saturate in the
   first segment, in later ones and never (the segments from there on are
   composited again);
-- the undo mode's gradients of the light scene within the same bound of the
-  float64 oracle;
+- the undo mode's gradients within the same bound of the float64 oracle;
 - a batch, replayed as a graph, gives every view's image bit for bit and the sum
   of the views' gradients.
 """
@@ -75,15 +74,17 @@ def test_segmented_lists_match_oracle(kind, ts):
     img = r.forward_tiled(*cam)
     assert np.abs(img - ref["rgba"]).max() <= 1e-4
     g = r.backward(dl)
-    if kind == "light":
-        f64 = {k: (np.asarray(v, np.float64) if np.asarray(v).dtype == np.float32 else v) for k, v in s.items()}
-        fw = orc.forward(f64, cam, W, H, ref["sorted_vals"], ref["ranges"], ts, dtype=np.float64)
-        go = orc.backward(f64, cam, W, H, ref["sorted_vals"], ref["ranges"], fw["rgba"], dl.astype(np.float64), ts,
-                          dtype=np.float64)
-        for k in KEYS:
-            assert _rel(g[k], go[k]) <= 1e-3, (k, _rel(g[k], go[k]))
-    else:
-        assert all(np.isfinite(np.asarray(g[k])).all() for k in KEYS)
+    # The undo starts from log(1 - alpha): 1 - alpha carries 6e-8 of the rounding of
+    # alpha, a share of T that the oracle takes from the exact image, and for a
+    # saturated pixel from the renderer's own alpha.
+    f64 = {k: (np.asarray(v, np.float64) if np.asarray(v).dtype == np.float32 else v) for k, v in s.items()}
+    fw = orc.forward(f64, cam, W, H, ref["sorted_vals"], ref["ranges"], ts, dtype=np.float64)
+    sat = 1.0 - fw["rgba"][..., 3] < np.exp(-13.8)
+    start = np.where(sat[..., None], np.asarray(img, np.float64).reshape(H, W, 4), fw["rgba"])
+    go = orc.backward(f64, cam, W, H, ref["sorted_vals"], ref["ranges"], start, dl.astype(np.float64), ts,
+                      dtype=np.float64)
+    for k in KEYS:
+        assert _rel(g[k], go[k]) <= 1e-3, (k, _rel(g[k], go[k]))
 
 
 @pytest.mark.parametrize("mode", ["undo", "checkpoint"])
