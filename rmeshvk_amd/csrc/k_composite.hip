@@ -1118,12 +1118,10 @@ struct BwdCfg {
     static constexpr int NREC = (CAP + NT - 1) / NT;  // records per lane
 };
 
-// Segmented inclusive sum on DPP; lanes with equal `key` form contiguous
-// segments (keys non-decreasing with the lane index).  Four row_shr steps sum
-// inside each 16-lane row, then row_bcast:15 (rows 1, 3) and row_bcast:31 (rows
-// 2, 3) carry the previous rows' partial sums.  Lanes whose DPP source lies
-// outside the row or the row mask read 0.  Masks are 0/1 floats (the summands
-// are finite: every gradient term is clamped to +-1e20 before it is summed).
+// Segmented inclusive sums on DPP inside each 16-lane row; lanes with equal `key`
+// form contiguous segments.  Lanes whose DPP source lies outside the row read 0.
+// Masks are 0/1 floats (the summands are finite: every gradient term is clamped
+// to +-1e20 before it is summed).
 template <int CTRL, int ROWS>
 __device__ __forceinline__ int dpp_i(int v, int old) {
     return __builtin_amdgcn_update_dpp(old, v, CTRL, ROWS, 0xF, false);
@@ -1133,36 +1131,6 @@ __device__ __forceinline__ float dpp_f(float v) {
     // full row mask: bound_ctrl (out-of-row lanes read 0) lets the shift fold into the FMA
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xF, ROWS == 0xF));
 }
-struct SegMasksDpp {
-    float m[6];
-};
-__device__ __forceinline__ SegMasksDpp seg_masks_dpp(int key) {
-    SegMasksDpp s;
-    s.m[0] = dpp_i<0x111, 0xF>(key, -1) == key ? 1.0f : 0.0f;  // row_shr:1
-    s.m[1] = dpp_i<0x112, 0xF>(key, -1) == key ? 1.0f : 0.0f;  // row_shr:2
-    s.m[2] = dpp_i<0x114, 0xF>(key, -1) == key ? 1.0f : 0.0f;  // row_shr:4
-    s.m[3] = dpp_i<0x118, 0xF>(key, -1) == key ? 1.0f : 0.0f;  // row_shr:8
-    s.m[4] = dpp_i<0x142, 0xA>(key, -1) == key ? 1.0f : 0.0f;  // row_bcast:15
-    s.m[5] = dpp_i<0x143, 0xC>(key, -1) == key ? 1.0f : 0.0f;  // row_bcast:31
-    return s;
-}
-// All N sums level by level (independent DPP reads back to back, no hazard stalls).
-template <int N>
-__device__ __forceinline__ void seg_scan_dpp(float* v, const SegMasksDpp& s) {
-#pragma unroll
-    for (int q = 0; q < N; ++q) v[q] = fmaf(dpp_f<0x111, 0xF>(v[q]), s.m[0], v[q]);
-#pragma unroll
-    for (int q = 0; q < N; ++q) v[q] = fmaf(dpp_f<0x112, 0xF>(v[q]), s.m[1], v[q]);
-#pragma unroll
-    for (int q = 0; q < N; ++q) v[q] = fmaf(dpp_f<0x114, 0xF>(v[q]), s.m[2], v[q]);
-#pragma unroll
-    for (int q = 0; q < N; ++q) v[q] = fmaf(dpp_f<0x118, 0xF>(v[q]), s.m[3], v[q]);
-#pragma unroll
-    for (int q = 0; q < N; ++q) v[q] = fmaf(dpp_f<0x142, 0xA>(v[q]), s.m[4], v[q]);
-#pragma unroll
-    for (int q = 0; q < N; ++q) v[q] = fmaf(dpp_f<0x143, 0xC>(v[q]), s.m[5], v[q]);
-}
-
 // The adjoint's scan of its 19 sums stays inside the 16-lane rows: four levels
 // instead of six.  A row's last lane ends its segment, so a tet leaves
 // one sum per row, and the flush adds the rows.  (The sums used to be added into
@@ -1202,6 +1170,27 @@ __device__ __forceinline__ void row_scan19(float* v, const RowMasks& s) {
 }
 #undef RMESH_SCAN_LEVEL
 #undef RMESH_FMAC_DPP
+// The same for other counts of sums.
+template <int N>
+__device__ __forceinline__ void row_scan(float* v, const RowMasks& s) {
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] = fmaf(dpp_f<0x111, 0xF>(v[q]), s.m[0], v[q]);
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] = fmaf(dpp_f<0x112, 0xF>(v[q]), s.m[1], v[q]);
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] = fmaf(dpp_f<0x114, 0xF>(v[q]), s.m[2], v[q]);
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] = fmaf(dpp_f<0x118, 0xF>(v[q]), s.m[3], v[q]);
+}
+// Sum over the rows of a tet whose records are rr (first | end << 16) of the row
+// sums part[tet + row][.] (stride floats a slot).
+__device__ __forceinline__ float sum_rows(const float* part, int stride, int k, uint32_t rr) {
+    const uint32_t lo = rr & 0xFFFFu, hi = rr >> 16;
+    float x = 0.0f;
+    if (lo < hi)
+        for (uint32_t r = lo >> 4; r < (hi + 15u) >> 4; ++r) x += part[((uint32_t)k + r) * (uint32_t)stride];
+    return x;
+}
 
 // Hit barycentrics of face fi's roles (a, b, c) placed at the tet's vertex
 // slots, 0 at the opposite vertex.  FACES = {0,2,1}, {1,2,3}, {0,3,2},
@@ -1855,10 +1844,11 @@ bool launch_backward(const BwdArgs& a, uint32_t tile_size, int variant, hipStrea
 // (record-parallel) keeps each covered pair's slab and optical depth; phase B
 // (pixel-sequential, depth order) applies the -5.5 log-transmittance cut-off
 // and turns a record into its weight T_val = exp(log T) od (0: no
-// contribution); phase C (record-parallel) forms the 14 weighted moments and
-// the pixel count, sums them per tet with the segmented DPP scan, and the batch
-// adds one atomic per statistic per (tile, tet); the max weight goes through an
-// LDS atomicMax.
+// contribution); phase C (record-parallel) forms the 14 weighted moments, the
+// pixel count and the largest weight, reduces them per tet inside 16-lane rows
+// (one stored result per (tet, row), as in the tiled adjoint), and the batch
+// adds one atomic per statistic per (tile, tet).  A pair's slab stays in the
+// registers of the lane that found it in phase A.
 // ---------------------------------------------------------------------------
 constexpr int kErrStats = 15;  // tet_err columns 0 1 2 5 6..15 (14), then the pixel count
 __device__ __forceinline__ int err_column(int q) { return q < 3 ? q : q + 2; }
@@ -1866,24 +1856,31 @@ __device__ __forceinline__ int err_column(int q) { return q < 3 ? q : q + 2; }
 template <class C>
 __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec, const uint32_t* __restrict__ sorted_vals,
                                                  const uint32_t* __restrict__ ranges,
-                                                 const ViewParams* __restrict__ views, const float* __restrict__ pixel_err,
+                                                 const ViewParams* __restrict__ views,
+                                                 const uint32_t* __restrict__ tile_order, const SplitPlan split,
+                                                 const float* __restrict__ pixel_err,
                                                  const float* __restrict__ ssim_err, float* __restrict__ tet_err,
                                                  int32_t* __restrict__ tet_count) {
     constexpr int TS = C::TS, NT = C::NT, B = C::B, CAP = C::CAP, SP = TS + 1;
     static_assert(B <= 64 && CAP % 32 == 0 && CAP / 32 <= NT && CAP >= TS * TS, "error pass geometry");
     __shared__ BatchLDS<TS, B, false> L;
-    __shared__ float s_r[3][CAP];  // t_min, t_max, optical depth -> weight (0: none)
+    __shared__ float s_w[CAP];  // optical depth -> weight (0: none)
     __shared__ float s_ray[3][TS * TS];
     __shared__ float s_pe[TS * TS], s_se[TS * TS];
     __shared__ uint32_t s_live[TS * TS];            // inside the image, log T >= -5.5
     __shared__ unsigned long long s_mask[TS * TS];  // covered tets of the batch per pixel
     __shared__ SegTab<CAP> G;
     __shared__ float4 s_cen[B];
-    __shared__ uint32_t s_tid[B];  // tet ids of the batch (the forward's LDS image has none)
-    __shared__ float s_acc[B][kErrStats];
-    __shared__ int32_t s_max[B];
+    constexpr int NREC = (CAP + NT - 1) / NT, NPART = B + CAP / 16;
+    __shared__ float4 s_part[NPART][(kErrStats + 1) / 4];  // row results: slot tet + row
+    constexpr int IDW = (2 * B + NT - 1) / NT;
+    __shared__ uint32_t s_ids[2 * B];  // tet ids from the batch's first on, as the forward keeps them
+    __shared__ uint32_t s_ftid[B];     // tet ids of the batch whose results s_part holds
+    static_assert(kErrStats == 15, "16 results a slot");
 
-    const uint32_t gtile = blockIdx.x;
+    // whole tiles, in the forward's order (of a split list the first item only)
+    if (split.seg && (blockIdx.x >= *split.n_items || split.seg[blockIdx.x] > 0u)) return;
+    const uint32_t gtile = tile_order ? tile_order[blockIdx.x] : blockIdx.x;
     const ViewParams& vw = views[0];
     const TileCtx tc = tile_ctx(vw, gtile);
     const int tid = threadIdx.x, wid = tid / 64, lane = (int)__lane_id();
@@ -1915,57 +1912,79 @@ __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec,
     const uint32_t count = re > rs ? re - rs : 0u;
     uint32_t done = 0;
     int nb = (int)min<uint32_t>(B, count);
-    TetFetch f;
-    QuadFetch qf{};
-    uint32_t ft = 0;
-    if (C::PF == 1 && tid < nb) fetch_tet(f, ft = sorted_vals[re - 1 - tid], rec, rec);
-    if (C::PF == 3 && tid < 4 * nb) fetch_quad(qf, ft = sorted_vals[re - 1 - (tid >> 2)], tid & 3, rec, rec);
-    while (done < count) {
-        if (__syncthreads_and(!active || log_t < -5.5f)) break;
+    auto fetch = [&](TetFetch& f, QuadFetch& qf, const uint32_t* ids, int dir, int n) {  // the tets ids[0], ids[dir], ...
+        if constexpr (C::PF == 3) fetch_quad(qf, ids[dir * min(tid >> 2, n - 1)], tid & 3, rec, rec);
+        else fetch_tet(f, ids[dir * min(tid, n - 1)], rec, rec);
+    };
+    auto load_ids = [&](uint32_t* idw, uint32_t d) {
+#pragma unroll
+        for (int u = 0; u < IDW; ++u) idw[u] = sorted_vals[re - 1 - min(d + (uint32_t)(u * NT + tid), count - 1u)];
+    };
+    auto stage = [&](const TetFetch& f, const QuadFetch& qf, const uint32_t* idw, int n) {
         if constexpr (C::PF == 3) {
-            store_quad<TS, B, false>(L, qf, tid >> 2, tid & 3, tid < 4 * nb, vw, tc);
+            store_quad<TS, B, false>(L, qf, tid >> 2, tid & 3, tid < 4 * n, vw, tc);
             const V3 a = qperm3<0x00>(qf.r), b = qperm3<0x55>(qf.r), c = qperm3<0xAA>(qf.r), d = qperm3<0xFF>(qf.r);
             const V3 cen = scl3(add3(add3(add3(a, b), c), d), 0.25f);
-            if (tid < 4 * nb && (tid & 3) == 0) {
-                s_cen[tid >> 2] = make_float4(cen.x, cen.y, cen.z, 0.0f);
-                s_tid[tid >> 2] = ft;
-            }
-        } else if (tid < nb) {
+            if (tid < 4 * n && (tid & 3) == 0) s_cen[tid >> 2] = make_float4(cen.x, cen.y, cen.z, 0.0f);
+        } else if (tid < n) {
             store_tet<TS, B, false>(L, tid, f, vw, tc);
             const V3 a = mk3(f.r[0].x, f.r[0].y, f.r[0].z), b = mk3(f.r[1].x, f.r[1].y, f.r[1].z),
                      c = mk3(f.r[2].x, f.r[2].y, f.r[2].z), d = mk3(f.r[3].x, f.r[3].y, f.r[3].z);
             const V3 cen = scl3(add3(add3(add3(a, b), c), d), 0.25f);
             s_cen[tid] = make_float4(cen.x, cen.y, cen.z, 0.0f);
-            s_tid[tid] = ft;
         }
         if (tid < TS * TS) s_mask[tid] = 0ull;
         if (tid < CAP / 32) G.starts()[tid] = 0u;
-        for (int i = tid; i < B * kErrStats; i += NT) (&s_acc[0][0])[i] = 0.0f;
-        if (tid < B) s_max[tid] = 0;
-        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < IDW; ++u)
+            if (u * NT + tid < 2 * B) s_ids[u * NT + tid] = idw[u];
+    };
+    if (count) {
+        TetFetch f;
+        QuadFetch qf;
+        uint32_t idw[IDW];
+        fetch(f, qf, sorted_vals + (re - 1), -1, nb);
+        load_ids(idw, 0u);
+        stage(f, qf, idw, nb);
+    }
+    while (done < count) {
+        if (__syncthreads_and(!active || log_t < -5.5f)) break;
         batch_layout<TS, B, false, true, CAP, NT>(L, nb, G.seg, G.starts());
         __syncthreads();
         const uint32_t nbp = L.nbp & 0xFFu;
         const uint32_t nrec = L.nbp >> 8;
         const uint32_t next = done + nbp;
-        const int nb_next = (int)min<uint32_t>(B, count - next);
-        if (C::PF == 1 && tid < nb_next) fetch_tet(f, ft = sorted_vals[re - 1 - next - tid], rec, rec);
-        if (C::PF == 3 && tid < 4 * nb_next) fetch_quad(qf, ft = sorted_vals[re - 1 - next - (tid >> 2)], tid & 3, rec, rec);
+        const int nb_next = next_batch<B>(nbp, nb, count - next);
+        TetFetch f;  // loaded for the end of this iteration
+        QuadFetch qf;
+        uint32_t idw[IDW];
+        fetch(f, qf, s_ids + nbp, 1, B);
+        load_ids(idw, next);
+        if (tid < (int)nbp) s_ftid[tid] = s_ids[tid];
         // phase A: slab and optical depth of every covered pair
-        for (uint32_t j = tid; j < nrec; j += NT) {
-            const RecordRef c = record_at(G.seg, G.starts(), j);
-            const int p = c.row * TS + c.col;
-            if (s_live[p]) {
-                TetRegs T;
-                tet_regs(L, c.k, T);
-                const V3 rd = mk3(s_ray[0][p], s_ray[1][p], s_ray[2][p]);
-                float t_min, t_max;
-                int fmin, fmax;
-                if (intersect(T, rd, min_t, t_min, t_max, fmin, fmax)) {
-                    s_r[0][j] = t_min;
-                    s_r[1][j] = t_max;
-                    s_r[2][j] = med_clip(T.dens * (t_max - t_min), 1e-8f, 88.0f);
-                    atomicOr(&s_mask[p], 1ull << c.k);
+        float r_t0[NREC], r_t1[NREC];
+        uint32_t r_m[NREC];  // tet | pixel << 6 | hit << 20
+#pragma unroll
+        for (int n = 0; n < NREC; ++n) {
+            const uint32_t j = (uint32_t)(n * NT + tid);
+            r_m[n] = 0u;
+            if (j < nrec) {
+                const RecordRef c = record_at(G.seg, G.starts(), j);
+                const int p = c.row * TS + c.col;
+                r_m[n] = (uint32_t)c.k;
+                if (s_live[p]) {
+                    TetRegs T;
+                    tet_regs(L, c.k, T);
+                    const V3 rd = mk3(s_ray[0][p], s_ray[1][p], s_ray[2][p]);
+                    float t_min, t_max;
+                    int fmin, fmax;
+                    if (intersect(T, rd, min_t, t_min, t_max, fmin, fmax)) {
+                        s_w[j] = med_clip(T.dens * (t_max - t_min), 1e-8f, 88.0f);
+                        r_t0[n] = t_min;
+                        r_t1[n] = t_max;
+                        r_m[n] |= ((uint32_t)p << 6) | (1u << 20);
+                        atomicOr(&s_mask[p], 1ull << c.k);
+                    }
                 }
             }
         }
@@ -1981,34 +2000,34 @@ __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec,
                 if (log_t >= -5.5f) {
                     const float trans = safe_exp(log_t);
                     if (trans >= 1e-6f) {
-                        const float od = s_r[2][slot];
+                        const float od = s_w[slot];
                         tv = trans * od;
                         log_t = log_t - od;
                     }
                 }
-                s_r[2][slot] = tv;
+                s_w[slot] = tv;
             }
             if (log_t < -5.5f) s_live[tid] = 0u;
         }
         __syncthreads();
-        // phase C: moments of the weighted pairs, summed per tet
-        for (uint32_t base = (uint32_t)wid * 64; base < nrec; base += NT) {
-            const uint32_t j = base + lane;
-            float acc[kErrStats];
+        // phase C: moments of the weighted pairs, reduced per tet
+#pragma unroll
+        for (int n = 0; n < NREC; ++n) {
+            const uint32_t j = (uint32_t)(n * NT + tid);
+            if ((uint32_t)(n * NT + wid * 64) >= nrec) break;  // per wave
+            float acc[kErrStats], top = 0.0f;
 #pragma unroll
             for (int q = 0; q < kErrStats; ++q) acc[q] = 0.0f;
-            int key = 0x7fffffff;
-            if (j < nrec) {
-                const RecordRef c = record_at(G.seg, G.starts(), j);
-                key = c.k;
-                const int p = c.row * TS + c.col;
-                const float tv = (s_mask[p] >> c.k) & 1ull ? s_r[2][j] : 0.0f;
+            const int key = j < nrec ? (int)(r_m[n] & 63u) : -2;  // a tet's records are contiguous, hit or not
+            if (r_m[n] >> 20) {
+                const float tv = s_w[j];
                 if (tv > 0.0f) {
+                    const int p = (int)((r_m[n] >> 6) & 1023u);
                     const V3 rd = mk3(s_ray[0][p], s_ray[1][p], s_ray[2][p]);
                     const V3 ro = add3(cam, scl3(rd, min_t));
-                    const V3 en = add3(ro, scl3(rd, s_r[0][j])), ex = add3(ro, scl3(rd, s_r[1][j]));
+                    const V3 en = add3(ro, scl3(rd, r_t0[n])), ex = add3(ro, scl3(rd, r_t1[n]));
                     const float pe = s_pe[p], se = s_se[p];
-                    const float4 cq = s_cen[c.k];
+                    const float4 cq = s_cen[key];
                     acc[0] = tv;
                     acc[1] = tv * pe;
                     acc[2] = (tv * pe) * pe;
@@ -2024,30 +2043,48 @@ __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec,
                     acc[12] = tv * cq.y;
                     acc[13] = tv * cq.z;
                     acc[14] = 1.0f;
-                    atomicMax(&s_max[c.k], sat_i32(65535.0f * tv));
+                    top = tv;
                 }
             }
-            const SegMasksDpp sm = seg_masks_dpp(key);
-            const int next_key = dpp_i<0x130, 0xF>(key, -1);  // wave_shl:1 (lane 63 reads -1)
-            const bool tail = key != 0x7fffffff && next_key != key;
-            seg_scan_dpp<kErrStats>(acc, sm);
-#pragma unroll
-            for (int q = 0; q < kErrStats; ++q)
-                if (tail && acc[q] != 0.0f) atomicAdd(&s_acc[key][q], acc[q]);
+            const RowMasks sm = row_masks(key);
+            const int next_key = dpp_i<0x101, 0xF>(key, -1);  // row_shl:1 (a row's last lane reads -1)
+            const bool tail = key >= 0 && next_key != key;
+            row_scan<kErrStats>(acc, sm);
+            // weights are >= 0, so a masked 0 leaves the maximum alone
+            top = fmaxf(top, dpp_f<0x111, 0xF>(top) * sm.m[0]);
+            top = fmaxf(top, dpp_f<0x112, 0xF>(top) * sm.m[1]);
+            top = fmaxf(top, dpp_f<0x114, 0xF>(top) * sm.m[2]);
+            top = fmaxf(top, dpp_f<0x118, 0xF>(top) * sm.m[3]);
+            if (tail) {
+                float4* const o = s_part[key + (int)(j >> 4)];
+                o[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+                o[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
+                o[2] = make_float4(acc[8], acc[9], acc[10], acc[11]);
+                o[3] = make_float4(acc[12], acc[13], acc[14], top);
+            }
         }
         __syncthreads();
-        // flush: one atomic per non-zero statistic per (tile, tet)
+        // the next batch's LDS image, then the flush: one atomic per non-zero
+        // statistic per (tile, tet), last because loads and atomics retire in order
+        if (nb_next > 0) stage(f, qf, idw, nb_next);
         for (int it = tid; it < (int)nbp * (kErrStats + 1); it += NT) {
             const int k = it / (kErrStats + 1), q = it % (kErrStats + 1);
-            const uint32_t t = s_tid[k];
+            const float* const part = reinterpret_cast<const float*>(s_part) + q;
+            const uint32_t rr = L.recs[k], t = s_ftid[k];
+            if (q == kErrStats) {
+                const uint32_t lo = rr & 0xFFFFu, hi = rr >> 16;
+                float top = 0.0f;
+                if (lo < hi)
+                    for (uint32_t r = lo >> 4; r < (hi + 15u) >> 4; ++r) top = fmaxf(top, part[((uint32_t)k + r) * (kErrStats + 1)]);
+                const int32_t n = sat_i32(65535.0f * top);
+                if (n > 0) atomicMax(tet_count + 2ull * t + 1, n);
+                continue;
+            }
+            const float v = sum_rows(part, kErrStats + 1, k, rr);
             if (q < kErrStats - 1) {
-                const float v = s_acc[k][q];
                 if (v != 0.0f) unsafeAtomicAdd(tet_err + 16ull * t + err_column(q), v);
-            } else if (q == kErrStats - 1) {
-                const int32_t n = (int32_t)s_acc[k][q];
-                if (n) atomicAdd(tet_count + 2ull * t, n);
-            } else if (s_max[k] > 0) {
-                atomicMax(tet_count + 2ull * t + 1, s_max[k]);
+            } else if ((int32_t)v) {
+                atomicAdd(tet_count + 2ull * t, (int32_t)v);
             }
         }
         done = next;
@@ -2055,11 +2092,14 @@ __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec,
     }
 }
 
+// (30,000 points in clusters at 803 x 601, tile 12: B 48 with CAP 768 and the heaviest tiles first 0.53 ms (0.62 in tile order), B 32
+// with 512 0.73; with LDS atomics for the results 0.83.)
 template <int TS>
 static void err_launch(const ErrArgs& a, hipStream_t s) {
-    using C = FwdCfg<TS, 32, (TS * TS > 512 ? TS * TS : 512), 3>;
-    hipLaunchKernelGGL((k_error<C>), dim3(a.num_tiles), dim3(C::NT), 0, s, a.rec, a.sorted_vals, a.ranges, a.views,
-                       a.pixel_err, a.ssim_err, a.tet_err, a.tet_count);
+    using C = FwdCfg<TS, (TS == 12 || TS == 16 ? 48 : 32), (TS > 16 ? TS * TS : TS == 8 ? 512 : 768), 3>;
+    const dim3 grid(a.split.seg ? a.split.grid : a.num_tiles);
+    hipLaunchKernelGGL((k_error<C>), grid, dim3(C::NT), 0, s, a.rec, a.sorted_vals, a.ranges, a.views,
+                       a.tile_order, a.split, a.pixel_err, a.ssim_err, a.tet_err, a.tet_count);
 }
 
 bool launch_error(const ErrArgs& a, uint32_t tile_size, hipStream_t s) {
@@ -2287,6 +2327,39 @@ __global__ __launch_bounds__(256) void k_interval_generate(const float4* __restr
     o[6] = base;
 }
 
+// A decomposition record on its way to the LDS image: lane j of a tet's quad
+// holds its float4 j and 4 + j.
+struct IvlFetch {
+    float4 a, b;
+};
+__device__ __forceinline__ void ivl_fetch(IvlFetch& f, uint32_t t, int j, const float4* __restrict__ ivr) {
+    f.a = ivr[(uint64_t)kIvlRec * t + j];
+    f.b = ivr[(uint64_t)kIvlRec * t + min(4 + j, kIvlRec - 1)];
+}
+// Every lane calls it (quad shuffles); on: the lane's tet is in the batch.
+template <int TS, int B>
+__device__ __forceinline__ void ivl_store(BatchLDS<TS, B, false>& L, const IvlFetch& f, int k, int j, bool on,
+                                          const TileCtx& tc) {
+    // the tet's four projected points: silhouette 0-2 and the inner vertex (3
+    // points) or silhouette 0-3
+    const float n = qperm<0x55>(f.b.w), cx = qperm<0x00>(f.b.x), cy = qperm<0x00>(f.b.y);
+    const bool inner = j == 3 && n == 3.0f;
+    const float x = (inner ? cx : f.a.x) - tc.tile_ox, y = (inner ? cy : f.a.y) - tc.tile_oy;
+    float ymin = fminf(y, qperm<0xB1>(y)), ymax = fmaxf(y, qperm<0xB1>(y));
+    ymin = fminf(ymin, qperm<0x4E>(ymin));
+    ymax = fmaxf(ymax, qperm<0x4E>(ymax));
+    if (!on) return;
+    L.tr[k * kIvlRec + j] = f.a;
+    if (j < kIvlRec - 4) L.tr[k * kIvlRec + 4 + j] = f.b;
+    L.pxy[j][k] = x;
+    L.pxy[4 + j][k] = y;
+    if (j == 0) {
+        const float r0 = fmaxf(ceilf(ymin) - 1.0f, 0.0f);
+        const float r1 = fminf(floorf(ymax), (float)(TS - 1));
+        L.rows[k] = n != 0.0f && r0 <= r1 ? (uint32_t)r0 | ((uint32_t)r1 << 8) : 0xFFu;
+    }
+}
+
 // Tiled compositing over the fan triangles: the batch machinery of the
 // tiled forward (spans of the tet's four projected points, which bound the
 // silhouette; pixels of a span outside it find no fan triangle), with one
@@ -2304,7 +2377,11 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     static_assert(B <= 64 && CAP >= TS * TS && CAP % 32 == 0 && CAP / 32 <= NT && CAP <= 2048, "batch geometry");
     static_assert(BatchLDS<TS, B, false>::TR == kIvlRec, "records live in the face rows");
     __shared__ BatchLDS<TS, B, false> L;
-    __shared__ float s_r[8][CAP];  // colour rgb, optical depth, depth, 1 - e^-u, m1 / T, self term / T^2
+    __shared__ float4 s_r0[CAP];  // colour rgb, optical depth
+    __shared__ float4 s_r1[CAP];  // depth, 1 - e^-u, m1 / T, self term / T^2
+    constexpr int IDW = (2 * B + NT - 1) / NT;
+    __shared__ uint32_t s_ids[2 * B];  // tet ids from the batch's first on, as the tiled forward keeps them
+    constexpr int FR = (4 * B + NT - 1) / NT;  // rounds of quads, one per tet
     __shared__ float s_rsc[TS * TS];
     __shared__ uint32_t s_live[TS * TS];
     __shared__ unsigned long long s_mask[TS * TS];
@@ -2336,48 +2413,42 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     const uint32_t count = re > rs_ ? re - rs_ : 0u;
     uint32_t done = 0;
     int nb = (int)min<uint32_t>(B, count);
-    float4 f[kIvlRec];
-    auto fetch = [&](uint32_t t) {
+    auto load_ids = [&](uint32_t* idw, uint32_t d) {
 #pragma unroll
-        for (int i = 0; i < kIvlRec; ++i) f[i] = ivr[(uint64_t)kIvlRec * t + i];
+        for (int u = 0; u < IDW; ++u) idw[u] = sorted_vals[re - 1 - min(d + (uint32_t)(u * NT + tid), count - 1u)];
     };
-    if (tid < nb) fetch(sorted_vals[re - 1 - tid]);
-    while (done < count) {
-        if (__syncthreads_and(!active || log_t < -13.8f)) break;
-        if (tid < nb) {
-            const int k = tid;
+    auto stage = [&](const IvlFetch* f, const uint32_t* idw, int n) {
 #pragma unroll
-            for (int i = 0; i < kIvlRec; ++i) L.tr[k * kIvlRec + i] = f[i];
-            // the tet's four projected points: silhouette 0-2 and the inner
-            // vertex (3 points) or silhouette 0-3
-            const bool tri = f[5].w == 3.0f;
-            const float qx[4] = {f[0].x, f[1].x, f[2].x, tri ? f[4].x : f[3].x};
-            const float qy[4] = {f[0].y, f[1].y, f[2].y, tri ? f[4].y : f[3].y};
-            uint32_t rr = 0xFFu;
-            if (f[5].w != 0.0f) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    L.pxy[i][k] = qx[i] - tc.tile_ox;
-                    L.pxy[4 + i][k] = qy[i] - tc.tile_oy;
-                }
-                const float ymin = fminf(fminf(qy[0], qy[1]), fminf(qy[2], qy[3])) - tc.tile_oy;
-                const float ymax = fmaxf(fmaxf(qy[0], qy[1]), fmaxf(qy[2], qy[3])) - tc.tile_oy;
-                const float r0 = fmaxf(ceilf(ymin) - 1.0f, 0.0f);
-                const float r1 = fminf(floorf(ymax), (float)(TS - 1));
-                if (r0 <= r1) rr = (uint32_t)r0 | ((uint32_t)r1 << 8);
-            }
-            L.rows[k] = rr;
-        }
+        for (int u = 0; u < FR; ++u)
+            ivl_store<TS, B>(L, f[u], min((u * NT + tid) >> 2, B - 1), tid & 3, u * NT + tid < 4 * n, tc);
         if (tid < TS * TS) s_mask[tid] = 0ull;
         if (tid < CAP / 32) G.starts()[tid] = 0u;
-        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < IDW; ++u)
+            if (u * NT + tid < 2 * B) s_ids[u * NT + tid] = idw[u];
+    };
+    if (count) {
+        IvlFetch f[FR];
+        uint32_t idw[IDW];
+#pragma unroll
+        for (int u = 0; u < FR; ++u)
+            ivl_fetch(f[u], sorted_vals[re - 1 - min((u * NT + tid) >> 2, nb - 1)], tid & 3, ivr);
+        load_ids(idw, 0u);
+        stage(f, idw, nb);
+    }
+    while (done < count) {
+        if (__syncthreads_and(!active || log_t < -13.8f)) break;
         batch_layout<TS, B, false, true, CAP, NT>(L, nb, G.seg, G.starts());
         __syncthreads();
         const uint32_t nbp = L.nbp & 0xFFu;
         const uint32_t nrec = L.nbp >> 8;
         const uint32_t next = done + nbp;
-        const int nb_next = (int)min<uint32_t>(B, count - next);
-        if (tid < nb_next) fetch(sorted_vals[re - 1 - next - tid]);
+        const int nb_next = next_batch<B>(nbp, nb, count - next);
+        IvlFetch f[FR];  // loaded for the end of this iteration
+        uint32_t idw[IDW];
+#pragma unroll
+        for (int u = 0; u < FR; ++u) ivl_fetch(f[u], s_ids[nbp + min((u * NT + tid) >> 2, B - 1)], tid & 3, ivr);
+        load_ids(idw, next);
         // record-parallel: fan triangle, interpolation and the per-pair terms
         // (interval_tiled_rasterize.wgsl:248-400)
         for (uint32_t j = tid; j < nrec; j += NT) {
@@ -2434,14 +2505,9 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             const float u = dens * (exit_d - enter);
             const float en = safe_exp(-u);
             const float ad = fmaxf(1.0f - en, 0.0f);
-            s_r[0][j] = cp.x;
-            s_r[1][j] = cp.y;
-            s_r[2][j] = cp.z;
-            s_r[3][j] = od;
-            s_r[4][j] = w0 * zb + w1 * zf;
-            s_r[5][j] = ad;
-            s_r[6][j] = enter * ad + safe_div(1.0f - (1.0f + u) * en, dens);
-            s_r[7][j] = safe_div(1.0f - 2.0f * u * en - en * en, dens);
+            s_r0[j] = make_float4(cp.x, cp.y, cp.z, od);
+            s_r1[j] = make_float4(w0 * zb + w1 * zf, ad, enter * ad + safe_div(1.0f - (1.0f + u) * en, dens),
+                                  safe_div(1.0f - 2.0f * u * en - en * en, dens));
             atomicOr(&s_mask[p], 1ull << c.k);
         }
         __syncthreads();
@@ -2455,14 +2521,15 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                 const uint32_t slot = (L.rpref[k * SP + row] + (uint32_t)colp) & 0xFFFFu;
                 const float Tj = safe_exp(log_t);
                 if (Tj >= 1e-6f) {
-                    cr = cr + s_r[0][slot] * Tj;
-                    cg = cg + s_r[1][slot] * Tj;
-                    cb = cb + s_r[2][slot] * Tj;
-                    log_t = log_t - s_r[3][slot];
-                    dep = dep + Tj * s_r[4][slot];
-                    const float m0 = Tj * s_r[5][slot];
-                    const float m1 = Tj * s_r[6][slot];
-                    const float sd = (Tj * Tj) * s_r[7][slot];
+                    const float4 q0 = s_r0[slot], q1 = s_r1[slot];
+                    cr = cr + q0.x * Tj;
+                    cg = cg + q0.y * Tj;
+                    cb = cb + q0.z * Tj;
+                    log_t = log_t - q0.w;
+                    dep = dep + Tj * q1.x;
+                    const float m0 = Tj * q1.y;
+                    const float m1 = Tj * q1.z;
+                    const float sd = (Tj * Tj) * q1.w;
                     ds0 = ds0 + 2.0f * m1 * ds2;
                     ds1 = ds1 + 2.0f * m0 * ds3;
                     ds2 = ds2 + m0;
@@ -2472,6 +2539,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             }
             if (log_t < -13.8f) s_live[tid] = 0u;
         }
+        if (nb_next > 0) stage(f, idw, nb_next);  // (the pixel phase reads neither the records nor other lanes' masks)
         done = next;
         nb = nb_next;
     }
@@ -2499,7 +2567,8 @@ struct IvlPair {
     V3 cf_raw, cb_raw, cf, cb, cp;
 };
 
-__device__ __forceinline__ bool ivl_pair(const float4* __restrict__ T, float pcx, float pcy, float rsc, IvlPair& q) {
+// The fan triangle holding the pixel centre and its barycentrics.
+__device__ __forceinline__ bool ivl_find(const float4* __restrict__ T, float pcx, float pcy, IvlPair& q) {
     const float4 q0 = T[0], q1 = T[1], q2 = T[2], q3 = T[3], q4 = T[4], q5 = T[5];
     const bool tri3 = q5.w == 3.0f;
     float4 ea = q0, eb = q1;
@@ -2521,6 +2590,11 @@ __device__ __forceinline__ bool ivl_pair(const float4* __restrict__ T, float pcx
     }
     if (!found) return false;
     ivl_bary(pcx, pcy, ea.x, ea.y, eb.x, eb.y, q4.x, q4.y, q.b0, q.b1, q.b2);
+    return true;
+}
+// The rest from b0, b1, b2, ai, bi.
+__device__ __forceinline__ void ivl_eval(const float4* __restrict__ T, float rsc, IvlPair& q) {
+    const float4 ea = T[q.ai], eb = T[q.bi], q4 = T[4], q5 = T[5];
     q.zfn = q.b0 * ea.z + q.b1 * eb.z + q.b2 * q4.z;
     q.zbn = q.b0 * ea.z + q.b1 * eb.z + q.b2 * q4.w;
     const float ofn = q.b0 * ea.w + q.b1 * eb.w + q.b2 * q5.x;
@@ -2544,7 +2618,6 @@ __device__ __forceinline__ bool ivl_pair(const float4* __restrict__ T, float pcx
     q.w1 = 1.0f - phv;
     q.cp = safe_clip3(mk3(q.cb.x * q.w0 + q.cf.x * q.w1, q.cb.y * q.w0 + q.cf.y * q.w1, q.cb.z * q.w0 + q.cf.z * q.w1),
                       0.0f, kMaxVal);
-    return true;
 }
 
 // Per-tet adjoint accumulators of the interval decomposition, in floats:
@@ -2558,8 +2631,10 @@ constexpr int kIvlGradTerms = 24, kIvlNormalTerms = 18, kIvlGradStride = 48;
 // batches: phase A evaluates each covered pair, phase B undoes the pixel's
 // colour / transmittance / distortion state in order and keeps the pair's
 // T_prev, the transmittance gradient before it and the m0 gradient, phase C
-// forms the pair's terms and reduces them per tet (segmented wave scan, LDS
-// adds, one global add per term per (tile, tet)).
+// forms the pair's terms and reduces them per tet as the tiled adjoint does
+// (segmented scan inside 16-lane rows, one stored sum per (tet, row), one global
+// add per term per (tile, tet)).  The pair's fan triangle and barycentrics stay
+// in the registers of the lane that found them in phase A.
 template <class C>
 __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE))) void k_interval_backward(
     const float4* __restrict__ ivr, const uint32_t* __restrict__ sorted_vals, const uint32_t* __restrict__ ranges,
@@ -2567,17 +2642,23 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     const float* __restrict__ dist_img, const float* __restrict__ dl_img, const float* __restrict__ dl_xyzd,
     const float* __restrict__ dl_dist, float* __restrict__ d_ivr) {
     constexpr int TS = C::TS, NT = C::NT, B = C::B, CAP = C::CAP, SP = TS + 1;
-    constexpr int KT = kIvlGradTerms + kIvlNormalTerms;
+    constexpr int KT = kIvlGradTerms + kIvlNormalTerms, NREC = (CAP + NT - 1) / NT;
+    constexpr int NPART = B + CAP / 16, PS = 11;  // row sums: slot tet + row, PS float4 each
+    constexpr int IDW = (2 * B + NT - 1) / NT;
     static_assert(B <= 64 && CAP >= TS * TS && CAP % 32 == 0 && CAP / 32 <= NT && CAP <= 2048, "batch geometry");
+    static_assert(kIvlGradTerms == 24 && kIvlNormalTerms <= 20, "row sum layout");
+    constexpr int FR = (4 * B + NT - 1) / NT;  // rounds of quads, one per tet
     __shared__ BatchLDS<TS, B, false> L;
-    __shared__ float s_r[6][CAP];  // A: colour rgb, od, 1 - e^-u, m1 / T; B: T_prev, -d log T, d m0
+    // A: optical depth, d colour . colour, 1 - e^-u, m1 / T; B: T_prev (0: no part), -d log T, d m0
+    __shared__ float4 s_r[CAP];
     __shared__ float s_rsc[TS * TS];
     __shared__ float s_dl[7][TS * TS];  // d colour rgb, d xyzd
     __shared__ uint32_t s_live[TS * TS];
     __shared__ unsigned long long s_mask[TS * TS];
     __shared__ SegTab<CAP> G;
-    __shared__ float s_acc[B][KT];
-    __shared__ uint32_t s_tid[B];
+    __shared__ float4 s_part[NPART][PS];
+    __shared__ uint32_t s_ids[2 * B];
+    __shared__ uint32_t s_ftid[B];  // tet ids of the batch whose sums s_part holds
 
     const uint32_t gtile = tile_order ? tile_order[blockIdx.x] : blockIdx.x;
     const ViewParams& vw = views[0];
@@ -2634,73 +2715,75 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     const uint32_t count = re > rs_ ? re - rs_ : 0u;
     uint32_t done = 0;
     int nb = (int)min<uint32_t>(B, count);
-    float4 f[kIvlRec];
-    uint32_t ft = 0;
-    auto fetch = [&](uint32_t t) {
-        ft = t;
+    auto load_ids = [&](uint32_t* idw, uint32_t d) {
 #pragma unroll
-        for (int i = 0; i < kIvlRec; ++i) f[i] = ivr[(uint64_t)kIvlRec * t + i];
+        for (int u = 0; u < IDW; ++u) idw[u] = sorted_vals[rs_ + min(d + (uint32_t)(u * NT + tid), count - 1u)];
     };
-    if (tid < nb) fetch(sorted_vals[rs_ + tid]);
-    while (done < count) {
-        __syncthreads();  // the previous batch's flush has read s_acc / s_tid
-        if (tid < nb) {
-            const int k = tid;
+    auto stage = [&](const IvlFetch* f, const uint32_t* idw, int n) {
 #pragma unroll
-            for (int i = 0; i < kIvlRec; ++i) L.tr[k * kIvlRec + i] = f[i];
-            s_tid[k] = ft;
-            const bool tri = f[5].w == 3.0f;
-            const float qx[4] = {f[0].x, f[1].x, f[2].x, tri ? f[4].x : f[3].x};
-            const float qy[4] = {f[0].y, f[1].y, f[2].y, tri ? f[4].y : f[3].y};
-            uint32_t rr = 0xFFu;
-            if (f[5].w != 0.0f) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    L.pxy[i][k] = qx[i] - tc.tile_ox;
-                    L.pxy[4 + i][k] = qy[i] - tc.tile_oy;
-                }
-                const float ymin = fminf(fminf(qy[0], qy[1]), fminf(qy[2], qy[3])) - tc.tile_oy;
-                const float ymax = fmaxf(fmaxf(qy[0], qy[1]), fmaxf(qy[2], qy[3])) - tc.tile_oy;
-                const float r0 = fmaxf(ceilf(ymin) - 1.0f, 0.0f);
-                const float r1 = fminf(floorf(ymax), (float)(TS - 1));
-                if (r0 <= r1) rr = (uint32_t)r0 | ((uint32_t)r1 << 8);
-            }
-            L.rows[k] = rr;
-        }
+        for (int u = 0; u < FR; ++u)
+            ivl_store<TS, B>(L, f[u], min((u * NT + tid) >> 2, B - 1), tid & 3, u * NT + tid < 4 * n, tc);
         if (tid < TS * TS) s_mask[tid] = 0ull;
         if (tid < CAP / 32) G.starts()[tid] = 0u;
-        for (int i = tid; i < B * KT; i += NT) (&s_acc[0][0])[i] = 0.0f;
+#pragma unroll
+        for (int u = 0; u < IDW; ++u)
+            if (u * NT + tid < 2 * B) s_ids[u * NT + tid] = idw[u];
+    };
+    if (count) {
+        IvlFetch f[FR];
+        uint32_t idw[IDW];
+#pragma unroll
+        for (int u = 0; u < FR; ++u)
+            ivl_fetch(f[u], sorted_vals[rs_ + min((u * NT + tid) >> 2, nb - 1)], tid & 3, ivr);
+        load_ids(idw, 0u);
+        stage(f, idw, nb);
+    }
+    while (done < count) {
         __syncthreads();
         batch_layout<TS, B, false, true, CAP, NT>(L, nb, G.seg, G.starts());
         __syncthreads();
         const uint32_t nbp = L.nbp & 0xFFu;
         const uint32_t nrec = L.nbp >> 8;
         const uint32_t next = done + nbp;
-        const int nb_next = (int)min<uint32_t>(B, count - next);
-        if (tid < nb_next) fetch(sorted_vals[rs_ + next + tid]);
+        const int nb_next = next_batch<B>(nbp, nb, count - next);
+        IvlFetch f[FR];  // loaded for the end of this iteration
+        uint32_t idw[IDW];
+#pragma unroll
+        for (int u = 0; u < FR; ++u) ivl_fetch(f[u], s_ids[nbp + min((u * NT + tid) >> 2, B - 1)], tid & 3, ivr);
+        load_ids(idw, next);
+        if (tid < (int)nbp) s_ftid[tid] = s_ids[tid];
         // phase A: the pair's colour, optical depth and distortion factors
-        for (uint32_t j = tid; j < nrec; j += NT) {
-            const RecordRef c = record_at(G.seg, G.starts(), j);
-            const int p = c.row * TS + c.col;
-            if (!s_live[p]) continue;
-            const float4* T = &L.tr[c.k * kIvlRec];
-            const float pcx = (float)(tc.tile_x * TS + (uint32_t)c.col) + 0.5f;
-            const float pcy = (float)(tc.tile_y * TS + (uint32_t)c.row) + 0.5f;
-            const float rsc = s_rsc[p];
-            IvlPair q;
-            if (!ivl_pair(T, pcx, pcy, rsc, q)) continue;
-            const float dens = T[5].z;
-            const float enter = q.z_f * rsc, exit_d = q.z_b * rsc;
-            const float u = dens * (exit_d - enter);
-            const float en = safe_exp(-u);
-            const float ad = fmaxf(1.0f - en, 0.0f);
-            s_r[0][j] = q.cp.x;
-            s_r[1][j] = q.cp.y;
-            s_r[2][j] = q.cp.z;
-            s_r[3][j] = q.od;
-            s_r[4][j] = ad;
-            s_r[5][j] = enter * ad + safe_div(1.0f - (1.0f + u) * en, dens);
-            atomicOr(&s_mask[p], 1ull << c.k);
+        float r_b0[NREC], r_b1[NREC], r_b2[NREC];
+        uint32_t r_m[NREC];  // tet | pixel << 6 | triangle's slots << 16, << 18 | hit << 20
+#pragma unroll
+        for (int n = 0; n < NREC; ++n) {
+            const uint32_t j = (uint32_t)(n * NT + tid);
+            r_m[n] = 0u;
+            if (j < nrec) {
+                const RecordRef c = record_at(G.seg, G.starts(), j);
+                const int p = c.row * TS + c.col;
+                r_m[n] = (uint32_t)c.k;
+                const float4* T = &L.tr[c.k * kIvlRec];
+                const float pcx = (float)(tc.tile_x * TS + (uint32_t)c.col) + 0.5f;
+                const float pcy = (float)(tc.tile_y * TS + (uint32_t)c.row) + 0.5f;
+                IvlPair q;
+                if (s_live[p] && ivl_find(T, pcx, pcy, q)) {
+                    const float rsc = s_rsc[p];
+                    ivl_eval(T, rsc, q);
+                    const float dens = T[5].z;
+                    const float enter = q.z_f * rsc, exit_d = q.z_b * rsc;
+                    const float u = dens * (exit_d - enter);
+                    const float en = safe_exp(-u);
+                    const float ad = fmaxf(1.0f - en, 0.0f);
+                    s_r[j] = make_float4(q.od, (s_dl[0][p] * q.cp.x + s_dl[1][p] * q.cp.y) + s_dl[2][p] * q.cp.z, ad,
+                                         enter * ad + safe_div(1.0f - (1.0f + u) * en, dens));
+                    r_b0[n] = q.b0;
+                    r_b1[n] = q.b1;
+                    r_b2[n] = q.b2;
+                    r_m[n] |= ((uint32_t)p << 6) | ((uint32_t)q.ai << 16) | ((uint32_t)q.bi << 18) | (1u << 20);
+                    atomicOr(&s_mask[p], 1ull << c.k);
+                }
+            }
         }
         __syncthreads();
         // phase B: undo back to front (backward_interval_tiled.wgsl:432-460, 602-630)
@@ -2710,52 +2793,54 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                 const uint32_t k = (uint32_t)__ffsll((long long)m) - 1u;
                 m &= m - 1ull;
                 const uint32_t slot = (L.rpref[k * SP + row] + (uint32_t)colp) & 0xFFFFu;
-                const float cr = s_r[0][slot], cg = s_r[1][slot], cb = s_r[2][slot], od = s_r[3][slot];
-                const float prev = fminf(log_t + od, 0.0f);
+                const float4 q = s_r[slot];
+                const float prev = fminf(log_t + q.x, 0.0f);
                 const float tp = safe_exp(prev);
                 log_t = prev;
                 if (tp < 1e-6f) {
-                    s_r[0][slot] = 0.0f;
+                    s_r[slot].x = 0.0f;
                     continue;
                 }
                 const float dos = -d_log_t;
-                d_log_t = safe_clip(d_log_t + ((dl_r * cr + dl_g * cg) + dl_b * cb) * tp, kMinVal, kMaxVal);
-                const float m0 = tp * s_r[4][slot];
-                const float m1 = tp * s_r[5][slot];
+                d_log_t = safe_clip(d_log_t + q.y * tp, kMinVal, kMaxVal);
+                const float m0 = tp * q.z;
+                const float m1 = tp * q.w;
                 st_z = st_z - m0;
                 st_w = st_w - m1;
                 const float dm0 = d_z + 2.0f * st_w * d_y;
                 d_z = d_z + 2.0f * m1 * d_x;
                 d_w = d_w + 2.0f * m0 * d_y;
-                s_r[0][slot] = tp;
-                s_r[1][slot] = dos;
-                s_r[2][slot] = dm0;
+                s_r[slot] = make_float4(tp, dos, dm0, 0.0f);
             }
         }
         __syncthreads();
         // phase C: the pair's terms, summed per tet (backward_interval_tiled.wgsl:460-660)
-        for (uint32_t base = (uint32_t)wid * 64; base < nrec; base += NT) {
-            const uint32_t j = base + lane;
+#pragma unroll
+        for (int n = 0; n < NREC; ++n) {
+            const uint32_t j = (uint32_t)(n * NT + tid);
+            if ((uint32_t)(n * NT + wid * 64) >= nrec) break;  // per wave
             float acc[kIvlGradTerms], accn[kIvlNormalTerms];
 #pragma unroll
             for (int i = 0; i < kIvlGradTerms; ++i) acc[i] = 0.0f;
 #pragma unroll
             for (int i = 0; i < kIvlNormalTerms; ++i) accn[i] = 0.0f;
-            int key = 0x7fffffff;
-            if (j < nrec) {
-                const RecordRef c = record_at(G.seg, G.starts(), j);
-                key = c.k;
-                const int p = c.row * TS + c.col;
-                const float tp = (s_mask[p] >> c.k) & 1ull ? s_r[0][j] : 0.0f;
+            const int key = j < nrec ? (int)(r_m[n] & 63u) : -2;  // a tet's records are contiguous, hit or not
+            if (r_m[n] >> 20) {
+                const int p = (int)((r_m[n] >> 6) & 1023u);
+                const float4 rr = s_r[j];
+                const float tp = rr.x;
                 if (tp > 0.0f) {
-                    const float4* T = &L.tr[c.k * kIvlRec];
-                    const float pcx = (float)(tc.tile_x * TS + (uint32_t)c.col) + 0.5f;
-                    const float pcy = (float)(tc.tile_y * TS + (uint32_t)c.row) + 0.5f;
+                    const float4* T = &L.tr[key * kIvlRec];
                     const float rsc = s_rsc[p];
                     IvlPair q;
-                    ivl_pair(T, pcx, pcy, rsc, q);
+                    q.b0 = r_b0[n];
+                    q.b1 = r_b1[n];
+                    q.b2 = r_b2[n];
+                    q.ai = (int)((r_m[n] >> 16) & 3u);
+                    q.bi = (int)((r_m[n] >> 18) & 3u);
+                    ivl_eval(T, rsc, q);
                     const float dens = T[5].z;
-                    const float dos = s_r[1][j], dm0 = s_r[2][j];
+                    const float dos = rr.y, dm0 = rr.z;
                     const V3 dcol = mk3(s_dl[0][p], s_dl[1][p], s_dl[2][p]);
                     const V3 d_cp = safe_clip3(scl3(dcol, tp), kMinVal, kMaxVal);
                     const float dphi = dphi_dx_f(q.od);
@@ -2834,26 +2919,34 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                     }
                 }
             }
-            const SegMasksDpp sm = seg_masks_dpp(key);
-            const int next_key = dpp_i<0x130, 0xF>(key, -1);  // wave_shl:1 (lane 63 reads -1)
-            const bool tail = key != 0x7fffffff && next_key != key;
-            seg_scan_dpp<kIvlGradTerms>(acc, sm);
+            const RowMasks sm = row_masks(key);
+            const int next_key = dpp_i<0x101, 0xF>(key, -1);  // row_shl:1 (a row's last lane reads -1)
+            const bool tail = key >= 0 && next_key != key;
+            float4* const o = s_part[max(key, 0) + (int)(j >> 4)];
+            row_scan<kIvlGradTerms>(acc, sm);
+            if (tail) {
 #pragma unroll
-            for (int i = 0; i < kIvlGradTerms; ++i)
-                if (tail && acc[i] != 0.0f) atomicAdd(&s_acc[key][i], acc[i]);
+                for (int i = 0; i < kIvlGradTerms / 4; ++i)
+                    o[i] = make_float4(acc[4 * i], acc[4 * i + 1], acc[4 * i + 2], acc[4 * i + 3]);
+            }
             if (has_dn) {
-                seg_scan_dpp<kIvlNormalTerms>(accn, sm);
+                row_scan<kIvlNormalTerms>(accn, sm);
+                if (tail) {
+                    float* const f = reinterpret_cast<float*>(o + kIvlGradTerms / 4);
 #pragma unroll
-                for (int i = 0; i < kIvlNormalTerms; ++i)
-                    if (tail && accn[i] != 0.0f) atomicAdd(&s_acc[key][kIvlGradTerms + i], accn[i]);
+                    for (int i = 0; i < kIvlNormalTerms; ++i) f[i] = accn[i];
+                }
             }
         }
         __syncthreads();
-        // flush: one global add per non-zero term per (tile, tet)
-        for (int it = tid; it < (int)nbp * KT; it += NT) {
-            const int k = it / KT, i = it % KT;
-            const float v = s_acc[k][i];
-            if (v != 0.0f) unsafeAtomicAdd(d_ivr + (uint64_t)kIvlGradStride * s_tid[k] + i, v);
+        // the next batch's LDS image, then the flush: one global add per non-zero
+        // term per (tile, tet), last because loads and atomics retire in order
+        if (nb_next > 0) stage(f, idw, nb_next);
+        const int terms = has_dn ? KT : kIvlGradTerms;
+        for (int it = tid; it < (int)nbp * terms; it += NT) {
+            const int k = it / terms, i = it % terms;
+            const float v = sum_rows(reinterpret_cast<const float*>(s_part) + i, 4 * PS, k, L.recs[k]);
+            if (v != 0.0f) unsafeAtomicAdd(d_ivr + (uint64_t)kIvlGradStride * s_ftid[k] + i, v);
         }
         done = next;
         nb = nb_next;
@@ -3084,9 +3177,18 @@ __global__ __launch_bounds__(256) void k_vertex_gather(const uint32_t* __restric
     d_vn[3ull * vtx + 2] = n2;
 }
 
+// Geometry of the interval kernels, bound by the batches of the longest lists:
+// fewer, larger ones up to a quad of lanes per tet in one round (50,000 points in
+// clusters at 637 x 479, tile 12, adjoint and forward: B 48 with three records a
+// lane 1.21 and 0.66 ms, B 32 1.37 and 0.81, B 64 1.24 and 0.67; with LDS atomics
+// for the sums, the search repeated in phase C and the records' loads waited for
+// in every batch, B 32, 1.89 and 0.93).
+template <int TS>
+using IvlCfg = FwdCfg<TS, (TS > 16 ? 16 : TS == 8 ? 32 : 48), (TS > 16 ? TS * TS : TS == 8 ? 512 : 3 * ((TS * TS + 63) / 64 * 64)), 1>;
+
 template <int TS>
 static void ivl_bwd_launch(const IvlBwdArgs& a, hipStream_t s) {
-    using C = FwdCfg<TS, (TS > 16 ? 16 : 32), (TS * TS > 512 ? TS * TS : 512), 1>;
+    using C = IvlCfg<TS>;
     hipLaunchKernelGGL((k_interval_backward<C>), dim3(a.num_tiles), dim3(C::NT), 0, s, a.ivr, a.sorted_vals, a.ranges,
                        a.views, a.tile_order, a.rgba, a.dist, a.dl_img, a.dl_xyzd, a.dl_dist, a.d_ivr);
 }
@@ -3110,7 +3212,7 @@ bool launch_interval_backward(const IvlBwdArgs& a, uint32_t tile_size, hipStream
 
 template <int TS>
 static void ivl_launch(const IvlArgs& a, hipStream_t s) {
-    using C = FwdCfg<TS, (TS > 16 ? 16 : 32), (TS * TS > 512 ? TS * TS : 512), 1>;
+    using C = IvlCfg<TS>;
     hipLaunchKernelGGL((k_interval_forward<C>), dim3(a.num_tiles), dim3(C::NT), 0, s, a.ivr, a.sorted_vals, a.ranges,
                        a.views, a.tile_order, a.rgba, a.xyzd, a.dist);
 }

@@ -1047,6 +1047,8 @@ extern "C" rmesh_status rmesh_forward_error(rmesh_renderer* h, const float* pixe
     a.ranges = h->ranges;
     a.views = h->d_views;
     a.num_tiles = h->T;
+    a.tile_order = h->tile_order;
+    if (h->order_split) a.split = split_plan(h);
     a.pixel_err = h->err_pe;
     a.ssim_err = h->err_se;
     a.tet_err = h->tet_err;

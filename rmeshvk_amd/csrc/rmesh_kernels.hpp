@@ -154,6 +154,8 @@ struct ErrArgs {
     const uint32_t* ranges;
     const ViewParams* views;  // views[0]
     uint32_t num_tiles;
+    const uint32_t* tile_order;  // nullable, as FwdArgs::tile_order
+    SplitPlan split;             // as FwdArgs::split (whole tiles all the same)
     const float* pixel_err;   // [H][W]
     const float* ssim_err;    // [H][W]
     float* tet_err;           // [M][16], accumulated
