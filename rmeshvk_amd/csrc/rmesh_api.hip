@@ -558,11 +558,10 @@ rmesh_status stage_forward(rmesh_renderer* h, uint32_t V, bool want_aux) {
 
 void zero_grads(rmesh_renderer* h, uint32_t V) {
     hipStream_t s = h->stream;
-    launch_fill_u32(reinterpret_cast<uint32_t*>(h->tet_g), 0u, 16ull * h->M, s);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(h->d_verts), 0u, 3ull * h->N, s);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(h->d_dens), 0u, h->M, s);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(h->d_grads), 0u, 3ull * h->M, s);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(h->d_colors), 0u, 3ull * h->color_len, s);
+    auto words = [](float* p) { return reinterpret_cast<uint32_t*>(p); };
+    launch_zero_ranges({{words(h->tet_g), words(h->d_verts), words(h->d_dens), words(h->d_grads), words(h->d_colors)},
+                        {16ull * h->M, 3ull * h->N, h->M, 3ull * h->M, 3ull * h->color_len}},
+                       s);
 }
 
 rmesh_status stage_backward(rmesh_renderer* h, uint32_t V, const float* dl, const float* gt, uint32_t loss_type) {

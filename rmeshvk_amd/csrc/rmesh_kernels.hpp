@@ -57,6 +57,13 @@ void launch_prep_records(const float* verts, const uint32_t* idx, const float* d
                          float4* rec, hipStream_t s);
 void launch_copy_colors(const float* base, uint32_t M, float4* col, hipStream_t s);
 void launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s);
+// n[r] words from the 16-byte aligned p[r] to 0, one launch
+struct ZeroRanges {
+    static constexpr int N = 5;
+    uint32_t* p[N];
+    uint64_t n[N];
+};
+void launch_zero_ranges(const ZeroRanges& z, hipStream_t s);
 // blocks x 256 lanes x per_thread float atomic adds over `lines` 64-byte lines (lines >= 977)
 void launch_atomic_probe(float* p, uint32_t lines, uint32_t blocks, uint32_t per_thread, hipStream_t s);
 void launch_copy_probe(const float4* src, float4* dst, uint64_t n16, hipStream_t s);
