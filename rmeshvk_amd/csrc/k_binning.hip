@@ -491,16 +491,14 @@ __global__ __launch_bounds__(1024) void k_spine_add(uint32_t* __restrict__ sums,
 }
 
 // K7 (+ K6 sentinel padding) for one item: its max_write pairs at
-// [start, start + max_write).  64-bit keys: (key tile << 32) | ~bits(depth);
-// 32-bit keys: the key tile alone (pairs already in depth order).
-template <bool POW2, typename KT>
+// [start, start + max_write), keys (key tile << 32) | ~bits(depth).
+template <bool POW2>
 __device__ __forceinline__ void emit_item_pairs(uint64_t item, uint32_t start, uint32_t max_write,
                                                 const float4* __restrict__ rec, const float4* __restrict__ circ,
                                                 const SceneRange* __restrict__ scenes, uint32_t n_scenes,
-                                                const ViewParams* __restrict__ views, KT* __restrict__ keys,
+                                                const ViewParams* __restrict__ views, uint64_t* __restrict__ keys,
                                                 uint32_t* __restrict__ vals, uint32_t cap,
                                                 uint32_t* __restrict__ overflow) {
-    constexpr bool FULL = sizeof(KT) == 8;
     uint32_t t, vv;
     item_tet_view(scenes, n_scenes, item, t, vv);
     V3 v[4];
@@ -522,8 +520,7 @@ __device__ __forceinline__ void emit_item_pairs(uint64_t item, uint32_t start, u
     uint32_t local = 0;
     TileBox b;
     if (tile_box<POW2>(proj, vw, T, invT, b)) {
-        uint32_t inv_depth = 0u;
-        if constexpr (FULL) inv_depth = depth_key(circ[t], vw);
+        const uint32_t inv_depth = depth_key(circ[t], vw);
         RowScan rs;
         rs.start(proj, b.y0, T);
         for (uint32_t ty = b.y0; ty <= b.y1 && local < max_write; ++ty) {
@@ -535,8 +532,7 @@ __device__ __forceinline__ void emit_item_pairs(uint64_t item, uint32_t start, u
                 uint32_t gt = vw.key_base + ty * vw.tiles_x + tx;
                 uint32_t wi = start + local;
                 if (wi < cap) {
-                    if constexpr (FULL) keys[wi] = ((uint64_t)gt << 32) | inv_depth;
-                    else keys[wi] = gt;
+                    keys[wi] = ((uint64_t)gt << 32) | inv_depth;
                     vals[wi] = t;
                 } else {
                     *overflow = 1u;
@@ -547,9 +543,7 @@ __device__ __forceinline__ void emit_item_pairs(uint64_t item, uint32_t start, u
     }
     // Slots counted by K1 but not produced by the division-based
     // re-projection keep the tile_fill sentinel (tile_gen_scan_compute.wgsl:202).
-    KT sentinel;
-    if constexpr (FULL) sentinel = ((uint64_t)vw.sentinel_tile << 32) | 0xFFFFFFFFull;
-    else sentinel = vw.sentinel_tile;
+    const uint64_t sentinel = ((uint64_t)vw.sentinel_tile << 32) | 0xFFFFFFFFull;
     for (; local < max_write; ++local) {
         uint32_t wi = start + local;
         if (wi < cap) {
@@ -577,7 +571,7 @@ __global__ __launch_bounds__(256) void k_pairs(const float4* __restrict__ rec, c
     uint32_t tot;
     const uint32_t start = block_excl_scan(max_write, red, tot) + block_off[blockIdx.x];
     if (max_write == 0) return;
-    emit_item_pairs<POW2, uint64_t>(item, start, max_write, rec, circ, scenes, n_scenes, views, keys, vals, cap,
+    emit_item_pairs<POW2>(item, start, max_write, rec, circ, scenes, n_scenes, views, keys, vals, cap,
                                     overflow);
 }
 
@@ -601,6 +595,24 @@ __global__ __launch_bounds__(256) void k_sorted_sums(const uint32_t* __restrict_
     if (threadIdx.x == 0) block_sums[blockIdx.x] = tot;
 }
 
+// Two levels of work per wave: the items' tile rows, one a lane, then the rows'
+// pairs, one a lane, so the longest item of a wave no longer sets its time and the
+// pair writes of a wave are consecutive (8 views of a 10,000-point scene, tile
+// 12: one lane per item 180 us, now 108; 60,000 points, one view: 72 and 54).  A row evaluates both of its border
+// lines (a lane's walk over its item's rows could carry one over).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// The last l of 64 with first[l] <= x (first[0] <= x, non-decreasing).
+__device__ __forceinline__ uint32_t last_at_most(const uint32_t* first, uint32_t x) {
+    uint32_t l = 0;
+#pragma unroll
+    for (uint32_t st = 32; st > 0; st >>= 1)
+        if (first[l + st] <= x) l += st;
+    return l;
+}
 template <bool POW2>
 __global__ __launch_bounds__(256) void k_pairs_sorted(const float4* __restrict__ rec,
                                                       const SceneRange* __restrict__ scenes, uint32_t n_scenes,
@@ -611,14 +623,122 @@ __global__ __launch_bounds__(256) void k_pairs_sorted(const float4* __restrict__
                                                       uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
                                                       uint32_t cap, uint32_t* __restrict__ overflow) {
     __shared__ uint32_t red[256 / kWave];
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ float s_proj[8][256];
+    __shared__ uint32_t s_box[3][256];                  // x0, x1, y0
+    __shared__ uint32_t s_row0[256], s_row1[256];       // tile rows of the wave up to the item's start and end
+    __shared__ uint32_t s_start[256], s_max[256];       // pair slots of the item
+    __shared__ uint32_t s_tet[256], s_view[256];
+    __shared__ uint32_t s_first[256], s_end[256];       // pairs of the wave before and up to the item's end
+    __shared__ uint32_t s_pre[256], s_key[256], s_item[256];  // 64 rows a wave: pairs before, first key, item
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, w0 = tid & ~63u;
+    const uint32_t i = blockIdx.x * blockDim.x + tid;
     const uint32_t sv = i < n_items ? sval[i] : 0u;
     const uint32_t max_write = i < n_items ? sorted_count(sv, counts) : 0u;
     uint32_t tot;
     const uint32_t start = block_excl_scan(max_write, red, tot) + block_off[blockIdx.x];
-    if (max_write == 0) return;
-    emit_item_pairs<POW2, uint32_t>(sv >> kCountBits, start, max_write, rec, nullptr, scenes, n_scenes, views, keys,
-                                    vals, cap, overflow);
+    const float T = (float)views[0].tile_size, invT = 1.0f / T;  // one tile size per renderer
+    uint32_t rows = 0u, vv = 0u;
+    if (max_write) {
+        uint32_t t;
+        item_tet_view(scenes, n_scenes, sv >> kCountBits, t, vv);
+        V3 v[4];
+        float dens;
+        V3 g;
+        load_rec(rec, t, v, dens, g);
+        const ViewParams& vw = views[vv];
+        float proj[4][2];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            float c[4];
+            mul_vp(vw.vp, v[k], c);
+            float nx = c[0] / (c[3] + 1e-6f);
+            float ny = c[1] / (c[3] + 1e-6f);
+            proj[k][0] = ((nx + 1.0f) * 0.5f) * vw.Wf;
+            proj[k][1] = ((1.0f - ny) * 0.5f) * vw.Hf;
+            s_proj[2 * k][tid] = proj[k][0];
+            s_proj[2 * k + 1][tid] = proj[k][1];
+        }
+        TileBox b;
+        if (tile_box<POW2>(proj, vw, T, invT, b) && b.y0 <= b.y1) {
+            rows = b.y1 - b.y0 + 1u;
+            s_box[0][tid] = b.x0;
+            s_box[1][tid] = b.x1;
+            s_box[2][tid] = b.y0;
+        }
+        s_start[tid] = start;
+        s_max[tid] = max_write;
+        s_tet[tid] = t;
+        s_view[tid] = vv;
+    }
+    const uint32_t row_end = wave_incl_scan(rows);
+    s_row0[tid] = row_end - rows;
+    s_row1[tid] = row_end;
+    const uint32_t n_rows = __shfl(row_end, 63, 64);
+    uint32_t carry = 0u;  // pairs of the rows before
+    wave_lds_sync();
+    for (uint32_t r0 = 0; r0 < n_rows; r0 += 64u) {
+        const uint32_t r = r0 + lane;
+        uint32_t n = 0u, l = 0u, key = 0u;
+        bool first = false;
+        if (r < n_rows) {
+            l = w0 + last_at_most(s_row0 + w0, r);
+            float proj[4][2];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                proj[k][0] = s_proj[2 * k][l];
+                proj[k][1] = s_proj[2 * k + 1][l];
+            }
+            const ViewParams& vw = views[s_view[l]];
+            TileBox b;
+            b.x0 = s_box[0][l];
+            b.x1 = s_box[1][l];
+            first = r == s_row0[l];
+            const uint32_t ty = s_box[2][l] + (r - s_row0[l]);
+            RowScan rs;
+            rs.start(proj, ty, T);
+            float xl, xr;
+            if (rs.row(proj, ty, T, xl, xr)) {
+                uint32_t tx0, tx1;
+                row_tiles<POW2>(xl, xr, T, invT, b, tx0, tx1);
+                n = tx0 <= tx1 ? tx1 - tx0 + 1u : 0u;
+                key = vw.key_base + ty * vw.tiles_x + tx0;
+            }
+        }
+        const uint32_t inc = wave_incl_scan(n);
+        if (first) s_first[l] = carry + inc - n;
+        if (r < n_rows && r + 1u == s_row1[l]) s_end[l] = carry + inc;
+        s_pre[tid] = inc - n;
+        s_key[tid] = key;
+        s_item[tid] = l;
+        const uint32_t q_end = __shfl(inc, 63, 64);
+        wave_lds_sync();
+        for (uint32_t q = lane; q < q_end; q += 64u) {
+            const uint32_t row = w0 + last_at_most(s_pre + w0, q);
+            const uint32_t it = s_item[row], local = carry + q - s_first[it];
+            if (local < s_max[it]) {
+                const uint32_t wi = s_start[it] + local;
+                if (wi < cap) {
+                    keys[wi] = s_key[row] + (q - s_pre[row]);
+                    vals[wi] = s_tet[it];
+                } else {
+                    *overflow = 1u;
+                }
+            }
+        }
+        carry += q_end;
+        wave_lds_sync();
+    }
+    // Slots counted by K1 but not produced by the division-based
+    // re-projection keep the tile_fill sentinel (tile_gen_scan_compute.wgsl:202).
+    for (uint32_t local = rows ? s_end[tid] - s_first[tid] : 0u; local < max_write; ++local) {
+        const uint32_t wi = start + local;
+        if (wi < cap) {
+            keys[wi] = views[vv].sentinel_tile;
+            vals[wi] = 0u;
+        } else {
+            *overflow = 1u;
+        }
+    }
 }
 
 // The 64-bit keys of depth-ordered pairs (key tile, sorted values): the depth
