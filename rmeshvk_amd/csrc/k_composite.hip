@@ -8,9 +8,9 @@
 //
 // MI355X design.  One workgroup per (view, tile).  The tile's depth-sorted tet
 // list is consumed in batches; per batch:
-//   1. one thread per tet gathers the 64-byte tet record and derives the inward
-//      face planes, the base colour at the camera and the tile-local projected
-//      vertices into LDS;
+//   1. a quad of lanes per tet takes the 64-byte tet record, loaded during the
+//      batch before, and derives the inward face planes, the base colour at the
+//      camera and the tile-local projected vertices into LDS;
 //   2. all lanes compute the per-row scanline spans of the batch; one wave
 //      turns them into a prefix over (tet, row), which enumerates every covered
 //      (pixel, tet) pair of the batch in a compact range [0, C);
@@ -994,9 +994,9 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         }
         if (tid < TS * TS) s_sat[tid] = sat;
         // the plan's counters are zero between forwards
-        for (uint32_t g = tid; g < n_seg; g += NT) split.dark[s_plan[3] + g] = 0.0f;
+        for (uint32_t g = tid; g < n_seg; g += NT) store_shared(split.dark + s_plan[3] + g, 0.0f);
         if (tid == 0) {
-            split.arrived[gtile] = 0u;
+            store_shared(split.arrived + gtile, 0u);
             s_merge = 0;
         }
     }

@@ -15,9 +15,9 @@ struct ViewParams;
 // multiples of 32 positions, as the transmittance checkpoints do.
 // The unit, 6 pairs per pixel: a tile's workgroup is a serial chain over its
 // list, and the chip holds some 1300 of them, so a list far above (all pairs) /
-// 1300 runs on after the rest of the grid is done (12 scenes, longest list 33,800
-// pairs at tile 16: forward 2.1 ms, adjoint 3.6 unsplit, 0.37 and 0.84 split; 4
-// clustered views, longest 16,300: 1.5 and 2.9, 0.34 and 0.79).  A segment costs a
+// 1300 runs on after the rest of the grid is done (uneven scenes, longest list
+// 33,800 pairs at tile 16: forward 2.1 ms, adjoint 3.6 unsplit, 0.37 and 0.84
+// split; 4 clustered views, longest 16,300: 1.5 and 2.9, 0.34 and 0.79).  A segment costs a
 // pixel record (16 bytes a pixel written, read by the tile's last workgroup and
 // by the adjoint) and the start of a workgroup: where no list is long for the
 // grid (config C) 2 % at 6, 4 % at 4 and 1 % at 8 pairs a pixel, while 8 leaves
