@@ -936,17 +936,20 @@ __device__ __forceinline__ uint32_t item_bucket(uint32_t c, int seg, const Split
     const uint32_t in = seg < 0 ? (uint32_t)kSegBuckets : (uint32_t)kSegBuckets - 1u - min((uint32_t)seg, (uint32_t)kSegBuckets - 1u);
     return lo + (min(b, hi) - lo) * (uint32_t)(kSegBuckets + 1) + in;
 }
+__device__ __forceinline__ uint32_t tile_unit(const ViewParams& vw, const SplitPlan& sp) {
+    return sp.unit_for(vw.tiles_x * vw.tiles_y);
+}
 // cnt: the tile's bucket counters (its scene's).
-__device__ __forceinline__ void count_items(uint32_t* cnt, uint32_t pairs, const SplitPlan& sp) {
-    const uint32_t n = sp.seg ? split_segments(pairs, sp.unit) : 1u;
+__device__ __forceinline__ void count_items(uint32_t* cnt, uint32_t pairs, uint32_t unit, const SplitPlan& sp) {
+    const uint32_t n = sp.seg ? split_segments(pairs, unit) : 1u;
     if (n == 1u) atomicAdd(&cnt[item_bucket(pairs, -1, sp)], 1u);
     else
-        for (uint32_t g = 0; g < n; ++g) atomicAdd(&cnt[item_bucket(split_length(pairs, sp.unit), (int)g, sp)], 1u);
+        for (uint32_t g = 0; g < n; ++g) atomicAdd(&cnt[item_bucket(split_length(pairs, unit), (int)g, sp)], 1u);
 }
 // off: the buckets' running item offsets; n_slots: the running slot count.
-__device__ __forceinline__ void place_items(uint32_t* off, uint32_t* n_slots, uint32_t t, uint32_t pairs,
+__device__ __forceinline__ void place_items(uint32_t* off, uint32_t* n_slots, uint32_t t, uint32_t pairs, uint32_t unit,
                                             uint32_t* __restrict__ order, const SplitPlan& sp) {
-    const uint32_t n = sp.seg ? split_segments(pairs, sp.unit) : 1u;
+    const uint32_t n = sp.seg ? split_segments(pairs, unit) : 1u;
     if (n == 1u) {
         const uint32_t i = atomicAdd(&off[item_bucket(pairs, -1, sp)], 1u);
         order[i] = t;
@@ -958,7 +961,7 @@ __device__ __forceinline__ void place_items(uint32_t* off, uint32_t* n_slots, ui
     sp.arrived[t] = 0u;
     sp.merged[t] = 0u;
     for (uint32_t g = 0; g < n; ++g) {
-        const uint32_t i = atomicAdd(&off[item_bucket(split_length(pairs, sp.unit), (int)g, sp)], 1u);
+        const uint32_t i = atomicAdd(&off[item_bucket(split_length(pairs, unit), (int)g, sp)], 1u);
         order[i] = t;
         sp.seg[i] = g;
         sp.dark[slot + g] = 0.0f;
@@ -966,6 +969,8 @@ __device__ __forceinline__ void place_items(uint32_t* off, uint32_t* n_slots, ui
 }
 
 __global__ __launch_bounds__(1024) void k_tile_order(const uint32_t* __restrict__ ranges, uint32_t n,
+                                                      const uint32_t* __restrict__ tile_view,
+                                                      const ViewParams* __restrict__ views,
                                                       uint32_t* __restrict__ order, SplitPlan sp) {
     __shared__ uint32_t cnt[kOrderBuckets];
     __shared__ uint32_t n_slots;
@@ -973,7 +978,7 @@ __global__ __launch_bounds__(1024) void k_tile_order(const uint32_t* __restrict_
     if (tid < kOrderBuckets) cnt[tid] = 0u;
     if (tid == 0) n_slots = 0u;
     __syncthreads();
-    for (uint32_t t = tid; t < n; t += blockDim.x) count_items(cnt, tile_pairs(ranges, t), sp);
+    for (uint32_t t = tid; t < n; t += blockDim.x) count_items(cnt, tile_pairs(ranges, t), tile_unit(views[tile_view[t]], sp), sp);
     __syncthreads();
     if (tid == 0) {
         uint32_t run = 0;
@@ -985,7 +990,8 @@ __global__ __launch_bounds__(1024) void k_tile_order(const uint32_t* __restrict_
         if (sp.seg) *sp.n_items = run;
     }
     __syncthreads();
-    for (uint32_t t = tid; t < n; t += blockDim.x) place_items(cnt, &n_slots, t, tile_pairs(ranges, t), order, sp);
+    for (uint32_t t = tid; t < n; t += blockDim.x)
+        place_items(cnt, &n_slots, t, tile_pairs(ranges, t), tile_unit(views[tile_view[t]], sp), order, sp);
 }
 
 // Scene-major order for batches of several scenes: the scenes one after
@@ -1009,8 +1015,9 @@ __global__ __launch_bounds__(1024) void k_tile_order_scenes(const uint32_t* __re
     if (tid == 0) n_slots = 0u;
     __syncthreads();
     for (uint32_t t = tid; t < n; t += blockDim.x) {
-        const uint32_t sc = views[tile_view[t]].scene, c = tile_pairs(ranges, t);
-        count_items(cnt + sc * kOrderBuckets, c, sp);
+        const ViewParams& vw = views[tile_view[t]];
+        const uint32_t sc = vw.scene, c = tile_pairs(ranges, t);
+        count_items(cnt + sc * kOrderBuckets, c, tile_unit(vw, sp), sp);
         atomicAdd(&s_pairs[sc], (unsigned long long)c);
     }
     __syncthreads();
@@ -1034,8 +1041,8 @@ __global__ __launch_bounds__(1024) void k_tile_order_scenes(const uint32_t* __re
     }
     __syncthreads();
     for (uint32_t t = tid; t < n; t += blockDim.x) {
-        const uint32_t sc = views[tile_view[t]].scene;
-        place_items(cnt + sc * kOrderBuckets, &n_slots, t, tile_pairs(ranges, t), order, sp);
+        const ViewParams& vw = views[tile_view[t]];
+        place_items(cnt + vw.scene * kOrderBuckets, &n_slots, t, tile_pairs(ranges, t), tile_unit(vw, sp), order, sp);
     }
 }
 
@@ -1047,8 +1054,10 @@ void launch_stamp_start(uint64_t* p, uint32_t n, hipStream_t s) {
     hipLaunchKernelGGL(k_stamp_start, dim3(1), dim3(64), 0, s, p, n);
 }
 
-void launch_tile_order(const uint32_t* ranges, uint32_t n_tiles, uint32_t* order, const SplitPlan& sp, hipStream_t s) {
-    if (n_tiles) hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, s, ranges, n_tiles, order, sp);
+void launch_tile_order(const uint32_t* ranges, uint32_t n_tiles, const uint32_t* tile_view, const ViewParams* views,
+                       uint32_t* order, const SplitPlan& sp, hipStream_t s) {
+    if (n_tiles)
+        hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, s, ranges, n_tiles, tile_view, views, order, sp);
 }
 
 bool launch_tile_order_scenes(const uint32_t* ranges, uint32_t n_tiles, const uint32_t* tile_view,

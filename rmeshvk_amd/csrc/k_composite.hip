@@ -750,15 +750,16 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     // list positions [done, end) of this workgroup
     uint32_t done = 0, end = count;
     bool skipped = false;
-    bool whole = AUX || !split.seg || split_segments(count, split.unit) == 1u;  // one workgroup, one list
+    const uint32_t unit = split.unit_for(vw.tiles_x * vw.tiles_y);
+    bool whole = AUX || !split.seg || split_segments(count, unit) == 1u;  // one workgroup, one list
     if (!whole) {
-        const uint32_t seg = split.seg[blockIdx.x], seg_len = split_length(count, split.unit);
+        const uint32_t seg = split.seg[blockIdx.x], seg_len = split_length(count, unit);
         const uint32_t slot = split.slot[gtile];
         done = seg * seg_len;
         end = min(done + seg_len, count);
         if (tid == 0) {  // (kept out of the registers until behind the loop)
             s_plan[0] = seg;
-            s_plan[1] = split_segments(count, split.unit);
+            s_plan[1] = split_segments(count, unit);
             s_plan[2] = seg_len;
             s_plan[3] = slot;
         }
@@ -1394,13 +1395,14 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     const uint32_t count = re > rs ? re - rs : 0u;
     // a list whose segment states the forward left is taken by segments too, the
     // first `merged` of them with the one behind
-    const bool by_seg = split.px && split_segments(count, split.unit) > 1u;
-    const uint32_t merged = by_seg ? split.merged[gtile] : 0u;
-    if (by_seg ? seg < merged : seg > 0u) return;
-    const uint32_t seg_len = by_seg ? split_length(count, split.unit) : count;
-    const uint32_t slot = by_seg ? split.slot[gtile] + seg : 0u;
     const uint32_t view = tile_view[gtile];
     const ViewParams& vw = views[view];
+    const uint32_t unit = split.unit_for(vw.tiles_x * vw.tiles_y);
+    const bool by_seg = split.px && split_segments(count, unit) > 1u;
+    const uint32_t merged = by_seg ? split.merged[gtile] : 0u;
+    if (by_seg ? seg < merged : seg > 0u) return;
+    const uint32_t seg_len = by_seg ? split_length(count, unit) : count;
+    const uint32_t slot = by_seg ? split.slot[gtile] + seg : 0u;
     const TileCtx tc = tile_ctx(vw, gtile);
     const float4* col_v = colors + vw.color_off;
     float* dcol_v = d_colors + 3 * vw.color_off;

@@ -352,10 +352,25 @@ void set_tiles(rmesh_renderer* h, uint32_t ts) {
     drop_graph(h);
 }
 
-// Pixel records of the segment slots for P pairs, at the tile size that needs most.
-uint64_t segment_pixels(uint64_t P) {
-    uint64_t n = 0;
-    for (uint32_t ts : {8u, 12u, 16u, 32u}) n = std::max<uint64_t>(n, split_slots(P, split_unit(ts)) * ts * ts);
+// The smallest segment unit of any of the renderer's views at tile size ts.
+uint32_t least_unit(const rmesh_renderer* h, uint32_t ts) {
+    for (const SceneHost& c : h->sc)
+        if ((uint64_t)((c.W + ts - 1) / ts) * ((c.H + ts - 1) / ts) <= kFewTiles) return split_unit_few(ts);
+    return split_unit(ts);
+}
+// Work items beyond one per tile, segment slots and their pixel records for P
+// pairs, each at the tile size that needs most.
+struct SegmentSizes {
+    uint64_t items = 0, slots = 0, pixels = 0;
+};
+SegmentSizes segment_sizes(const rmesh_renderer* h, uint64_t P) {
+    SegmentSizes n;
+    for (uint32_t ts : {8u, 12u, 16u, 32u}) {
+        const uint32_t unit = least_unit(h, ts);
+        n.items = std::max(n.items, split_extra_items(P, unit));
+        n.slots = std::max(n.slots, split_slots(P, unit));
+        n.pixels = std::max<uint64_t>(n.pixels, split_slots(P, unit) * ts * ts);
+    }
     return n;
 }
 
@@ -387,11 +402,11 @@ rmesh_status ensure_capacity(rmesh_renderer* h, uint64_t need) {
     HIP_TRY(dalloc(&h->vals_a, c));
     HIP_TRY(dalloc(&h->vals_b, c));
     HIP_TRY(dalloc(&h->hist, std::max(radix_hist_words((uint32_t)c), radix_hist_words32((uint32_t)c))));
-    // work items and segment slots of any tile size (most at the smallest)
-    HIP_TRY(dalloc(&h->tile_order, h->tile_cap + split_extra_items(c, split_unit(8))));
-    HIP_TRY(dalloc(&h->seg, h->tile_cap + split_extra_items(c, split_unit(8))));
-    HIP_TRY(dalloc(&h->seg_dark, split_slots(c, split_unit(8))));
-    HIP_TRY(dalloc(&h->seg_px, segment_pixels(c)));
+    const SegmentSizes ns = segment_sizes(h, c);
+    HIP_TRY(dalloc(&h->tile_order, h->tile_cap + ns.items));
+    HIP_TRY(dalloc(&h->seg, h->tile_cap + ns.items));
+    HIP_TRY(dalloc(&h->seg_dark, ns.slots));
+    HIP_TRY(dalloc(&h->seg_px, ns.pixels));
     h->cap = (uint32_t)c;
     drop_graph(h);
     return RMESH_OK;
@@ -413,7 +428,7 @@ rmesh_status ensure_checkpoints(rmesh_renderer* h, uint32_t V) {
         drop_graph(h);
     }
     if (!h->seg_stop) {
-        HIP_TRY(dalloc(&h->seg_stop, segment_pixels(h->cap)));
+        HIP_TRY(dalloc(&h->seg_stop, segment_sizes(h, h->cap).pixels));
         drop_graph(h);
     }
     if (!h->fin) HIP_TRY(dalloc(&h->fin, (size_t)h->pix_cap));
@@ -494,6 +509,7 @@ void launch_sort_stage(rmesh_renderer* h, hipStream_t s) {
 SplitPlan split_plan(const rmesh_renderer* h) {
     SplitPlan p;
     p.unit = split_unit(h->TS);
+    p.unit_few = split_unit_few(h->TS);
     p.seg = h->seg;
     p.n_items = h->n_seg_items;
     p.slot = h->seg_slot;
@@ -502,7 +518,7 @@ SplitPlan split_plan(const rmesh_renderer* h) {
     p.dark = h->seg_dark;
     p.px = h->seg_px;
     p.stop = h->seg_stop;
-    p.grid = h->n_gt + (uint32_t)split_extra_items(h->cap, p.unit);
+    p.grid = h->n_gt + (uint32_t)split_extra_items(h->cap, least_unit(h, h->TS));
     return p;
 }
 // split: long lists as several work items (the plain forward and the adjoint);
@@ -518,7 +534,7 @@ void launch_ranges_stage(rmesh_renderer* h, bool split, hipStream_t s) {
     if (h->scene_order != RMESH_SCENE_ORDER_BY_SCENE ||
         !launch_tile_order_scenes(h->ranges, h->n_gt, h->d_tile_view, h->d_views, (uint32_t)h->sc.size(),
                                   h->tile_order, sp, s))
-        launch_tile_order(h->ranges, h->n_gt, h->tile_order, sp, s);
+        launch_tile_order(h->ranges, h->n_gt, h->d_tile_view, h->d_views, h->tile_order, sp, s);
 }
 
 rmesh_status stage_binning_back(rmesh_renderer* h, uint32_t V, bool split) {

@@ -23,10 +23,19 @@ struct ViewParams;
 // grid (config C) 2 % at 6, 4 % at 4 and 1 % at 8 pairs a pixel, while 8 leaves
 // the clustered views 7 % slower than 6.
 constexpr uint32_t split_unit(uint32_t tile_size) { return 6u * tile_size * tile_size; }
+// A view of at most kFewTiles tiles (a 256 x 256 image at tile 12) leaves most of
+// the chip idle, and its workgroups, one a CU, issue far below the rate of
+// several: there the unit is one pair per pixel (2,000-point mesh: forward 87 ->
+// 55 us, adjoint 175 -> 105; two pairs 73 and 158).  On larger views that costs
+// 8 % (8 views at 512 x 512, where the grid is full).
+constexpr uint32_t kFewTiles = 512;
+constexpr uint32_t split_unit_few(uint32_t tile_size) {
+    return tile_size <= 16u ? tile_size * tile_size : split_unit(tile_size);
+}
 __host__ __device__ inline uint32_t split_length(uint32_t pairs, uint32_t unit) {
     if (pairs <= unit) return pairs;
     const uint32_t n = (pairs - 1u) / unit + 1u;
-    return ((pairs - 1u) / n + 1u + 31u) & ~31u;  // <= unit, a multiple of 32
+    return ((pairs - 1u) / n + 1u + 31u) & ~31u;  // a multiple of 32
 }
 __host__ __device__ inline uint32_t split_segments(uint32_t pairs, uint32_t unit) {
     return pairs <= unit ? 1u : (pairs - 1u) / split_length(pairs, unit) + 1u;
@@ -37,7 +46,8 @@ inline uint64_t split_extra_items(uint64_t P, uint32_t unit) { return P / unit; 
 inline uint64_t split_slots(uint64_t P, uint32_t unit) { return 2u * (P / unit) + 2u; }
 
 struct SplitPlan {
-    uint32_t unit = 0;
+    uint32_t unit = 0, unit_few = 0;
+    __host__ __device__ uint32_t unit_for(uint32_t view_tiles) const { return view_tiles <= kFewTiles ? unit_few : unit; }
     uint32_t* seg = nullptr;      // [item] segment of the item's tile; null: one item per tile, no segments
     uint32_t* n_items = nullptr;
     uint32_t* slot = nullptr;     // [tile] first segment slot (tiles with more than one segment)
@@ -104,7 +114,8 @@ void launch_ranges32(const uint32_t* keys, const uint32_t* n_ptr, uint32_t cap, 
 // Work items (tile, segment) in launch order, heaviest first: order[item] the
 // global tile, sp.seg[item] its segment; without a plan (sp.seg null) a
 // permutation of the tiles.
-void launch_tile_order(const uint32_t* ranges, uint32_t n_tiles, uint32_t* order, const SplitPlan& sp, hipStream_t s);
+void launch_tile_order(const uint32_t* ranges, uint32_t n_tiles, const uint32_t* tile_view, const ViewParams* views,
+                       uint32_t* order, const SplitPlan& sp, hipStream_t s);
 // Scene-major heaviest-first order (scenes by ascending pair count); false
 // (nothing launched) above 64 scenes.
 bool launch_tile_order_scenes(const uint32_t* ranges, uint32_t n_tiles, const uint32_t* tile_view,

@@ -1,5 +1,6 @@
-"""GPU: tile lists longer than a segment (6 pairs per pixel of the tile), which
-several workgroups composite, against the oracle's single pass over each list.
+"""GPU: tile lists longer than a segment (6 pairs per pixel of the tile, one in
+views of at most 512 tiles), which several workgroups composite, against the
+oracle's single pass over each list.
 
 - images within 1e-4 max-abs and checkpointed gradients within 1e-3 relative L2
   of the float32 oracle, the bounds of the unsegmented path, at every tile size,
@@ -39,11 +40,11 @@ def _scene(kind):
     return s
 
 
-def _renderer(s, **kw):
+def _renderer(s, w=W, h=H, **kw):
     from rmeshvk_amd import RMeshRenderer
 
     return RMeshRenderer(s["vertices"], s["indices"], s["base_colors"], s["densities"], s["color_grads"],
-                         s["circumdata"], W, H, device_id=0, **kw)
+                         s["circumdata"], w, h, device_id=0, **kw)
 
 
 def _longest(ref):
@@ -83,6 +84,28 @@ def test_segmented_lists_match_oracle(kind, ts):
     start = np.where(sat[..., None], np.asarray(img, np.float64).reshape(H, W, 4), fw["rgba"])
     go = orc.backward(f64, cam, W, H, ref["sorted_vals"], ref["ranges"], start, dl.astype(np.float64), ts,
                       dtype=np.float64)
+    for k in KEYS:
+        assert _rel(g[k], go[k]) <= 1e-3, (k, _rel(g[k], go[k]))
+
+
+@pytest.mark.parametrize("kind", ["plain", "saturating"])
+@pytest.mark.parametrize("ts,w", [(8, 200), (12, 280), (16, 376)])
+def test_segmented_lists_of_a_large_view_match_oracle(kind, ts, w):
+    """Views of more than 512 tiles, the mesh in a few of them (a wide angle: seen
+    from far away the float32 slabs lose digits on either side).  Image bound: the
+    float32 oracle is up to 8.6e-5 from its float64 evaluation here, so two float32
+    evaluations may be 2e-4 apart."""
+    s, cam = _scene(kind), fibonacci_cameras(2, 3.0, 140.0, w, w)[1]
+    ref = orc.render(s, cam, w, w, ts)
+    assert len(ref["ranges"].reshape(-1, 2)) > 512 and _longest(ref) > 2 * (6 * ts * ts)
+    dl = np.random.default_rng(ts).normal(0, 1e-2, (w, w, 4)).astype(np.float32)
+    fw = orc.forward(s, cam, w, w, ref["sorted_vals"], ref["ranges"], ts, want_checkpoints=True)
+    go = orc.backward(s, cam, w, w, ref["sorted_vals"], ref["ranges"], fw["rgba"], dl, ts, checkpoints=fw)
+    r = _renderer(s, w, w, tile_size=ts)
+    r.set_adjoint_mode("checkpoint")
+    img = r.forward_tiled(*cam)
+    assert np.abs(img - ref["rgba"]).max() <= 2e-4
+    g = r.backward(dl)
     for k in KEYS:
         assert _rel(g[k], go[k]) <= 1e-3, (k, _rel(g[k], go[k]))
 
