@@ -803,219 +803,219 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             if (u * NT + tid < 2 * B) s_ids[u * NT + tid] = idw[u];
     };
     for (;;) {
-    int nb = (int)min<uint32_t>(B, end - done);
-    if (nb > 0) {
-        TetFetch f;
-        QuadFetch qf;
-        uint32_t idw[IDW];
-        fetch(f, qf, sorted_vals + (re - 1 - done), -1, nb);
-        load_ids(idw, done);
-        stage(f, qf, idw, nb);
-    }
-    while (done < end) {
-        if (__syncthreads_and(!run || log_t < -13.8f)) break;
-        batch_layout<TS, B, false, true, CAP, NT>(L, nb, G.seg, G.starts());
-        __syncthreads();
-        const uint32_t nbp = L.nbp & 0xFFu;
-        const uint32_t nrec = L.nbp >> 8;
-        // The next batch's tet records and the ids of the one after it are
-        // loaded while this batch is processed, by every lane (a lane without a
-        // tet takes the last one) into registers declared here and consumed in
-        // this iteration: joined with an older value, by a branch or around
-        // the loop, they were copied right behind the loads, and every batch
-        // waited for the whole latency.
-        const uint32_t next = done + nbp;
-        const int nb_next = next_batch<B>(nbp, nb, end - next);
-        TetFetch f;
-        QuadFetch qf;
-        uint32_t idw[IDW];
-        fetch(f, qf, s_ids + nbp, 1, B);
-        load_ids(idw, next);
-        // record-parallel: intersection + volume integral of one (pixel, tet)
-        // record per lane
-        for (uint32_t j = tid; j < nrec; j += NT) {
-            const RecordRef c = record_at(G.seg, G.starts(), j);
-            const int p = c.row * TS + c.col;
-            const float4 rq = s_ray[p];
-            // saturated pixels skip the rest of the tile's tets (their compositing loop would)
-            if (rq.w != 0.0f) {
-                TetRegs T;
-                tet_regs(L, c.k, T);
-                const V3 rd = mk3(rq.x, rq.y, rq.z);
-                float t_min, t_max;
-                int fmin, fmax;
-                if (intersect(T, rd, min_t, t_min, t_max, fmin, fmax)) {
-                    Integral I;
-                    integral(T, rd, t_min, t_max, min_t != 0.0f ? min_t * dot3(T.g, rd) : 0.0f, 0.0f, I);
-                    s_pr[j] = make_float4(I.cp[0], I.cp[1], I.cp[2], I.od);
-                    if (AUX) {
-                        s_aux[0][j] = t_min;
-                        s_aux[1][j] = t_max;
-                        s_aux[2][j] = I.w0;
-                        s_ent[j] = t_min == kNoEntry ? 4u : (uint32_t)fmin;
-                    }
-                    atomicOr(&s_mask[p], 1ull << c.k);
-                }
-            }
+        int nb = (int)min<uint32_t>(B, end - done);
+        if (nb > 0) {
+            TetFetch f;
+            QuadFetch qf;
+            uint32_t idw[IDW];
+            fetch(f, qf, sorted_vals + (re - 1 - done), -1, nb);
+            load_ids(idw, done);
+            stage(f, qf, idw, nb);
         }
-        __syncthreads();
-        // pixel-sequential compositing in depth order over this pixel's covered
-        // tets (rasterize_compute.wgsl:336-463), two tets per round: both
-        // records' LDS reads (row base, then record) are in flight together,
-        // and only the arithmetic on log T stays sequential
-        if (run) {
-            unsigned long long m = s_mask[tid];
-            while (m != 0ull && !(log_t < -13.8f)) {
-                const uint32_t k0 = (uint32_t)__ffsll((long long)m) - 1u;
-                m &= m - 1ull;
-                const bool two = m != 0ull;
-                const uint32_t k1 = two ? (uint32_t)__ffsll((long long)m) - 1u : k0;
-                m &= m - 1ull;
-                const uint32_t slot0 = (L.rpref[k0 * SP + row] + (uint32_t)colp) & 0xFFFFu;
-                const uint32_t slot1 = (L.rpref[k1 * SP + row] + (uint32_t)colp) & 0xFFFFu;
-                const float4 q0 = s_pr[slot0], q1 = s_pr[slot1];
-                auto step = [&](uint32_t k, uint32_t slot, float4 q) {
-                    if constexpr (CK) {
-                        const uint32_t pos = done + k;
-                        for (; next_ck <= pos; next_ck += kCkGroup)
-                            store_shared(ck + (ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)), log_t);
-                        stop = pos + 1u;
-                    }
-                    // log_t is in [-13.8, 0] here: the reference's clamp of the
-                    // exponent and its test T >= 1e-6 (exp(-13.8) = 1.01e-6) hold
-                    const float Tj = fast_exp(log_t);
-                    const float od = q.w;
-                    cr = cr + q.x * Tj;
-                    cg = cg + q.y * Tj;
-                    cb = cb + q.z * Tj;
-                    log_t = log_t - od;
-                    if (AUX) {
-                        // rasterize_compute.wgsl:434-456
-                        float alpha_t = fast_safe_exp(-od);
-                        float alpha = 1.0f - alpha_t;
-                        float w0 = s_aux[2][slot];
-                        float w1 = 1.0f - (w0 + alpha_t);
-                        float t_min = s_aux[0][slot], t_max = s_aux[1][slot];
-                        int entry = (int)s_ent[slot];
-                        V3 en = mk3(0.f, 0.f, 0.f);
-                        if (entry < 4) {
-                            const float4 q = L.tr[k * L.TR + entry];
-                            en = normalize3(neg3(mk3(q.x, q.y, q.z)));
+        while (done < end) {
+            if (__syncthreads_and(!run || log_t < -13.8f)) break;
+            batch_layout<TS, B, false, true, CAP, NT>(L, nb, G.seg, G.starts());
+            __syncthreads();
+            const uint32_t nbp = L.nbp & 0xFFu;
+            const uint32_t nrec = L.nbp >> 8;
+            // The next batch's tet records and the ids of the one after it are
+            // loaded while this batch is processed, by every lane (a lane without a
+            // tet takes the last one) into registers declared here and consumed in
+            // this iteration: joined with an older value, by a branch or around
+            // the loop, they were copied right behind the loads, and every batch
+            // waited for the whole latency.
+            const uint32_t next = done + nbp;
+            const int nb_next = next_batch<B>(nbp, nb, end - next);
+            TetFetch f;
+            QuadFetch qf;
+            uint32_t idw[IDW];
+            fetch(f, qf, s_ids + nbp, 1, B);
+            load_ids(idw, next);
+            // record-parallel: intersection + volume integral of one (pixel, tet)
+            // record per lane
+            for (uint32_t j = tid; j < nrec; j += NT) {
+                const RecordRef c = record_at(G.seg, G.starts(), j);
+                const int p = c.row * TS + c.col;
+                const float4 rq = s_ray[p];
+                // saturated pixels skip the rest of the tile's tets (their compositing loop would)
+                if (rq.w != 0.0f) {
+                    TetRegs T;
+                    tet_regs(L, c.k, T);
+                    const V3 rd = mk3(rq.x, rq.y, rq.z);
+                    float t_min, t_max;
+                    int fmin, fmax;
+                    if (intersect(T, rd, min_t, t_min, t_max, fmin, fmax)) {
+                        Integral I;
+                        integral(T, rd, t_min, t_max, min_t != 0.0f ? min_t * dot3(T.g, rd) : 0.0f, 0.0f, I);
+                        s_pr[j] = make_float4(I.cp[0], I.cp[1], I.cp[2], I.od);
+                        if (AUX) {
+                            s_aux[0][j] = t_min;
+                            s_aux[1][j] = t_max;
+                            s_aux[2][j] = I.w0;
+                            s_ent[j] = t_min == kNoEntry ? 4u : (uint32_t)fmin;
                         }
-                        float depth_premul = w0 * t_max + w1 * t_min;
-                        float ta = Tj * alpha;
-                        nx = nx + ta * en.x;
-                        ny = ny + ta * en.y;
-                        nz = nz + ta * en.z;
-                        dep = dep + Tj * depth_premul;
-                        float wt = alpha * Tj;
-                        float c_mid = (t_min + t_max) * 0.5f;
-                        float wc = wt * c_mid;
-                        e0 = e0 + wt;
-                        e1 = e1 + (wt > 1e-20f ? wt * logf(wt) : 0.0f);
-                        e2 = e2 + wt * c_mid;
-                        e3 = e3 + (wc > 1e-20f ? wc * logf(wc) : 0.0f);
-                    }
-                };
-                step(k0, slot0, q0);
-                if (two && !(log_t < -13.8f)) step(k1, slot1, q1);
-            }
-            if (log_t < -13.8f) s_ray[tid].w = 0.0f;
-            else if constexpr (CK)  // positions up to the batch's end that this pixel passed uncovered
-                for (; next_ck <= next && next_ck < count; next_ck += kCkGroup)
-                    store_shared(ck + (ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)), log_t);
-        }
-        // The next batch's LDS image follows the pixel phase without a barrier
-        // between them (that phase reads only the row bases and the pair
-        // records, which the image does not touch; each lane clears its own
-        // pixel's mask after reading it).  The aux outputs' phase reads the
-        // face planes too.
-        if (AUX) __syncthreads();
-        if (nb_next > 0) stage(f, qf, idw, nb_next);
-        done = next;
-        nb = nb_next;
-    }
-    if (whole) break;
-    const uint32_t seg = s_plan[0], n_seg = s_plan[1], seg_len = s_plan[2];
-    float4* const px = split.px + ((uint64_t)s_plan[3] * (TS * TS) + (uint64_t)tid);
-    if (!joined) {
-        // One segment: its pixel states go to its slot, and all but the tile's
-        // last workgroup to get here are done.  (log T of a segment that was
-        // skipped, or in which the pixel saturated by itself, is short of its
-        // pairs: below -13.8.)
-        if (tid < TS * TS) {
-            store_shared(px + (uint64_t)seg * (TS * TS), make_float4(cr, cg, cb, skipped ? -1e30f : log_t));
-            if constexpr (CK) store_shared(split.stop + (px - split.px) + (uint64_t)seg * (TS * TS), stop);
-        }
-        float d = active ? (skipped ? 0.0f : log_t) : -3.0e38f;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) d = fmaxf(d, __shfl_xor(d, o, 64));
-        __syncthreads();  // s_red's readers at the start are done
-        if ((tid & 63) == 0) s_red[tid >> 6] = d;
-        drain_stores();  // this wave's states and checkpoints
-        __syncthreads();
-        if (tid == 0) {
-            for (int w = 1; w < NT / 64; ++w) d = fmaxf(d, s_red[w]);
-            store_shared(split.dark + s_plan[3] + seg, d);
-            drain_stores();
-            s_arrived = (int)atomicAdd(split.arrived + gtile, 1u);
-        }
-        __syncthreads();
-        if (s_arrived != (int)n_seg - 1) return;
-        joined = true;
-        // Front to back: log T at each segment's end, colour and log T of the
-        // pixel, up to the segment in which it saturates (s_sat).
-        uint32_t sat = n_seg;
-        cr = cg = cb = log_t = 0.0f;
-        stop = 0u;
-        if (active) {
-            constexpr int U = 4;
-            for (uint32_t g0 = 0; g0 < n_seg && sat == n_seg; g0 += U) {
-                float4 q[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) q[u] = load_shared(px + (uint64_t)min(g0 + u, n_seg - 1u) * (TS * TS));
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const uint32_t g = g0 + u;
-                    if (g >= n_seg || sat < n_seg) continue;
-                    const float lt = log_t + q[u].w;
-                    store_shared(&px[(uint64_t)g * (TS * TS)].w, lt);
-                    if (lt < -13.8f) sat = g;
-                    if (sat == n_seg || g == 0u) {  // (in the first segment the pixel stopped where it has to)
-                        const float w = expf(log_t);
-                        cr += q[u].x * w;
-                        cg += q[u].y * w;
-                        cb += q[u].z * w;
-                        log_t = lt;
-                        if constexpr (CK)
-                            stop = max(stop, load_shared(split.stop + (px - split.px) + (uint64_t)g * (TS * TS)));
+                        atomicOr(&s_mask[p], 1ull << c.k);
                     }
                 }
             }
+            __syncthreads();
+            // pixel-sequential compositing in depth order over this pixel's covered
+            // tets (rasterize_compute.wgsl:336-463), two tets per round: both
+            // records' LDS reads (row base, then record) are in flight together,
+            // and only the arithmetic on log T stays sequential
+            if (run) {
+                unsigned long long m = s_mask[tid];
+                while (m != 0ull && !(log_t < -13.8f)) {
+                    const uint32_t k0 = (uint32_t)__ffsll((long long)m) - 1u;
+                    m &= m - 1ull;
+                    const bool two = m != 0ull;
+                    const uint32_t k1 = two ? (uint32_t)__ffsll((long long)m) - 1u : k0;
+                    m &= m - 1ull;
+                    const uint32_t slot0 = (L.rpref[k0 * SP + row] + (uint32_t)colp) & 0xFFFFu;
+                    const uint32_t slot1 = (L.rpref[k1 * SP + row] + (uint32_t)colp) & 0xFFFFu;
+                    const float4 q0 = s_pr[slot0], q1 = s_pr[slot1];
+                    auto step = [&](uint32_t k, uint32_t slot, float4 q) {
+                        if constexpr (CK) {
+                            const uint32_t pos = done + k;
+                            for (; next_ck <= pos; next_ck += kCkGroup)
+                                store_shared(ck + (ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)), log_t);
+                            stop = pos + 1u;
+                        }
+                        // log_t is in [-13.8, 0] here: the reference's clamp of the
+                        // exponent and its test T >= 1e-6 (exp(-13.8) = 1.01e-6) hold
+                        const float Tj = fast_exp(log_t);
+                        const float od = q.w;
+                        cr = cr + q.x * Tj;
+                        cg = cg + q.y * Tj;
+                        cb = cb + q.z * Tj;
+                        log_t = log_t - od;
+                        if (AUX) {
+                            // rasterize_compute.wgsl:434-456
+                            float alpha_t = fast_safe_exp(-od);
+                            float alpha = 1.0f - alpha_t;
+                            float w0 = s_aux[2][slot];
+                            float w1 = 1.0f - (w0 + alpha_t);
+                            float t_min = s_aux[0][slot], t_max = s_aux[1][slot];
+                            int entry = (int)s_ent[slot];
+                            V3 en = mk3(0.f, 0.f, 0.f);
+                            if (entry < 4) {
+                                const float4 q = L.tr[k * L.TR + entry];
+                                en = normalize3(neg3(mk3(q.x, q.y, q.z)));
+                            }
+                            float depth_premul = w0 * t_max + w1 * t_min;
+                            float ta = Tj * alpha;
+                            nx = nx + ta * en.x;
+                            ny = ny + ta * en.y;
+                            nz = nz + ta * en.z;
+                            dep = dep + Tj * depth_premul;
+                            float wt = alpha * Tj;
+                            float c_mid = (t_min + t_max) * 0.5f;
+                            float wc = wt * c_mid;
+                            e0 = e0 + wt;
+                            e1 = e1 + (wt > 1e-20f ? wt * logf(wt) : 0.0f);
+                            e2 = e2 + wt * c_mid;
+                            e3 = e3 + (wc > 1e-20f ? wc * logf(wc) : 0.0f);
+                        }
+                    };
+                    step(k0, slot0, q0);
+                    if (two && !(log_t < -13.8f)) step(k1, slot1, q1);
+                }
+                if (log_t < -13.8f) s_ray[tid].w = 0.0f;
+                else if constexpr (CK)  // positions up to the batch's end that this pixel passed uncovered
+                    for (; next_ck <= next && next_ck < count; next_ck += kCkGroup)
+                        store_shared(ck + (ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)), log_t);
+            }
+            // The next batch's LDS image follows the pixel phase without a barrier
+            // between them (that phase reads only the row bases and the pair
+            // records, which the image does not touch; each lane clears its own
+            // pixel's mask after reading it).  The aux outputs' phase reads the
+            // face planes too.
+            if (AUX) __syncthreads();
+            if (nb_next > 0) stage(f, qf, idw, nb_next);
+            done = next;
+            nb = nb_next;
         }
-        if (tid < TS * TS) s_sat[tid] = sat;
-        // the plan's counters are zero between forwards
-        for (uint32_t g = tid; g < n_seg; g += NT) store_shared(split.dark + s_plan[3] + g, 0.0f);
-        if (tid == 0) {
-            store_shared(split.arrived + gtile, 0u);
-            s_merge = 0;
+        if (whole) break;
+        const uint32_t seg = s_plan[0], n_seg = s_plan[1], seg_len = s_plan[2];
+        float4* const px = split.px + ((uint64_t)s_plan[3] * (TS * TS) + (uint64_t)tid);
+        if (!joined) {
+            // One segment: its pixel states go to its slot, and all but the tile's
+            // last workgroup to get here are done.  (log T of a segment that was
+            // skipped, or in which the pixel saturated by itself, is short of its
+            // pairs: below -13.8.)
+            if (tid < TS * TS) {
+                store_shared(px + (uint64_t)seg * (TS * TS), make_float4(cr, cg, cb, skipped ? -1e30f : log_t));
+                if constexpr (CK) store_shared(split.stop + (px - split.px) + (uint64_t)seg * (TS * TS), stop);
+            }
+            float d = active ? (skipped ? 0.0f : log_t) : -3.0e38f;
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) d = fmaxf(d, __shfl_xor(d, o, 64));
+            __syncthreads();  // s_red's readers at the start are done
+            if ((tid & 63) == 0) s_red[tid >> 6] = d;
+            drain_stores();  // this wave's states and checkpoints
+            __syncthreads();
+            if (tid == 0) {
+                for (int w = 1; w < NT / 64; ++w) d = fmaxf(d, s_red[w]);
+                store_shared(split.dark + s_plan[3] + seg, d);
+                drain_stores();
+                s_arrived = (int)atomicAdd(split.arrived + gtile, 1u);
+            }
+            __syncthreads();
+            if (s_arrived != (int)n_seg - 1) return;
+            joined = true;
+            // Front to back: log T at each segment's end, colour and log T of the
+            // pixel, up to the segment in which it saturates (s_sat).
+            uint32_t sat = n_seg;
+            cr = cg = cb = log_t = 0.0f;
+            stop = 0u;
+            if (active) {
+                constexpr int U = 4;
+                for (uint32_t g0 = 0; g0 < n_seg && sat == n_seg; g0 += U) {
+                    float4 q[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) q[u] = load_shared(px + (uint64_t)min(g0 + u, n_seg - 1u) * (TS * TS));
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const uint32_t g = g0 + u;
+                        if (g >= n_seg || sat < n_seg) continue;
+                        const float lt = log_t + q[u].w;
+                        store_shared(&px[(uint64_t)g * (TS * TS)].w, lt);
+                        if (lt < -13.8f) sat = g;
+                        if (sat == n_seg || g == 0u) {  // (in the first segment the pixel stopped where it has to)
+                            const float w = expf(log_t);
+                            cr += q[u].x * w;
+                            cg += q[u].y * w;
+                            cb += q[u].z * w;
+                            log_t = lt;
+                            if constexpr (CK)
+                                stop = max(stop, load_shared(split.stop + (px - split.px) + (uint64_t)g * (TS * TS)));
+                        }
+                    }
+                }
+            }
+            if (tid < TS * TS) s_sat[tid] = sat;
+            // the plan's counters are zero between forwards
+            for (uint32_t g = tid; g < n_seg; g += NT) store_shared(split.dark + s_plan[3] + g, 0.0f);
+            if (tid == 0) {
+                store_shared(split.arrived + gtile, 0u);
+                s_merge = 0;
+            }
         }
-    }
-    // Pixels that saturate in a later segment run in it once more, segment by
-    // segment, from the pixel state in front of it; their colour starts from 0.
-    if (tid == 0) s_first = (int)n_seg;
-    __syncthreads();
-    const uint32_t sat = tid < TS * TS ? s_sat[tid] : 0u;
-    if (active && sat > again && sat < n_seg) atomicMin(&s_first, (int)sat);
-    __syncthreads();
-    again = (uint32_t)s_first;
-    if (again == n_seg) break;
-    run = active && sat == again;
-    if (run) cr = cg = cb = 0.0f;
-    if (tid < TS * TS) s_ray[tid].w = run ? 1.0f : 0.0f;
-    done = again * seg_len;
-    end = min(done + seg_len, ranges[2ull * gtile + 1] - ranges[2ull * gtile]);
-    next_ck = 0xFFFFFFFFu;  // the segment's checkpoints stand
+        // Pixels that saturate in a later segment run in it once more, segment by
+        // segment, from the pixel state in front of it; their colour starts from 0.
+        if (tid == 0) s_first = (int)n_seg;
+        __syncthreads();
+        const uint32_t sat = tid < TS * TS ? s_sat[tid] : 0u;
+        if (active && sat > again && sat < n_seg) atomicMin(&s_first, (int)sat);
+        __syncthreads();
+        again = (uint32_t)s_first;
+        if (again == n_seg) break;
+        run = active && sat == again;
+        if (run) cr = cg = cb = 0.0f;
+        if (tid < TS * TS) s_ray[tid].w = run ? 1.0f : 0.0f;
+        done = again * seg_len;
+        end = min(done + seg_len, ranges[2ull * gtile + 1] - ranges[2ull * gtile]);
+        next_ck = 0xFFFFFFFFu;  // the segment's checkpoints stand
     }
     if (!whole) {
         // Back to front: every segment's slot gets what lies behind the segment, the
@@ -1354,7 +1354,8 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     const float4* __restrict__ rec, const float4* __restrict__ colors,
     const uint32_t* __restrict__ sorted_vals, const uint32_t* __restrict__ ranges,
     const ViewParams* __restrict__ views, const uint32_t* __restrict__ tile_view, const uint32_t* __restrict__ tile_order,
-    const SplitPlan split, const float* __restrict__ rgba, const float* __restrict__ dl_img, const float* __restrict__ gt, uint32_t loss_type,
+    const SplitPlan split, const float* __restrict__ rgba, const float* __restrict__ dl_img,
+    const float* __restrict__ gt, uint32_t loss_type,
     float* __restrict__ loss_partial, float* __restrict__ tet_g, float* __restrict__ d_colors,
     const float* __restrict__ ck, const float2* __restrict__ fin, uint64_t* __restrict__ scene_done) {
     constexpr int TS = C::TS, NT = C::NT, B = C::B, CAP = C::CAP, SP = TS + 1, NW = NT / 64, NREC = C::NREC;
@@ -1659,8 +1660,8 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                     const int p = (int)((r_m[n] >> 6) & 1023u);
                     const float4 rq = s_ray[p];
                     const float2 dq = s_dc[p];
-                    pair_grad<TS, B>(L, key, cam, mk3(rq.x, rq.y, rq.z), rq.w, dq.x, dq.y, -q.x, q.y, r_t0[n], r_t1[n], r_at[n], r_ph[n], (int)((r_m[n] >> 16) & 3u), (int)((r_m[n] >> 18) & 3u),
-                                     acc);
+                    pair_grad<TS, B>(L, key, cam, mk3(rq.x, rq.y, rq.z), rq.w, dq.x, dq.y, -q.x, q.y, r_t0[n], r_t1[n],
+                                     r_at[n], r_ph[n], (int)((r_m[n] >> 16) & 3u), (int)((r_m[n] >> 18) & 3u), acc);
                     have = true;
                 }
             }
@@ -2094,8 +2095,9 @@ __global__ __launch_bounds__(C::NT) void k_error(const float4* __restrict__ rec,
     }
 }
 
-// (30,000 points in clusters at 803 x 601, tile 12: B 48 with CAP 768 and the heaviest tiles first 0.53 ms (0.62 in tile order), B 32
-// with 512 0.73; with LDS atomics for the results 0.83.)
+// (30,000 points in clusters at 803 x 601, tile 12: B 48 with CAP 768 and the
+// heaviest tiles first 0.53 ms (0.62 in tile order), B 32 with 512 0.73; with LDS
+// atomics for the results 0.83.)
 template <int TS>
 static void err_launch(const ErrArgs& a, hipStream_t s) {
     using C = FwdCfg<TS, (TS == 12 || TS == 16 ? 48 : 32), (TS > 16 ? TS * TS : TS == 8 ? 512 : 768), 3>;
@@ -3186,7 +3188,8 @@ __global__ __launch_bounds__(256) void k_vertex_gather(const uint32_t* __restric
 // for the sums, the search repeated in phase C and the records' loads waited for
 // in every batch, B 32, 1.89 and 0.93).
 template <int TS>
-using IvlCfg = FwdCfg<TS, (TS > 16 ? 16 : TS == 8 ? 32 : 48), (TS > 16 ? TS * TS : TS == 8 ? 512 : 3 * ((TS * TS + 63) / 64 * 64)), 1>;
+using IvlCfg = FwdCfg<TS, (TS > 16 ? 16 : TS == 8 ? 32 : 48),
+                      (TS > 16 ? TS * TS : TS == 8 ? 512 : 3 * ((TS * TS + 63) / 64 * 64)), 1>;
 
 template <int TS>
 static void ivl_bwd_launch(const IvlBwdArgs& a, hipStream_t s) {
