@@ -1019,21 +1019,23 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     }
     if (!whole) {
         // Back to front: every segment's slot gets what lies behind the segment, the
-        // adjoint's start: colour and log T.  The undo of a saturated pixel begins
-        // at its alpha and passes over the pairs behind its stop too, so that it
-        // reaches log T = 0, and stays there, before the front: from a segment in
-        // which it does (or whose sum is short) on, the adjoint takes the rest of
-        // the list in one.
+        // adjoint's start: colour and log T.  Without checkpoints log T is the undo's,
+        // which starts at log(1 - alpha) whatever the list's length, adds the pairs'
+        // optical depths from the back (a saturated pixel's behind its stop too) and
+        // stays at 0 once it reaches 0.  Where it gets there before the pixel's first
+        // pair (or a segment's sum is short), the colours in front are not the
+        // forward's: from that segment on, the adjoint takes the rest of the list in one.
         const uint32_t n_seg = s_plan[1];
         float4* const px = split.px + ((uint64_t)s_plan[3] * (TS * TS) + (uint64_t)tid);
         const uint32_t sat = tid < TS * TS ? s_sat[tid] : 0u;
         uint32_t merge = 0u;
         if (active) {
-            const bool undo = !CK && sat < n_seg;
+            constexpr bool undo = !CK;
             const float end_r = cr, end_g = cg, end_b = cb;  // of the saturating segment
             float br = 0.f, bg = 0.f, bb = 0.f;              // behind the segment
             float tr = 0.f, tg = 0.f, tb = 0.f;              // the pixel's, if it ran again
             float x = undo ? logf(fmaxf(1.0f - (1.0f - safe_exp(log_t)), 1e-20f)) : 0.0f;
+            float shift = 0.0f;  // undo: its log T minus the forward's, from the saturating segment (or the end) on
             bool lost = false;
             constexpr int U = 4;
             for (int g0 = (int)n_seg - 1; g0 >= 0; g0 -= U) {
@@ -1054,12 +1056,16 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                         tb += q[u].z * w;
                     }
                     if (undo) {
-                        const float sum = (uint32_t)g <= sat ? q[u].w - front : q[u].w;
-                        const float xf = x - sum;
-                        if (!lost && (sum < -13.79f || xf > 0.0f)) {
+                        const bool known = (uint32_t)g <= sat;  // q.w and front are log T seen from the camera
+                        const float sum = known ? q[u].w - front : q[u].w;
+                        if ((uint32_t)g == min(sat, n_seg - 1u)) shift = x - q[u].w;
+                        float xf = known ? front + shift : x - sum;
+                        // (up to 1e-6 above 0 is rounding; with front 0 there is no pair of the pixel in front)
+                        if (!lost && (sum < -13.79f || (xf > 1e-6f && !(known && front == 0.0f)))) {
                             lost = true;
                             merge = (uint32_t)g;
                         }
+                        xf = fminf(xf, 0.0f);
                         if (!lost) {
                             const float wx = expf(xf);
                             br += q[u].x * wx;
