@@ -697,7 +697,15 @@ __device__ __forceinline__ void drain_stores() { asm volatile("s_waitcnt vmcnt(0
 // 32 j it reaches (coalesced: the tile's pixels write one 4 TS^2-byte slot),
 // and at the end its final log T and stop position (1 + the last position it
 // composited).
-template <class C, bool AUX, bool CK>
+//
+// ONE: a list's first segment composites all of it, in the rounding of an unsplit
+// list, and leaves the segments' states for the adjoint.  The steps with the L1
+// loss need that: their gradient is the sign of image - target, and joining the
+// segments moves a third of the channels by an ulp, of which one in some 10^6
+// changes its sign (one such channel: 2.1e-4 of the vertex gradients of 8 views).
+// A saturated pixel's sums behind its stop are not known here; its tile's undo
+// takes the list in one.
+template <class C, bool AUX, bool CK, bool ONE>
 __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE))) void k_forward(
     const float4* __restrict__ rec, const float4* __restrict__ colors,
     const uint32_t* __restrict__ sorted_vals, const uint32_t* __restrict__ ranges, const ViewParams* __restrict__ views,
@@ -744,6 +752,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     }
     float cr = 0.f, cg = 0.f, cb = 0.f, log_t = 0.f;
     float nx = 0.f, ny = 0.f, nz = 0.f, dep = 0.f, e0 = 0.f, e1 = 0.f, e2 = 0.f, e3 = 0.f;
+    float sr = 0.f, sg = 0.f, sb = 0.f, front_lt = 0.f;  // ONE: the segment's colour, log T in front of it
 
     const uint32_t rs = ranges[2ull * gtile], re = ranges[2ull * gtile + 1];
     const uint32_t count = re > rs ? re - rs : 0u;
@@ -755,6 +764,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     if (!whole) {
         const uint32_t seg = split.seg[blockIdx.x], seg_len = split_length(count, unit);
         const uint32_t slot = split.slot[gtile];
+        if (ONE && seg > 0u) return;
         done = seg * seg_len;
         end = min(done + seg_len, count);
         if (tid == 0) {  // (kept out of the registers until behind the loop)
@@ -762,6 +772,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             s_plan[1] = split_segments(count, unit);
             s_plan[2] = seg_len;
             s_plan[3] = slot;
+            if constexpr (ONE) s_merge = 0;
         }
         // nothing to do once the segments in front are known to saturate every
         // pixel (with a margin for the rounding of the sum): their last pixel
@@ -878,7 +889,8 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                         if constexpr (CK) {
                             const uint32_t pos = done + k;
                             for (; next_ck <= pos; next_ck += kCkGroup)
-                                store_shared(ck + (ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)), log_t);
+                                store_shared(ck + (ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)),
+                                             ONE ? log_t - front_lt : log_t);
                             stop = pos + 1u;
                         }
                         // log_t is in [-13.8, 0] here: the reference's clamp of the
@@ -889,6 +901,11 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                         cg = cg + q.y * Tj;
                         cb = cb + q.z * Tj;
                         log_t = log_t - od;
+                        if constexpr (ONE) {
+                            sr = sr + q.x * Tj;
+                            sg = sg + q.y * Tj;
+                            sb = sb + q.z * Tj;
+                        }
                         if (AUX) {
                             // rasterize_compute.wgsl:434-456
                             float alpha_t = fast_safe_exp(-od);
@@ -923,7 +940,8 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                 if (log_t < -13.8f) s_ray[tid].w = 0.0f;
                 else if constexpr (CK)  // positions up to the batch's end that this pixel passed uncovered
                     for (; next_ck <= next && next_ck < count; next_ck += kCkGroup)
-                        store_shared(ck + (ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)), log_t);
+                        store_shared(ck + (ck_base + (uint64_t)(next_ck / kCkGroup) * (TS * TS)),
+                                     ONE ? log_t - front_lt : log_t);
             }
             // The next batch's LDS image follows the pixel phase without a barrier
             // between them (that phase reads only the row bases and the pair
@@ -938,6 +956,25 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         if (whole) break;
         const uint32_t seg = s_plan[0], n_seg = s_plan[1], seg_len = s_plan[2];
         float4* const px = split.px + ((uint64_t)s_plan[3] * (TS * TS) + (uint64_t)tid);
+        if constexpr (ONE) {
+            // the segment's own colour, log T at its end; all further ones empty
+            // once no pixel composites any more
+            const bool last = done < end || end == count;
+            if (tid < TS * TS) {
+                const float w = expf(-fmaxf(front_lt, -14.0f));  // (below, the pixel is saturated: no colour)
+                store_shared(px + (uint64_t)again * (TS * TS), make_float4(sr * w, sg * w, sb * w, log_t));
+                if (last)
+                    for (uint32_t g = again + 1u; g < n_seg; ++g)
+                        store_shared(px + (uint64_t)g * (TS * TS), make_float4(0.f, 0.f, 0.f, log_t));
+            }
+            if (last) break;
+            ++again;
+            sr = sg = sb = 0.0f;
+            front_lt = log_t;
+            done = end;
+            end = min(done + seg_len, count);
+            continue;
+        }
         if (!joined) {
             // One segment: its pixel states go to its slot, and all but the tile's
             // last workgroup to get here are done.  (log T of a segment that was
@@ -1027,7 +1064,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         // forward's: from that segment on, the adjoint takes the rest of the list in one.
         const uint32_t n_seg = s_plan[1];
         float4* const px = split.px + ((uint64_t)s_plan[3] * (TS * TS) + (uint64_t)tid);
-        const uint32_t sat = tid < TS * TS ? s_sat[tid] : 0u;
+        const uint32_t sat = ONE ? n_seg : tid < TS * TS ? s_sat[tid] : 0u;
         uint32_t merge = 0u;
         if (active) {
             constexpr bool undo = !CK;
@@ -1036,7 +1073,8 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             float tr = 0.f, tg = 0.f, tb = 0.f;              // the pixel's, if it ran again
             float x = undo ? logf(fmaxf(1.0f - (1.0f - safe_exp(log_t)), 1e-20f)) : 0.0f;
             float shift = 0.0f;  // undo: its log T minus the forward's, from the saturating segment (or the end) on
-            bool lost = false;
+            bool lost = ONE && undo && log_t < -13.8f;
+            if (lost) merge = n_seg - 1u;
             constexpr int U = 4;
             for (int g0 = (int)n_seg - 1; g0 >= 0; g0 -= U) {
                 float4 q[U + 1];
@@ -1708,18 +1746,19 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
 template <class C>
 static void fwd_launch(const FwdArgs& a, hipStream_t s) {
     const dim3 grid(a.split.seg ? a.split.grid : a.num_gtiles);
+    auto launch = [&](auto kernel, float* aux, float* ck, float2* fin) {
+        hipLaunchKernelGGL(kernel, grid, dim3(C::NT), 0, s, a.rec, a.colors, a.sorted_vals, a.ranges, a.views,
+                           a.tile_view, a.tile_order, a.split, a.rgba, aux, ck, fin);
+    };
+    const bool one = a.one_pass && a.split.seg;
     if (a.aux)  // the aux outputs serve the forward-only API: no checkpoints with them
-        hipLaunchKernelGGL((k_forward<C, true, false>), grid, dim3(C::NT), 0, s, a.rec, a.colors,
-                           a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order, a.split,
-                           a.rgba, a.aux, nullptr, nullptr);
+        launch(k_forward<C, true, false, false>, a.aux, nullptr, nullptr);
     else if (a.ck)
-        hipLaunchKernelGGL((k_forward<C, false, true>), grid, dim3(C::NT), 0, s, a.rec, a.colors,
-                           a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order, a.split,
-                           a.rgba, nullptr, a.ck, a.fin);
+        one ? launch(k_forward<C, false, true, true>, nullptr, a.ck, a.fin)
+            : launch(k_forward<C, false, true, false>, nullptr, a.ck, a.fin);
     else
-        hipLaunchKernelGGL((k_forward<C, false, false>), grid, dim3(C::NT), 0, s, a.rec, a.colors,
-                           a.sorted_vals, a.ranges, a.views, a.tile_view, a.tile_order, a.split,
-                           a.rgba, nullptr, nullptr, nullptr);
+        one ? launch(k_forward<C, false, false, true>, nullptr, nullptr, nullptr)
+            : launch(k_forward<C, false, false, false>, nullptr, nullptr, nullptr);
 }
 
 // Forward geometries.  The defaults measured best over a batch of small views,

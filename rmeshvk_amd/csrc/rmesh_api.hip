@@ -547,8 +547,8 @@ rmesh_status stage_binning_back(rmesh_renderer* h, uint32_t V, bool split) {
 
 const uint32_t* sorted_vals(const rmesh_renderer* h) { return h->sorted_in_b ? h->vals_b : h->vals_a; }
 
-
-rmesh_status stage_forward(rmesh_renderer* h, uint32_t V, bool want_aux) {
+// one_pass: FwdArgs::one_pass, for the steps with the L1 loss (loss type 0).
+rmesh_status stage_forward(rmesh_renderer* h, uint32_t V, bool want_aux, bool one_pass) {
     FwdArgs a;
     a.rec = h->rec;
     a.colors = h->colors;
@@ -559,6 +559,7 @@ rmesh_status stage_forward(rmesh_renderer* h, uint32_t V, bool want_aux) {
     a.num_gtiles = h->n_gt;
     a.tile_order = h->tile_order;
     if (h->order_split) a.split = split_plan(h);
+    a.one_pass = one_pass;
     a.rgba = h->rgba;
     a.aux = want_aux ? h->aux : nullptr;
     const bool ck = h->adj_ck && !want_aux;  // the aux forward keeps no checkpoints
@@ -725,7 +726,7 @@ rmesh_status record_stage(rmesh_renderer* h, int stage, uint32_t V, const float*
         case 3:
             launch_ranges_stage(h, true, s);
             return RMESH_OK;
-        case 4: return stage_forward(h, V, false);
+        case 4: return stage_forward(h, V, false, loss_type == 0);
         case 5: return stage_backward(h, V, nullptr, gt, loss_type);
         default: return stage_adam(h, V, lr_v, lr_d, lr_g, lr_sh);
     }
@@ -1010,7 +1011,7 @@ static rmesh_status forward_views(rmesh_renderer* h, uint32_t V, const float* ca
         HIP_TRY(dalloc(&h->aux, 8ull * h->W * h->H * h->max_views));
         h->aux_alloc = true;
     }
-    st = stage_forward(h, V, want_aux);
+    st = stage_forward(h, V, want_aux, false);
     if (st != RMESH_OK) return st;
     h->last_views = V;
     h->have_forward = true;
@@ -1540,7 +1541,7 @@ static rmesh_status autotune_layout(rmesh_renderer* h, const uint32_t* per_user,
         for (int f = 0; f < fwd_variants(ts) && result == RMESH_OK; ++f) {
             h->fwd_var = f;
             float t = 0.0f;
-            result = timed([&]() { return stage_forward(h, V, false); }, t);
+            result = timed([&]() { return stage_forward(h, V, false, loss_type == 0); }, t);
             if (t < t_fwd) {
                 t_fwd = t;
                 bf = f;
@@ -1548,7 +1549,7 @@ static rmesh_status autotune_layout(rmesh_renderer* h, const uint32_t* per_user,
         }
         if (result != RMESH_OK) break;
         h->fwd_var = bf;
-        if ((result = stage_forward(h, V, false)) != RMESH_OK) break;  // image of the chosen variant
+        if ((result = stage_forward(h, V, false, loss_type == 0)) != RMESH_OK) break;  // image of the chosen variant
         for (int b = 0; b < bwd_variants(ts) && result == RMESH_OK; ++b) {
             h->bwd_var = b;
             float t = 0.0f;
@@ -1715,7 +1716,7 @@ extern "C" rmesh_status rmesh_forward_multi(rmesh_renderer* h, const uint32_t* v
     const uint32_t V = h->n_views;
     if ((st = stage_binning_front(h, V, false)) != RMESH_OK) return st;
     if ((st = stage_binning_back(h, V, true)) != RMESH_OK) return st;
-    if ((st = stage_forward(h, V, false)) != RMESH_OK) return st;
+    if ((st = stage_forward(h, V, false, false)) != RMESH_OK) return st;
     h->last_views = V;
     h->have_forward = !h->multi();
     if (out_rgba) HIP_TRY(hipMemcpyAsync(out_rgba, h->rgba, 16ull * h->pix_len, hipMemcpyDeviceToHost, h->stream));

@@ -148,6 +148,7 @@ struct FwdArgs {
     uint32_t num_gtiles;
     const uint32_t* tile_order;  // nullable: work item -> global tile (identity when null)
     SplitPlan split;             // the plan tile_order was made with
+    bool one_pass;               // split lists composited by one workgroup each (the steps with the L1 loss)
     float* rgba;
     float* aux;  // nullable: [V][H][W][8]
     // nullable: transmittance checkpoints for the checkpointed adjoint.

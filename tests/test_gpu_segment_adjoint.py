@@ -62,3 +62,41 @@ def test_undo_starts_at_the_image_alpha(ts, w, h, fov, scale):
     g32 = orc.backward(s, cam, w, h, ref["sorted_vals"], ref["ranges"], img, dl, ts)
     for k in KEYS:
         assert _rel(g[k], go[k]) <= 4 * _rel(g32[k], go[k]), (k, _rel(g[k], go[k]), _rel(g32[k], go[k]))
+
+
+@pytest.mark.parametrize("mode", ["undo", "checkpoint"])
+@pytest.mark.parametrize("kind", ["plain", "saturating"])
+@pytest.mark.parametrize("ts", [8, 12, 16, 32])
+def test_l1_step_composites_in_list_order(ts, kind, mode):
+    """The L1 gradient is the sign of image - target, so its image has the
+    rounding of one pass over each list.  Towards the image of such a pass (the
+    aux forward's) nothing is left: loss and gradients 0; and towards a far
+    target the gradients are the unsplit lists'."""
+    s, cam = _scene(), fibonacci_cameras(2, 3.0, 50.0, W, H)[1]
+    if kind == "saturating":
+        x = s["vertices"].reshape(-1, 3)[s["indices"].reshape(-1, 4).astype(int)].mean(1)[:, 0]
+        s["densities"] = (s["densities"] * np.where(x > 0.1, 30.0, np.where(x < -0.3, 0.5, 6.0))).astype(np.float32)
+    ref = orc.render(s, cam, W, H, ts)
+    assert _longest(ref) > 2 * (6 * ts * ts)
+    assert ((1.0 - ref["rgba"][..., 3]).min() < 1e-6) == (kind == "saturating") and ref["rgba"].max() < 20.0
+    r = _renderer(s, tile_size=ts)
+    r.set_adjoint_mode(mode)
+    img = np.asarray(r.forward_tiled(*cam, render_aux=True)[0]).reshape(H, W, 4)
+    assert r.train_step(*cam, np.ascontiguousarray(img[..., :3]), 0.0, 0.0, 0.0, 0) == 0.0
+    np.testing.assert_array_equal(r.read_buffer(0, H * W * 4).reshape(H, W, 4), img)
+    for k, v in r.gradients().items():
+        assert not np.any(v), k
+    gt = np.random.default_rng(3).uniform(20.0, 30.0, (H, W, 3)).astype(np.float32)  # brighter than any pixel
+    for _ in range(2):
+        r.train_step(*cam, gt, 0.0, 0.0, 0.0, 0)
+        g = r.gradients()
+    dl = np.concatenate([np.full((H, W, 3), -1.0 / (W * H)), np.zeros((H, W, 1))], -1).astype(np.float32)
+    if mode == "checkpoint":
+        fw = orc.forward(s, cam, W, H, ref["sorted_vals"], ref["ranges"], ts, want_checkpoints=True)
+        go = orc.backward(s, cam, W, H, ref["sorted_vals"], ref["ranges"], fw["rgba"], dl, ts, checkpoints=fw)
+    else:
+        f64 = {k: (np.asarray(v, np.float64) if np.asarray(v).dtype == np.float32 else v) for k, v in s.items()}
+        go = orc.backward(f64, cam, W, H, ref["sorted_vals"], ref["ranges"], img.astype(np.float64),
+                          dl.astype(np.float64), ts, dtype=np.float64)
+    for k in ("d_vertices", "d_densities", "d_color_grads"):
+        assert _rel(g[k], go[k]) <= 1e-3, (k, _rel(g[k], go[k]))
