@@ -136,7 +136,6 @@ struct rmesh_renderer {
     // block sums of the depth-ordered pair scan
     uint32_t *dkey_a = nullptr, *dkey_b = nullptr, *ditem_a = nullptr, *ditem_b = nullptr;
     uint32_t *ihist = nullptr, *d_nitems = nullptr, *block_sums2 = nullptr;
-    bool pairs_depth_ordered = false;  // the last pair generation emitted items in depth order
     uint32_t* ranges = nullptr;
     uint32_t* tile_order = nullptr;  // compositing work item -> global tile, heaviest first
     // segments of long tile lists (SplitPlan); px also per tet-sorted pair capacity
@@ -144,13 +143,18 @@ struct rmesh_renderer {
     float* seg_dark = nullptr;
     float4* seg_px = nullptr;
     uint32_t* seg_stop = nullptr;
-    bool order_split = false;        // tile_order holds (tile, segment) items
-    bool have_segs = false;          // the last forward left segment states for these tile lists
-    bool sorted_in_b = false;
+    // What the stages left in the buffers above, set where they are launched or
+    // recorded.  A graph leaves what was recorded, whatever ran between its replays.
+    struct Left {
+        bool pairs_depth_ordered = false;  // items were emitted in depth order
+        bool sorted_in_b = false;
+        bool order_split = false;          // tile_order holds (tile, segment) items
+        bool have_segs = false;            // the forward's segment states for these tile lists
+        bool have_ck = false;              // the forward's checkpoints
+    } left, graph_left;
     // adjoint mode: false = the reference's undo from the image alpha, true =
     // the checkpointed adjoint (transmittance checkpoints stored by the forward)
     bool adj_ck = false;
-    bool have_ck = false;        // the last forward stored checkpoints
     float* ck = nullptr;         // [slots][TS*TS]
     uint64_t ck_floats = 0;
     float2* fin = nullptr;       // [max_views][H][W]: final log T, stop position
@@ -478,7 +482,7 @@ uint32_t* keys32(uint64_t* k) { return reinterpret_cast<uint32_t*>(k); }
 void launch_pair_gen_item_order(rmesh_renderer* h, hipStream_t s) {
     launch_pairs(h->rec, reinterpret_cast<const float4*>(h->circ), h->d_scenes, (uint32_t)h->sc.size(), h->n_items,
                  h->d_views, h->TS, h->counts, h->block_sums, h->keys_a, h->vals_a, h->cap, h->overflow, s);
-    h->pairs_depth_ordered = false;
+    h->left.pairs_depth_ordered = false;
 }
 // Pair generation.  Depth-first: the items (M V 32-bit keys) are sorted by
 // depth key, and their pairs emitted in that order, so the pair sort that
@@ -493,17 +497,17 @@ void launch_pair_gen(rmesh_renderer* h, hipStream_t s) {
     launch_pairs_depth_ordered(h->rec, h->d_scenes, (uint32_t)h->sc.size(), in_b ? h->ditem_b : h->ditem_a,
                                (uint32_t)h->n_items, h->d_views, h->TS, h->counts, h->block_sums2, h->n_pairs,
                                keys32(h->keys_a), h->vals_a, h->cap, h->overflow, h->spine_part, s);
-    h->pairs_depth_ordered = true;
+    h->left.pairs_depth_ordered = true;
 }
 // Depth-ordered pairs carry 32-bit keys (the key tile) and are sorted on the
 // tile bits; item-ordered pairs carry the 64-bit (tile, depth) keys.
 void launch_sort_stage(rmesh_renderer* h, hipStream_t s) {
-    if (h->pairs_depth_ordered)
-        h->sorted_in_b = launch_radix_sort32(keys32(h->keys_a), h->vals_a, keys32(h->keys_b), h->vals_b, h->n_pairs,
-                                             h->cap, h->hist, s, h->sort_db, h->sorting_bits(0) - 32u);
+    if (h->left.pairs_depth_ordered)
+        h->left.sorted_in_b = launch_radix_sort32(keys32(h->keys_a), h->vals_a, keys32(h->keys_b), h->vals_b,
+                                                  h->n_pairs, h->cap, h->hist, s, h->sort_db, h->sorting_bits(0) - 32u);
     else
-        h->sorted_in_b = launch_radix_sort(h->keys_a, h->vals_a, h->keys_b, h->vals_b, h->n_pairs, h->cap,
-                                           h->sorting_bits(0), h->hist, s, h->sort_db);
+        h->left.sorted_in_b = launch_radix_sort(h->keys_a, h->vals_a, h->keys_b, h->vals_b, h->n_pairs, h->cap,
+                                                h->sorting_bits(0), h->hist, s, h->sort_db);
 }
 // The segment plan of the current tile size, for the order kernel and the forward.
 SplitPlan split_plan(const rmesh_renderer* h) {
@@ -525,11 +529,11 @@ SplitPlan split_plan(const rmesh_renderer* h) {
 // the aux, error and interval kernels take whole tiles.
 void launch_ranges_stage(rmesh_renderer* h, bool split, hipStream_t s) {
     const SplitPlan sp = split ? split_plan(h) : SplitPlan();
-    h->order_split = split;
-    h->have_segs = false;
+    h->left.order_split = split;
+    h->left.have_segs = false;
     launch_fill_u32(h->ranges, 0u, 2ull * h->n_gt, s);
-    uint64_t* sk = h->sorted_in_b ? h->keys_b : h->keys_a;
-    if (h->pairs_depth_ordered) launch_ranges32(keys32(sk), h->n_pairs, h->cap, h->ranges, h->d_ktile, h->n_kt, s);
+    uint64_t* sk = h->left.sorted_in_b ? h->keys_b : h->keys_a;
+    if (h->left.pairs_depth_ordered) launch_ranges32(keys32(sk), h->n_pairs, h->cap, h->ranges, h->d_ktile, h->n_kt, s);
     else launch_ranges(sk, h->n_pairs, h->cap, h->ranges, h->d_ktile, h->n_kt, s);
     if (h->scene_order != RMESH_SCENE_ORDER_BY_SCENE ||
         !launch_tile_order_scenes(h->ranges, h->n_gt, h->d_tile_view, h->d_views, (uint32_t)h->sc.size(),
@@ -545,7 +549,7 @@ rmesh_status stage_binning_back(rmesh_renderer* h, uint32_t V, bool split) {
     return RMESH_OK;
 }
 
-const uint32_t* sorted_vals(const rmesh_renderer* h) { return h->sorted_in_b ? h->vals_b : h->vals_a; }
+const uint32_t* sorted_vals(const rmesh_renderer* h) { return h->left.sorted_in_b ? h->vals_b : h->vals_a; }
 
 // one_pass: FwdArgs::one_pass, for the steps with the L1 loss (loss type 0).
 rmesh_status stage_forward(rmesh_renderer* h, uint32_t V, bool want_aux, bool one_pass) {
@@ -558,7 +562,7 @@ rmesh_status stage_forward(rmesh_renderer* h, uint32_t V, bool want_aux, bool on
     a.tile_view = h->d_tile_view;
     a.num_gtiles = h->n_gt;
     a.tile_order = h->tile_order;
-    if (h->order_split) a.split = split_plan(h);
+    if (h->left.order_split) a.split = split_plan(h);
     a.one_pass = one_pass;
     a.rgba = h->rgba;
     a.aux = want_aux ? h->aux : nullptr;
@@ -566,10 +570,10 @@ rmesh_status stage_forward(rmesh_renderer* h, uint32_t V, bool want_aux, bool on
     a.ck = ck ? h->ck : nullptr;
     a.fin = ck ? h->fin : nullptr;
     if (!launch_forward(a, h->TS, h->fwd_var, h->stream)) return fail(RMESH_ERR_INVALID, "unsupported tile size");
-    h->have_ck = ck;
+    h->left.have_ck = ck;
     // A near limit cuts the forward's slabs and not the adjoint's, whose undo runs
     // from the image alpha alone: its list stays one chain then.
-    h->have_segs = h->order_split && (h->min_t == 0.0f || ck);
+    h->left.have_segs = h->left.order_split && (h->min_t == 0.0f || ck);
     return RMESH_OK;
 }
 
@@ -591,9 +595,9 @@ rmesh_status stage_backward(rmesh_renderer* h, uint32_t V, const float* dl, cons
     a.tile_view = h->d_tile_view;
     a.num_gtiles = h->n_gt;
     a.tile_order = h->tile_order;
-    if (h->order_split) {
+    if (h->left.order_split) {
         a.split = split_plan(h);
-        if (!h->have_segs) a.split.px = nullptr;
+        if (!h->left.have_segs) a.split.px = nullptr;
     }
     a.rgba = h->rgba;
     a.dl_img = dl;
@@ -606,7 +610,7 @@ rmesh_status stage_backward(rmesh_renderer* h, uint32_t V, const float* dl, cons
     a.fin = nullptr;
     a.scene_done = h->scene_timing ? h->scene_clock : nullptr;
     if (h->adj_ck) {
-        if (!h->have_ck)
+        if (!h->left.have_ck)
             return fail(RMESH_ERR_INVALID,
                         "checkpointed adjoint: the last forward kept no checkpoints (a render_aux forward, or the "
                         "mode was switched after it); run forward_tiled again");
@@ -1064,7 +1068,7 @@ extern "C" rmesh_status rmesh_forward_error(rmesh_renderer* h, const float* pixe
     a.views = h->d_views;
     a.num_tiles = h->T;
     a.tile_order = h->tile_order;
-    if (h->order_split) a.split = split_plan(h);
+    if (h->left.order_split) a.split = split_plan(h);
     a.pixel_err = h->err_pe;
     a.ssim_err = h->err_se;
     a.tet_err = h->tet_err;
@@ -1330,7 +1334,7 @@ extern "C" rmesh_status rmesh_set_adjoint_mode(rmesh_renderer* h, int32_t mode) 
         DeviceGuard g(h->device);
         drop_graph(h);
         h->adj_ck = ck;
-        h->have_ck = false;
+        h->left.have_ck = false;
         h->have_forward = false;  // the next backward needs a forward in this mode
         if (!ck) {
             HIP_TRY(hipStreamSynchronize(h->stream));
@@ -1635,25 +1639,34 @@ static rmesh_status train_layout(rmesh_renderer* h, const uint32_t* per_user, co
     }
     if (h->graph_mode && h->cap > 0 && !graph_ok) {
         drop_graph(h);
-        for (int p = 0; p < parts; ++p) {
-            HIP_TRY(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-            rmesh_status cst = RMESH_OK;
-            for (int i = (parts == 1 ? 0 : p); i < (parts == 1 ? kStages : p + 1) && cst == RMESH_OK; ++i)
-                cst = record_stage(h, i, V, h->gt, loss_type, lr_v, lr_d, lr_g, lr_sh, true);
-            hipGraph_t graph = nullptr;
-            hipError_t e = hipStreamEndCapture(h->stream, &graph);
-            if (cst != RMESH_OK || e != hipSuccess) {
-                if (graph) (void)hipGraphDestroy(graph);
-                drop_graph(h);
-                if (cst != RMESH_OK) return cst;
-                return fail(RMESH_ERR_DEVICE, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
+        // (recording launches nothing: what is left stays as it was)
+        const rmesh_renderer::Left before = h->left;
+        auto record = [&]() -> rmesh_status {
+            for (int p = 0; p < parts; ++p) {
+                HIP_TRY(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
+                rmesh_status cst = RMESH_OK;
+                for (int i = (parts == 1 ? 0 : p); i < (parts == 1 ? kStages : p + 1) && cst == RMESH_OK; ++i)
+                    cst = record_stage(h, i, V, h->gt, loss_type, lr_v, lr_d, lr_g, lr_sh, true);
+                hipGraph_t graph = nullptr;
+                hipError_t e = hipStreamEndCapture(h->stream, &graph);
+                if (cst != RMESH_OK || e != hipSuccess) {
+                    if (graph) (void)hipGraphDestroy(graph);
+                    if (cst != RMESH_OK) return cst;
+                    return fail(RMESH_ERR_DEVICE, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
+                }
+                h->graph[p] = graph;
+                hipError_t ie = hipGraphInstantiate(&h->graph_exec[p], graph, nullptr, nullptr, 0);
+                if (ie != hipSuccess)
+                    return fail(RMESH_ERR_DEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(ie));
             }
-            h->graph[p] = graph;
-            hipError_t ie = hipGraphInstantiate(&h->graph_exec[p], graph, nullptr, nullptr, 0);
-            if (ie != hipSuccess) {
-                drop_graph(h);
-                return fail(RMESH_ERR_DEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(ie));
-            }
+            return RMESH_OK;
+        };
+        st = record();
+        h->graph_left = h->left;
+        h->left = before;
+        if (st != RMESH_OK) {
+            drop_graph(h);
+            return st;
         }
         h->graph_parts = parts;
         h->graph_views = V;
@@ -1667,6 +1680,7 @@ static rmesh_status train_layout(rmesh_renderer* h, const uint32_t* per_user, co
             if (h->graph_parts > 1) mark(h, p);
             HIP_TRY(hipGraphLaunch(h->graph_exec[p], h->stream));
         }
+        h->left = h->graph_left;
         if (h->graph_parts > 1) mark(h, kStages);
         st = finish_train(h, V, out_loss, out_view_losses);
         if (st == RMESH_ERR_CAPACITY) {
@@ -1883,10 +1897,10 @@ extern "C" rmesh_status rmesh_debug_sorted(rmesh_renderer* h, uint64_t* keys, ui
     HIP_TRY(hipMemcpy(&P, h->n_pairs, 4, hipMemcpyDeviceToHost));
     *n_pairs = P;
     uint64_t n = std::min<uint64_t>(P, cap);
-    uint64_t* sk = h->sorted_in_b ? h->keys_b : h->keys_a;
-    if (keys && n && h->pairs_depth_ordered) {
+    uint64_t* sk = h->left.sorted_in_b ? h->keys_b : h->keys_a;
+    if (keys && n && h->left.pairs_depth_ordered) {
         // 32-bit key tiles: rebuild the 64-bit (tile, depth) keys in the free key buffer
-        uint64_t* full = h->sorted_in_b ? h->keys_a : h->keys_b;
+        uint64_t* full = h->left.sorted_in_b ? h->keys_a : h->keys_b;
         launch_full_keys(keys32(sk), sorted_vals(h), h->n_pairs, h->cap, reinterpret_cast<const float4*>(h->circ),
                          h->d_views, h->d_ktile, h->n_kt, h->d_tile_view, full, P, h->stream);
         HIP_TRY(hipStreamSynchronize(h->stream));
