@@ -571,9 +571,9 @@ rmesh_status stage_forward(rmesh_renderer* h, uint32_t V, bool want_aux, bool on
     a.fin = ck ? h->fin : nullptr;
     if (!launch_forward(a, h->TS, h->fwd_var, h->stream)) return fail(RMESH_ERR_INVALID, "unsupported tile size");
     h->left.have_ck = ck;
-    // A near limit cuts the forward's slabs and not the adjoint's, whose undo runs
-    // from the image alpha alone: its list stays one chain then.
-    h->left.have_segs = h->left.order_split && (h->min_t == 0.0f || ck);
+    // (with a near offset too: min_t shifts the forward's ray parameter and cuts
+    // no slab, so the states are those of the adjoint, which takes no offset)
+    h->left.have_segs = h->left.order_split;
     return RMESH_OK;
 }
 
@@ -987,7 +987,6 @@ extern "C" void rmesh_destroy(rmesh_renderer* h) {
 
 extern "C" rmesh_status rmesh_set_min_t(rmesh_renderer* h, float min_t) {
     if (!h) return fail(RMESH_ERR_INVALID, "null handle");
-    if ((min_t != 0.0f) != (h->min_t != 0.0f)) drop_graph(h);  // the captured adjoint depends on it
     h->min_t = min_t;
     return RMESH_OK;
 }

@@ -4,7 +4,9 @@
   as on a whole one: against the float64 oracle started from the renderer's own
   image, within four times the distance of the float32 oracle from it.  Pixels
   down to T = 3e-6, where the rounding of alpha moves the gradients by 1.5e-4 to
-  5e-4 of those from an exact image.
+  5e-4 of those from an exact image;
+- an L1 step has the image of one pass over each list, and the adjoint of it;
+- both adjoints with a near offset.
 """
 
 import numpy as np
@@ -99,4 +101,32 @@ def test_l1_step_composites_in_list_order(ts, kind, mode):
         go = orc.backward(f64, cam, W, H, ref["sorted_vals"], ref["ranges"], img.astype(np.float64),
                           dl.astype(np.float64), ts, dtype=np.float64)
     for k in ("d_vertices", "d_densities", "d_color_grads"):
+        assert _rel(g[k], go[k]) <= 1e-3, (k, _rel(g[k], go[k]))
+
+
+@pytest.mark.parametrize("mode", ["undo", "checkpoint"])
+@pytest.mark.parametrize("min_t", [0.5, 3.0])
+@pytest.mark.parametrize("ts", [8, 12, 16, 32])
+def test_near_offset(ts, min_t, mode):
+    """min_t shifts the forward's ray parameter only; the adjoint of a split list
+    starts its segments from that forward's states.  The bounds of the unsplit
+    path: image 1e-4, gradients 1e-3 relative L2."""
+    s, cam = _scene(), fibonacci_cameras(2, 3.0, 50.0, W, H)[1]
+    ref = orc.render(s, cam, W, H, ts, min_t=min_t)
+    assert _longest(ref) > 2 * (6 * ts * ts)
+    dl = np.random.default_rng(ts).normal(0, 1e-2, (H, W, 4)).astype(np.float32)
+    r = _renderer(s, tile_size=ts)
+    r.set_adjoint_mode(mode)
+    r.set_min_t(min_t)
+    img = np.asarray(r.forward_tiled(*cam)).reshape(H, W, 4)
+    assert np.abs(img - ref["rgba"]).max() <= 1e-4
+    g = r.backward(dl)
+    if mode == "checkpoint":
+        fw = orc.forward(s, cam, W, H, ref["sorted_vals"], ref["ranges"], ts, min_t=min_t, want_checkpoints=True)
+        go = orc.backward(s, cam, W, H, ref["sorted_vals"], ref["ranges"], fw["rgba"], dl, ts, checkpoints=fw)
+    else:
+        f64 = {k: (np.asarray(v, np.float64) if np.asarray(v).dtype == np.float32 else v) for k, v in s.items()}
+        go = orc.backward(f64, cam, W, H, ref["sorted_vals"], ref["ranges"], img.astype(np.float64),
+                          dl.astype(np.float64), ts, dtype=np.float64)
+    for k in KEYS:
         assert _rel(g[k], go[k]) <= 1e-3, (k, _rel(g[k], go[k]))
