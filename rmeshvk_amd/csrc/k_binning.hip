@@ -936,8 +936,10 @@ __device__ __forceinline__ uint32_t item_bucket(uint32_t c, int seg, const Split
     const uint32_t in = seg < 0 ? (uint32_t)kSegBuckets : (uint32_t)kSegBuckets - 1u - min((uint32_t)seg, (uint32_t)kSegBuckets - 1u);
     return lo + (min(b, hi) - lo) * (uint32_t)(kSegBuckets + 1) + in;
 }
-__device__ __forceinline__ uint32_t tile_unit(const ViewParams& vw, const SplitPlan& sp) {
-    return sp.unit_for(vw.tiles_x * vw.tiles_y);
+// (without a plan not read)
+__device__ __forceinline__ uint32_t call_unit(uint32_t n_tiles, const uint32_t* __restrict__ n_pairs, uint32_t cap,
+                                              const SplitPlan& sp) {
+    return sp.seg ? split_unit_of(sp.unit, sp.unit_few, n_tiles, min(*n_pairs, cap)) : 0u;
 }
 // cnt: the tile's bucket counters (its scene's).
 __device__ __forceinline__ void count_items(uint32_t* cnt, uint32_t pairs, uint32_t unit, const SplitPlan& sp) {
@@ -969,16 +971,16 @@ __device__ __forceinline__ void place_items(uint32_t* off, uint32_t* n_slots, ui
 }
 
 __global__ __launch_bounds__(1024) void k_tile_order(const uint32_t* __restrict__ ranges, uint32_t n,
-                                                      const uint32_t* __restrict__ tile_view,
-                                                      const ViewParams* __restrict__ views,
+                                                      const uint32_t* __restrict__ n_pairs, uint32_t cap,
                                                       uint32_t* __restrict__ order, SplitPlan sp) {
     __shared__ uint32_t cnt[kOrderBuckets];
     __shared__ uint32_t n_slots;
     const uint32_t tid = threadIdx.x;
     if (tid < kOrderBuckets) cnt[tid] = 0u;
     if (tid == 0) n_slots = 0u;
+    const uint32_t unit = call_unit(n, n_pairs, cap, sp);
     __syncthreads();
-    for (uint32_t t = tid; t < n; t += blockDim.x) count_items(cnt, tile_pairs(ranges, t), tile_unit(views[tile_view[t]], sp), sp);
+    for (uint32_t t = tid; t < n; t += blockDim.x) count_items(cnt, tile_pairs(ranges, t), unit, sp);
     __syncthreads();
     if (tid == 0) {
         uint32_t run = 0;
@@ -987,11 +989,14 @@ __global__ __launch_bounds__(1024) void k_tile_order(const uint32_t* __restrict_
             cnt[b] = run;
             run += k;
         }
-        if (sp.seg) *sp.n_items = run;
+        if (sp.seg) {
+            sp.n_items[0] = run;
+            sp.n_items[1] = unit;
+        }
     }
     __syncthreads();
     for (uint32_t t = tid; t < n; t += blockDim.x)
-        place_items(cnt, &n_slots, t, tile_pairs(ranges, t), tile_unit(views[tile_view[t]], sp), order, sp);
+        place_items(cnt, &n_slots, t, tile_pairs(ranges, t), unit, order, sp);
 }
 
 // Scene-major order for batches of several scenes: the scenes one after
@@ -1002,6 +1007,7 @@ __global__ __launch_bounds__(1024) void k_tile_order(const uint32_t* __restrict_
 // in LDS, then offsets by one thread.
 constexpr uint32_t kOrderMaxScenes = 64;
 __global__ __launch_bounds__(1024) void k_tile_order_scenes(const uint32_t* __restrict__ ranges, uint32_t n,
+                                                            const uint32_t* __restrict__ n_pairs, uint32_t cap,
                                                             const uint32_t* __restrict__ tile_view,
                                                             const ViewParams* __restrict__ views, uint32_t n_scenes,
                                                             uint32_t* __restrict__ order, SplitPlan sp) {
@@ -1013,11 +1019,11 @@ __global__ __launch_bounds__(1024) void k_tile_order_scenes(const uint32_t* __re
     for (uint32_t i = tid; i < n_scenes * kOrderBuckets; i += blockDim.x) cnt[i] = 0u;
     if (tid < n_scenes) s_pairs[tid] = 0ull;
     if (tid == 0) n_slots = 0u;
+    const uint32_t unit = call_unit(n, n_pairs, cap, sp);
     __syncthreads();
     for (uint32_t t = tid; t < n; t += blockDim.x) {
-        const ViewParams& vw = views[tile_view[t]];
-        const uint32_t sc = vw.scene, c = tile_pairs(ranges, t);
-        count_items(cnt + sc * kOrderBuckets, c, tile_unit(vw, sp), sp);
+        const uint32_t sc = views[tile_view[t]].scene, c = tile_pairs(ranges, t);
+        count_items(cnt + sc * kOrderBuckets, c, unit, sp);
         atomicAdd(&s_pairs[sc], (unsigned long long)c);
     }
     __syncthreads();
@@ -1037,12 +1043,15 @@ __global__ __launch_bounds__(1024) void k_tile_order_scenes(const uint32_t* __re
                 run += k;
             }
         }
-        if (sp.seg) *sp.n_items = run;
+        if (sp.seg) {
+            sp.n_items[0] = run;
+            sp.n_items[1] = unit;
+        }
     }
     __syncthreads();
     for (uint32_t t = tid; t < n; t += blockDim.x) {
-        const ViewParams& vw = views[tile_view[t]];
-        place_items(cnt + vw.scene * kOrderBuckets, &n_slots, t, tile_pairs(ranges, t), tile_unit(vw, sp), order, sp);
+        const uint32_t sc = views[tile_view[t]].scene;
+        place_items(cnt + sc * kOrderBuckets, &n_slots, t, tile_pairs(ranges, t), unit, order, sp);
     }
 }
 
@@ -1054,19 +1063,18 @@ void launch_stamp_start(uint64_t* p, uint32_t n, hipStream_t s) {
     hipLaunchKernelGGL(k_stamp_start, dim3(1), dim3(64), 0, s, p, n);
 }
 
-void launch_tile_order(const uint32_t* ranges, uint32_t n_tiles, const uint32_t* tile_view, const ViewParams* views,
-                       uint32_t* order, const SplitPlan& sp, hipStream_t s) {
-    if (n_tiles)
-        hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, s, ranges, n_tiles, tile_view, views, order, sp);
+void launch_tile_order(const uint32_t* ranges, uint32_t n_tiles, const uint32_t* n_pairs, uint32_t cap, uint32_t* order,
+                       const SplitPlan& sp, hipStream_t s) {
+    if (n_tiles) hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, s, ranges, n_tiles, n_pairs, cap, order, sp);
 }
 
-bool launch_tile_order_scenes(const uint32_t* ranges, uint32_t n_tiles, const uint32_t* tile_view,
-                              const ViewParams* views, uint32_t n_scenes, uint32_t* order, const SplitPlan& sp,
-                              hipStream_t s) {
+bool launch_tile_order_scenes(const uint32_t* ranges, uint32_t n_tiles, const uint32_t* n_pairs, uint32_t cap,
+                              const uint32_t* tile_view, const ViewParams* views, uint32_t n_scenes, uint32_t* order,
+                              const SplitPlan& sp, hipStream_t s) {
     if (n_scenes == 0 || n_scenes > kOrderMaxScenes) return false;
     if (n_tiles)
-        hipLaunchKernelGGL(k_tile_order_scenes, dim3(1), dim3(1024), 0, s, ranges, n_tiles, tile_view, views, n_scenes,
-                           order, sp);
+        hipLaunchKernelGGL(k_tile_order_scenes, dim3(1), dim3(1024), 0, s, ranges, n_tiles, n_pairs, cap, tile_view,
+                           views, n_scenes, order, sp);
     return true;
 }
 

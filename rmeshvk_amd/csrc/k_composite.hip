@@ -759,7 +759,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     // list positions [done, end) of this workgroup
     uint32_t done = 0, end = count;
     bool skipped = false;
-    const uint32_t unit = split.unit_for(vw.tiles_x * vw.tiles_y);
+    const uint32_t unit = split.seg ? split.unit_now() : 0u;
     bool whole = AUX || !split.seg || split_segments(count, unit) == 1u;  // one workgroup, one list
     if (!whole) {
         const uint32_t seg = split.seg[blockIdx.x], seg_len = split_length(count, unit);
@@ -1442,7 +1442,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     // first `merged` of them with the one behind
     const uint32_t view = tile_view[gtile];
     const ViewParams& vw = views[view];
-    const uint32_t unit = split.unit_for(vw.tiles_x * vw.tiles_y);
+    const uint32_t unit = split.px ? split.unit_now() : 0u;
     const bool by_seg = split.px && split_segments(count, unit) > 1u;
     const uint32_t merged = by_seg ? split.merged[gtile] : 0u;
     if (by_seg ? seg < merged : seg > 0u) return;

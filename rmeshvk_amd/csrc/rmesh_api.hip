@@ -356,24 +356,17 @@ void set_tiles(rmesh_renderer* h, uint32_t ts) {
     drop_graph(h);
 }
 
-// The smallest segment unit of any of the renderer's views at tile size ts.
-uint32_t least_unit(const rmesh_renderer* h, uint32_t ts) {
-    for (const SceneHost& c : h->sc)
-        if ((uint64_t)((c.W + ts - 1) / ts) * ((c.H + ts - 1) / ts) <= kFewTiles) return split_unit_few(ts);
-    return split_unit(ts);
-}
-// Work items beyond one per tile, segment slots and their pixel records for P
-// pairs, each at the tile size that needs most.
+// Work items beyond one per tile, segment slots and their pixel records for calls
+// of at most P pairs, each at the tile size that needs most.
 struct SegmentSizes {
     uint64_t items = 0, slots = 0, pixels = 0;
 };
-SegmentSizes segment_sizes(const rmesh_renderer* h, uint64_t P) {
+SegmentSizes segment_sizes(uint64_t P) {
     SegmentSizes n;
     for (uint32_t ts : {8u, 12u, 16u, 32u}) {
-        const uint32_t unit = least_unit(h, ts);
-        n.items = std::max(n.items, split_extra_items(P, unit));
-        n.slots = std::max(n.slots, split_slots(P, unit));
-        n.pixels = std::max<uint64_t>(n.pixels, split_slots(P, unit) * ts * ts);
+        n.items = std::max(n.items, split_extra_items(P, ts, 0u));
+        n.slots = std::max(n.slots, split_slots(P, ts));
+        n.pixels = std::max(n.pixels, split_slots(P, ts) * ts * ts);
     }
     return n;
 }
@@ -406,7 +399,7 @@ rmesh_status ensure_capacity(rmesh_renderer* h, uint64_t need) {
     HIP_TRY(dalloc(&h->vals_a, c));
     HIP_TRY(dalloc(&h->vals_b, c));
     HIP_TRY(dalloc(&h->hist, std::max(radix_hist_words((uint32_t)c), radix_hist_words32((uint32_t)c))));
-    const SegmentSizes ns = segment_sizes(h, c);
+    const SegmentSizes ns = segment_sizes(c);
     HIP_TRY(dalloc(&h->tile_order, h->tile_cap + ns.items));
     HIP_TRY(dalloc(&h->seg, h->tile_cap + ns.items));
     HIP_TRY(dalloc(&h->seg_dark, ns.slots));
@@ -432,7 +425,7 @@ rmesh_status ensure_checkpoints(rmesh_renderer* h, uint32_t V) {
         drop_graph(h);
     }
     if (!h->seg_stop) {
-        HIP_TRY(dalloc(&h->seg_stop, segment_sizes(h, h->cap).pixels));
+        HIP_TRY(dalloc(&h->seg_stop, segment_sizes(h->cap).pixels));
         drop_graph(h);
     }
     if (!h->fin) HIP_TRY(dalloc(&h->fin, (size_t)h->pix_cap));
@@ -522,7 +515,7 @@ SplitPlan split_plan(const rmesh_renderer* h) {
     p.dark = h->seg_dark;
     p.px = h->seg_px;
     p.stop = h->seg_stop;
-    p.grid = h->n_gt + (uint32_t)split_extra_items(h->cap, least_unit(h, h->TS));
+    p.grid = h->n_gt + (uint32_t)split_extra_items(h->cap, h->TS, h->n_gt);
     return p;
 }
 // split: long lists as several work items (the plain forward and the adjoint);
@@ -536,9 +529,9 @@ void launch_ranges_stage(rmesh_renderer* h, bool split, hipStream_t s) {
     if (h->left.pairs_depth_ordered) launch_ranges32(keys32(sk), h->n_pairs, h->cap, h->ranges, h->d_ktile, h->n_kt, s);
     else launch_ranges(sk, h->n_pairs, h->cap, h->ranges, h->d_ktile, h->n_kt, s);
     if (h->scene_order != RMESH_SCENE_ORDER_BY_SCENE ||
-        !launch_tile_order_scenes(h->ranges, h->n_gt, h->d_tile_view, h->d_views, (uint32_t)h->sc.size(),
-                                  h->tile_order, sp, s))
-        launch_tile_order(h->ranges, h->n_gt, h->d_tile_view, h->d_views, h->tile_order, sp, s);
+        !launch_tile_order_scenes(h->ranges, h->n_gt, h->n_pairs, h->cap, h->d_tile_view, h->d_views,
+                                  (uint32_t)h->sc.size(), h->tile_order, sp, s))
+        launch_tile_order(h->ranges, h->n_gt, h->n_pairs, h->cap, h->tile_order, sp, s);
 }
 
 rmesh_status stage_binning_back(rmesh_renderer* h, uint32_t V, bool split) {
@@ -955,7 +948,7 @@ static rmesh_status create_impl(const rmesh_scene_desc* descs, uint32_t n_scenes
     CREATE_TRY(dalloc(&h->d_step, 1));
     CREATE_TRY(hipMemset(h->d_step, 0, 4));
     CREATE_TRY(dalloc(&h->ranges, 2ull * h->tile_cap));
-    CREATE_TRY(dalloc(&h->n_seg_items, 1));
+    CREATE_TRY(dalloc(&h->n_seg_items, 2));
     CREATE_TRY(dalloc(&h->seg_slot, (size_t)h->tile_cap));
     CREATE_TRY(dalloc(&h->seg_arrived, (size_t)h->tile_cap));
     CREATE_TRY(dalloc(&h->seg_merged, (size_t)h->tile_cap));

@@ -10,9 +10,8 @@ namespace rmesh {
 struct ViewParams;
 
 // Tile lists longer than a unit are composited by several workgroups, a segment
-// of at most `unit` pairs each (a rule of the list's own length, so a view's
-// image does not depend on what it is batched with).  Segments start at
-// multiples of 32 positions, as the transmittance checkpoints do.
+// of at most `unit` pairs each.  Segments start at multiples of 32 positions, as
+// the transmittance checkpoints do.
 // The unit, 6 pairs per pixel: a tile's workgroup is a serial chain over its
 // list, and the chip holds some 1300 of them, so a list far above (all pairs) /
 // 1300 runs on after the rest of the grid is done (uneven scenes, longest list
@@ -23,14 +22,21 @@ struct ViewParams;
 // grid (config C) 2 % at 6, 4 % at 4 and 1 % at 8 pairs a pixel, while 8 leaves
 // the clustered views 7 % slower than 6.
 constexpr uint32_t split_unit(uint32_t tile_size) { return 6u * tile_size * tile_size; }
-// A view of at most kFewTiles tiles (a 256 x 256 image at tile 12) leaves most of
-// the chip idle, and its workgroups, one a CU, issue far below the rate of
-// several: there the unit is one pair per pixel (2,000-point mesh: forward 87 ->
-// 55 us, adjoint 175 -> 105; two pairs 73 and 158).  On larger views that costs
-// 8 % (8 views at 512 x 512, where the grid is full).
-constexpr uint32_t kFewTiles = 512;
+// A call of at most kFewItems work items at that unit leaves part of the chip
+// idle, and its workgroups, a few a CU, issue far below the rate of more: there
+// the unit is one pair per pixel.  Train step and forward call in us, six pairs
+// and one: 484 tiles (2,000 points, 256 x 256) 502 -> 436, 343 -> 309; 784 tiles
+// (10,000 points) 719 -> 584, 415 -> 365; 968 (two views) 698 -> 608, 400 -> 372;
+// 1,156 (clustered) 669 -> 560, 386 -> 358; 1,849 829 -> 864, 466 -> 487; 3,528
+// (8 views, tile 16) 1,405 -> 1,504, 722 -> 788; 7,744 (16 views at 256 x 256)
+// 2,264 -> 2,570, 1,217 -> 1,426.
+constexpr uint32_t kFewItems = 1536;
 constexpr uint32_t split_unit_few(uint32_t tile_size) {
     return tile_size <= 16u ? tile_size * tile_size : split_unit(tile_size);
+}
+// The unit of a call of n_tiles tiles and P pairs.
+__host__ __device__ inline uint32_t split_unit_of(uint32_t unit, uint32_t unit_few, uint32_t n_tiles, uint64_t P) {
+    return n_tiles + P / unit <= kFewItems ? unit_few : unit;
 }
 __host__ __device__ inline uint32_t split_length(uint32_t pairs, uint32_t unit) {
     if (pairs <= unit) return pairs;
@@ -40,16 +46,30 @@ __host__ __device__ inline uint32_t split_length(uint32_t pairs, uint32_t unit) 
 __host__ __device__ inline uint32_t split_segments(uint32_t pairs, uint32_t unit) {
     return pairs <= unit ? 1u : (pairs - 1u) / split_length(pairs, unit) + 1u;
 }
-// Bounds for P pairs: items beyond one per tile, and segment slots.  A tile of c >
-// unit pairs has at most (c - 1) / unit + 1 < 2 c / unit segments.
-inline uint64_t split_extra_items(uint64_t P, uint32_t unit) { return P / unit; }
-inline uint64_t split_slots(uint64_t P, uint32_t unit) { return 2u * (P / unit) + 2u; }
+// Bounds for calls of at most P pairs (and n_tiles tiles) at a tile size: items
+// beyond one per tile, and segment slots.  A tile of c > unit pairs has at most
+// (c - 1) / unit + 1 segments, below 2 c / unit and c / unit + 1; calls at
+// unit_few have at most kFewItems tiles and below (kFewItems + 1) unit pairs.
+inline uint64_t split_few_pairs(uint64_t P, uint32_t tile_size) {
+    const uint64_t most = (uint64_t)(kFewItems + 1u) * split_unit(tile_size);
+    return P < most ? P : most;
+}
+inline uint64_t split_extra_items(uint64_t P, uint32_t tile_size, uint32_t n_tiles) {
+    const uint64_t n = P / split_unit(tile_size);
+    const uint64_t few = n_tiles <= kFewItems ? split_few_pairs(P, tile_size) / split_unit_few(tile_size) : 0u;
+    return n > few ? n : few;
+}
+inline uint64_t split_slots(uint64_t P, uint32_t tile_size) {
+    const uint64_t n = 2u * (P / split_unit(tile_size)) + 2u;
+    const uint64_t few = split_few_pairs(P, tile_size) / split_unit_few(tile_size) + kFewItems;
+    return n > few ? n : few;
+}
 
 struct SplitPlan {
     uint32_t unit = 0, unit_few = 0;
-    __host__ __device__ uint32_t unit_for(uint32_t view_tiles) const { return view_tiles <= kFewTiles ? unit_few : unit; }
     uint32_t* seg = nullptr;      // [item] segment of the item's tile; null: one item per tile, no segments
-    uint32_t* n_items = nullptr;
+    uint32_t* n_items = nullptr;  // then the call's unit (split_unit_of)
+    __device__ uint32_t unit_now() const { return n_items[1]; }
     uint32_t* slot = nullptr;     // [tile] first segment slot (tiles with more than one segment)
     uint32_t* arrived = nullptr;  // [tile] segments composited
     uint32_t* merged = nullptr;   // [tile] the adjoint takes segments 0 .. merged in one
@@ -114,13 +134,13 @@ void launch_ranges32(const uint32_t* keys, const uint32_t* n_ptr, uint32_t cap, 
 // Work items (tile, segment) in launch order, heaviest first: order[item] the
 // global tile, sp.seg[item] its segment; without a plan (sp.seg null) a
 // permutation of the tiles.
-void launch_tile_order(const uint32_t* ranges, uint32_t n_tiles, const uint32_t* tile_view, const ViewParams* views,
-                       uint32_t* order, const SplitPlan& sp, hipStream_t s);
+void launch_tile_order(const uint32_t* ranges, uint32_t n_tiles, const uint32_t* n_pairs, uint32_t cap, uint32_t* order,
+                       const SplitPlan& sp, hipStream_t s);
 // Scene-major heaviest-first order (scenes by ascending pair count); false
 // (nothing launched) above 64 scenes.
-bool launch_tile_order_scenes(const uint32_t* ranges, uint32_t n_tiles, const uint32_t* tile_view,
-                              const ViewParams* views, uint32_t n_scenes, uint32_t* order, const SplitPlan& sp,
-                              hipStream_t s);
+bool launch_tile_order_scenes(const uint32_t* ranges, uint32_t n_tiles, const uint32_t* n_pairs, uint32_t cap,
+                              const uint32_t* tile_view, const ViewParams* views, uint32_t n_scenes, uint32_t* order,
+                              const SplitPlan& sp, hipStream_t s);
 // p[0..n) = 0, p[n] = the wall clock now (start of a step's per-scene timing)
 void launch_stamp_start(uint64_t* p, uint32_t n, hipStream_t s);
 

@@ -6,7 +6,9 @@
   down to T = 3e-6, where the rounding of alpha moves the gradients by 1.5e-4 to
   5e-4 of those from an exact image;
 - an L1 step has the image of one pass over each list, and the adjoint of it;
-- both adjoints with a near offset.
+- both adjoints with a near offset, in calls of many tiles, under the scene-major
+  order and through the autotuner;
+- segment buffers sized by what calls with short segments can need.
 """
 
 import numpy as np
@@ -130,3 +132,78 @@ def test_near_offset(ts, min_t, mode):
                           dl.astype(np.float64), ts, dtype=np.float64)
     for k in KEYS:
         assert _rel(g[k], go[k]) <= 1e-3, (k, _rel(g[k], go[k]))
+
+
+@pytest.mark.parametrize("mode", ["undo", "checkpoint"])
+@pytest.mark.parametrize("ts,w,fov", [(8, 328, 140.0), (12, 480, 145.0), (16, 640, 145.0)])
+def test_calls_of_many_tiles(ts, w, fov, mode):
+    """Above 1,536 work items, where the segments hold six pairs per pixel: the mesh
+    in a few of the tiles of a wide angle.  Image 2e-4 (two float32 evaluations, each
+    up to 5.3e-5 from float64 here), gradients 1e-3 relative L2, or four times the
+    float32 oracle's own error where that is more (vertices far from the axis)."""
+    s, cam = _scene(), fibonacci_cameras(2, 3.0, fov, w, w)[1]
+    ref = orc.render(s, cam, w, w, ts)
+    assert len(ref["ranges"].reshape(-1, 2)) > 1536 and _longest(ref) > 2 * (6 * ts * ts)
+    dl = np.random.default_rng(ts).normal(0, 1e-2, (w, w, 4)).astype(np.float32)
+    r = _renderer(s, w, w, tile_size=ts)
+    r.set_adjoint_mode(mode)
+    img = np.asarray(r.forward_tiled(*cam)).reshape(w, w, 4)
+    assert np.abs(img - ref["rgba"]).max() <= 2e-4
+    g = r.backward(dl)
+    f64 = {k: (np.asarray(v, np.float64) if np.asarray(v).dtype == np.float32 else v) for k, v in s.items()}
+    go = orc.backward(f64, cam, w, w, ref["sorted_vals"], ref["ranges"], img.astype(np.float64), dl.astype(np.float64),
+                      ts, dtype=np.float64)
+    g32 = orc.backward(s, cam, w, w, ref["sorted_vals"], ref["ranges"], img, dl, ts)
+    for k in KEYS:
+        assert _rel(g[k], go[k]) <= max(1e-3, 4 * _rel(g32[k], go[k])), (k, _rel(g[k], go[k]))
+
+
+def test_a_thumbnail_scene_does_not_size_the_segments():
+    """Segment buffers are sized by the pairs that a call with short segments can
+    have, not by all of a renderer that has a small view."""
+    from rmeshvk_amd import MultiSceneRenderer, RMeshRenderer
+
+    rng = np.random.default_rng(5)
+    big, small = make_scene(uniform_points(40000, rng), rng), make_scene(uniform_points(300, rng), rng)
+    cams = fibonacci_cameras(4, 3.0, 50.0, 512, 512)
+    one = RMeshRenderer(big["vertices"], big["indices"], big["base_colors"], big["densities"], big["color_grads"],
+                        big["circumdata"], 512, 512, device_id=0, max_views=4)
+    one.forward_batched(cams, copy_out=False)
+    assert one.pair_count() > 2_000_000
+    thumb = _renderer(small, 64, 64)
+    thumb.forward_tiled(*fibonacci_cameras(1, 3.0, 50.0, 64, 64)[0])
+    both = MultiSceneRenderer([dict(big, width=512, height=512, max_views=4), dict(small, width=64, height=64, max_views=1)])
+    both.forward([4, 1], cams + fibonacci_cameras(1, 3.0, 50.0, 64, 64))
+    # (what the two hold apart, the larger pair buffer's growth step and the rest of a few MB)
+    assert both.device_bytes() <= 1.1 * (one.device_bytes() + thumb.device_bytes())
+
+
+def test_segments_in_scene_major_order():
+    from rmeshvk_amd import MultiSceneRenderer
+
+    a, b = _scene(0.2), _scene(1.0)
+    cams = fibonacci_cameras(3, 3.0, 50.0, W, H)
+    got = []
+    for order in ("interleaved", "by_scene"):
+        r = MultiSceneRenderer([dict(s, width=W, height=H, max_views=2) for s in (a, b)])
+        r.set_scene_order(order)
+        r.set_targets([2, 1], [np.full((n, H, W, 3), 0.4, np.float32) for n in (2, 1)])
+        r.train_step([2, 1], cams, 1, 0.0, 0.0, 0.0, 0.0)
+        got.append((r.read_buffer(0, 3 * H * W * 4), r.gradients()))
+    np.testing.assert_array_equal(got[0][0], got[1][0])
+    for k, v in got[0][1].items():
+        assert _rel(got[1][1][k], v) <= 1e-5, k
+
+
+def test_segments_through_the_autotuner():
+    s, cam = _scene(0.2), fibonacci_cameras(2, 3.0, 50.0, W, H)[1]
+    gt = np.full((1, H, W, 3), 0.4, np.float32)
+    r = _renderer(s)
+    r.set_targets(gt)
+    r.autotune([cam], reps=1)
+    r.train_step_batched([cam], 1, 0.0, 0.0, 0.0)
+    fresh = _renderer(s, tile_size=r.get_tuning()[0])
+    fresh.set_tuning(*r.get_tuning())
+    fresh.train_step(*cam, gt[0], 0.0, 0.0, 0.0, 1)
+    for k, v in fresh.gradients().items():
+        assert _rel(r.gradients()[k], v) <= 1e-5, k
