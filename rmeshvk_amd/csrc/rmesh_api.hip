@@ -371,28 +371,38 @@ SegmentSizes segment_sizes(uint64_t P) {
     return n;
 }
 
+void free_segments(rmesh_renderer* h) {
+    (void)hipFree(h->seg);
+    (void)hipFree(h->seg_dark);
+    (void)hipFree(h->seg_px);
+    (void)hipFree(h->seg_stop);
+    h->seg = h->seg_stop = nullptr;
+    h->seg_dark = nullptr;
+    h->seg_px = nullptr;
+}
+
+// The buffers of the lists for at least `need` pairs; what they held is gone when
+// they grow, and with it the graph and the last forward.  Without memory for the
+// segments' (seg_px null) the lists stay whole.
 rmesh_status ensure_capacity(rmesh_renderer* h, uint64_t need) {
-    if (need <= h->cap && h->keys_a && h->hist && h->seg_px) return RMESH_OK;
+    if (need <= h->cap && h->keys_a && h->hist && h->tile_order) return RMESH_OK;
     if (need > 0xFFFFFFF0ull) return fail(RMESH_ERR_CAPACITY, "tile-tet pair count exceeds 2^32");
     uint64_t c = std::max<uint64_t>(need + need / 4 + (1u << 16), 1u << 20);
     if (c > 0xFFFFFFF0ull) c = 0xFFFFFFF0ull;
     HIP_TRY(hipStreamSynchronize(h->stream));
+    drop_graph(h);
+    h->have_forward = h->have_interval = false;
     (void)hipFree(h->keys_a);
     (void)hipFree(h->keys_b);
     (void)hipFree(h->vals_a);
     (void)hipFree(h->vals_b);
     (void)hipFree(h->hist);
     (void)hipFree(h->tile_order);
-    (void)hipFree(h->seg);
-    (void)hipFree(h->seg_dark);
-    (void)hipFree(h->seg_px);
-    (void)hipFree(h->seg_stop);
+    free_segments(h);
     h->keys_a = h->keys_b = nullptr;
     h->vals_a = h->vals_b = nullptr;
     h->hist = nullptr;
-    h->tile_order = h->seg = h->seg_stop = nullptr;
-    h->seg_dark = nullptr;
-    h->seg_px = nullptr;
+    h->tile_order = nullptr;
     h->cap = 0;
     HIP_TRY(dalloc(&h->keys_a, c));
     HIP_TRY(dalloc(&h->keys_b, c));
@@ -401,11 +411,12 @@ rmesh_status ensure_capacity(rmesh_renderer* h, uint64_t need) {
     HIP_TRY(dalloc(&h->hist, std::max(radix_hist_words((uint32_t)c), radix_hist_words32((uint32_t)c))));
     const SegmentSizes ns = segment_sizes(c);
     HIP_TRY(dalloc(&h->tile_order, h->tile_cap + ns.items));
-    HIP_TRY(dalloc(&h->seg, h->tile_cap + ns.items));
-    HIP_TRY(dalloc(&h->seg_dark, ns.slots));
-    HIP_TRY(dalloc(&h->seg_px, ns.pixels));
+    if (dalloc(&h->seg, h->tile_cap + ns.items) != hipSuccess || dalloc(&h->seg_dark, ns.slots) != hipSuccess ||
+        dalloc(&h->seg_px, ns.pixels) != hipSuccess) {
+        (void)hipGetLastError();
+        free_segments(h);
+    }
     h->cap = (uint32_t)c;
-    drop_graph(h);
     return RMESH_OK;
 }
 
@@ -416,17 +427,23 @@ rmesh_status ensure_checkpoints(rmesh_renderer* h, uint32_t V) {
     const uint64_t need = checkpoint_slots(h->cap, h->n_gt) * h->TS * h->TS;
     if (need > h->ck_floats || !h->ck) {
         HIP_TRY(hipStreamSynchronize(h->stream));
+        drop_graph(h);
+        h->have_forward = false;
         (void)hipFree(h->ck);
         h->ck = nullptr;
         h->ck_floats = 0;
         const uint64_t c = need + need / 8;
         HIP_TRY(dalloc(&h->ck, c));
         h->ck_floats = c;
-        drop_graph(h);
     }
-    if (!h->seg_stop) {
-        HIP_TRY(dalloc(&h->seg_stop, segment_sizes(h->cap).pixels));
+    if (h->seg_px && !h->seg_stop) {
         drop_graph(h);
+        if (dalloc(&h->seg_stop, segment_sizes(h->cap).pixels) != hipSuccess) {
+            (void)hipGetLastError();
+            HIP_TRY(hipStreamSynchronize(h->stream));
+            h->have_forward = false;
+            free_segments(h);
+        }
     }
     if (!h->fin) HIP_TRY(dalloc(&h->fin, (size_t)h->pix_cap));
     return RMESH_OK;
@@ -521,6 +538,7 @@ SplitPlan split_plan(const rmesh_renderer* h) {
 // split: long lists as several work items (the plain forward and the adjoint);
 // the aux, error and interval kernels take whole tiles.
 void launch_ranges_stage(rmesh_renderer* h, bool split, hipStream_t s) {
+    split = split && h->seg_px;
     const SplitPlan sp = split ? split_plan(h) : SplitPlan();
     h->left.order_split = split;
     h->left.have_segs = false;
