@@ -1769,6 +1769,7 @@ static void fwd_launch(const FwdArgs& a, hipStream_t s) {
 // for 1.50 with B 48, CAP 768).
 template <int TS>
 static bool fwd_variant(const FwdArgs& a, int v, hipStream_t s) {
+    if (fwd_is_default(TS, v)) v = 0;
     switch (v) {
         case 0:
             if constexpr (TS == 12) fwd_launch<FwdCfg<TS, 32, 1152, 3>>(a, s);
@@ -1784,8 +1785,7 @@ static bool fwd_variant(const FwdArgs& a, int v, hipStream_t s) {
         case 4: fwd_launch<FwdCfg<TS, 64, 768, 3, 5>>(a, s); return true;
         case 5: fwd_launch<FwdCfg<TS, 56, 896, 3>>(a, s); return true;
         case 6:
-            if constexpr (TS == 16) fwd_launch<FwdCfg<TS, 64, 1024, 3, 4>>(a, s);
-            else fwd_launch<FwdCfg<TS, 56, 768, 3, 5>>(a, s);
+            if constexpr (TS != 16) fwd_launch<FwdCfg<TS, 56, 768, 3, 5>>(a, s);
             return true;
         case 7: fwd_launch<FwdCfg<TS, 64, 896, 3>>(a, s); return true;
         default: return false;
@@ -1843,9 +1843,9 @@ template <int TS, int B, int N>
 using BwdGeo = BwdCfg<TS, (TS == 8 ? B / 2 : B), (TS == 8 ? N + 1 : N) * ((TS * TS + 63) / 64 * 64), 3, 4>;
 template <int TS>
 static bool bwd_variant(const BwdArgs& a, int v, hipStream_t s) {
+    if (bwd_is_default(TS, v)) v = 0;
     switch (v) {
         case 0:
-        case 10:
             if constexpr (TS == 12) bwd_launch<BwdGeo<TS, 32, 5>>(a, s);
             else bwd_launch<BwdGeo<TS, 48, 3>>(a, s);
             return true;

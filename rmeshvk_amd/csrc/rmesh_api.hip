@@ -1553,6 +1553,7 @@ static rmesh_status autotune_layout(rmesh_renderer* h, const uint32_t* per_user,
         h->sort_db = bdb;
         if ((result = stage_binning_back(h, V, true)) != RMESH_OK) break;  // lists of the chosen width
         for (int f = 0; f < fwd_variants(ts) && result == RMESH_OK; ++f) {
+            if (fwd_is_default(ts, f)) continue;
             h->fwd_var = f;
             float t = 0.0f;
             result = timed([&]() { return stage_forward(h, V, false, loss_type == 0); }, t);
@@ -1565,6 +1566,7 @@ static rmesh_status autotune_layout(rmesh_renderer* h, const uint32_t* per_user,
         h->fwd_var = bf;
         if ((result = stage_forward(h, V, false, loss_type == 0)) != RMESH_OK) break;  // image of the chosen variant
         for (int b = 0; b < bwd_variants(ts) && result == RMESH_OK; ++b) {
+            if (bwd_is_default(ts, b)) continue;
             h->bwd_var = b;
             float t = 0.0f;
             result = timed([&]() { return stage_backward(h, V, nullptr, h->gt, loss_type); }, t);

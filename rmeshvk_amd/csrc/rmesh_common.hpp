@@ -150,14 +150,6 @@ __device__ __forceinline__ V3 med_clip3(V3 v, float lo, float hi) {
 }
 __device__ __forceinline__ float relu(float v) { return __builtin_amdgcn_fmed3f(v, 0.0f, __builtin_huge_valf()); }
 __device__ __forceinline__ float fast_safe_exp(float v) { return fast_exp(clampf(v, -88.0f, kLogMaxVal)); }
-__device__ __forceinline__ float fast_phi(float x, float ex) {  // ex = exp(-x)
-    if (fabsf(x) < 0.02f) return 1.0f + x * (-0.5f + x * ((float)(1.0 / 6.0) + x * ((float)(-1.0 / 24.0))));
-    return fast_safe_div(1.0f - ex, x);
-}
-__device__ __forceinline__ float fast_dphi(float x, float ex) {
-    if (fabsf(x) < 0.02f) return -0.5f + x * ((float)(1.0 / 3.0) + x * ((float)(-1.0 / 8.0) + x * ((float)(1.0 / 30.0))));
-    return fast_safe_div(ex * (x + 1.0f) - 1.0f, x * x);
-}
 
 // WGSL-style saturating conversions (explicit: no reliance on UB rules).
 __device__ __forceinline__ uint32_t sat_u32(float x) {

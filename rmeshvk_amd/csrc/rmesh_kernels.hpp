@@ -184,6 +184,9 @@ constexpr int kBwdVariants = 11;
 // tile 32 compiles fewer geometries (a batch must hold one tet's 1024 pixels)
 inline int fwd_variants(uint32_t tile_size) { return tile_size == 32 ? 2 : kFwdVariants; }
 inline int bwd_variants(uint32_t tile_size) { return tile_size == 32 ? 2 : kBwdVariants; }
+// Numbers that programs hold and whose geometry has become variant 0's.
+inline bool fwd_is_default(uint32_t tile_size, int variant) { return variant == 6 && tile_size == 16; }
+inline bool bwd_is_default(uint32_t, int variant) { return variant == 10; }
 bool launch_forward(const FwdArgs& a, uint32_t tile_size, int variant, hipStream_t s);
 
 // Per-tet error statistics (forward_error) over one view's tile lists.

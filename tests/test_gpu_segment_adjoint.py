@@ -207,3 +207,19 @@ def test_segments_through_the_autotuner():
     fresh.train_step(*cam, gt[0], 0.0, 0.0, 0.0, 1)
     for k, v in fresh.gradients().items():
         assert _rel(r.gradients()[k], v) <= 1e-5, k
+
+
+def test_the_autotuner_times_a_geometry_once():
+    """Forward 6 at tile 16 and adjoint 10 are variant 0's geometries: accepted, and
+    never what the autotuner keeps (with both timed it kept either by chance)."""
+    s, cam = _scene(0.2), fibonacci_cameras(2, 3.0, 50.0, W, H)[1]
+    r = _renderer(s, tile_size=16)
+    r.set_targets(np.full((1, H, W, 3), 0.4, np.float32))
+    imgs = []
+    for f, b in ((0, 0), (6, 10)):
+        r.set_tuning(16, f, b)
+        imgs.append(r.forward_tiled(*cam))
+    np.testing.assert_array_equal(*imgs)
+    for _ in range(4):
+        ts, f, b = r.autotune([cam], reps=1)["tuning"]
+        assert b != 10 and (ts, f) != (16, 6)
