@@ -913,7 +913,7 @@ void launch_pairs_depth_ordered(const float4* rec, const SceneRange* scenes, uin
 // next two bits (four buckets per octave), descending; among segments of a bucket
 // those nearer the camera first (a segment behind others that already block the
 // tile's light need not run).  The order inside a bucket and the slot bases are
-// whatever the LDS atomics give (no result depends on either).
+// whatever the LDS atomics give; no image depends on either (k_forward).
 constexpr int kPairBuckets = 33 * 4;
 constexpr int kSegBuckets = 16;   // per pair bucket that segments fall into: segments 0 .. 14, 15 and later
 constexpr int kOrderBuckets = kPairBuckets + 5 * kSegBuckets;  // (unit / 2 .. unit pairs: at most five)

@@ -552,9 +552,11 @@ __device__ __forceinline__ float fdot3(V3 a, V3 b) { return fmaf(a.x, b.x, fmaf(
 // reciprocals overlap, and a wave never splits over the faces.  The reference
 // skips a face whose |n . d| is below 1e-20 and calls the tet missed if its
 // plane faces the ray (num > 0).  Sorting the faces by the sign bit of n . d
-// gives the same without the test: an (almost) parallel face divides to
-// +-inf, entry +inf or exit -inf where num > 0 (no slab left), a value that
-// max / min ignore otherwise (0 * inf = NaN for num = 0 included).
+// gives the same without the test: a parallel face divides to +-inf, one below
+// 1e-20 to a number beyond any scene; as entry or exit that leaves no slab where
+// num > 0 and is ignored by max / min otherwise (0 * inf = NaN for num = 0
+// included).  Faces whose planes are themselves of the order of 1e-20 (edges
+// below 1e-9) are divided all the same.
 // min_face / max_face: the first face in table order that attains the bound
 // (0 where no face does, as the reference's adjoint assumes).
 // Written with per-face branches, a face cost 14 scalar and branch
@@ -691,6 +693,10 @@ __device__ __forceinline__ void drain_stores() { asm volatile("s_waitcnt vmcnt(0
 // this shows to saturate (log T < -13.8, from where the serial pass composites
 // nothing) in a later segment than the first is composited again from that
 // segment's start, so that it stops behind the same pair as in a serial pass.
+// Which segments are skipped behind dark ones depends on the order in which the
+// workgroups run.  The image does not: what is skipped lies behind the pixels'
+// stops.  The undo of a saturated tile does, in its rounding: a skipped segment's
+// sum is not known, and the adjoint takes the list from there on in one.
 //
 // CK: also store the transmittance checkpoints of the checkpointed adjoint:
 // a pixel still compositing writes its log T before every tile-list position
