@@ -926,15 +926,21 @@ __device__ __forceinline__ uint32_t pair_bucket(uint32_t c) {
     const uint32_t len = 32u - (uint32_t)__clz((int)c);  // >= 3
     return len * 4u + ((c >> (len - 3u)) & 3u);           // 3 leading bits: 1xx
 }
-// Bucket of segment seg of a tile whose segments hold c pairs, or (seg -1) of a
-// whole tile of c pairs.  Whole tiles come first in their pair bucket.
+// Bucket of segment seg of a tile whose segments hold c pairs, or (seg -1) of an
+// item that takes a list of c pairs whole.  Those come first in their pair bucket.
 __device__ __forceinline__ uint32_t item_bucket(uint32_t c, int seg, const SplitPlan& sp) {
     const uint32_t b = pair_bucket(c);
     if (!sp.seg) return b;
     const uint32_t lo = pair_bucket(sp.unit / 2u), hi = pair_bucket(sp.unit);
     if (b < lo) return b;
+    if (b > hi) return lo + (hi - lo) * (uint32_t)(kSegBuckets + 1) + (uint32_t)kSegBuckets + (b - hi);  // (whole)
     const uint32_t in = seg < 0 ? (uint32_t)kSegBuckets : (uint32_t)kSegBuckets - 1u - min((uint32_t)seg, (uint32_t)kSegBuckets - 1u);
-    return lo + (min(b, hi) - lo) * (uint32_t)(kSegBuckets + 1) + in;
+    return lo + (b - lo) * (uint32_t)(kSegBuckets + 1) + in;
+}
+// Segment g of a list of `pairs`.  Where the first one's workgroup composites the
+// whole list (one_pass) its item is as heavy as that.
+__device__ __forceinline__ uint32_t segment_bucket(uint32_t pairs, uint32_t unit, uint32_t g, const SplitPlan& sp) {
+    return sp.one_pass && g == 0u ? item_bucket(pairs, -1, sp) : item_bucket(split_length(pairs, unit), (int)g, sp);
 }
 // (without a plan not read)
 __device__ __forceinline__ uint32_t call_unit(uint32_t n_tiles, const uint32_t* __restrict__ n_pairs, uint32_t cap,
@@ -946,7 +952,7 @@ __device__ __forceinline__ void count_items(uint32_t* cnt, uint32_t pairs, uint3
     const uint32_t n = sp.seg ? split_segments(pairs, unit) : 1u;
     if (n == 1u) atomicAdd(&cnt[item_bucket(pairs, -1, sp)], 1u);
     else
-        for (uint32_t g = 0; g < n; ++g) atomicAdd(&cnt[item_bucket(split_length(pairs, unit), (int)g, sp)], 1u);
+        for (uint32_t g = 0; g < n; ++g) atomicAdd(&cnt[segment_bucket(pairs, unit, g, sp)], 1u);
 }
 // off: the buckets' running item offsets; n_slots: the running slot count.
 __device__ __forceinline__ void place_items(uint32_t* off, uint32_t* n_slots, uint32_t t, uint32_t pairs, uint32_t unit,
@@ -963,7 +969,7 @@ __device__ __forceinline__ void place_items(uint32_t* off, uint32_t* n_slots, ui
     sp.arrived[t] = 0u;
     sp.merged[t] = 0u;
     for (uint32_t g = 0; g < n; ++g) {
-        const uint32_t i = atomicAdd(&off[item_bucket(split_length(pairs, unit), (int)g, sp)], 1u);
+        const uint32_t i = atomicAdd(&off[segment_bucket(pairs, unit, g, sp)], 1u);
         order[i] = t;
         sp.seg[i] = g;
         sp.dark[slot + g] = 0.0f;

@@ -1756,7 +1756,7 @@ static void fwd_launch(const FwdArgs& a, hipStream_t s) {
         hipLaunchKernelGGL(kernel, grid, dim3(C::NT), 0, s, a.rec, a.colors, a.sorted_vals, a.ranges, a.views,
                            a.tile_view, a.tile_order, a.split, a.rgba, aux, ck, fin);
     };
-    const bool one = a.one_pass && a.split.seg;
+    const bool one = a.split.one_pass && a.split.seg;
     if (a.aux)  // the aux outputs serve the forward-only API: no checkpoints with them
         launch(k_forward<C, true, false, false>, a.aux, nullptr, nullptr);
     else if (a.ck)

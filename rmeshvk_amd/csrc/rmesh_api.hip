@@ -519,9 +519,11 @@ void launch_sort_stage(rmesh_renderer* h, hipStream_t s) {
         h->left.sorted_in_b = launch_radix_sort(h->keys_a, h->vals_a, h->keys_b, h->vals_b, h->n_pairs, h->cap,
                                                 h->sorting_bits(0), h->hist, s, h->sort_db);
 }
-// The segment plan of the current tile size, for the order kernel and the forward.
-SplitPlan split_plan(const rmesh_renderer* h) {
+// The segment plan of the current tile size, for the order kernel and the
+// compositing kernels.  one_pass: in a step with the L1 loss (loss type 0).
+SplitPlan split_plan(const rmesh_renderer* h, bool one_pass = false) {
     SplitPlan p;
+    p.one_pass = one_pass;
     p.unit = split_unit(h->TS);
     p.unit_few = split_unit_few(h->TS);
     p.seg = h->seg;
@@ -537,9 +539,9 @@ SplitPlan split_plan(const rmesh_renderer* h) {
 }
 // split: long lists as several work items (the plain forward and the adjoint);
 // the aux, error and interval kernels take whole tiles.
-void launch_ranges_stage(rmesh_renderer* h, bool split, hipStream_t s) {
+void launch_ranges_stage(rmesh_renderer* h, bool split, bool one_pass, hipStream_t s) {
     split = split && h->seg_px;
-    const SplitPlan sp = split ? split_plan(h) : SplitPlan();
+    const SplitPlan sp = split ? split_plan(h, one_pass) : SplitPlan();
     h->left.order_split = split;
     h->left.have_segs = false;
     launch_fill_u32(h->ranges, 0u, 2ull * h->n_gt, s);
@@ -552,17 +554,17 @@ void launch_ranges_stage(rmesh_renderer* h, bool split, hipStream_t s) {
         launch_tile_order(h->ranges, h->n_gt, h->n_pairs, h->cap, h->tile_order, sp, s);
 }
 
-rmesh_status stage_binning_back(rmesh_renderer* h, uint32_t V, bool split) {
+rmesh_status stage_binning_back(rmesh_renderer* h, uint32_t V, bool split, bool one_pass = false) {
     hipStream_t s = h->stream;
     launch_pair_gen(h, s);
     launch_sort_stage(h, s);
-    launch_ranges_stage(h, split, s);
+    launch_ranges_stage(h, split, one_pass, s);
     return RMESH_OK;
 }
 
 const uint32_t* sorted_vals(const rmesh_renderer* h) { return h->left.sorted_in_b ? h->vals_b : h->vals_a; }
 
-// one_pass: FwdArgs::one_pass, for the steps with the L1 loss (loss type 0).
+// one_pass: as split_plan.
 rmesh_status stage_forward(rmesh_renderer* h, uint32_t V, bool want_aux, bool one_pass) {
     FwdArgs a;
     a.rec = h->rec;
@@ -573,8 +575,7 @@ rmesh_status stage_forward(rmesh_renderer* h, uint32_t V, bool want_aux, bool on
     a.tile_view = h->d_tile_view;
     a.num_gtiles = h->n_gt;
     a.tile_order = h->tile_order;
-    if (h->left.order_split) a.split = split_plan(h);
-    a.one_pass = one_pass;
+    if (h->left.order_split) a.split = split_plan(h, one_pass);
     a.rgba = h->rgba;
     a.aux = want_aux ? h->aux : nullptr;
     const bool ck = h->adj_ck && !want_aux;  // the aux forward keeps no checkpoints
@@ -739,7 +740,7 @@ rmesh_status record_stage(rmesh_renderer* h, int stage, uint32_t V, const float*
             launch_sort_stage(h, s);
             return RMESH_OK;
         case 3:
-            launch_ranges_stage(h, true, s);
+            launch_ranges_stage(h, true, loss_type == 0, s);
             return RMESH_OK;
         case 4: return stage_forward(h, V, false, loss_type == 0);
         case 5: return stage_backward(h, V, nullptr, gt, loss_type);
@@ -1541,7 +1542,7 @@ static rmesh_status autotune_layout(rmesh_renderer* h, const uint32_t* per_user,
             result = timed([&]() {
                 rmesh_status s2 = stage_binning_front(h, V, true);
                 if (s2 != RMESH_OK) return s2;
-                return stage_binning_back(h, V, true);
+                return stage_binning_back(h, V, true, loss_type == 0);
             }, t);
             if (result != RMESH_OK) break;
             if (t < t_bin) {
@@ -1551,7 +1552,7 @@ static rmesh_status autotune_layout(rmesh_renderer* h, const uint32_t* per_user,
         }
         if (result != RMESH_OK) break;
         h->sort_db = bdb;
-        if ((result = stage_binning_back(h, V, true)) != RMESH_OK) break;  // lists of the chosen width
+        if ((result = stage_binning_back(h, V, true, loss_type == 0)) != RMESH_OK) break;  // lists of the chosen width
         for (int f = 0; f < fwd_variants(ts) && result == RMESH_OK; ++f) {
             if (fwd_is_default(ts, f)) continue;
             h->fwd_var = f;

@@ -67,6 +67,7 @@ inline uint64_t split_slots(uint64_t P, uint32_t tile_size) {
 
 struct SplitPlan {
     uint32_t unit = 0, unit_few = 0;
+    bool one_pass = false;        // the forward composites each list by one workgroup (the steps with the L1 loss)
     uint32_t* seg = nullptr;      // [item] segment of the item's tile; null: one item per tile, no segments
     uint32_t* n_items = nullptr;  // then the call's unit (split_unit_of)
     __device__ uint32_t unit_now() const { return n_items[1]; }
@@ -168,7 +169,6 @@ struct FwdArgs {
     uint32_t num_gtiles;
     const uint32_t* tile_order;  // nullable: work item -> global tile (identity when null)
     SplitPlan split;             // the plan tile_order was made with
-    bool one_pass;               // split lists composited by one workgroup each (the steps with the L1 loss)
     float* rgba;
     float* aux;  // nullable: [V][H][W][8]
     // nullable: transmittance checkpoints for the checkpointed adjoint.
