@@ -15,7 +15,7 @@ struct ViewParams;
 // The unit, 6 pairs per pixel: a tile's workgroup is a serial chain over its
 // list, and the chip holds some 1300 of them, so a list far above (all pairs) /
 // 1300 runs on after the rest of the grid is done (uneven scenes, longest list
-// 33,800 pairs at tile 16: forward 2.1 ms, adjoint 3.6 unsplit, 0.37 and 0.84
+// 33,800 pairs at tile 16: forward 2.1 ms, adjoint 3.6 unsplit, 0.41 and 0.86
 // split; 4 clustered views, longest 16,300: 1.5 and 2.9, 0.34 and 0.79).  A segment costs a
 // pixel record (16 bytes a pixel written, read by the tile's last workgroup and
 // by the adjoint) and the start of a workgroup: where no list is long for the
@@ -61,6 +61,7 @@ inline uint64_t split_extra_items(uint64_t P, uint32_t tile_size, uint32_t n_til
 }
 inline uint64_t split_slots(uint64_t P, uint32_t tile_size) {
     const uint64_t n = 2u * (P / split_unit(tile_size)) + 2u;
+    if (split_unit_few(tile_size) == split_unit(tile_size)) return n;
     const uint64_t few = split_few_pairs(P, tile_size) / split_unit_few(tile_size) + kFewItems;
     return n > few ? n : few;
 }
