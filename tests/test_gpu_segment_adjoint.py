@@ -223,3 +223,27 @@ def test_the_autotuner_times_a_geometry_once():
     for _ in range(4):
         ts, f, b = r.autotune([cam], reps=1)["tuning"]
         assert b != 10 and (ts, f) != (16, 6)
+
+
+@pytest.mark.parametrize("mode", ["undo", "checkpoint"])
+def test_a_view_alone_and_in_a_batch(mode):
+    """Alone (484 tiles) a view's lists are split at one pair per pixel, among eight
+    (3,872) at six: the same image to the rounding of the joined sums (1e-6 a
+    channel of order 1, bound 1e-5), and the gradients to what that moves them."""
+    s = _scene()
+    cams = fibonacci_cameras(8, 3.0, 50.0, 256, 256)
+    gts = np.random.default_rng(5).random((8, 256, 256, 3)).astype(np.float32)
+    rb, r1 = _renderer(s, 256, 256, max_views=8), _renderer(s, 256, 256)
+    for r in (rb, r1):
+        r.set_adjoint_mode(mode)
+    rb.set_targets(gts)
+    rb.train_step_batched(cams, 1, 0.0, 0.0, 0.0)
+    images = rb.read_buffer(0, 8 * 256 * 256 * 4).reshape(8, 256, 256, 4)
+    total = {}
+    for i, (c, gt) in enumerate(zip(cams, gts)):
+        r1.train_step(*c, gt, 0.0, 0.0, 0.0, 1)
+        assert np.abs(r1.read_buffer(0, 256 * 256 * 4).reshape(256, 256, 4) - images[i]).max() <= 1e-5
+        for k, v in r1.gradients().items():
+            total[k] = total.get(k, 0.0) + np.asarray(v, np.float64)
+    for k, v in rb.gradients().items():
+        assert _rel(v, total[k]) <= 2e-5, (k, _rel(v, total[k]))
