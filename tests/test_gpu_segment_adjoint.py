@@ -7,7 +7,7 @@
   5e-4 of those from an exact image;
 - an L1 step has the image of one pass over each list, and the adjoint of it;
 - both adjoints with a near offset, in calls of many tiles, under the scene-major
-  order and through the autotuner;
+  order and through the autotuner; a view alone and in a batch;
 - segment buffers sized by what calls with short segments can need.
 """
 
